@@ -73,9 +73,6 @@ void free_sim(gsim_sim *s) {
     for (hipEvent_t e : s->event_pool) (void)hipEventDestroy(e);
     for (hipEvent_t e : s->order_ev)
         if (e) (void)hipEventDestroy(e);
-    if (s->ev_fork) (void)hipEventDestroy(s->ev_fork);
-    if (s->ev_join) (void)hipEventDestroy(s->ev_join);
-    if (s->side) (void)hipStreamDestroy(s->side);
     if (s->stream) (void)hipStreamDestroy(s->stream);
     delete s;
 }
@@ -371,12 +368,6 @@ gsim_status gsim_create(const gsim_params *params, const float *pos_xy, const fl
         e = gsim::bh_alloc(&s->bh, na, gsim::kTreeDepth);
         if (e != hipSuccess)
             return bail(fail(GSIM_ERROR_OUT_OF_MEMORY, "Barnes-Hut buffers: %s", hipGetErrorString(e)));
-        // the heavy list's walks run on a second stream (default priority),
-        // forked from and joined back to s->stream by events
-        e = hipStreamCreateWithFlags(&s->side, hipStreamNonBlocking);
-        if (e == hipSuccess) e = hipEventCreateWithFlags(&s->ev_fork, hipEventDisableTiming);
-        if (e == hipSuccess) e = hipEventCreateWithFlags(&s->ev_join, hipEventDisableTiming);
-        if (e != hipSuccess) return bail(hip_fail(e, "side stream"));
     }
     *out = s;
     return GSIM_OK;
@@ -466,8 +457,7 @@ gsim_status gsim_set_ds_shape(gsim_sim *s, uint32_t R, uint32_t S) {
 gsim_status gsim_set_tuning(gsim_sim *s, int32_t knob, uint32_t value) {
     gsim::clear_error();
     if (!s) return fail(GSIM_ERROR_INVALID_ARGUMENT, "gsim_set_tuning: NULL handle");
-    // A W = 32 handle has one traversal launch (bh_traverse32_kernel): the
-    // W = 64 launch-shape knobs would be silently ignored, so they are refused.
+    // the W = 64 launch-shape knobs are refused on a W = 32 handle
     if (s->params.algorithm == GSIM_BARNES_HUT && s->W == 32 &&
         (knob == GSIM_TUNE_BH_WAVES_PER_SIMD || knob == GSIM_TUNE_BH_TRAVERSAL ||
          knob == GSIM_TUNE_BH_SPLIT || knob == GSIM_TUNE_BH_SEGMENTS))
@@ -481,12 +471,10 @@ gsim_status gsim_set_tuning(gsim_sim *s, int32_t knob, uint32_t value) {
         case GSIM_TUNE_BH_WAVES_PER_SIMD:
             if (value < 1 || value > 8)
                 return fail(GSIM_ERROR_INVALID_ARGUMENT, "waves per SIMD must be in [1, 8]");
-            s->trav_waves_per_simd = value;
             return GSIM_OK;
         case GSIM_TUNE_BH_TRAVERSAL:
             if (value > 3 && value != 6)
                 return fail(GSIM_ERROR_INVALID_ARGUMENT, "traversal mode must be 0..3 or 6");
-            s->trav_mode = value;
             return GSIM_OK;
         case GSIM_TUNE_BH_ADAPTIVE_BOX:
             if (s->params.algorithm != GSIM_BARNES_HUT)
@@ -517,7 +505,6 @@ gsim_status gsim_set_tuning(gsim_sim *s, int32_t knob, uint32_t value) {
         }
         case GSIM_TUNE_BH_SPLIT:
             if (value > 1000) return fail(GSIM_ERROR_INVALID_ARGUMENT, "split threshold must be in [0, 1000]");
-            s->trav_split = value;
             return GSIM_OK;
         case GSIM_TUNE_BH_ORDER:
             if (value > 2) return fail(GSIM_ERROR_INVALID_ARGUMENT, "group order must be 0, 1 or 2");
@@ -535,7 +522,6 @@ gsim_status gsim_set_tuning(gsim_sim *s, int32_t knob, uint32_t value) {
         case GSIM_TUNE_BH_SEGMENTS:
             if (value < 1 || value > 65536)
                 return fail(GSIM_ERROR_INVALID_ARGUMENT, "segments must be in [1, 65536]");
-            s->trav_segments = value;
             return GSIM_OK;
         case GSIM_TUNE_DS_SYMMETRIC:
         case GSIM_TUNE_DS_SYM_COLS: {
@@ -677,7 +663,18 @@ gsim_status gsim_debug_dump(gsim_sim *s, int32_t what, void *buf, size_t bytes, 
         case GSIM_DUMP_COUNTS:
             *written = sizeof(uint32_t) * nodes;
             if (bytes < *written || (!buf && nodes)) return fail(GSIM_ERROR_CAPACITY, "buffer too small");
-            if (nodes) GSIM_HIP(hipMemcpy(buf, s->bh.ncount, *written, hipMemcpyDeviceToHost));
+            if (nodes) {  // a particle's subtree is itself, a cell's its children's
+                std::vector<float4> rec(nodes);
+                std::vector<uint4> ch(nodes);
+                GSIM_HIP(hipMemcpy(rec.data(), s->bh.node4, sizeof(float4) * nodes, hipMemcpyDeviceToHost));
+                GSIM_HIP(hipMemcpy(ch.data(), s->bh.child, sizeof(uint4) * nodes, hipMemcpyDeviceToHost));
+                uint32_t *u = (uint32_t *)buf;
+                for (size_t k = 0; k < nodes; ++k)
+                    u[k] = rec[k].w <= 0.0f ? 1u
+                           : ch[k].w == gsim::kLeafMark
+                               ? ch[k].x + 1u
+                               : ch[k].x + ch[k].y + ch[k].z + ch[k].w + 1u;
+            }
             return GSIM_OK;
         case GSIM_DUMP_RADII:
         case GSIM_DUMP_NODE_POS:
@@ -690,7 +687,7 @@ gsim_status gsim_debug_dump(gsim_sim *s, int32_t what, void *buf, size_t bytes, 
             GSIM_HIP(hipMemcpy(tmp.data(), s->bh.node4, sizeof(float4) * nodes, hipMemcpyDeviceToHost));
             float *f = (float *)buf;
             for (size_t k = 0; k < nodes; ++k) {
-                if (what == GSIM_DUMP_RADII) f[k] = tmp[k].w > 0.0f ? tmp[k].w : 0.0f;  // run length -> 0
+                if (what == GSIM_DUMP_RADII) f[k] = tmp[k].w;
                 else if (what == GSIM_DUMP_NODE_MASS) f[k] = tmp[k].z;
                 else { f[2 * k] = tmp[k].x; f[2 * k + 1] = tmp[k].y; }
             }

@@ -47,9 +47,9 @@ void free_batch(gsim_batch *b) {
     void *ptrs[] = {d.pos[0], d.pos[1], d.vel[0], d.vel[1], d.mass, d.partial, d.desc, d.remaining,
                     d.bh_sys, d.bh_prefix, d.ds_sys, d.ds_prefix, d.items, d.counts, d.stats,
                     d.keys[0], d.keys[1], d.idx[0], d.idx[1], d.status, d.digit_total,
-                    d.block_cells, d.block_leaves, d.sdep, d.cpos, d.sorted_src, d.prod,
+                    d.block_cells, d.block_leaves, d.sdep, d.cpos, d.sorted_src,
                     d.leaf_sum, d.leaf_first, d.leaf_key, d.tile_range, d.live_tiles, d.top, d.node4,
-                    d.ncount, d.breaker, d.wave_acc, d.ichunk};
+                    d.child, d.wave_acc, d.ichunk};
     for (void *p : ptrs) (void)hipFree(p);
     if (b->stream) (void)hipStreamDestroy(b->stream);
     delete b;
@@ -263,7 +263,6 @@ gsim_status gsim_batch_create(int32_t device, size_t capacity_particles, uint32_
     GSIM_BALLOC(d.sdep, cap);
     GSIM_BALLOC(d.cpos, cap);
     GSIM_BALLOC(d.sorted_src, cap);
-    GSIM_BALLOC(d.prod, cap);
     GSIM_BALLOC(d.leaf_sum, cap);
     GSIM_BALLOC(d.leaf_first, cap + 1);
     GSIM_BALLOC(d.leaf_key, cap);
@@ -271,15 +270,14 @@ gsim_status gsim_batch_create(int32_t device, size_t capacity_particles, uint32_
     GSIM_BALLOC(d.live_tiles, (size_t)gsim::kTiles * max_systems);
     GSIM_BALLOC(d.top, (size_t)gsim::kTiles * max_systems);
     GSIM_BALLOC(d.node4, b->node_capacity);
-    GSIM_BALLOC(d.ncount, b->node_capacity);
-    GSIM_BALLOC(d.breaker, b->node_capacity);
+    GSIM_BALLOC(d.child, b->node_capacity);
     GSIM_BALLOC(d.wave_acc, 2 * gsim::kMaxForceWaves);
     GSIM_BALLOC(d.ichunk, b->item_capacity);
 #undef GSIM_BALLOC
     if (e == hipSuccess) e = hipMemset(d.counts, 0, sizeof(gsim::BatchCounts));
     if (e == hipSuccess) e = hipMemset(d.wave_acc, 0, sizeof(unsigned long long) * 2 * gsim::kMaxForceWaves);
     if (e == hipSuccess) e = hipMemset(d.ichunk, 0, sizeof(uint32_t) * b->item_capacity);
-    if (e == hipSuccess) e = hipMemset(d.ncount, 0, sizeof(uint32_t) * b->node_capacity);
+    if (e == hipSuccess) e = hipMemset(d.child, 0, sizeof(uint4) * b->node_capacity);
     if (e == hipSuccess) e = hipMemset(d.node4, 0, sizeof(float4) * b->node_capacity);
     if (e != hipSuccess) {
         gsim_status st = fail(GSIM_ERROR_OUT_OF_MEMORY, "batch allocation failed: %s", hipGetErrorString(e));
@@ -491,8 +489,8 @@ gsim_status gsim_batch_query(const gsim_batch *b, gsim_batch_info *out) {
 }
 
 size_t gsim_batch_bytes_per_particle(void) {
-    // state 36 B, Barnes-Hut scratch 67 B, 3 node slots x 28 B, partials 32 B
-    return 36 + 67 + 3 * 28 + 32;
+    // state 36 B, Barnes-Hut scratch 55 B, 3 node slots x 32 B, partials 32 B
+    return 36 + 55 + 3 * 32 + 32;
 }
 
 gsim_status gsim_batch_set_waves(gsim_batch *b, uint32_t waves_per_simd) {
@@ -621,7 +619,6 @@ gsim_status gsim_batch_autotune(gsim_batch *b, uint32_t steps_per_trial, uint32_
     const Knob knobs[] = {
         {&gsim_batch_tuning::waves_per_simd, {2, 4, 6, 8}},
         {&gsim_batch_tuning::sort_tile, {2048, 3072, 4096}},
-        {&gsim_batch_tuning::run_queue, {16, 32, 64}},
         {&gsim_batch_tuning::prio_step, {0, 16, 32, 64}},
         {&gsim_batch_tuning::prio_carry, {0, 8, 16, 32}},
     };

@@ -81,7 +81,7 @@ struct BatchTune {
     // round of waves)
     uint32_t waves_per_simd = 6;
     uint32_t sort_rounds = kBatchSortRoundsDefault;
-    uint32_t run_queue = 64;   // <= kRunQueue
+    uint32_t run_queue = 64;   // <= kRunQueue (kept for the interface: the walk has no run queue)
     uint32_t prio_step = 32;   // summed chunks per priority level
     uint32_t prio_carry = 16;  // last step's chunks / this = the starting level
 };
@@ -115,14 +115,14 @@ struct BatchDevice {
     uint32_t *block_cells = nullptr, *block_leaves = nullptr;
     int8_t *sdep = nullptr;
     uint32_t *cpos = nullptr, *sorted_src = nullptr;
-    float4 *prod = nullptr, *leaf_sum = nullptr;
+    float4 *leaf_sum = nullptr;
     uint32_t *leaf_first = nullptr, *leaf_key = nullptr;
     uint32_t *tile_range = nullptr;
     uint32_t *live_tiles = nullptr;  // [kLiveLists][live_per_list] tiles with leaves, any order
     TileCell *top = nullptr;
     // nodes of all trees
     float4 *node4 = nullptr;
-    uint32_t *ncount = nullptr, *breaker = nullptr;
+    uint4 *child = nullptr;           // a cell's children (kLeafMark)
     // each force wave's Barnes-Hut acceptances, then its node visits, in the
     // last step, summed into counts->accepts / visits by the step's last
     // kernel (a same-address atomic per wave costs more than the sum)

@@ -228,10 +228,10 @@ __global__ __launch_bounds__(256) void bb_emit_kernel(
     const float2 *__restrict__ pos, const float *__restrict__ mass,
     BatchCounts *__restrict__ counts, const uint32_t *__restrict__ bh_prefix,
     const uint32_t *__restrict__ block_cells, const uint32_t *__restrict__ block_leaves,
-    int8_t *__restrict__ sdep, uint32_t *__restrict__ cpos, float4 *__restrict__ prod,
+    int8_t *__restrict__ sdep, uint32_t *__restrict__ cpos,
     uint32_t *__restrict__ leaf_first, uint32_t *__restrict__ leaf_key,
-    float4 *__restrict__ node4, uint32_t *__restrict__ ncount, uint32_t *__restrict__ sorted_src,
-    uint32_t *__restrict__ breaker, RankStats *__restrict__ stats) {
+    float4 *__restrict__ node4, uint32_t *__restrict__ sorted_src,
+    RankStats *__restrict__ stats) {
     __shared__ uint32_t wa[4], wb[4];
     const uint32_t n = counts->n_bh_particles;
     const uint32_t nblocks = (n + 255) / 256;
@@ -269,16 +269,13 @@ __global__ __launch_bounds__(256) void bb_emit_kernel(
         }
         const uint32_t slot = k + C + q.ns;
         node4[slot] = make_float4(p.x, p.y, m, 0.0f);
-        ncount[slot] = 1u;
         sorted_src[k] = i;
         sdep[k] = (int8_t)q.sk;
         cpos[k] = C;
-        prod[k] = make_float4(p.x * m, p.y * m, m, 0.0f);
         if (q.lf) {
             leaf_first[L] = k;
             leaf_key[L] = q.key;
         }
-        for (uint32_t j = 0; j < q.ns; ++j) breaker[C + j] = k;
         if (q.sk < 0) stats[q.rank].root = k + C;
         if (q.sk1 < 0) {
             stats[q.rank].end_slot = k + 1 + C + q.ns;
@@ -287,7 +284,7 @@ __global__ __launch_bounds__(256) void bb_emit_kernel(
     }
 }
 
-// ---- leaf sums and particle runs ------------------------------------------------
+// ---- leaf sums ----------------------------------------------------------------
 
 // The live list of (system r, depth-5 tile c), T = r kTiles + c: (c + 23 r)
 // mod 64.  Each system gives each list exactly kTiles / 64 of its tiles, so a
@@ -301,74 +298,84 @@ __device__ __forceinline__ uint32_t tile_of(uint32_t key) {
     return (key >> kBatchRankShift) * kTiles + ((key >> 10) & (kTiles - 1));
 }
 
+// One leaf of system r: its record and, with two or more particles, its cell
+// node, which comes right before its first particle's (node slot `first`).
+__device__ __forceinline__ void bb_emit_leaf(const float4 &r, uint32_t L, uint32_t first,
+                                             uint32_t n, float4 *__restrict__ leaf_sum,
+                                             float4 *__restrict__ node4,
+                                             uint4 *__restrict__ child) {
+    leaf_sum[L] = make_float4(r.x, r.y, r.z, __uint_as_float(n));
+    if (n >= 2u)
+        emit_cell_at(TileCell{n, n + 1u, 0u, 0u, r.x, r.y, r.z, 0.0f}, (int)kTreeDepth, first - 1u,
+                     make_uint4(n, 0u, 0u, kLeafMark), node4, child);
+}
+
+// The particles of leaf L, [f, e), and the node slot of the first: f + C(f + 1).
+// The positions after a system's last in-domain one hold no C, but that one's
+// C(f + 1) is what its tree ends with: end_slot - 1 - f.
+struct LeafSpan {
+    uint32_t f, e, first;
+};
+
+__device__ __forceinline__ LeafSpan leaf_span(uint32_t L, uint32_t key,
+                                              const uint32_t *__restrict__ leaf_first,
+                                              const uint32_t *__restrict__ bh_prefix,
+                                              const RankStats *__restrict__ stats,
+                                              const uint32_t *__restrict__ cpos) {
+    const uint32_t r = key >> kBatchRankShift;
+    const RankStats st = stats[r];
+    const uint32_t sys_end = bh_prefix[r] + st.n_in;
+    const uint32_t e = min(leaf_first[L + 1], sys_end);
+    const uint32_t f = min(leaf_first[L], e);
+    const uint32_t first = f + 1 < sys_end ? f + cpos[f + 1] : st.end_slot - 1u;
+    return LeafSpan{f, e, first};
+}
+
 __global__ __launch_bounds__(256) void bb_leaf_kernel(
     const uint32_t *__restrict__ leaf_first, const uint32_t *__restrict__ leaf_key,
-    const float4 *__restrict__ prod, const uint32_t *__restrict__ keys,
-    const uint32_t *__restrict__ cpos, const uint32_t *__restrict__ breaker,
-    BatchCounts *counts, const uint32_t *__restrict__ bh_prefix,
-    const RankStats *__restrict__ stats, float4 *__restrict__ leaf_sum,
-    uint32_t *__restrict__ tile_range, uint32_t *__restrict__ live_tiles, uint32_t live_per_list,
-    float4 *__restrict__ node4) {
+    const uint32_t *__restrict__ cpos, BatchCounts *counts,
+    const uint32_t *__restrict__ bh_prefix, const RankStats *__restrict__ stats,
+    float4 *__restrict__ leaf_sum, uint32_t *__restrict__ tile_range,
+    uint32_t *__restrict__ live_tiles, uint32_t live_per_list, float4 *__restrict__ node4,
+    uint4 *__restrict__ child) {
     __shared__ float4 stage[4][64];
-    const uint32_t n = counts->n_bh_particles, nl = counts->n_leaves, ncells = counts->n_cells;
+    const uint32_t nl = counts->n_leaves;
     const uint32_t waves = gridDim.x * 4;
     const uint32_t lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const uint32_t wave_id = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + w);
     // small leaves: each wave takes 64 consecutive leaves, one per lane
     for (uint32_t base = wave_id * 64; base < nl; base += waves * 64) {
         const uint32_t L = base + lane;
-        const bool valid = L < nl;
-        uint32_t f = 0, e = 0, key = 0;
-        if (valid) {
-            key = leaf_key[L];
-            const uint32_t r = key >> kBatchRankShift;
-            const uint32_t sys_end = bh_prefix[r] + stats[r].n_in;
-            e = min(leaf_first[L + 1], sys_end);
-            f = min(leaf_first[L], e);
+        if (L >= nl) continue;
+        const uint32_t key = leaf_key[L];
+        const LeafSpan p = leaf_span(L, key, leaf_first, bh_prefix, stats, cpos);
+        if (p.e - p.f <= kSmallLeaf)
+            bb_emit_leaf(lane_leaf_sum(node4, p.first, p.first + (p.e - p.f)), L, p.first,
+                         p.e - p.f, leaf_sum, node4, child);
+        const uint32_t T = tile_of(key);
+        if (L == 0 || tile_of(leaf_key[L - 1]) != T) {
+            tile_range[2 * T] = L;
+            const uint32_t q = live_list(T);
+            live_tiles[q * live_per_list + atomicAdd(&counts->n_live[q], 1u)] = T;
         }
-        const bool small = valid && e - f <= kSmallLeaf;
-        if (small) {
-            const float4 r = lane_leaf_sum(prod, f, e);
-            leaf_sum[L] = make_float4(r.x, r.y, r.z, __uint_as_float(e - f));
-        }
-        if (valid) {
-            const uint32_t T = tile_of(key);
-            if (L == 0 || tile_of(leaf_key[L - 1]) != T) {
-                tile_range[2 * T] = L;
-                const uint32_t q = live_list(T);
-                live_tiles[q * live_per_list + atomicAdd(&counts->n_live[q], 1u)] = T;
-            }
-            if (L + 1 == nl || tile_of(leaf_key[L + 1]) != T) tile_range[2 * T + 1] = L + 1;
-        }
+        if (L + 1 == nl || tile_of(leaf_key[L + 1]) != T) tile_range[2 * T + 1] = L + 1;
     }
     // larger leaves: leaf L goes to wave L mod waves (neighbouring dense
     // leaves to different waves), streamed by the whole wave
     for (uint32_t i0 = 0; wave_id + i0 * waves < nl; i0 += 64) {
         const uint32_t L = wave_id + (i0 + lane) * waves;
-        uint32_t f = 0, e = 0;
-        if (L < nl) {
-            const uint32_t r = leaf_key[L] >> kBatchRankShift;
-            e = min(leaf_first[L + 1], bh_prefix[r] + stats[r].n_in);
-            f = min(leaf_first[L], e);
-        }
-        unsigned long long big = __ballot(L < nl && e - f > kSmallLeaf);
+        LeafSpan p{0u, 0u, 0u};
+        if (L < nl) p = leaf_span(L, leaf_key[L], leaf_first, bh_prefix, stats, cpos);
+        unsigned long long big = __ballot(L < nl && p.e - p.f > kSmallLeaf);
         while (big) {
             const uint32_t j = (uint32_t)__builtin_ctzll(big);
             big &= big - 1;
-            const uint32_t bf = __builtin_amdgcn_readfirstlane(__shfl(f, j, 64));
-            const uint32_t be = __builtin_amdgcn_readfirstlane(__shfl(e, j, 64));
-            const float4 r = wave_leaf_sum(stage[w], prod, bf, be, lane);
+            const uint32_t n = __builtin_amdgcn_readfirstlane(__shfl(p.e - p.f, j, 64));
+            const uint32_t first = __builtin_amdgcn_readfirstlane(__shfl(p.first, j, 64));
+            const float4 r = wave_leaf_sum(stage[w], node4, first, first + n, lane);
             if (lane == 0)
-                leaf_sum[wave_id + (i0 + j) * waves] = make_float4(r.x, r.y, r.z, __uint_as_float(be - bf));
+                bb_emit_leaf(r, wave_id + (i0 + j) * waves, first, n, leaf_sum, node4, child);
         }
-    }
-    for (uint32_t k = blockIdx.x * 256 + threadIdx.x; k < n; k += gridDim.x * 256) {
-        const BPos q = bpos_info(keys, n, k);
-        if (!q.inside) continue;
-        const uint32_t c1 = cpos[k] + q.ns;  // C(k+1)
-        uint32_t run_end = c1 < ncells ? breaker[c1] : n;
-        run_end = min(run_end, bh_prefix[q.rank] + stats[q.rank].n_in);
-        set_run_length(node4, k + c1, run_end > k ? run_end - k : 1u);
     }
 }
 
@@ -383,7 +390,7 @@ __global__ __launch_bounds__(256) void bb_tile_kernel(
     const uint32_t *__restrict__ leaf_key, const float4 *__restrict__ leaf_sum,
     const int8_t *__restrict__ sdep, const uint32_t *__restrict__ cpos,
     const BatchCounts *__restrict__ counts, const uint32_t *__restrict__ live_tiles,
-    uint32_t live_per_list, float4 *__restrict__ node4, uint32_t *__restrict__ ncount,
+    uint32_t live_per_list, float4 *__restrict__ node4, uint4 *__restrict__ child,
     TileCell *__restrict__ top) {
     __shared__ TileCell l10[1024];
     __shared__ TileCell up[341];
@@ -401,9 +408,7 @@ __global__ __launch_bounds__(256) void bb_tile_kernel(
             const uint32_t c = leaf_key[L] & 1023u;
             const float4 s = leaf_sum[L];
             const uint32_t n = __float_as_uint(s.w);
-            TileCell cell{n, n + (n >= 2u ? 1u : 0u), leaf_first[L], 0u, s.x, s.y, s.z, 0.0f};
-            l10[c] = cell;
-            emit_cell(cell, 10, sdep, cpos, node4, ncount);
+            l10[c] = TileCell{n, n + (n >= 2u ? 1u : 0u), leaf_first[L], 0u, s.x, s.y, s.z, 0.0f};
         }
         __syncthreads();
         up[t] = reduce4(l10[4 * t], l10[4 * t + 1], l10[4 * t + 2], l10[4 * t + 3]);
@@ -418,7 +423,10 @@ __global__ __launch_bounds__(256) void bb_tile_kernel(
         }
         for (uint32_t c = t; c < 341; c += 256) {
             const int d = c < 256 ? 9 : c < 320 ? 8 : c < 336 ? 7 : c < 340 ? 6 : 5;
-            emit_cell(up[c], d, sdep, cpos, node4, ncount);
+            const TileCell *kids = d == 9 ? l10 + 4 * c
+                                          : up + tile_level_offset(d + 1) +
+                                                4 * (c - tile_level_offset(d));
+            emit_cell(up[c], d, sizes4(kids), sdep, cpos, node4, child);
         }
         if (t == 0) top[T] = up[340];
         __syncthreads();
@@ -435,7 +443,7 @@ __global__ __launch_bounds__(1024) void bb_top_kernel(const TileCell *__restrict
                                                       const uint32_t *__restrict__ cpos,
                                                       const BatchCounts *__restrict__ counts,
                                                       float4 *__restrict__ node4,
-                                                      uint32_t *__restrict__ ncount) {
+                                                      uint4 *__restrict__ child) {
     __shared__ TileCell lv[1365];
     const uint32_t t = threadIdx.x;
     for (uint32_t r = blockIdx.x; r < counts->n_bh; r += gridDim.x) {
@@ -455,7 +463,8 @@ __global__ __launch_bounds__(1024) void bb_top_kernel(const TileCell *__restrict
         if (t < 341) {
             const uint32_t c = 1024 + t;
             const int d = c < 1280 ? 4 : c < 1344 ? 3 : c < 1360 ? 2 : c < 1364 ? 1 : 0;
-            emit_cell(lv[c], d, sdep, cpos, node4, ncount);
+            const TileCell *kids = lv + top_level_offset(d + 1) + 4 * (c - top_level_offset(d));
+            emit_cell(lv[c], d, sizes4(kids), sdep, cpos, node4, child);
         }
         __syncthreads();
     }
@@ -464,62 +473,42 @@ __global__ __launch_bounds__(1024) void bb_top_kernel(const TileCell *__restrict
 // ---- one persistent force launch for every system ------------------------------
 
 // Barnes-Hut group g of one system: the walk of bh_kernels.hip over the
-// system's node range [root, end_slot) with its own constants.
-// kHalf: a group of the W = 32 vote (the published runs' subgroup width), one
-// 32-particle group per wave with sorted position g * 32 + l held by lanes l
-// and l + 32, walked exactly as bh_traverse32_kernel walks it (both halves
-// vote alike; each half sums its part of every chunk (sum_run_queue), and the
-// halves' partials are added before the acceleration), so the result is that
-// kernel's bit for bit.
-template <bool kHalf>
-__device__ void bb_walk_group(uint32_t g, const SysDesc &d, const RankStats &st, float4 *stage,
-                              uint2 *queue, const uint32_t *__restrict__ sorted_src,
+// system's node range with its own constants, one wave per group.
+template <int W, bool kWide>
+__device__ void bb_walk_group(uint32_t g, const SysDesc &d, const RankStats &st, WalkShared &sh,
+                              const uint32_t *__restrict__ sorted_src,
                               const float2 *__restrict__ pos, const float2 *__restrict__ vel,
-                              const float4 *__restrict__ node4,
-                              const uint32_t *__restrict__ ncount, float2 *__restrict__ pos_out,
-                              float2 *__restrict__ vel_out, uint32_t node_cap,
-                              unsigned long long &vis, unsigned long long &acc,
+                              const float4 *__restrict__ node4, const uint4 *__restrict__ child,
+                              float2 *__restrict__ pos_out, float2 *__restrict__ vel_out,
+                              uint32_t node_cap, unsigned long long &vis, unsigned long long &acc,
                               uint32_t *__restrict__ chunks_io, const BatchTune &tune) {
+    constexpr int R = W / 8;
+    constexpr uint32_t kLanes = 8 / R;  // lanes that end with a target
     const uint32_t lane = threadIdx.x & 63;
-    const uint32_t src = kHalf ? sorted_src[d.sorted_base + g * 32 + (lane & 31u)]
-                               : sorted_src[d.sorted_base + g * 64 + lane];
-    const bool real = src != kBatchSentinel;
-    const uint32_t nreal = kHalf ? (uint32_t)__popcll(__ballot(real) & 0xffffffffull)
-                                 : (uint32_t)__popcll(__ballot(real));
-    float px = 0.0f, py = 0.0f;
-    if (real) {
-        const float2 p = pos[src];
-        px = p.x;
-        py = p.y;
-    }
-    const uint32_t end = __builtin_amdgcn_readfirstlane(min(st.end_slot, node_cap));
-    const uint32_t root = __builtin_amdgcn_readfirstlane(st.root);
-    Partials P;
+    const uint32_t vsrc = sorted_src[d.sorted_base + g * W + (lane & (W - 1u))];
+    const bool real = vsrc != kBatchSentinel;
+    float2 vp = real ? pos[vsrc] : make_float2(0.0f, 0.0f);
+    const unsigned long long rb = __ballot(real);
+    const uint32_t nreal = (uint32_t)__popcll(W == 64 ? rb : rb & 0xffffffffull);
+    // the killed sort last, so the group's first particle is real if any is
+    vp.x = real ? vp.x : lane_value(vp.x, 0);
+    vp.y = real ? vp.y : lane_value(vp.y, 0);
+    const WalkTree tree{node4, child, uniform(st.root),
+                        uniform(min(st.end_slot, node_cap)),
+                        uniform(st.n_in)};
     // start at the issue priority this work item reached in the last step
     const uint32_t prio0 = tune.prio_carry ? *chunks_io / tune.prio_carry : 0u;
+    float ax, ay;
     uint32_t chunks = 0;
-    (void)walk_partials<true, kHalf>(root, end, stage, queue, node4, ncount, px, py, real, nreal,
-                                     d.eps2, d.theta2, 0xfu, P, vis, acc, tune.prio_step, prio0,
-                                     &chunks, tune.run_queue);
+    walk_group<W, R, kWide>(tree, sh, 0u, vp.x, vp.y, nreal, d.eps2, d.theta2, tune.prio_step,
+                     prio0, ax, ay, vis, acc, chunks);
     if (lane == 0) *chunks_io = chunks;
-    if (kHalf) {
-        P.x0 += __shfl_xor(P.x0, 32, 64);
-        P.y0 += __shfl_xor(P.y0, 32, 64);
-        P.x1 += __shfl_xor(P.x1, 32, 64);
-        P.y1 += __shfl_xor(P.y1, 32, 64);
-        P.x2 += __shfl_xor(P.x2, 32, 64);
-        P.y2 += __shfl_xor(P.y2, 32, 64);
-        P.x3 += __shfl_xor(P.x3, 32, 64);
-        P.y3 += __shfl_xor(P.y3, 32, 64);
-    }
-    if (real && (!kHalf || lane < 32)) {
-        float ax, ay;
-        partial_sum(P, ax, ay);
-        const float2 v = vel[src];
-        const float nvx = v.x + ax * d.kv, nvy = v.y + ay * d.kv;
-        pos_out[src] = make_float2(px + (v.x + nvx) * d.kp, py + (v.y + nvy) * d.kp);
-        vel_out[src] = make_float2(nvx, nvy);
-    }
+    const uint32_t src = sorted_src[d.sorted_base + g * W + lane / kLanes];
+    if (lane % kLanes != 0u || src == kBatchSentinel) return;
+    const float2 p = pos[src], v = vel[src];
+    const float nvx = v.x + ax * d.kv, nvy = v.y + ay * d.kv;
+    pos_out[src] = make_float2(p.x + (v.x + nvx) * d.kp, p.y + (v.y + nvy) * d.kp);
+    vel_out[src] = make_float2(nvx, nvy);
 }
 
 // Direct-sum tile: 128 targets (two per lane) x one source slice; the same
@@ -563,18 +552,18 @@ __device__ void bb_ds_tile(uint32_t sub, const SysDesc &d, const float2 *__restr
     if (t1 < d.na) dst[t1] = make_float2(ax1, ay1);
 }
 
+template <bool kWide>
 __global__ __launch_bounds__(256) void bb_force_kernel(
     const uint2 *__restrict__ items, const SysDesc *__restrict__ desc,
     const uint32_t *__restrict__ remaining, const RankStats *__restrict__ stats,
     BatchCounts *__restrict__ counts,
     const uint32_t *__restrict__ sorted_src, const float2 *__restrict__ pos,
     const float2 *__restrict__ vel, const float *__restrict__ mass,
-    const float4 *__restrict__ node4, const uint32_t *__restrict__ ncount,
+    const float4 *__restrict__ node4, const uint4 *__restrict__ child,
     float2 *__restrict__ pos_out, float2 *__restrict__ vel_out, float2 *__restrict__ partial,
     uint32_t node_cap, unsigned long long *__restrict__ wave_acc, uint32_t *__restrict__ ichunk,
     BatchTune tune) {
-    __shared__ float4 stage[4][64];
-    __shared__ uint2 runq[4][kRunQueue];
+    __shared__ WalkShared sh[4];
     const uint32_t w = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const uint32_t nitems = counts->n_items;
     // this wave's queue (kForceQueues queues, each shared by the waves of
@@ -602,13 +591,11 @@ __global__ __launch_bounds__(256) void bb_force_kernel(
             // kernel has already written the system's output)
             if (!live || st.n_in == 0) continue;
             if (d.w == 32)
-                bb_walk_group<true>(item.y, d, st, stage[w], runq[w], sorted_src, pos, vel, node4,
-                                    ncount, pos_out, vel_out, node_cap, vis, acc, &ichunk[it],
-                                    tune);
+                bb_walk_group<32, kWide>(item.y, d, st, sh[w], sorted_src, pos, vel, node4, child,
+                                  pos_out, vel_out, node_cap, vis, acc, &ichunk[it], tune);
             else
-                bb_walk_group<false>(item.y, d, st, stage[w], runq[w], sorted_src, pos, vel,
-                                     node4, ncount, pos_out, vel_out, node_cap, vis, acc,
-                                     &ichunk[it], tune);
+                bb_walk_group<64, kWide>(item.y, d, st, sh[w], sorted_src, pos, vel, node4, child,
+                                  pos_out, vel_out, node_cap, vis, acc, &ichunk[it], tune);
         } else if (live) {
             bb_ds_tile(item.y, d, pos, mass, partial);
         }
@@ -731,21 +718,22 @@ hipError_t batch_launch_step(gsim_batch *b, int in, int out) {
     bb_prep_kernel<<<g_blk, 256, 0, st>>>(sk, d.counts, d.block_cells, d.block_leaves);
     bb_block_scan_kernel<<<2, 1024, 0, st>>>(d.block_cells, d.block_leaves, d.counts);
     bb_emit_kernel<<<g_blk, 256, 0, st>>>(sk, si, d.pos[in], d.mass, d.counts, d.bh_prefix,
-                                          d.block_cells, d.block_leaves, d.sdep, d.cpos, d.prod,
-                                          d.leaf_first, d.leaf_key, d.node4, d.ncount,
-                                          d.sorted_src, d.breaker, d.stats);
-    bb_leaf_kernel<<<4096, 256, 0, st>>>(d.leaf_first, d.leaf_key, d.prod, sk, d.cpos, d.breaker,
-                                         d.counts, d.bh_prefix, d.stats, d.leaf_sum,
-                                         d.tile_range, d.live_tiles, live_per_list, d.node4);
+                                          d.block_cells, d.block_leaves, d.sdep, d.cpos,
+                                          d.leaf_first, d.leaf_key, d.node4, d.sorted_src,
+                                          d.stats);
+    bb_leaf_kernel<<<4096, 256, 0, st>>>(d.leaf_first, d.leaf_key, d.cpos, d.counts, d.bh_prefix,
+                                         d.stats, d.leaf_sum, d.tile_range, d.live_tiles,
+                                         live_per_list, d.node4, d.child);
     const uint32_t g_tile = 4096;  // 64 workgroups per live list
     bb_tile_kernel<<<g_tile, 256, 0, st>>>(d.tile_range, d.leaf_first, d.leaf_key, d.leaf_sum,
                                            d.sdep, d.cpos, d.counts, d.live_tiles, live_per_list,
-                                           d.node4, d.ncount, d.top);
+                                           d.node4, d.child, d.top);
     bb_top_kernel<<<std::min<uint32_t>(b->max_systems, 256), 1024, 0, st>>>(
-        d.top, d.tile_range, d.sdep, d.cpos, d.counts, d.node4, d.ncount);
+        d.top, d.tile_range, d.sdep, d.cpos, d.counts, d.node4, d.child);
     const uint32_t waves = 1024u * b->tune.waves_per_simd;
-    bb_force_kernel<<<waves / 4, 256, 0, st>>>(d.items, d.desc, d.remaining, d.stats, d.counts, d.sorted_src,
-                                               d.pos[in], d.vel[in], d.mass, d.node4, d.ncount,
+    auto *force = b->node_capacity >= kNarrowNodes ? bb_force_kernel<true> : bb_force_kernel<false>;
+    force<<<waves / 4, 256, 0, st>>>(d.items, d.desc, d.remaining, d.stats, d.counts, d.sorted_src,
+                                               d.pos[in], d.vel[in], d.mass, d.node4, d.child,
                                                d.pos[out], d.vel[out], d.partial,
                                                (uint32_t)b->node_capacity, d.wave_acc, d.ichunk,
                                                tune);

@@ -134,18 +134,18 @@ __device__ __forceinline__ TileCell reduce4(const TileCell &a, const TileCell &b
     return r;
 }
 
-// The depth-d cell node c (first particle c.f) at its pre-order slot, given.
-__device__ __forceinline__ void emit_cell_at(const TileCell &c, int d, uint32_t slot,
+// The depth-d cell node c (first particle c.f) at its pre-order slot, given,
+// with its children's subtree sizes (kLeafMark: a leaf cell's particles).
+__device__ __forceinline__ void emit_cell_at(const TileCell &c, int d, uint32_t slot, uint4 sizes,
                                              float4 *__restrict__ node4,
-                                             uint32_t *__restrict__ ncount,
-                                             float r0 = kFixedR0) {
+                                             uint4 *__restrict__ child, float r0 = kFixedR0) {
     if (c.y <= 1u) return;
     float px = c.sx, py = c.sy;
     if (c.sm != 0.0f) {  // TreeMoveShader.comp:66-67
         px = px / c.sm;
         py = py / c.sm;
     }
-    ncount[slot] = c.y;
+    child[slot] = sizes;
     node4[slot] = make_float4(px, py, c.sm, cell_radius(d, r0));
 }
 
@@ -155,23 +155,18 @@ __device__ __forceinline__ uint32_t cell_slot(uint32_t f, int d, const int8_t *_
     return f + cpos[f] + (uint32_t)(d - (int)sdep[f] - 1);
 }
 
-__device__ __forceinline__ void emit_cell(const TileCell &c, int d,
+__device__ __forceinline__ void emit_cell(const TileCell &c, int d, uint4 sizes,
                                           const int8_t *__restrict__ sdep,
                                           const uint32_t *__restrict__ cpos,
-                                          float4 *__restrict__ node4,
-                                          uint32_t *__restrict__ ncount,
+                                          float4 *__restrict__ node4, uint4 *__restrict__ child,
                                           float r0 = kFixedR0) {
     if (c.y <= 1u) return;
-    emit_cell_at(c, d, cell_slot(c.f, d, sdep, cpos), node4, ncount, r0);
+    emit_cell_at(c, d, cell_slot(c.f, d, sdep, cpos), sizes, node4, child, r0);
 }
 
-// A particle node's fourth word (the reference's radius 0): minus the number
-// of particle nodes from it to the next cell node, capped at 2^24 so it is
-// exact in FP32 (a longer run continues from the next slot, which holds its
-// own count).  Every reader takes w <= 0 as a particle node.
-__device__ __forceinline__ void set_run_length(float4 *__restrict__ node4, uint32_t slot,
-                                               uint32_t n) {
-    reinterpret_cast<float *>(node4)[4 * (size_t)slot + 3] = -(float)min(n, 1u << 24);
+// The subtree sizes of four sibling cells.
+__device__ __forceinline__ uint4 sizes4(const TileCell *c) {
+    return make_uint4(c[0].y, c[1].y, c[2].y, c[3].y);
 }
 
 // Exclusive scan of data[0, count) in place by one workgroup of 1024 threads:
@@ -251,18 +246,20 @@ __device__ __forceinline__ void wave_scan2(uint32_t &a, uint32_t &b) {
 }
 
 // ---- leaf sums: m*x, m*y, m of a leaf's particles in ascending sorted order --
-// Both forms add the products one after another in the same order, so a leaf
-// gets the same bits whichever sums it.
+// A leaf's particle nodes are consecutive, [f, e) of node4: their products
+// (pos *= mass, InitShader.comp:102) are formed here.  Both forms add the
+// products one after another in the same order, so a leaf gets the same bits
+// whichever sums it.
 
 // Leaves of at most kSmallLeaf particles are summed by one lane.
 constexpr uint32_t kSmallLeaf = 24;
 
 // Loads go out eight at a time (one round trip per eight products); the
 // additions keep the sequential order.
-__device__ __forceinline__ float4 lane_leaf_sum(const float4 *__restrict__ prod, uint32_t f,
+__device__ __forceinline__ float4 lane_leaf_sum(const float4 *__restrict__ node4, uint32_t f,
                                                 uint32_t e) {
     typedef float v4 __attribute__((ext_vector_type(4)));  // stays in registers
-    const v4 *vp = reinterpret_cast<const v4 *>(prod);
+    const v4 *vp = reinterpret_cast<const v4 *>(node4);
     const v4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
     float sx = 0.0f, sy = 0.0f, sm = 0.0f;
     for (uint32_t k = f; k < e; k += 8) {
@@ -272,8 +269,8 @@ __device__ __forceinline__ float4 lane_leaf_sum(const float4 *__restrict__ prod,
 #pragma unroll
         for (uint32_t u = 0; u < 8; ++u) {
             const bool in = k + u < e;
-            sx = in ? sx + q[u].x : sx;
-            sy = in ? sy + q[u].y : sy;
+            sx = in ? sx + q[u].x * q[u].z : sx;
+            sy = in ? sy + q[u].y * q[u].z : sy;
             sm = in ? sm + q[u].z : sm;
         }
     }
@@ -286,10 +283,10 @@ __device__ __forceinline__ float4 lane_leaf_sum(const float4 *__restrict__ prod,
 // Lanes 0, 1 and 2 each sum one component, reading it 16 bytes at a time, so
 // the wave issues one add per product; each component's order is the leaf's
 // particle order, from +0.  The dependent chain of adds is what remains.
-__device__ __forceinline__ float4 wave_leaf_sum(float4 *stage, const float4 *__restrict__ prod,
+__device__ __forceinline__ float4 wave_leaf_sum(float4 *stage, const float4 *__restrict__ node4,
                                                 uint32_t f, uint32_t e, uint32_t lane) {
     typedef float v4 __attribute__((ext_vector_type(4)));  // stays in registers
-    const v4 *vp = reinterpret_cast<const v4 *>(prod);
+    const v4 *vp = reinterpret_cast<const v4 *>(node4);
     float *st = reinterpret_cast<float *>(stage);
     const uint32_t comp = lane < 3u ? lane : 0u;  // the component this lane sums
     const v4 *sc = reinterpret_cast<const v4 *>(st + 64 * comp);
@@ -304,8 +301,8 @@ __device__ __forceinline__ float4 wave_leaf_sum(float4 *stage, const float4 *__r
         for (uint32_t u = 0; u < 4; ++u) {
             const uint32_t cb = base + 64 * u;
             if (cb >= e) break;
-            st[lane] = q[u].x;
-            st[64 + lane] = q[u].y;
+            st[lane] = q[u].x * q[u].z;
+            st[64 + lane] = q[u].y * q[u].z;
             st[128 + lane] = q[u].z;
             __builtin_amdgcn_wave_barrier();
             q[u] = vp[min(cb + 256 + lane, e - 1)];
@@ -333,187 +330,241 @@ __device__ __forceinline__ float4 wave_leaf_sum(float4 *stage, const float4 *__r
     return make_float4(__shfl(s, 0, 64), __shfl(s, 1, 64), __shfl(s, 2, 64), 0.0f);
 }
 
-// ---- the walk of one W = 64 group --------------------------------------------
-// Summation order, the same in every W = 64 launch, single-system or batched:
-// accepted cells are added in walk order into c; the particle runs (leaf
-// buckets) are cut into 64-node chunks numbered in walk order across runs;
-// chunk j is summed node by node from zero and its sum added to partial
-// j mod 4; the acceleration is (((c + p0) + p1) + p2) + p3.  One wave can
-// compute all of them, or four waves one partial each (a dense-core group
-// split across waves; the wave of p0 also adds the cells and hands over
-// c + p0), with the same bits.
-// Native 4-float vector: conditional copies stay in registers (HIP's float4
-// is a union-based struct whose selects the compiler may route through
-// private memory).
-typedef float f4v __attribute__((ext_vector_type(4)));
+// ---- the walk of one vote group --------------------------------------------
+// A vote group is W = 64 or 32 consecutive sorted particles that take every
+// cell together (ForceShader.comp:111-141): a cell is accepted iff every real
+// particle has radius <= (dx*dx + dy*dy + eps2) * theta2, rounded as the
+// shader writes it, and opened otherwise; particles are always accepted.
+//
+// One wave walks the cells 64 at a time, one per lane, from a stack in LDS.
+// Rounding is monotonic, so the shader's own expression at the nearest point
+// of the group's bounding box is a lower bound of every particle's value: a
+// cell whose radius is within it is accepted by all, and the others are voted
+// on, eight at a time.  The accepted set is therefore the shader's, exactly.
+// An opened cell pushes its children (their slots follow from their subtree
+// sizes, `child`); an opened leaf cell and every accepted node append their
+// slots to the list of sources.
+//
+// The sources are summed eight at a time: lane = 8 * slot + stream holds
+// R targets (t = slot * R + r) and sums every eighth source (its stream) for
+// each, straight from the node records; at the end a target's eight streams
+// are added in a fixed order.  A target's sum depends only on the order of
+// the list, so the same group gives the same bits whichever R its targets
+// are dealt to waves by.
+//
+// What bounds it: the VALU, 9 operations (a SIMD issues one every 2 clocks from
+// two waves in turn where all operands are vector registers, otherwise one
+// every 4) and one v_rsq_f32 (8 to 12 clocks) per source and target.  They are
+// kept in the order written: interleaved over pairs by the compiler the same
+// operations took 43 clocks a pair, in sequence 34-37 (500,000 particles, W =
+// 32: 226 against 199 us).  Matrix instructions for the differences bring
+// nothing: v_mfma_f32_32x32x2_f32 holds up the VALU for as long as the
+// subtractions it saves.  Measured against one cell at a time per wave, with
+// runs staged in LDS (us per walk): 500,000 particles at W = 32 214 -> 176, a
+// million at W = 64 929 -> 881, 200,017 with 15-bit leaves 124 -> 39, 5,003 at
+// theta 0.5 109 -> 25.
 
-// The (x, y, mass) words of node i, or zeros: a run sum uses no more, and a
-// 16-byte load whose fourth word is dead lets the compiler reuse that
-// register while the load is still in flight, which forces a wait for the
-// load at the reuse (a prefetch issued before the previous chunk's sum would
-// then stall at that sum's first instruction).
+// Cells pushed but not yet visited, and sources not yet summed, of one wave.
+// Visiting n cells pushes at most 4 n, so n is kept small enough to leave
+// kWalkMargin free, more than the 3 entries a level that visiting one cell at
+// a time can add down to depth 15.
+constexpr uint32_t kWalkStack = 512;
+constexpr uint32_t kWalkList = 512;
+constexpr uint32_t kWalkMargin = 64;
+struct WalkShared {
+    uint4 list4[kWalkList / 4];
+    uint32_t stack[kWalkStack + 64];  // a read of 64 entries may start at any of them
+    float4 cell[64];                  // cells being voted on
+};
+
+// Orders one wave's LDS accesses (a wave's LDS operations complete in order:
+// this holds the compiler to it).
+__device__ __forceinline__ void wave_lds_order() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
+    __builtin_amdgcn_wave_barrier();
+}
+
+__device__ __forceinline__ uint32_t uniform(uint32_t v) {
+    return (uint32_t)__builtin_amdgcn_readfirstlane((int)v);
+}
+
+__device__ __forceinline__ uint32_t lane_rank(unsigned long long m) {  // set bits below this lane
+    return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+}
+
+template <int kCtrl>
+__device__ __forceinline__ float dpp(float v) {
+    return __builtin_bit_cast(
+        float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), kCtrl, 0xF, 0xF, true));
+}
+constexpr int kDppXor1 = 0xB1, kDppXor2 = 0x4E, kDppXor7 = 0x141, kDppXor15 = 0x140;
+
+__device__ __forceinline__ float lane_value(float v, uint32_t lane) {
+    return __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(v), lane));
+}
+
+// Minimum (kMax: maximum) over the wave, in every lane.
+template <bool kMax>
+__device__ __forceinline__ float wave_extreme(float v) {
+    auto op = [](float a, float b) { return kMax ? fmaxf(a, b) : fminf(a, b); };
+    v = op(v, dpp<kDppXor1>(v));
+    v = op(v, dpp<kDppXor2>(v));
+    v = op(v, dpp<kDppXor7>(v));
+    v = op(v, dpp<kDppXor15>(v));
+    v = op(v, __shfl_xor(v, 16, 64));
+    return op(v, __shfl_xor(v, 32, 64));
+}
+
+// The (x, y, mass) words of a node record.
 typedef float f3v __attribute__((ext_vector_type(3)));
-__device__ __forceinline__ f3v load_node3(const float4 *__restrict__ node4, uint32_t i, bool ok) {
-    f3v r = {0.0f, 0.0f, 0.0f};
-    if (ok) {
-        const float *p = reinterpret_cast<const float *>(node4 + i);
-        r.x = p[0];
-        r.y = p[1];
-        r.z = p[2];
+
+struct BoxXY {
+    float x0, x1, y0, y1;
+};
+
+// One source (x, y, mass) against this lane's targets.
+template <int R>
+__device__ __forceinline__ void add_source(f3v q, const float (&tx)[R], const float (&ty)[R],
+                                           float eps2, float (&ax)[R], float (&ay)[R]) {
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        accumulate(q.x, q.y, q.z, tx[r], ty[r], eps2, ax[r], ay[r]);
+        __builtin_amdgcn_sched_barrier(0);
     }
+}
+
+// A list entry: the byte offset of the node's record, or with kWide (node
+// arrays of 4 GiB and more) its slot.
+template <bool kWide>
+__device__ __forceinline__ uint32_t source_key(uint32_t slot) {
+    return kWide ? slot : slot * 16u;
+}
+
+template <bool kWide>
+__device__ __forceinline__ f3v load_source(const float4 *__restrict__ node4, uint32_t key) {
+    const float *p = kWide ? reinterpret_cast<const float *>(node4 + key)
+                           : reinterpret_cast<const float *>(
+                                 reinterpret_cast<const char *>(node4) + key);
+    f3v r;
+    r.x = p[0];
+    r.y = p[1];
+    r.z = p[2];
     return r;
 }
 
-struct Partials {
-    float xc = 0.0f, yc = 0.0f;  // accepted cells
-    float x0 = 0.0f, y0 = 0.0f, x1 = 0.0f, y1 = 0.0f, x2 = 0.0f, y2 = 0.0f, x3 = 0.0f, y3 = 0.0f;
+// Record `slot` of an array of 16-byte records.
+template <bool kWide, typename T>
+__device__ __forceinline__ T tree_record(const T *__restrict__ base, uint32_t slot) {
+    static_assert(sizeof(T) == 16, "16-byte records");
+    return kWide ? base[slot]
+                 : *reinterpret_cast<const T *>(reinterpret_cast<const char *>(base) + slot * 16u);
+}
+
+// Four sources for each stream from a block of 32 list entries: stream s
+// takes entries 4s .. 4s + 3.
+struct SourceBlock {
+    f3v q[4];
 };
 
-// Adds a chunk's sum to partial k (wave-uniform).  Selects rather than a
-// switch: a switch over the fields lets the compiler index Partials as an
-// array in private memory.
-__device__ __forceinline__ void add_partial(Partials &P, uint32_t k, float cx, float cy) {
-    const float ax0 = P.x0 + cx, ay0 = P.y0 + cy, ax1 = P.x1 + cx, ay1 = P.y1 + cy;
-    const float ax2 = P.x2 + cx, ay2 = P.y2 + cy, ax3 = P.x3 + cx, ay3 = P.y3 + cy;
-    P.x0 = k == 0u ? ax0 : P.x0;
-    P.y0 = k == 0u ? ay0 : P.y0;
-    P.x1 = k == 1u ? ax1 : P.x1;
-    P.y1 = k == 1u ? ay1 : P.y1;
-    P.x2 = k == 2u ? ax2 : P.x2;
-    P.y2 = k == 2u ? ay2 : P.y2;
-    P.x3 = k == 3u ? ax3 : P.x3;
-    P.y3 = k == 3u ? ay3 : P.y3;
+template <bool kWide>
+__device__ __forceinline__ SourceBlock load_block(const WalkShared &sh, uint32_t block,
+                                                  uint32_t stream,
+                                                  const float4 *__restrict__ node4) {
+    const uint4 i = sh.list4[block * 8 + stream];
+    SourceBlock b;
+    b.q[0] = load_source<kWide>(node4, i.x);
+    b.q[1] = load_source<kWide>(node4, i.y);
+    b.q[2] = load_source<kWide>(node4, i.z);
+    b.q[3] = load_source<kWide>(node4, i.w);
+    return b;
 }
 
-__device__ __forceinline__ void partial_sum(const Partials &P, float &ax, float &ay) {
-    ax = (((P.xc + P.x0) + P.x1) + P.x2) + P.x3;
-    ay = (((P.yc + P.y0) + P.y1) + P.y2) + P.y3;
+template <int R>
+__device__ __forceinline__ void add_block(const SourceBlock &b, const float (&tx)[R],
+                                          const float (&ty)[R], float eps2, float (&ax)[R],
+                                          float (&ay)[R]) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) add_source<R>(b.q[j], tx, ty, eps2, ax, ay);
 }
 
-// What the wave computing partial k of a split group hands over: c + p0 for
-// k = 0, else pk; added in order they give partial_sum's bits.
-__device__ __forceinline__ void split_share(const Partials &P, uint32_t k, float &ax, float &ay) {
-    switch (k) {
-        case 0: ax = P.xc + P.x0; ay = P.yc + P.y0; break;
-        case 1: ax = P.x1; ay = P.y1; break;
-        case 2: ax = P.x2; ay = P.y2; break;
-        default: ax = P.x3; ay = P.y3; break;
+// The whole blocks of 32 of the first `count` list entries, each block's
+// loads in flight while the block before is summed.
+template <int R, bool kWide>
+__device__ __forceinline__ void sum_blocks(const WalkShared &sh, uint32_t blocks, uint32_t stream,
+                                           const float4 *__restrict__ node4, const float (&tx)[R],
+                                           const float (&ty)[R], float eps2, float (&ax)[R],
+                                           float (&ay)[R]) {
+    if (!blocks) return;
+    SourceBlock a = load_block<kWide>(sh, 0, stream, node4);
+    for (uint32_t b = 0; b < blocks; b += 2) {
+        const SourceBlock c = load_block<kWide>(sh, min(b + 1, blocks - 1), stream, node4);
+        add_block<R>(a, tx, ty, eps2, ax, ay);
+        if (b + 1 == blocks) break;
+        a = load_block<kWide>(sh, min(b + 2, blocks - 1), stream, node4);
+        add_block<R>(c, tx, ty, eps2, ax, ay);
     }
 }
 
-
-// The run chunks [queue[0], queue[qn]) of one queue batch, chunk numbers from
-// ch0: each chunk this wave owns ((parts >> (chunk & 3)) & 1) is loaded with
-// one coalesced load while the previous one is summed (across run
-// boundaries; a chunk is staged in LDS before the next one's load is issued),
-// staged in the wave's LDS as packed 12-byte (x, y, m) records,
-// summed node by node from zero and added to its partial.  kHalf: the wave
-// holds one 32-particle group twice (lane l and l + 32 the same particle) and
-// each half sums part of every chunk: lanes 0-31 its first s nodes, lanes
-// 32-63 the rest, s = the chunk's node count halved and rounded up to a
-// multiple of 4 (32 for a full chunk), so a partial chunk costs the wave
-// about half its nodes rather than up to all of them.
-template <bool kHalf = false>
-__device__ __forceinline__ void sum_run_queue(const uint2 *queue, uint32_t qn, uint32_t ch0,
-                                              float4 *stage, const float4 *__restrict__ node4,
-                                              float px, float py, float eps2, uint32_t parts,
-                                              Partials &P) {
-    const uint32_t lane = threadIdx.x & 63;
-    float *st = reinterpret_cast<float *>(stage);
-    const f4v *st4 = reinterpret_cast<const f4v *>(stage);
-    // cursor: run e, chunk start base, run end rend, chunk number ch
-    uint32_t e = 0, base = 0, rend = 0, ch = ch0;
-    auto run_at = [&](uint32_t i, uint32_t &b, uint32_t &r) {
-        const uint2 q = queue[i];
-        b = __builtin_amdgcn_readfirstlane(q.x);
-        r = b + __builtin_amdgcn_readfirstlane(q.y);
-    };
-    auto owned = [&](uint32_t c) { return ((parts >> (c & 3u)) & 1u) != 0u; };
-    auto step = [&](uint32_t &ee, uint32_t &bb, uint32_t &rr, uint32_t &cc) {
-        bb += 64u;
-        ++cc;
-        if (bb >= rr) {
-            ++ee;
-            if (ee < qn) run_at(ee, bb, rr);
-        }
-    };
-    if (qn == 0) return;
-    run_at(0, base, rend);
-    while (e < qn && !owned(ch)) step(e, base, rend, ch);
-    f3v cur = load_node3(node4, base + lane, e < qn && lane < min(64u, rend - base));
-    while (e < qn) {
-        const uint32_t cnt = min(64u, rend - base), k = ch & 3u;
-        // stage this chunk first: its load (the previous iteration's
-        // prefetch) is the only one in flight, so the wait for it cannot
-        // also wait for the next chunk's load, issued right after
-        st[3 * lane] = cur.x;
-        st[3 * lane + 1] = cur.y;
-        st[3 * lane + 2] = cur.z;
-        uint32_t ne = e, nb = base, nr = rend, nch = ch;
-        do {
-            step(ne, nb, nr, nch);
-        } while (ne < qn && !owned(nch));
-        const f3v next = load_node3(node4, nb + lane, ne < qn && lane < min(64u, nr - nb));
-        __builtin_amdgcn_wave_barrier();
-        float cx = 0.0f, cy = 0.0f;
-        uint32_t j = 0, jend = cnt;
-        if (kHalf) {
-            const uint32_t split = ((cnt + 7u) >> 3) << 2;  // a multiple of 4: float4 reads
-            j = lane < 32u ? 0u : split;
-            jend = lane < 32u ? min(split, cnt) : cnt;
-        }
-        for (; j + 8 <= jend; j += 8) {
-            f4v r[6];
-#pragma unroll
-            for (int u = 0; u < 6; ++u) r[u] = st4[3 * (j / 4) + u];
-            const float *q = reinterpret_cast<const float *>(r);
-#pragma unroll
-            for (int u = 0; u < 8; ++u)
-                accumulate(q[3 * u], q[3 * u + 1], q[3 * u + 2], px, py, eps2, cx, cy);
-        }
-        for (; j < jend; ++j)
-            accumulate(st[3 * j], st[3 * j + 1], st[3 * j + 2], px, py, eps2, cx, cy);
-        add_partial(P, k, cx, cy);
-        __builtin_amdgcn_wave_barrier();
-        cur = next;
-        e = ne;
-        base = nb;
-        rend = nr;
-        ch = nch;
+// The last count < 32 entries, stream s taking entry 8 j + s of each eight; a
+// stream without one adds a massless source far away (exactly nothing).
+template <int R, bool kWide>
+__device__ __forceinline__ void sum_rest(const WalkShared &sh, uint32_t first, uint32_t count,
+                                         uint32_t stream, const float4 *__restrict__ node4,
+                                         const float (&tx)[R], const float (&ty)[R], float eps2,
+                                         float (&ax)[R], float (&ay)[R]) {
+    const uint32_t *list = reinterpret_cast<const uint32_t *>(sh.list4);
+    for (uint32_t j = 0; j < count; j += 8) {
+        const bool in = j + stream < count;
+        f3v q = load_source<kWide>(node4, list[first + (in ? j + stream : j)]);
+        q.x = in ? q.x : 1e18f;
+        q.z = in ? q.z : 0.0f;
+        add_source<R>(q, tx, ty, eps2, ax, ay);
     }
 }
 
-// Walks the pre-order nodes [ind, end) for the group's lanes (ForceShader.comp
-// :111-141): a cell is accepted iff every real lane has radius <= (dx*dx +
-// dy*dy + eps2) * theta2, rounded as the shader writes it, then ind += count,
-// else ind++.  Particle nodes are always accepted, so a run of them is a plain
-// direct sum; a particle node's fourth word (the reference's radius 0) holds
-// minus the number of particle nodes from it to the next cell node, so one
-// 16-byte record tells a cell from a run and gives the run's length.  `parts` (bit k) selects the partials this wave computes; the
-// wave computing partial 0 adds the cells and counts the real-lane visits
-// and acceptances.  kStaged: the walk decides first and queues the particle
-// runs (up to qmax <= kRunQueue, `queue` is the wave's LDS; where the queue
-// is cut changes no sum, as chunks are numbered across runs) -- no decision
-// depends on
-// a force -- then sums the queued runs with the next chunk always in flight
-// (sum_run_queue), raising the wave's issue priority one level per prio_step
-// chunks summed (0: never); the node record, its count and its run length are loaded
-// together, so each step of the walk is one round trip.  Otherwise runs are
-// summed as they come, through scalar loads.  Returns the walk's VALU weight
-// (a cell visit ~12 instructions, a particle ~10) in units of 4, capped at
-// 65535.
-// Issue-priority steps of the staged walk, in summed chunks of 64 source
-// particles per priority level (s_setprio 1..3).  Dense-core groups are the
-// tail of a launch whose groups are all resident from the start; letting them
-// take issue slots ahead of lighter waves shortens it.  Measured best: 56-72
-// for the single-system 500k two-disk step (traversal -4.5%), 32 for the
-// batched workload (+1.8%; the batch's step and carry are autotuner knobs,
-// BatchTune); 0 turns it off.
+// The sum of a target's eight streams: the lanes of a slot exchange with
+// stream ^ 7, ^ 2 and ^ 1, halving the targets each still holds, so that lane
+// l ends with target l / (8 / R) and the order of additions is the same for
+// every R.
+template <int R>
+__device__ __forceinline__ float sum_streams(const float (&a)[R], uint32_t lane) {
+    if constexpr (R == 8) {
+        float b[4];
+        const bool up = (lane & 4u) != 0;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            b[i] = (up ? a[i + 4] : a[i]) + dpp<kDppXor7>(up ? a[i] : a[i + 4]);
+        const bool u2 = (lane & 2u) != 0;
+        const float c0 = (u2 ? b[2] : b[0]) + dpp<kDppXor2>(u2 ? b[0] : b[2]);
+        const float c1 = (u2 ? b[3] : b[1]) + dpp<kDppXor2>(u2 ? b[1] : b[3]);
+        const bool u1 = (lane & 1u) != 0;
+        return (u1 ? c1 : c0) + dpp<kDppXor1>(u1 ? c0 : c1);
+    } else if constexpr (R == 4) {
+        const bool up = (lane & 4u) != 0, u2 = (lane & 2u) != 0;
+        const float b0 = (up ? a[2] : a[0]) + dpp<kDppXor7>(up ? a[0] : a[2]);
+        const float b1 = (up ? a[3] : a[1]) + dpp<kDppXor7>(up ? a[1] : a[3]);
+        const float c = (u2 ? b1 : b0) + dpp<kDppXor2>(u2 ? b0 : b1);
+        return c + dpp<kDppXor1>(c);
+    } else if constexpr (R == 2) {
+        const bool up = (lane & 4u) != 0;
+        const float b = (up ? a[1] : a[0]) + dpp<kDppXor7>(up ? a[0] : a[1]);
+        const float c = b + dpp<kDppXor2>(b);
+        return c + dpp<kDppXor1>(c);
+    } else {
+        static_assert(R == 1, "targets per lane");
+        const float b = a[0] + dpp<kDppXor7>(a[0]);
+        const float c = b + dpp<kDppXor2>(b);
+        return c + dpp<kDppXor1>(c);
+    }
+}
+
+// Issue priority of a walking wave: dense-core groups are the tail of a
+// launch whose groups are all resident from the start, so a wave rises one
+// level (s_setprio 1..3) per prio_step chunks of 64 sources it has summed (0:
+// never), and starts at level prio0.
 constexpr uint32_t kPrioStepSingle = 64;
-// A single-system group also starts at level (chunks it summed last step) /
-// kPrioCarry: the heavy groups lead from the first instruction.  Measured on
-// the same workload: 24 -> traversal a further -4% (16: none, 32: -2%, 64: +1%).
-// The batched force launch does the same per work item.
+// A single-system group starts at level (chunks it summed last step) /
+// kPrioCarry; the batched force launch does the same per work item.
 constexpr uint32_t kPrioCarry = 24;
 
 __device__ __forceinline__ void set_issue_priority(uint32_t level) {
@@ -523,111 +574,196 @@ __device__ __forceinline__ void set_issue_priority(uint32_t level) {
     else __builtin_amdgcn_s_setprio(0);
 }
 
-// kHalf (staged only): one 32-particle group held twice by the wave, see
-// sum_run_queue; the votes are the group's, as both halves vote alike.
-template <bool kStaged, bool kHalf = false>
-__device__ __forceinline__ uint32_t walk_partials(
-    uint32_t ind, uint32_t end, float4 *stage, uint2 *queue, const float4 *__restrict__ node4,
-    const uint32_t *__restrict__ ncount, float px, float py, bool real, uint32_t nreal,
-    float eps2, float theta2, uint32_t parts, Partials &P, unsigned long long &vis,
-    unsigned long long &acc, uint32_t prio_step, uint32_t prio0 = 0,
-    uint32_t *chunks_out = nullptr, uint32_t qmax = kRunQueue) {
-    static_assert(kStaged || !kHalf, "half-wave groups need the staged walk");
-    const uint32_t lane = threadIdx.x & 63;
-    const bool first = (parts & 1u) != 0;
-    uint32_t chunk = 0, cells = 0, runs = 0, qn = 0, qch = 0;
-    uint32_t level = 0;
-    if (kStaged && prio_step && prio0) {
-        level = min(prio0, 3u);
-        set_issue_priority(level);
+struct WalkTree {
+    const float4 *__restrict__ node4;
+    const uint4 *__restrict__ child;
+    uint32_t root, end;  // first node slot, one past the last
+    uint32_t n_in;       // particles in the tree
+};
+
+// Walks one group for R * 8 of its W targets, t = part * 8 R + slot * R + r of
+// the group.  px, py: the group's particle lane & (W - 1), or any real one of
+// the group in place of one that is not; nreal: its real particles.  Returns in lane l the acceleration of
+// target part * 8 R + l / (8 / R); vis and acc grow by the group's real-lane
+// visits and acceptances, chunks becomes the sources summed / 64.
+template <int W, int R, bool kWide>
+__device__ __forceinline__ void walk_group(const WalkTree &tree, WalkShared &sh, uint32_t part,
+                                           float px, float py, uint32_t nreal, float eps2, float theta2, uint32_t prio_step,
+                                           uint32_t prio0, float &ax_out, float &ay_out,
+                                           unsigned long long &vis, unsigned long long &acc,
+                                           uint32_t &chunks) {
+    const uint32_t lane = threadIdx.x & 63, stream = lane & 7u;
+    uint32_t *const stack = sh.stack;
+    uint32_t *const list = reinterpret_cast<uint32_t *>(sh.list4);
+    float tx[R], ty[R], ax[R], ay[R];
+    float vx[W / 8], vy[W / 8];  // this slot's share of the group, for the votes
+    BoxXY box;
+    {
+        // the group through LDS: the targets are R consecutive particles a slot
+        float2 *const xy = reinterpret_cast<float2 *>(stack);
+        xy[lane] = make_float2(px, py);
+        wave_lds_order();
+        const uint32_t t0 = part * (8 * R) + (lane >> 3) * R, v0 = (lane >> 3) * (W / 8);
+#pragma unroll
+        for (int i = 0; i < W / 8; ++i) {
+            const float2 p = xy[v0 + i];
+            vx[i] = p.x;
+            vy[i] = p.y;
+        }
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const float2 p = xy[t0 + r];
+            tx[r] = p.x;
+            ty[r] = p.y;
+            ax[r] = 0.0f;
+            ay[r] = 0.0f;
+        }
+        wave_lds_order();
+        box.x0 = wave_extreme<false>(px);
+        box.x1 = wave_extreme<true>(px);
+        box.y0 = wave_extreme<false>(py);
+        box.y1 = wave_extreme<true>(py);
     }
+    float ev = eps2;  // in a vector register: a scalar operand costs the second issue
+    asm volatile("" : "+v"(ev));
+    uint32_t sp = 0, sc = 0, sources = 0;
+    uint32_t visited = 0, accepted = 0;  // nodes, of this group
+    if (nreal && tree.n_in) {            // one particle alone has no cell above it
+        if (tree.n_in > 1u) {
+            stack[lane] = tree.root;
+            sp = 1;
+        } else {
+            list[lane] = source_key<kWide>(tree.root);
+            sc = visited = accepted = 1;
+        }
+        wave_lds_order();
+    }
+    uint32_t level = prio_step ? min(prio0, 3u) : 0u;
+    if (level) set_issue_priority(level);
+    unsigned long long runs = 0;  // lanes whose opened leaf cell is not yet listed
+    uint32_t run_first = 0, run_left = 0;
+    uint32_t slot = 0, count = 0;
     while (true) {
-      while (ind < end && qn < qmax) {
-        const float4 nd = node4[ind];
-        const uint32_t cnt = ncount[ind];
-        // one round trip per step: both loads are issued here and waited for
-        // together (otherwise the compiler sinks the x, y half of the record
-        // and the count into the branches that use them, three dependent
-        // round trips for an accepted cell)
-        asm volatile("" ::"s"(nd.x), "s"(nd.y), "s"(nd.z), "s"(nd.w), "s"(cnt));
-        if (nd.w <= 0.0f) {  // a particle node: w = -(particle nodes left in its run)
-            const uint32_t pr = (uint32_t)(-nd.w);
-            const uint32_t n = __builtin_amdgcn_readfirstlane(min(max(pr, 1u), end - ind));
-            if (first) {
-                vis += (unsigned long long)n * nreal;
-                acc += (unsigned long long)n * nreal;
-            }
-            runs += n;
-            if (kStaged) {
-                if (lane == 0) queue[qn] = make_uint2(ind, n);
-                ++qn;
-                chunk += (n + 63u) >> 6;
-                ind += n;
+        while (sc <= kWalkList - 64u && (run_left || runs || sp)) {
+            if (run_left || runs) {
+                if (!run_left) {
+                    const uint32_t j = (uint32_t)__builtin_ctzll(runs);
+                    runs &= runs - 1;
+                    run_first = (uint32_t)__builtin_amdgcn_readlane(slot, j) + 1u;
+                    run_left = min((uint32_t)__builtin_amdgcn_readlane(count, j),
+                                   tree.end - min(run_first, tree.end));
+                    visited += run_left;
+                    accepted += run_left;
+                }
+                const uint32_t take = min(run_left, 64u);
+                // entries past `take` are overwritten by the next append
+                list[sc + lane] = source_key<kWide>(run_first + lane);
+                sc += take;
+                run_first += take;
+                run_left -= take;
                 continue;
             }
-            const uint32_t rend = ind + n;
-            for (uint32_t base = ind; base < rend; base += 64, ++chunk) {
-                const uint32_t k = chunk & 3u;
-                if (!((parts >> k) & 1u)) continue;
-                const uint32_t ce = base + min(64u, rend - base);
-                float cx = 0.0f, cy = 0.0f;
-                uint32_t j = base;
-                for (; j + 4 <= ce; j += 4) {
-                    float4 q[4];
+            // visit the top n cells of the stack (at least four entries stay
+            // free, whatever the tree)
+            sp = min(sp, kWalkStack - 4u);
+            const uint32_t room = kWalkStack - kWalkMargin;
+            uint32_t n = min(sp, 64u);
+            if (sp + 3u * n > room) n = max(1u, (room - min(sp, room)) / 3u);
+            n = uniform(n);
+            sp -= n;
+            const unsigned long long on = ~0ull >> (64u - n);
+            wave_lds_order();
+            slot = min(stack[sp + lane], tree.end - 1u);  // lanes past n: any node
+            wave_lds_order();
+            const float4 nd = tree_record<kWide>(tree.node4, slot);
+            const uint4 ch = tree_record<kWide>(tree.child, slot);
+            // ForceShader.comp:124-125 at the nearest point of the box
+            const float nx = nd.x - __builtin_amdgcn_fmed3f(nd.x, box.x0, box.x1);
+            const float ny = nd.y - __builtin_amdgcn_fmed3f(nd.y, box.y0, box.y1);
+            const float near2 = (nx * nx + ny * ny) + eps2;
+            // a particle's node has radius 0
+            unsigned long long take = (__builtin_amdgcn_ballot_w64(nd.w <= 0.0f) |
+                                       __builtin_amdgcn_ballot_w64(nd.w <= near2 * theta2)) &
+                                      on;
+            // the others eight at a time: this lane's stream names the cell,
+            // its slot W / 8 of the particles.  Rounding is monotonic, so the
+            // particle with the smallest dx*dx + dy*dy decides for them all.
+            const unsigned long long vote = on & ~take;
+            if (vote) {
+                const uint32_t rank = lane_rank(vote), voted = (uint32_t)__popcll(vote);
+                if (__builtin_amdgcn_inverse_ballot_w64(vote)) sh.cell[rank] = nd;
+                wave_lds_order();
+                unsigned long long opened = 0;  // by rank
+                for (uint32_t base = 0; base < voted; base += 8) {
+                    const float4 c = sh.cell[base + stream];
+                    float least = 0.0f;
 #pragma unroll
-                    for (int u = 0; u < 4; ++u) q[u] = node4[j + u];
+                    for (int i = 0; i < W / 8; ++i) {
+                        const float dx = c.x - vx[i], dy = c.y - vy[i];
+                        const float d2 = dx * dx + dy * dy;
+                        least = i ? fminf(least, d2) : d2;
+                    }
+                    unsigned long long m =
+                        __builtin_amdgcn_ballot_w64(!(c.w <= (least + eps2) * theta2));
+                    m |= m >> 32;  // over the slots
+                    m |= m >> 16;
+                    m |= m >> 8;
+                    opened |= (m & 0xffull) << base;
+                }
+                take |= __builtin_amdgcn_ballot_w64(((opened >> rank) & 1ull) == 0ull) & vote;
+            }
+            visited += n;
+            const uint32_t taken = (uint32_t)__popcll(take);
+            accepted += taken;
+            if (__builtin_amdgcn_inverse_ballot_w64(take))
+                list[sc + lane_rank(take)] = source_key<kWide>(slot);
+            sc += taken;
+            const unsigned long long open = on & ~take;
+            runs = __builtin_amdgcn_ballot_w64(ch.w == kLeafMark) & open;
+            count = ch.x;
+            // the children of the others, by quadrant
+            const unsigned long long inner = open & ~runs;
+            if (inner) {
+                const uint32_t size[4] = {ch.x, ch.y, ch.z, ch.w};
+                uint32_t at = slot + 1u;
 #pragma unroll
-                    for (int u = 0; u < 4; ++u)
-                        accumulate(q[u].x, q[u].y, q[u].z, px, py, eps2, cx, cy);
+                for (int q = 0; q < 4; ++q) {
+                    const unsigned long long m = __builtin_amdgcn_ballot_w64(size[q] != 0u) & inner;
+                    if (__builtin_amdgcn_inverse_ballot_w64(m)) stack[sp + lane_rank(m)] = at;
+                    sp += (uint32_t)__popcll(m);
+                    at += size[q];
                 }
-                for (; j < ce; ++j) {
-                    const float4 q = node4[j];
-                    accumulate(q.x, q.y, q.z, px, py, eps2, cx, cy);
-                }
-                add_partial(P, k, cx, cy);
             }
-            ind = rend;
-            continue;
         }
-        ++cells;
-        const float dx = nd.x - px;
-        const float dy = nd.y - py;
-        const float r2 = (dx * dx + dy * dy) + eps2;  // ForceShader.comp:124-125
-        const bool ok = (nd.w <= r2 * theta2) || !real;
-        if (first) vis += nreal;
-        if (__ballot(ok) == ~0ull) {
-            if (first) {
-                const float inv = __builtin_amdgcn_rsqf(r2);
-                const float sc = (nd.z * inv) * (inv * inv);
-                P.xc = __builtin_fmaf(dx, sc, P.xc);
-                P.yc = __builtin_fmaf(dy, sc, P.yc);
-                acc += nreal;
+        wave_lds_order();
+        const uint32_t blocks = sc >> 5;
+        sources += sc & ~31u;
+        if (prio_step) {  // this wave's walk so far, in chunks
+            const uint32_t want = min((sources >> 6) / prio_step, 3u);
+            if (want > level) {
+                level = want;
+                set_issue_priority(level);
             }
-            ind = __builtin_amdgcn_readfirstlane(ind + max(cnt, 1u));
-        } else {
-            ind = __builtin_amdgcn_readfirstlane(ind + 1u);
         }
-      }
-      if (kStaged && qn) {  // the one place queued runs are summed
-          // a wave that has summed many chunks is a dense-core group, the
-          // tail of the launch: it takes issue priority over lighter waves
-          if (prio_step) {
-              const uint32_t want = min(chunk / prio_step, 3u);
-              if (want > level) {
-                  level = want;
-                  set_issue_priority(level);
-              }
-          }
-          __builtin_amdgcn_wave_barrier();
-          sum_run_queue<kHalf>(queue, qn, qch, stage, node4, px, py, eps2, parts, P);
-          qn = 0;
-          qch = chunk;
-      }
-      if (ind >= end) break;
+        sum_blocks<R, kWide>(sh, blocks, stream, tree.node4, tx, ty, ev, ax, ay);
+        const uint32_t rest = sc & 31u;
+        if (!run_left && !runs && !sp) {
+            sum_rest<R, kWide>(sh, sc - rest, rest, stream, tree.node4, tx, ty, ev, ax, ay);
+            sources += rest;
+            break;
+        }
+        wave_lds_order();
+        const uint32_t keep = lane < rest ? list[sc - rest + lane] : 0u;
+        wave_lds_order();
+        if (lane < rest) list[lane] = keep;
+        sc = rest;
     }
-    if (kStaged && level) __builtin_amdgcn_s_setprio(0);  // a persistent wave goes on to other work
-    if (chunks_out) *chunks_out = chunk;
-    return min((cells * 12u + runs * 10u) >> 2, 65535u);
+    if (level) __builtin_amdgcn_s_setprio(0);  // a persistent wave goes on to other work
+    vis += (unsigned long long)visited * nreal;
+    acc += (unsigned long long)accepted * nreal;
+    chunks = (sources + 63u) >> 6;
+    ax_out = sum_streams<R>(ax, lane);
+    ay_out = sum_streams<R>(ay, lane);
 }
 
 }  // namespace gsim

@@ -17,18 +17,20 @@
 //                slot: particle k -> k + C(k+1); the depth-d cell starting at
 //                k -> k + C(k) + (d - s(k) - 1).  Per-block counts here.
 //   4. emit      the scan (each block adds up the counts before it), particle
-//                nodes, sorted_src, m*p products, leaf records.
-//   5. leafsum   leaf sums in ascending particle index (the canonical order of
-//                the reference's float atomics, InitShader.comp:107-109).
+//                nodes, sorted_src, leaf records.
+//   5. leaf      leaf sums in ascending particle index (the canonical order of
+//                the reference's float atomics, InitShader.comp:107-109) and
+//                the leaf cells' nodes.
 //   6. tile      one workgroup per depth-5 cell: the 32x32 leaf tile is
 //                reduced in LDS level by level with ((c0+c1)+c2)+c3 exactly as
 //                TreeInitShader.comp:78-83, counts y = sum + [sum > 1]; cells
-//                with y > 1 are written as nodes (TreeMoveShader.comp:60-77).
+//                with y > 1 are written as nodes (TreeMoveShader.comp:60-77),
+//                with their children's subtree sizes.
 //   7. top       the last tile workgroup to finish reduces the 1024 depth-5
 //                cells to the root.
-//   8. traverse  groups of W sorted slots walk one path; a node is accepted
-//                iff all W lanes accept it (ForceShader.comp:111-141), then
-//                integrate (ForceShader.comp:145-150).
+//   8. walk      groups of W sorted slots take the same cells; a node is
+//                accepted iff all W particles accept it (ForceShader.comp:111-
+//                141), then integrate (ForceShader.comp:145-150).
 #include "bh_device.hpp"
 #include "radix_device.hpp"
 
@@ -146,7 +148,6 @@ __global__ __launch_bounds__(kSortThreads) void bh_keys_kernel(
     for (uint32_t j = g; j < kDigitCopies * 1024; j += stride) digit_next[j] = 0;
     for (uint32_t j = g; j < status_words; j += stride) status[j] = 0;
     if (g == 0) {
-        ctr->next_group = 0;
         ctr->sort_stall = 0;
         ctr->tiles_busy = 0;
         ctr->tiles_done = 0;
@@ -288,10 +289,9 @@ __global__ __launch_bounds__(256) void bh_emit_kernel(
     float2 *__restrict__ pos_out, float2 *__restrict__ vel_out, float *__restrict__ mass_out,
     uint32_t *__restrict__ perm_out, uint2 *__restrict__ ncells, uint32_t na, int bits,
     const uint32_t *__restrict__ block_cells, const uint32_t *__restrict__ block_leaves,
-    int8_t *__restrict__ sdep, uint32_t *__restrict__ cpos, float4 *__restrict__ prod,
+    int8_t *__restrict__ sdep, uint32_t *__restrict__ cpos,
     uint32_t *__restrict__ leaf_first, uint32_t *__restrict__ leaf_key,
-    float4 *__restrict__ node4, uint32_t *__restrict__ ncount,
-    uint32_t *__restrict__ sorted_src, uint32_t *__restrict__ breaker,
+    float4 *__restrict__ node4, uint32_t *__restrict__ sorted_src,
     BhCounters *__restrict__ ctr, const uint32_t *__restrict__ block_gran,
     uint32_t *__restrict__ gran_first, uint32_t *__restrict__ gran_key) {
     __shared__ uint32_t wa[4], wb[4], wc[4], pa[4], pb[4], pc[4];
@@ -379,16 +379,13 @@ __global__ __launch_bounds__(256) void bh_emit_kernel(
     const uint32_t slot = k + C + q.ns;
     // ParticleSortShader.comp:99-107 (canonical order)
     node4[slot] = make_float4(p.x, p.y, m, 0.0f);
-    ncount[slot] = 1u;
     sorted_src[k] = i;
     sdep[k] = (int8_t)q.sk;
     cpos[k] = C;
-    prod[k] = make_float4(p.x * m, p.y * m, m, 0.0f);  // pos *= mass, InitShader.comp:102
     if (q.lf) {
         leaf_first[L] = k;
         leaf_key[L] = q.key;
     }
-    for (uint32_t j = 0; j < q.ns; ++j) breaker[C + j] = k;
     if (gran_first && q.g10) {
         gran_first[ec] = k;
         gran_key[ec] = q.key >> 10;  // the 20-bit cell
@@ -404,41 +401,43 @@ __global__ __launch_bounds__(256) void bh_emit_kernel(
     }
 }
 
-// ---- 5. leaf sums and particle runs ------------------------------------------
+// ---- 5. leaf sums --------------------------------------------------------------
 
 constexpr uint32_t kLeafBlocks = 4096;
 constexpr uint32_t kBoxParts = 256;  // blocks of the box reduction
 
-// Phase A, one wave per leaf: the sum runs over the leaf's particles in
-// sorted (= ascending index) order, the canonical order of the reference's
-// float atomics; the wave stages 64 products at a time in LDS with one
-// coalesced load and adds them in order.  Phase B, one thread per sorted position: the
-// number of consecutive particle nodes from that particle's slot, i.e. up to
-// the next position where a cell node starts (breaker[C(k+1)]).
-// With 15-bit leaves (nsum != nullptr) a leaf of two or more particles is
-// written as its depth-15 cell node at once, with its sums in nsum for the
-// level reduction; there are no tiles.
-__device__ __forceinline__ void emit_deep_leaf(const float4 &r, uint32_t f, uint32_t n,
-                                               const int8_t *__restrict__ sdep,
-                                               const uint32_t *__restrict__ cpos,
-                                               float4 *__restrict__ node4,
-                                               uint32_t *__restrict__ ncount,
-                                               float4 *__restrict__ nsum, float r0) {
-    if (n < 2u) return;
-    const TileCell c{n, n + 1u, f, 0u, r.x, r.y, r.z, 0.0f};
-    emit_cell(c, (int)kDeepBits, sdep, cpos, node4, ncount, r0);
-    const uint32_t slot = f + cpos[f] + (uint32_t)((int)kDeepBits - (int)sdep[f] - 1);
-    nsum[slot] = make_float4(r.x, r.y, r.z, __uint_as_float(n));
+// The node slot of the particle at sorted position f: f + C(f + 1).
+__device__ __forceinline__ uint32_t particle_slot(uint32_t f, uint32_t n_in, uint32_t n_cells,
+                                                  const uint32_t *__restrict__ cpos) {
+    return f + (f + 1 < n_in ? cpos[f + 1] : n_cells);
 }
 
+// A leaf's record: its sums to leaf_sum (15-bit leaves: to nsum at its cell
+// node, for the level reduction) and, with two or more particles, its cell
+// node, which comes right before its first particle's.
+__device__ __forceinline__ void emit_leaf(const float4 &r, uint32_t L, uint32_t first,
+                                          uint32_t n, int bits, float4 *__restrict__ leaf_sum,
+                                          float4 *__restrict__ node4,
+                                          uint4 *__restrict__ child, float4 *__restrict__ nsum,
+                                          float r0) {
+    const float4 sum = make_float4(r.x, r.y, r.z, __uint_as_float(n));
+    if (!nsum) leaf_sum[L] = sum;
+    if (n < 2u) return;
+    emit_cell_at(TileCell{n, n + 1u, 0u, 0u, r.x, r.y, r.z, 0.0f}, bits, first - 1u,
+                 make_uint4(n, 0u, 0u, kLeafMark), node4, child, r0);
+    if (nsum) nsum[first - 1u] = sum;
+}
+
+// The sum runs over the leaf's particles in sorted (= ascending index) order,
+// the canonical order of the reference's float atomics: small leaves one per
+// lane, larger ones one per wave (wave_leaf_sum).  nsum != nullptr: 15-bit
+// leaves, which have no tiles.
 __global__ __launch_bounds__(256) void bh_leaf_kernel(
     const uint32_t *__restrict__ leaf_first, const uint32_t *__restrict__ leaf_key,
-    const float4 *__restrict__ prod, const uint32_t *__restrict__ keys, uint32_t na, int bits,
-    const uint32_t *__restrict__ cpos, const uint32_t *__restrict__ breaker,
-    const BhCounters *__restrict__ ctr, float4 *__restrict__ leaf_sum,
-    uint32_t *__restrict__ tile_range, const int8_t *__restrict__ sdep,
-    float4 *__restrict__ node4, uint32_t *__restrict__ ncount,
-    float4 *__restrict__ nsum, const float *__restrict__ box, uint32_t *__restrict__ tiles_busy) {
+    const uint32_t *__restrict__ cpos, const BhCounters *__restrict__ ctr, int bits,
+    float4 *__restrict__ leaf_sum, uint32_t *__restrict__ tile_range,
+    float4 *__restrict__ node4, uint4 *__restrict__ child, float4 *__restrict__ nsum,
+    const float *__restrict__ box, uint32_t *__restrict__ tiles_busy) {
     __shared__ float4 stage[4][64];
     const uint32_t n_in = ctr->n_in, nl = ctr->n_leaves, ncells = ctr->n_cells;
     const bool deep = nsum != nullptr;
@@ -446,18 +445,10 @@ __global__ __launch_bounds__(256) void bh_leaf_kernel(
     const uint32_t waves = gridDim.x * 4;
     const uint32_t lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const uint32_t wave_id = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + w);
-    // the first particle's run length: its loads go out first, its dependent
-    // load (breaker) once the leaves are summed
-    const uint32_t k0 = blockIdx.x * 256 + threadIdx.x;
-    const bool has0 = k0 < n_in;
-    const uint32_t kk0 = has0 ? k0 : 0u;
-    const uint32_t key0 = keys[kk0], cpos0 = cpos[kk0];
-    const uint32_t keyp = keys[kk0 ? kk0 - 1 : 0], keyn = keys[kk0 + 1 < na ? kk0 + 1 : kk0];
     // larger leaves: leaf L goes to wave (waves - 1 - L) mod waves, so the
     // largest ones (dense cores, low L when few) avoid the first waves, which
     // hold the small leaves; neighbouring dense leaves go to different waves;
-    // each is streamed by the whole wave; the 10-bit leaf's cell node is
-    // written here (15-bit leaves: its depth-15 cell)
+    // each is streamed by the whole wave
     const uint32_t rw = waves - 1u - wave_id;
     for (uint32_t i0 = 0; rw + i0 * waves < nl; i0 += 64) {
         const uint32_t L = rw + (i0 + lane) * waves;
@@ -472,42 +463,25 @@ __global__ __launch_bounds__(256) void bh_leaf_kernel(
             big &= big - 1;
             const uint32_t bf = __builtin_amdgcn_readfirstlane(__shfl(f, j, 64));
             const uint32_t be = __builtin_amdgcn_readfirstlane(__shfl(e, j, 64));
-            const uint32_t slot = deep ? 0u : cell_slot(bf, (int)kTreeDepth, sdep, cpos);
-            const float4 r = wave_leaf_sum(stage[w], prod, bf, be, lane);
-            if (lane == 0) {
-                const uint32_t nb = be - bf;
-                if (deep) {
-                    emit_deep_leaf(r, bf, nb, sdep, cpos, node4, ncount, nsum, r0);
-                } else {
-                    leaf_sum[rw + (i0 + j) * waves] = make_float4(r.x, r.y, r.z, __uint_as_float(nb));
-                    emit_cell_at(TileCell{nb, nb + 1u, bf, 0u, r.x, r.y, r.z, 0.0f},
-                                 (int)kTreeDepth, slot, node4, ncount, r0);
-                }
-            }
+            const uint32_t first = particle_slot(bf, n_in, ncells, cpos);
+            const float4 r = wave_leaf_sum(stage[w], node4, first, first + (be - bf), lane);
+            if (lane == 0)
+                emit_leaf(r, rw + (i0 + j) * waves, first, be - bf, bits, leaf_sum, node4, child,
+                          nsum, r0);
         }
     }
     // small leaves: each wave takes 64 consecutive leaves, one per lane
     for (uint32_t base = wave_id * 64; base < nl; base += waves * 64) {
         const uint32_t L = base + lane;
-        const bool valid = L < nl;
-        uint32_t f = 0, e = 0;
-        if (valid) {
-            e = min(leaf_first[L + 1], n_in);
-            f = min(leaf_first[L], e);
+        if (L >= nl) continue;
+        const uint32_t e = min(leaf_first[L + 1], n_in);
+        const uint32_t f = min(leaf_first[L], e);
+        if (e - f <= kSmallLeaf) {
+            const uint32_t first = particle_slot(f, n_in, ncells, cpos);
+            emit_leaf(lane_leaf_sum(node4, first, first + (e - f)), L, first, e - f, bits,
+                      leaf_sum, node4, child, nsum, r0);
         }
-        const bool small = valid && e - f <= kSmallLeaf;
-        if (small) {
-            const float4 r = lane_leaf_sum(prod, f, e);
-            const uint32_t nb = e - f;
-            if (deep) {
-                emit_deep_leaf(r, f, nb, sdep, cpos, node4, ncount, nsum, r0);
-            } else {
-                leaf_sum[L] = make_float4(r.x, r.y, r.z, __uint_as_float(nb));
-                emit_cell(TileCell{nb, nb + (nb >= 2u ? 1u : 0u), f, 0u, r.x, r.y, r.z, 0.0f},
-                          (int)kTreeDepth, sdep, cpos, node4, ncount, r0);
-            }
-        }
-        if (valid && !deep) {
+        if (!deep) {
             const uint32_t T = leaf_key[L] >> 10;
             if (L == 0 || (leaf_key[L - 1] >> 10) != T) {
                 tile_range[2 * T] = L;
@@ -516,88 +490,76 @@ __global__ __launch_bounds__(256) void bh_leaf_kernel(
             if (L + 1 == nl || (leaf_key[L + 1] >> 10) != T) tile_range[2 * T + 1] = L + 1;
         }
     }
-    uint32_t slot0 = 0, end0 = 0;
-    if (has0) {
-        // pos_info(keys, na, k0, bits) from the loads above
-        const uint32_t killed = 1u << (2 * bits);
-        const int sk = k0 == 0 ? -1 : shared_depth_bits(keyp, key0, bits);
-        const int sk1 = k0 + 1 < na && keyn < killed ? shared_depth_bits(key0, keyn, bits) : -1;
-        const uint32_t c1 = cpos0 + (sk1 > sk ? (uint32_t)(sk1 - sk) : 0u);  // C(k+1)
-        slot0 = k0 + c1;
-        end0 = c1 < ncells ? breaker[c1] : n_in;
-    }
-    if (k0 < n_in) set_run_length(node4, slot0, end0 > k0 ? end0 - k0 : 1u);
-    for (uint32_t k = k0 + gridDim.x * 256; k < n_in; k += gridDim.x * 256) {
-        const PosInfo q = pos_info(keys, na, k, bits);
-        const uint32_t c1 = cpos[k] + q.ns;  // C(k+1)
-        const uint32_t run_end = c1 < ncells ? breaker[c1] : n_in;
-        set_run_length(node4, k + c1, run_end > k ? run_end - k : 1u);
-    }
 }
 
 // ---- 6'. sparse level reduction (15-bit leaves) ---------------------------------
 
 // The sums of the depth-d cell (>= 2 particles) that starts at sorted position
-// k, from its children in pre-order at slot + 1 on: a particle node (count 1)
-// contributes 0 + m*p, a cell node its sums in nsum; each child's quadrant
-// comes from the key bits of its first particle.  Sums are ((c0 + c1) + c2) + c3
-// with an empty quadrant +0: the dense tile reduction's rule, evaluated only
-// where particles are.  Returns (sx, sy, sm) and the particle count n and
-// subtree size y.
+// k, from its children in pre-order at slot + 1 on: a particle node contributes
+// 0 + m*p, a cell node its sums in nsum; each child's quadrant comes from the
+// key bits of its first particle.  Sums are ((c0 + c1) + c2) + c3 with an
+// empty quadrant +0: the dense tile reduction's rule, evaluated only where
+// particles are.  Returns (sx, sy, sm), the particle count n, the subtree size
+// y and the children's sizes by quadrant.
 struct CellSums {
-    float sx, sy, sm;
-    uint32_t n, y;
+    TileCell c;
+    uint4 sizes;
 };
 
+__device__ __forceinline__ uint32_t subtree_size(uint4 ch) {
+    return ch.w == kLeafMark ? ch.x + 1u : ch.x + ch.y + ch.z + ch.w + 1u;
+}
+
 __device__ __forceinline__ CellSums child_sums(const uint32_t *__restrict__ keys,
-                                               const float4 *__restrict__ prod,
-                                               const uint32_t *__restrict__ ncount,
+                                               const float4 *__restrict__ node4,
+                                               const uint4 *__restrict__ child,
                                                const float4 *__restrict__ nsum, uint32_t k,
                                                uint32_t slot, int d, uint32_t n_in,
                                                uint32_t n_nodes) {
     const uint32_t shift = 2u * (kDeepBits - 1u - (uint32_t)d);  // child quadrant bits
     const uint32_t prefix = keys[k] >> (shift + 2u);
     float4 v0 = make_float4(0.0f, 0.0f, 0.0f, 0.0f), v1 = v0, v2 = v0, v3 = v0;
+    uint4 sizes = make_uint4(0u, 0u, 0u, 0u);
     uint32_t c = slot + 1u, f = k, n = 0u, y = 1u;
     // at most four children (distinct quadrants)
     for (int it = 0; it < 4 && f < n_in && c < n_nodes; ++it) {
-        // one round of loads per child: both candidate sums are read before
-        // the count says which one the child is
+        // one round of loads per child: everything a cell or a particle needs
+        // is read before the record says which one the child is
         const uint32_t key = keys[f];
-        const uint32_t cy = ncount[c];
-        const float4 p = prod[f];
+        const float4 p = node4[c];
+        const uint4 ch = child[c];
         const float4 s = nsum[c];
         if ((key >> (shift + 2u)) != prefix) break;
         float4 v;
-        uint32_t cn;
-        if (cy == 1u) {  // a particle node
-            v = make_float4(0.0f + p.x, 0.0f + p.y, 0.0f + p.z, 0.0f);
-            cn = 1u;
+        uint32_t cn = 1u, cy = 1u;
+        if (p.w <= 0.0f) {  // a particle node: pos *= mass, InitShader.comp:102
+            v = make_float4(0.0f + p.x * p.z, 0.0f + p.y * p.z, 0.0f + p.z, 0.0f);
         } else {
             v = s;
             cn = __float_as_uint(v.w);
+            cy = subtree_size(ch);
         }
         const uint32_t q = (key >> shift) & 3u;
-        if (q == 0u) v0 = v;
-        else if (q == 1u) v1 = v;
-        else if (q == 2u) v2 = v;
-        else v3 = v;
+        if (q == 0u) { v0 = v; sizes.x = cy; }
+        else if (q == 1u) { v1 = v; sizes.y = cy; }
+        else if (q == 2u) { v2 = v; sizes.z = cy; }
+        else { v3 = v; sizes.w = cy; }
         n += cn;
         y += cy;
         f += cn;
         c += cy;
     }
-    return CellSums{((v0.x + v1.x) + v2.x) + v3.x, ((v0.y + v1.y) + v2.y) + v3.y,
-                    ((v0.z + v1.z) + v2.z) + v3.z, n, y};
+    return CellSums{TileCell{n, y, k, 0u, ((v0.x + v1.x) + v2.x) + v3.x,
+                             ((v0.y + v1.y) + v2.y) + v3.y, ((v0.z + v1.z) + v2.z) + v3.z, 0.0f},
+                    sizes};
 }
 
 // One launch per depth d = 14..11: every cell node of depth d (a sorted
 // position k with s(k) < d <= s(k+1) starts one) gets its node and its sums.
 __global__ __launch_bounds__(256) void bh_level_kernel(
     const uint32_t *__restrict__ keys, const int8_t *__restrict__ sdep,
-    const uint32_t *__restrict__ cpos, const float4 *__restrict__ prod,
-    const BhCounters *__restrict__ ctr, float4 *__restrict__ node4,
-    uint32_t *__restrict__ ncount, float4 *__restrict__ nsum, int d,
+    const uint32_t *__restrict__ cpos, const BhCounters *__restrict__ ctr,
+    float4 *__restrict__ node4, uint4 *__restrict__ child, float4 *__restrict__ nsum, int d,
     const float *__restrict__ box) {
     const uint32_t n_in = ctr->n_in, n_nodes = ctr->n_nodes;
     const float r0 = box ? box[3] : kFixedR0;
@@ -606,45 +568,43 @@ __global__ __launch_bounds__(256) void bh_level_kernel(
         const int sk1 = k + 1 < n_in ? (int)sdep[k + 1] : -1;
         if (!(sk < d && d <= sk1)) continue;
         const uint32_t slot = k + cpos[k] + (uint32_t)(d - sk - 1);
-        const CellSums c = child_sums(keys, prod, ncount, nsum, k, slot, d, n_in, n_nodes);
-        float px = c.sx, py = c.sy;
-        if (c.sm != 0.0f) {
-            px = px / c.sm;
-            py = py / c.sm;
-        }
-        ncount[slot] = c.y;
-        node4[slot] = make_float4(px, py, c.sm, cell_radius(d, r0));
-        nsum[slot] = make_float4(c.sx, c.sy, c.sm, __uint_as_float(c.n));
+        const CellSums r = child_sums(keys, node4, child, nsum, k, slot, d, n_in, n_nodes);
+        emit_cell_at(r.c, d, slot, r.sizes, node4, child, r0);
+        nsum[slot] = make_float4(r.c.sx, r.c.sy, r.c.sm, __uint_as_float(r.c.n));
     }
 }
 
 // Depth 10 and up with 15-bit leaves: the cells of depth <= 10 are those of a
 // 10-bit tree over the same particles, so the dense tile and top kernels
 // reduce them once each occupied depth-10 cell (granule) has its record: the
-// sums of its depth-10 cell (child_sums) when it holds >= 2 particles, else
-// 0 + m*p of its one particle; particle count; subtree size.  Also marks each
-// depth-5 tile's granule range for the tile kernel.
+// sums of its depth-10 cell (child_sums; its node is written here) when it
+// holds >= 2 particles, else 0 + m*p of its one particle; particle count;
+// subtree size.  Also marks each depth-5 tile's granule range for the tile
+// kernel.
 __global__ __launch_bounds__(256) void bh_gran_kernel(
     const uint32_t *__restrict__ keys, const int8_t *__restrict__ sdep,
-    const uint32_t *__restrict__ cpos, const float4 *__restrict__ prod,
-    const BhCounters *__restrict__ ctr, const uint32_t *__restrict__ ncount,
+    const uint32_t *__restrict__ cpos, const BhCounters *__restrict__ ctr,
+    float4 *__restrict__ node4, uint4 *__restrict__ child,
     const float4 *__restrict__ nsum, const uint32_t *__restrict__ gran_first,
     const uint32_t *__restrict__ gran_key, float4 *__restrict__ gran_sum,
     uint32_t *__restrict__ gran_y, uint32_t *__restrict__ tile_range,
-    uint32_t *__restrict__ tiles_busy) {
+    uint32_t *__restrict__ tiles_busy, const float *__restrict__ box) {
     const uint32_t n_in = ctr->n_in, n_nodes = ctr->n_nodes, ng = ctr->n_gran;
+    const float r0 = box ? box[3] : kFixedR0;
     for (uint32_t L = blockIdx.x * 256 + threadIdx.x; L < ng; L += gridDim.x * 256) {
         const uint32_t k = gran_first[L];
         const int sk = sdep[k];
         const int sk1 = k + 1 < n_in ? (int)sdep[k + 1] : -1;
         if (sk1 >= 10) {
             const uint32_t slot = k + cpos[k] + (uint32_t)(10 - sk - 1);
-            const CellSums c = child_sums(keys, prod, ncount, nsum, k, slot, 10, n_in, n_nodes);
-            gran_sum[L] = make_float4(c.sx, c.sy, c.sm, __uint_as_float(c.n));
-            gran_y[L] = c.y;
+            const CellSums r = child_sums(keys, node4, child, nsum, k, slot, 10, n_in, n_nodes);
+            emit_cell_at(r.c, 10, slot, r.sizes, node4, child, r0);
+            gran_sum[L] = make_float4(r.c.sx, r.c.sy, r.c.sm, __uint_as_float(r.c.n));
+            gran_y[L] = r.c.y;
         } else {
-            const float4 p = prod[k];
-            gran_sum[L] = make_float4(0.0f + p.x, 0.0f + p.y, 0.0f + p.z, __uint_as_float(1u));
+            const float4 p = node4[particle_slot(k, n_in, ctr->n_cells, cpos)];
+            gran_sum[L] = make_float4(0.0f + p.x * p.z, 0.0f + p.y * p.z, 0.0f + p.z,
+                                      __uint_as_float(1u));
             gran_y[L] = 1u;
         }
         const uint32_t T = gran_key[L] >> 10;
@@ -674,11 +634,12 @@ __global__ __launch_bounds__(256) void bh_tile_kernel(
     const uint32_t *__restrict__ tile_range, const uint32_t *__restrict__ leaf_first,
     const uint32_t *__restrict__ leaf_key, const float4 *__restrict__ leaf_sum,
     const int8_t *__restrict__ sdep, const uint32_t *__restrict__ cpos,
-    float4 *__restrict__ node4, uint32_t *__restrict__ ncount, TileCell *__restrict__ top,
+    float4 *__restrict__ node4, uint4 *__restrict__ child, TileCell *__restrict__ top,
     const float *__restrict__ box, const uint32_t *__restrict__ leaf_y,
     BhCounters *__restrict__ ctr) {
     // leaf_y (15-bit leaves): the depth-10 records are granules whose subtree
-    // size is given; otherwise leaves of n particles, y = n + [n >= 2]
+    // size is given; otherwise leaves of n particles, y = n + [n >= 2].  The
+    // depth-10 nodes themselves are already written.
     __shared__ TileCell l10[1024];
     __shared__ TileCell up[341];
     __shared__ uint32_t last;
@@ -690,7 +651,7 @@ __global__ __launch_bounds__(256) void bh_tile_kernel(
         l10[c] = TileCell{0u, 0u, 0xffffffffu, 0u, 0.0f, 0.0f, 0.0f, 0.0f};
     lds_barrier();
     // a tile holds at most 1024 leaves (granules): four per thread, loaded
-    // together; a 10-bit leaf's own cell node was written with its sum
+    // together
 #pragma unroll
     for (uint32_t u = 0; u < 4; ++u) {
         const uint32_t L = lb + t + 256 * u;
@@ -699,9 +660,7 @@ __global__ __launch_bounds__(256) void bh_tile_kernel(
         const float4 s = leaf_sum[L];
         const uint32_t n = __float_as_uint(s.w);
         const uint32_t y = leaf_y ? leaf_y[L] : n + (n >= 2u ? 1u : 0u);
-        TileCell cell{n, y, leaf_first[L], 0u, s.x, s.y, s.z, 0.0f};
-        l10[c] = cell;
-        if (leaf_y) emit_cell(cell, 10, sdep, cpos, node4, ncount, r0);
+        l10[c] = TileCell{n, y, leaf_first[L], 0u, s.x, s.y, s.z, 0.0f};
     }
     lds_barrier();
     {
@@ -719,7 +678,9 @@ __global__ __launch_bounds__(256) void bh_tile_kernel(
     }
     for (uint32_t c = t; c < 341; c += 256) {
         const int d = c < 256 ? 9 : c < 320 ? 8 : c < 336 ? 7 : c < 340 ? 6 : 5;
-        emit_cell(up[c], d, sdep, cpos, node4, ncount, r0);
+        const TileCell *kids =
+            d == 9 ? l10 + 4 * c : up + tile_level_offset(d + 1) + 4 * (c - tile_level_offset(d));
+        emit_cell(up[c], d, sizes4(kids), sdep, cpos, node4, child, r0);
     }
     if (t == 0) {
         top[T] = up[340];
@@ -741,6 +702,7 @@ __global__ __launch_bounds__(256) void bh_tile_kernel(
                     : TileCell{0u, 0u, 0xffffffffu, 0u, 0.0f, 0.0f, 0.0f, 0.0f};
     }
     up[t] = reduce4(c4[0], c4[1], c4[2], c4[3]);
+    emit_cell(up[t], 4, sizes4(c4), sdep, cpos, node4, child, r0);
     lds_barrier();
     for (int d = 3; d >= 0; --d) {
         const uint32_t cnt = 1u << (2 * d);
@@ -750,20 +712,17 @@ __global__ __launch_bounds__(256) void bh_tile_kernel(
                                 up[oc + 4 * t + 3]);
         lds_barrier();
     }
-    for (uint32_t c = t; c < 341; c += 256) {
-        const int d = c < 256 ? 4 : c < 320 ? 3 : c < 336 ? 2 : c < 340 ? 1 : 0;
-        emit_cell(up[c], d, sdep, cpos, node4, ncount, r0);
+    if (t < 85) {  // depths 3..0
+        const uint32_t c = 256 + t;
+        const int d = c < 320 ? 3 : c < 336 ? 2 : c < 340 ? 1 : 0;
+        const TileCell *kids =
+            up + tile_level_offset(d + 6) + 4 * (c - tile_level_offset(d + 5));
+        emit_cell(up[c], d, sizes4(kids), sdep, cpos, node4, child, r0);
     }
 }
 
 // ---- 8. traversal + integrate ----------------------------------------------------
 
-// W = 64: one wave is one group, so the node index is wave-uniform and node
-// records arrive through scalar loads.  A particle node (radius 0) is accepted
-// by every lane, so a run of consecutive particle nodes (a leaf bucket) is
-// streamed as a plain direct sum without votes; cell nodes are voted on with
-// r2 = (dx*dx + dy*dy) + eps2 rounded exactly as the reference's shader, so
-// the visited and accepted node sets are the reference's.
 // The next build's sort input, written by the walk on the fixed domain: the
 // cell of the particle's new position (InitShader.comp:73-119), at the
 // particle's caller index o = perm[slot] (cells[o] = {cell, slot}), so the
@@ -781,138 +740,7 @@ __device__ __forceinline__ void write_next_key(const NextKeys &nk, uint32_t slot
     nk.cells[nk.perm[slot]] = make_uint2(c, slot);
 }
 
-// One group's walk (all four partials) and integrate.
-template <bool kDebugAccel, bool kStaged>
-__device__ __forceinline__ void walk_group(
-    uint32_t g, uint32_t total, float4 *stage, uint2 *queue, const uint32_t *__restrict__ sorted_src,
-    const float2 *__restrict__ pos, const float2 *__restrict__ vel,
-    const float4 *__restrict__ node4, const uint32_t *__restrict__ ncount,
-    float2 *__restrict__ pos_out,
-    float2 *__restrict__ vel_out, float2 *__restrict__ acc_dbg, uint32_t na, float eps2,
-    float theta2, float kv, float kp, unsigned long long *__restrict__ gvis,
-    unsigned long long *__restrict__ gacc, const NextKeys &nk, uint32_t *__restrict__ gcost = nullptr,
-    uint32_t *__restrict__ gchunk = nullptr, const uint8_t *__restrict__ heavy = nullptr) {
-    if (heavy && heavy[g]) return;  // walked by bh_traverse_heavy_kernel
-    const uint32_t lane = threadIdx.x & 63;
-    const uint32_t dst = g * 64 + lane;  // this particle's slot in the next order
-    const uint32_t src = sorted_src[dst];
-    const bool real = src < na;  // ForceShader.comp:80-92
-    float px = 0.0f, py = 0.0f;
-    if (real) {
-        const float2 p = pos[src];
-        px = p.x;
-        py = p.y;
-    }
-    const uint32_t nreal = (uint32_t)__popcll(__ballot(real));
-    Partials P;
-    unsigned long long vis = 0, acc = 0;
-    // start at the issue priority this group reached in the last step
-    const uint32_t prio0 = gchunk ? gchunk[g] / kPrioCarry : 0u;
-    uint32_t chunks = 0;
-    const uint32_t cost = walk_partials<kStaged>(0u, total, stage, queue, node4, ncount, px, py,
-                                                 real, nreal, eps2, theta2, 0xfu, P, vis, acc,
-                                                 kPrioStepSingle, prio0, &chunks);
-    if (gchunk && lane == 0) gchunk[g] = chunks;
-    if (lane == 0) {  // this group's visits and acceptances, summed on a dump
-        gvis[g] = vis;
-        gacc[g] = acc;
-    }
-    if (real) {
-        float ax, ay;
-        partial_sum(P, ax, ay);
-        const float2 v = vel[src];
-        const float nvx = v.x + ax * kv, nvy = v.y + ay * kv;
-        const float2 np = make_float2(px + (v.x + nvx) * kp, py + (v.y + nvy) * kp);
-        pos_out[dst] = np;
-        vel_out[dst] = make_float2(nvx, nvy);
-        if (nk.cells) write_next_key(nk, dst, np);
-        if (kDebugAccel) acc_dbg[dst] = make_float2(ax, ay);
-    }
-    if (gcost && lane == 0) gcost[g] = cost;
-}
-
-// The static traversal's heavy list from the last step's chunk counts
-// (gchunk): with q = floor(4 x chunks / mean) - 4 x split_x, the groups with
-// q >= qt go to plan[0, n_heavy) and are flagged in heavy[] (every other flag
-// is cleared), qt >= 0 the smallest threshold that lists at most `cap` groups
-// (the heaviest, whatever their index); q saturates at 63, and if more than
-// `cap` groups reach it the first `cap` of them by index are listed.  With no
-// counts yet (the first step) the list is empty.  One workgroup.
-__global__ __launch_bounds__(1024) void bh_heavy_plan_kernel(const uint32_t *__restrict__ gchunk,
-                                                             uint32_t groups, uint32_t split_x,
-                                                             uint32_t cap,
-                                                             uint32_t *__restrict__ plan,
-                                                             uint8_t *__restrict__ heavy,
-                                                             BhCounters *__restrict__ ctr) {
-    __shared__ uint32_t wsum[16];
-    __shared__ uint32_t hist[64];
-    __shared__ uint32_t qt_sh;
-    __shared__ unsigned long long total_sh;
-    const uint32_t t = threadIdx.x, lane = t & 63, wave = t >> 6;
-    unsigned long long part = 0;
-    for (uint32_t g = t; g < groups; g += 1024) part += gchunk[g];
-    if (t == 0) total_sh = 0;
-    if (t < 64) hist[t] = 0;
-    lds_barrier();
-    atomicAdd(&total_sh, part);
-    lds_barrier();
-    const unsigned long long total = total_sh;
-    const bool any = total > 0 && split_x > 0 && cap > 0;
-    auto quarter = [&](uint32_t g) -> uint32_t {  // q as above, 64 below the multiple
-        const unsigned long long q = 4ull * gchunk[g] * groups / total;
-        const unsigned long long lo = 4ull * split_x;
-        return q < lo ? 64u : (q - lo > 63ull ? 63u : (uint32_t)(q - lo));
-    };
-    if (any)
-        for (uint32_t g = t; g < groups; g += 1024) {
-            const uint32_t q = quarter(g);
-            if (q < 64) atomicAdd(&hist[q], 1u);
-        }
-    lds_barrier();
-    if (t == 0) {
-        uint32_t qt = 64;  // 64: nothing listed
-        if (any) {
-            uint32_t above = 0;  // groups with q >= k
-            for (int k = 63; k >= 0; --k) {
-                above += hist[k];
-                if (above > cap && k < 63) break;
-                qt = (uint32_t)k;
-            }
-        }
-        qt_sh = qt;
-    }
-    lds_barrier();
-    const uint32_t qt = qt_sh;
-    uint32_t carry = 0;  // heavy groups before this chunk of 1024
-    for (uint32_t base = 0; base < groups; base += 1024) {
-        const uint32_t g = base + t;
-        uint32_t q = 64;
-        if (g < groups && qt < 64) q = quarter(g);
-        const bool h = q < 64 && q >= qt;
-        uint32_t x = h ? 1u : 0u;
-#pragma unroll
-        for (int off = 1; off < 64; off <<= 1) {
-            const uint32_t y = __shfl_up(x, off, 64);
-            if (lane >= (uint32_t)off) x += y;
-        }
-        if (lane == 63) wsum[wave] = x;
-        lds_barrier();
-        uint32_t before = carry + (h ? x - 1u : x);
-        uint32_t chunk_total = 0;
-        for (uint32_t w = 0; w < 16; ++w) {
-            if (w < wave) before += wsum[w];
-            chunk_total += wsum[w];
-        }
-        const bool listed = h && before < cap;
-        if (listed) plan[before] = g;
-        if (g < groups) heavy[g] = listed ? 1u : 0u;
-        carry += chunk_total;
-        lds_barrier();  // wsum is rewritten by the next chunk
-    }
-    if (t == 0) ctr->n_heavy = min(carry, cap);
-}
-
-// The W = 32 launch order, by workgroup (four consecutive groups, the launch
+// The walk's launch order, by workgroup (four consecutive groups, the launch
 // unit): by last step's walk cost (the four groups' real-lane visits, gvis),
 // heaviest first, in buckets of a quarter of the mean (the last bucket holds
 // everything from 7.75x the mean up) and by index within a bucket, so the
@@ -1031,399 +859,60 @@ __global__ __launch_bounds__(1024) void bh_order_plan_kernel(
     }
 }
 
-// The heavy list, one workgroup of four waves per group, beside the main
-// traversal (which skips these groups): wave 0 decides -- the walk of
-// walk_partials, same votes and counts -- and queues the particle runs in the
-// workgroup's LDS, then all four waves sum the queued chunks, wave k those of
-// partial k, wave 0 also holding the accepted cells; at the end the shares
-// (split_share) are added in order by wave 0, which integrates.  The same
-// bits as one wave walking the group, with the summing spread over four SIMDs.
-template <bool kDebugAccel>
-__global__ __launch_bounds__(256) void bh_traverse_heavy_kernel(
-    const uint32_t *__restrict__ plan, const BhCounters *__restrict__ ctr,
+// One wave per part of a group: R * 8 of its W targets (walk_group), W / (8 R)
+// parts.  Part 0 counts the group's visits and acceptances.
+template <int W, int R, bool kWide, bool kDebugAccel>
+__global__ __launch_bounds__(256) void bh_walk_kernel(
     const uint32_t *__restrict__ sorted_src, const float2 *__restrict__ pos,
     const float2 *__restrict__ vel, const float4 *__restrict__ node4,
-    const uint32_t *__restrict__ ncount, float2 *__restrict__ pos_out,
-    float2 *__restrict__ vel_out, float2 *__restrict__ acc_dbg, uint32_t na, uint32_t cap,
-    float eps2, float theta2, float kv, float kp, unsigned long long *__restrict__ gvis,
-    unsigned long long *__restrict__ gacc, uint32_t *__restrict__ gchunk, NextKeys nk) {
-    __shared__ float4 stage[4][64];
-    __shared__ uint2 runq[kRunQueue];
-    __shared__ uint32_t qs[3];  // queued runs, their first chunk number, walk finished
-    __shared__ float2 share[4][64];
-    if (blockIdx.x >= ctr->n_heavy) return;  // the whole workgroup
-    const uint32_t lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const uint32_t g = __builtin_amdgcn_readfirstlane(plan[blockIdx.x]);
-    // node count is bounded by the node arrays; every step advances ind by at
-    // least one, so the walk ends
-    const uint32_t end = __builtin_amdgcn_readfirstlane(min(ctr->n_nodes, cap));
-    const uint32_t dst = g * 64 + lane;  // this particle's slot in the next order
-    const uint32_t src = sorted_src[dst];
-    const bool real = src < na;  // ForceShader.comp:80-92
-    float px = 0.0f, py = 0.0f;
-    if (real) {
-        const float2 p = pos[src];
-        px = p.x;
-        py = p.y;
-    }
-    const uint32_t nreal = (uint32_t)__popcll(__ballot(real));
-    __builtin_amdgcn_s_setprio(3);  // these groups are the launch's tail
-    Partials P;
-    unsigned long long vis = 0, acc = 0;
-    uint32_t ind = 0, chunk = 0;  // wave 0's walk
-    while (true) {
-        if (w == 0) {
-            const uint32_t qch = chunk;
-            uint32_t qn = 0;
-            while (ind < end && qn < kRunQueue) {
-                const float4 nd = node4[ind];
-                const uint32_t cnt = ncount[ind];
-                // one round trip per step, as in walk_partials
-                asm volatile("" ::"s"(nd.x), "s"(nd.y), "s"(nd.z), "s"(nd.w), "s"(cnt));
-                if (nd.w <= 0.0f) {  // a particle node: w = -(particle nodes left in its run)
-                    const uint32_t pr = (uint32_t)(-nd.w);
-                    const uint32_t n = __builtin_amdgcn_readfirstlane(min(max(pr, 1u), end - ind));
-                    vis += (unsigned long long)n * nreal;
-                    acc += (unsigned long long)n * nreal;
-                    if (lane == 0) runq[qn] = make_uint2(ind, n);
-                    ++qn;
-                    chunk += (n + 63u) >> 6;
-                    ind += n;
-                    continue;
-                }
-                const float dx = nd.x - px;
-                const float dy = nd.y - py;
-                const float r2 = (dx * dx + dy * dy) + eps2;  // ForceShader.comp:124-125
-                const bool ok = (nd.w <= r2 * theta2) || !real;
-                vis += nreal;
-                if (__ballot(ok) == ~0ull) {
-                    const float inv = __builtin_amdgcn_rsqf(r2);
-                    const float sc = (nd.z * inv) * (inv * inv);
-                    P.xc = __builtin_fmaf(dx, sc, P.xc);
-                    P.yc = __builtin_fmaf(dy, sc, P.yc);
-                    acc += nreal;
-                    ind = __builtin_amdgcn_readfirstlane(ind + max(cnt, 1u));
-                } else {
-                    ind = __builtin_amdgcn_readfirstlane(ind + 1u);
-                }
-            }
-            if (lane == 0) {
-                qs[0] = qn;
-                qs[1] = qch;
-                qs[2] = ind >= end ? 1u : 0u;
-            }
-        }
-        lds_barrier();
-        const uint32_t qn = __builtin_amdgcn_readfirstlane(qs[0]);
-        const uint32_t qch = __builtin_amdgcn_readfirstlane(qs[1]);
-        const uint32_t done = __builtin_amdgcn_readfirstlane(qs[2]);
-        if (qn) sum_run_queue(runq, qn, qch, stage[w], node4, px, py, eps2, 1u << w, P);
-        lds_barrier();  // runq and qs are rewritten by the next batch
-        if (done) break;
-    }
-    float ax, ay;
-    split_share(P, w, ax, ay);
-    share[w][lane] = make_float2(ax, ay);
-    lds_barrier();
-    __builtin_amdgcn_s_setprio(0);
-    if (w != 0) return;
-    if (lane == 0) {
-        gvis[g] = vis;
-        gacc[g] = acc;
-        gchunk[g] = chunk;
-    }
-    if (real) {
-        ax = ((share[0][lane].x + share[1][lane].x) + share[2][lane].x) + share[3][lane].x;
-        ay = ((share[0][lane].y + share[1][lane].y) + share[2][lane].y) + share[3][lane].y;
-        const float2 v = vel[src];
-        const float nvx = v.x + ax * kv, nvy = v.y + ay * kv;
-        const float2 np = make_float2(px + (v.x + nvx) * kp, py + (v.y + nvy) * kp);
-        pos_out[dst] = np;
-        vel_out[dst] = make_float2(nvx, nvy);
-        if (nk.cells) write_next_key(nk, dst, np);
-        if (kDebugAccel) acc_dbg[dst] = make_float2(ax, ay);
-    }
-}
-
-// Exclusive prefix of (cost + 1) over the groups, and the total at [groups]
-// (one workgroup).  The +1 makes the first step, with no costs yet, split the
-// groups evenly by count.
-__global__ __launch_bounds__(1024) void bh_cost_scan_kernel(const uint32_t *__restrict__ gcost,
-                                                            uint32_t groups,
-                                                            uint32_t *__restrict__ gpre) {
-    __shared__ uint32_t part[1024];
-    const uint32_t t = threadIdx.x;
-    const uint32_t per = (groups + 1023) / 1024;
-    const uint32_t lo = min(groups, t * per), hi = min(groups, lo + per);
-    uint32_t sum = 0;
-    for (uint32_t g = lo; g < hi; ++g) sum += gcost[g] + 1u;
-    part[t] = sum;
-    lds_barrier();
-    for (uint32_t off = 1; off < 1024; off <<= 1) {
-        const uint32_t v = t >= off ? part[t - off] : 0u;
-        lds_barrier();
-        part[t] += v;
-        lds_barrier();
-    }
-    uint32_t run = t ? part[t - 1] : 0u;
-    for (uint32_t g = lo; g < hi; ++g) {
-        gpre[g] = run;
-        run += gcost[g] + 1u;
-    }
-    if (t == 1023) gpre[groups] = part[1023];
-}
-
-// Cost-balanced traversal: workgroup k of P walks the contiguous groups whose
-// cost prefix starts in [k T / P, (k+1) T / P) (T = total cost of the last
-// walk), so every workgroup gets the same estimated work while neighbouring
-// groups -- which share their near field in the caches -- stay together.
-// Dense-core groups (last cost above `split_x` times the mean) would still
-// bound the launch alone on one wave (one walks ~5,400 particle nodes at the
-// 500k workload), so up to kSplitSlots of them per segment are split into
-// four units, one per partial of the canonical summation (walk_partials);
-// the four waves leave their partials in LDS and the last to finish adds them
-// in order and integrates -- the same bits as one wave walking the group.
-// The 16 waves take units from an LDS counter: split parts first, then the
-// segment's other groups.  Which wave walks what never changes a result.
-// Measured at 500k (two disks, theta 1), traversal ms: static one wave per
-// group 0.336, balanced 0.320, balanced with groups above 5x the mean split
-// 0.311-0.316 (per-CU work max/mean 1.45 -> 1.13).
-constexpr uint32_t kSplitSlots = 16;
-constexpr uint32_t kSegList = 1024;
-
-// kSplit = false: every unit is a whole group (one specialised walk in the
-// kernel, all four partials on one wave).
-template <bool kDebugAccel, bool kSplit>
-__global__ __launch_bounds__(1024) void bh_traverse_bal_kernel(
-    const uint32_t *__restrict__ sorted_src, const float2 *__restrict__ pos,
-    const float2 *__restrict__ vel, const float4 *__restrict__ node4,
-    const uint32_t *__restrict__ ncount,
-    BhCounters *__restrict__ ctr, float2 *__restrict__ pos_out, float2 *__restrict__ vel_out,
-    float2 *__restrict__ acc_dbg, uint32_t na, uint32_t cap, float eps2, float theta2,
-    float kv, float kp, const uint32_t *__restrict__ gpre, uint32_t *__restrict__ gcost,
-    uint32_t split_x, unsigned long long *__restrict__ gvis,
-    unsigned long long *__restrict__ gacc, NextKeys nk) {
-    __shared__ float4 stage[16][64];
-    __shared__ uint2 runq[16][kRunQueue];
-    __shared__ uint32_t seg[4];            // first group, end, next unit, list fill
-    __shared__ uint32_t list[kSegList];    // split groups first, then the others
-    __shared__ float2 hpart[kSplitSlots][4][64];
-    __shared__ uint32_t hdone[kSplitSlots];
-    const uint32_t lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const uint32_t groups = na / 64;
-    const unsigned long long total_cost = gpre[groups];
-    if (threadIdx.x == 0) {
-        const uint32_t tl = (uint32_t)(total_cost * blockIdx.x / gridDim.x);
-        const uint32_t th = (uint32_t)(total_cost * (blockIdx.x + 1) / gridDim.x);
-        auto first_at_least = [&](uint32_t v) -> uint32_t {  // first g with gpre[g] >= v
-            uint32_t a = 0, b = groups;
-            while (a < b) {
-                const uint32_t m = (a + b) >> 1;
-                if (gpre[m] < v) a = m + 1;
-                else b = m;
-            }
-            return a;
-        };
-        seg[0] = first_at_least(tl);
-        seg[1] = blockIdx.x + 1 == gridDim.x ? groups : first_at_least(th);
-        seg[2] = 0;
-        seg[3] = 0;
-    }
-    if (threadIdx.x < kSplitSlots) hdone[threadIdx.x] = 0;
-    lds_barrier();
-    const uint32_t lo = seg[0], hi = seg[1];
-    const uint32_t count = hi - lo, listed = min(count, kSegList);
-    const uint32_t i = threadIdx.x;  // one listed group per thread (kSegList == blockDim)
-    bool split = false;
-    if (kSplit && split_x && i < listed &&
-        (unsigned long long)(gcost[lo + i] + 1u) * groups > split_x * total_cost) {
-        const uint32_t slot = atomicAdd(&seg[3], 1u);
-        if (slot < kSplitSlots) {
-            list[slot] = lo + i;
-            split = true;
-        }
-    }
-    lds_barrier();
-    const uint32_t nsplit = min(seg[3], kSplitSlots);
-    lds_barrier();
-    if (threadIdx.x == 0) seg[3] = nsplit;
-    lds_barrier();
-    if (i < listed && !split) list[atomicAdd(&seg[3], 1u)] = lo + i;
-    lds_barrier();
-    const uint32_t total_nodes = __builtin_amdgcn_readfirstlane(min(ctr->n_nodes, cap));
-    const uint32_t units = 4 * nsplit + (count - nsplit);
-    while (true) {
-        uint32_t u = 0;
-        if (lane == 0) u = atomicAdd(&seg[2], 1u);
-        u = __builtin_amdgcn_readfirstlane(__shfl(u, 0, 64));
-        if (u >= units) break;
-        // a whole group (all partials), or one partial of a split group; one
-        // walk call for both keeps a single copy of the walk in the kernel
-        const bool whole = !kSplit || u >= 4 * nsplit;
-        const uint32_t v = u - 4 * nsplit + nsplit;
-        const uint32_t h = u >> 2, part = u & 3u;
-        uint32_t g;
-        if (whole) g = v < listed ? list[v] : lo + v;
-        else g = list[h];  // h < nsplit <= kSplitSlots
-        g = __builtin_amdgcn_readfirstlane(g);
-        const uint32_t parts = !kSplit ? 0xfu : whole ? 0xfu : 1u << part;
-        const uint32_t dst = g * 64 + lane;  // this particle's slot in the next order
-        const uint32_t src = sorted_src[dst];
-        const bool real = src < na;  // ForceShader.comp:80-92
-        float px = 0.0f, py = 0.0f;
-        if (real) {
-            const float2 p = pos[src];
-            px = p.x;
-            py = p.y;
-        }
-        const uint32_t nreal = (uint32_t)__popcll(__ballot(real));
-        Partials P;
-        unsigned long long vis = 0, acc = 0;
-        const uint32_t cost = walk_partials<true>(0u, total_nodes, stage[w], runq[w], node4, ncount,
-                                                  px, py, real, nreal, eps2, theta2, parts, P, vis,
-                                                  acc, kPrioStepSingle);
-        if (lane == 0 && (parts & 1u)) {  // the counting wave of the group
-            gvis[g] = vis;
-            gacc[g] = acc;
-        }
-        float ax = 0.0f, ay = 0.0f;
-        if (whole) {
-            partial_sum(P, ax, ay);
-            if (lane == 0) gcost[g] = cost;
-        } else {
-            split_share(P, part, ax, ay);
-            hpart[h][part][lane] = make_float2(ax, ay);
-            if (part == 0 && lane == 0) gcost[g] = cost;
-            __threadfence_block();
-            uint32_t done = 0;
-            if (lane == 0) done = atomicAdd(&hdone[h], 1u);
-            done = __builtin_amdgcn_readfirstlane(__shfl(done, 0, 64));
-            if (done != 3u) continue;
-            __threadfence_block();  // the last of the four adds the shares in order
-            ax = ((hpart[h][0][lane].x + hpart[h][1][lane].x) + hpart[h][2][lane].x) +
-                 hpart[h][3][lane].x;
-            ay = ((hpart[h][0][lane].y + hpart[h][1][lane].y) + hpart[h][2][lane].y) +
-                 hpart[h][3][lane].y;
-        }
-        if (real) {
-            const float2 vv = vel[src];
-            const float nvx = vv.x + ax * kv, nvy = vv.y + ay * kv;
-            const float2 np = make_float2(px + (vv.x + nvx) * kp, py + (vv.y + nvy) * kp);
-            pos_out[dst] = np;
-            vel_out[dst] = make_float2(nvx, nvy);
-            if (nk.cells) write_next_key(nk, dst, np);
-            if (kDebugAccel) acc_dbg[dst] = make_float2(ax, ay);
-        }
-    }
-}
-
-// kPersistent: waves take groups from a device counter until all na/64 are
-// done (every wave leaves once the counter passes the last group); otherwise
-// wave i walks group i.
-template <bool kDebugAccel, bool kStaged, bool kPersistent>
-__global__ __launch_bounds__(256) void bh_traverse64_kernel(
-    const uint32_t *__restrict__ sorted_src, const float2 *__restrict__ pos,
-    const float2 *__restrict__ vel, const float4 *__restrict__ node4,
-    const uint32_t *__restrict__ ncount,
-    BhCounters *__restrict__ ctr, float2 *__restrict__ pos_out, float2 *__restrict__ vel_out,
-    float2 *__restrict__ acc_dbg, uint32_t na, uint32_t cap, float eps2, float theta2,
-    float kv, float kp, unsigned long long *__restrict__ gvis,
-    unsigned long long *__restrict__ gacc, uint32_t *__restrict__ gchunk,
-    const uint8_t *__restrict__ heavy, uint32_t xcd, NextKeys nk,
-    const uint32_t *__restrict__ order) {
-    __shared__ float4 stage[kStaged ? 4 : 1][64];
-    __shared__ uint2 runq[kStaged ? 4 : 1][kStaged ? kRunQueue : 1];
-    const uint32_t lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const uint32_t groups = na / 64;
-    // node count is bounded by the node arrays; every iteration advances ind by
-    // at least one, so each walk ends
-    const uint32_t total = __builtin_amdgcn_readfirstlane(min(ctr->n_nodes, cap));
-    float4 *st = stage[kStaged ? w : 0];
-    uint2 *rq = runq[kStaged ? w : 0];
-    if (kPersistent) {
-        while (true) {
-            uint32_t g = 0;
-            if (lane == 0) g = atomicAdd(&ctr->next_group, 1u);
-            g = __builtin_amdgcn_readfirstlane(__shfl(g, 0, 64));
-            if (g >= groups) break;
-            walk_group<kDebugAccel, kStaged>(g, total, st, rq, sorted_src, pos, vel, node4,
-                                             ncount, pos_out, vel_out, acc_dbg, na, eps2,
-                                             theta2, kv, kp, gvis, gacc, nk, nullptr, gchunk);
-        }
-    } else {
-        const uint32_t b0 = xcd_block(blockIdx.x, gridDim.x, xcd);
-        // order: a permutation of the gridDim.x workgroups' units
-        const uint32_t b = order ? __builtin_amdgcn_readfirstlane(order[b0]) : b0;
-        const uint32_t g = b * 4 + w;
-        if (g >= groups) return;  // whole wave beyond the last group
-        walk_group<kDebugAccel, kStaged>(g, total, st, rq, sorted_src, pos, vel, node4, ncount,
-                                         pos_out, vel_out, acc_dbg, na, eps2, theta2, kv,
-                                         kp, gvis, gacc, nk, nullptr, gchunk, heavy);
-    }
-}
-
-// W = 32 (the published runs' subgroup width): one 32-particle group per
-// wave, particle slot g * 32 + l held by lanes l and l + 32, walked by the
-// staged W = 64 walk (both halves vote alike, so the 64-lane vote is the
-// group's: the same visits and acceptances); each half sums its part of every
-// chunk (sum_run_queue).  Per partial k the halves' sums are added, then the
-// acceleration is (((c + p0) + p1) + p2) + p3 as at W = 64.
-template <bool kDebugAccel>
-__global__ __launch_bounds__(256) void bh_traverse32_kernel(
-    const uint32_t *__restrict__ sorted_src, const float2 *__restrict__ pos,
-    const float2 *__restrict__ vel, const float4 *__restrict__ node4,
-    const uint32_t *__restrict__ ncount, BhCounters *__restrict__ ctr,
+    const uint4 *__restrict__ child, const BhCounters *__restrict__ ctr,
     float2 *__restrict__ pos_out, float2 *__restrict__ vel_out, float2 *__restrict__ acc_dbg,
     uint32_t na, uint32_t cap, float eps2, float theta2, float kv, float kp,
-    unsigned long long *__restrict__ gvis, unsigned long long *__restrict__ gacc, uint32_t xcd,
-    NextKeys nk, const uint32_t *__restrict__ order) {
-    __shared__ float4 stage[4][64];
-    __shared__ uint2 runq[4][kRunQueue];
+    unsigned long long *__restrict__ gvis, unsigned long long *__restrict__ gacc,
+    uint32_t *__restrict__ gchunk, uint32_t xcd, NextKeys nk,
+    const uint32_t *__restrict__ order) {
+    constexpr uint32_t kParts = W / (8 * R), kLanes = 8 / R;  // lanes that end with a target
+    __shared__ WalkShared sh[4];
     const uint32_t lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const uint32_t b0 = xcd_block(blockIdx.x, gridDim.x, xcd);
     // order: a permutation of the gridDim.x workgroups' units
     const uint32_t b = order ? __builtin_amdgcn_readfirstlane(order[b0]) : b0;
-    const uint32_t g = b * 4 + w;
-    if (g >= na / 32) return;  // whole wave beyond the last group
-    // node count is bounded by the node arrays; every step advances the walk
-    const uint32_t total = __builtin_amdgcn_readfirstlane(min(ctr->n_nodes, cap));
-    const uint32_t dst = g * 32 + (lane & 31u);  // this particle's slot in the next order
-    const uint32_t src = sorted_src[dst];
-    const bool real = src < na;  // ForceShader.comp:80-92
-    float px = 0.0f, py = 0.0f;
-    if (real) {
-        const float2 p = pos[src];
-        px = p.x;
-        py = p.y;
-    }
-    const uint32_t nreal = (uint32_t)__popcll(__ballot(real) & 0xffffffffull);
-    Partials P;
+    const uint32_t u = b * 4 + w, g = u / kParts, part = u % kParts;
+    if (g >= na / W) return;  // whole wave beyond the last group
+    const uint32_t vsrc = sorted_src[g * W + (lane & (W - 1u))];
+    const bool real = vsrc < na;  // ForceShader.comp:80-92
+    float2 vp = real ? pos[vsrc] : make_float2(0.0f, 0.0f);
+    const unsigned long long rb = __ballot(real);
+    const uint32_t nreal = (uint32_t)__popcll(W == 64 ? rb : rb & 0xffffffffull);
+    // the killed sort last, so the group's first particle is real if any is
+    vp.x = real ? vp.x : lane_value(vp.x, 0);
+    vp.y = real ? vp.y : lane_value(vp.y, 0);
+    // start at the issue priority this group reached in the last step (it
+    // gains at W = 64 and nothing at W = 32)
+    const uint32_t prio0 = W == 64 ? gchunk[g] / kPrioCarry : 0u;
+    const WalkTree tree{node4, child, 0u, uniform(min(ctr->n_nodes, cap)),
+                        uniform(ctr->n_in)};
+    float ax, ay;
     unsigned long long vis = 0, acc = 0;
-    (void)walk_partials<true, true>(0u, total, stage[w], runq[w], node4, ncount, px, py, real,
-                                    nreal, eps2, theta2, 0xfu, P, vis, acc, kPrioStepSingle);
-    P.x0 += __shfl_xor(P.x0, 32, 64);
-    P.y0 += __shfl_xor(P.y0, 32, 64);
-    P.x1 += __shfl_xor(P.x1, 32, 64);
-    P.y1 += __shfl_xor(P.y1, 32, 64);
-    P.x2 += __shfl_xor(P.x2, 32, 64);
-    P.y2 += __shfl_xor(P.y2, 32, 64);
-    P.x3 += __shfl_xor(P.x3, 32, 64);
-    P.y3 += __shfl_xor(P.y3, 32, 64);
-    if (lane == 0) {  // this group's visits and acceptances, summed on a dump
+    uint32_t chunks = 0;
+    walk_group<W, R, kWide>(tree, sh[w], part, vp.x, vp.y, nreal, eps2, theta2, kPrioStepSingle,
+                     prio0, ax, ay, vis, acc, chunks);
+    if (part == 0 && lane == 0) {  // summed on a dump
         gvis[g] = vis;
         gacc[g] = acc;
+        if (W == 64) gchunk[g] = chunks;
     }
-    if (real && lane < 32) {
-        float ax, ay;
-        partial_sum(P, ax, ay);
-        const float2 v = vel[src];
-        const float nvx = v.x + ax * kv, nvy = v.y + ay * kv;
-        const float2 np = make_float2(px + (v.x + nvx) * kp, py + (v.y + nvy) * kp);
-        pos_out[dst] = np;
-        vel_out[dst] = make_float2(nvx, nvy);
-        if (nk.cells) write_next_key(nk, dst, np);
-        if (kDebugAccel) acc_dbg[dst] = make_float2(ax, ay);
-    }
+    const uint32_t dst = g * W + part * (8 * R) + lane / kLanes;  // slot in the next order
+    const uint32_t src = sorted_src[dst];
+    if (lane % kLanes != 0u || src >= na) return;
+    const float2 p = pos[src], v = vel[src];
+    // ForceShader.comp:145-150
+    const float nvx = v.x + ax * kv, nvy = v.y + ay * kv;
+    const float2 np = make_float2(p.x + (v.x + nvx) * kp, p.y + (v.y + nvy) * kp);
+    pos_out[dst] = np;
+    vel_out[dst] = make_float2(nvx, nvy);
+    if (nk.cells) write_next_key(nk, dst, np);
+    if (kDebugAccel) acc_dbg[dst] = make_float2(ax, ay);
 }
 
 // 30-bit Morton codes (15 bits per axis) of the same normalised coordinate;
@@ -1471,19 +960,17 @@ hipError_t bh_alloc(BhBuffers *b, size_t na, uint32_t bits) {
     // four passes of tile words and group words
     GSIM_ALLOC(b->status, 4 * 256 * (b->sort_blocks + (b->sort_blocks + kLookGroup - 1) / kLookGroup));
     GSIM_ALLOC(b->digit_total, 2 * kDigitCopies * 1024);
-    GSIM_ALLOC(b->breaker, b->cap);
     GSIM_ALLOC(b->block_cells, b->prep_blocks);
     GSIM_ALLOC(b->block_leaves, b->prep_blocks);
     GSIM_ALLOC(b->sdep, na + 1);
     GSIM_ALLOC(b->cpos, na);
-    GSIM_ALLOC(b->prod, na);
     GSIM_ALLOC(b->leaf_first, na + 1);
     GSIM_ALLOC(b->leaf_key, na);
     GSIM_ALLOC(b->leaf_sum, na);
     GSIM_ALLOC(b->tile_range, 2 * kTiles);
     GSIM_ALLOC(b->top, kTiles);
     GSIM_ALLOC(b->node4, b->cap);
-    GSIM_ALLOC(b->ncount, b->cap);
+    GSIM_ALLOC(b->child, b->cap);
     if (bits == kDeepBits) {
         GSIM_ALLOC(b->nsum, b->cap);
         GSIM_ALLOC(b->gran_first, na + 1);
@@ -1495,22 +982,17 @@ hipError_t bh_alloc(BhBuffers *b, size_t na, uint32_t bits) {
     GSIM_ALLOC(b->ctr, 1);
     GSIM_ALLOC(b->box, 4);
     GSIM_ALLOC(b->box_part, kBoxParts);
-    GSIM_ALLOC(b->gcost, na / 64);
     GSIM_ALLOC(b->gchunk, na / 64 + 1);
-    GSIM_ALLOC(b->plan, kMaxHeavy);
     GSIM_ALLOC(b->order, na / 128 + 1);
-    GSIM_ALLOC(b->heavy, na / 64 + 1);
     GSIM_ALLOC(b->gvis, na / 32 + 1);  // one slot per group of W = 32 or 64
     GSIM_ALLOC(b->gacc, na / 32 + 1);
-    GSIM_ALLOC(b->gpre, na / 64 + 1);
 #undef GSIM_ALLOC
     if (e == hipSuccess) e = hipMemset(b->ctr, 0, sizeof(BhCounters));
     if (e == hipSuccess) e = hipMemset(b->digit_total, 0, sizeof(uint32_t) * 2 * kDigitCopies * 1024);
-    if (e == hipSuccess) e = hipMemset(b->gcost, 0, sizeof(uint32_t) * (na / 64));
     if (e == hipSuccess) e = hipMemset(b->gchunk, 0, sizeof(uint32_t) * (na / 64 + 1));
     if (e == hipSuccess) e = hipMemset(b->gvis, 0, sizeof(unsigned long long) * (na / 32 + 1));
     if (e == hipSuccess) e = hipMemset(b->gacc, 0, sizeof(unsigned long long) * (na / 32 + 1));
-    if (e == hipSuccess) e = hipMemset(b->ncount, 0, sizeof(uint32_t) * b->cap);
+    if (e == hipSuccess) e = hipMemset(b->child, 0, sizeof(uint4) * b->cap);
     if (e == hipSuccess) e = hipMemset(b->node4, 0, sizeof(float4) * b->cap);
     return e;
 }
@@ -1521,10 +1003,10 @@ void bh_free(BhBuffers *b) {
         (void)hipFree(b->idx[k]);
         (void)hipFree(b->cells[k]);
     }
-    void *ptrs[] = {b->status, b->digit_total, b->breaker, b->block_cells, b->block_leaves, b->sdep, b->cpos, b->prod,
-                    b->leaf_first, b->leaf_key, b->leaf_sum, b->tile_range, b->top,
-                    b->node4, b->ncount, b->nsum, b->gran_first, b->gran_key, b->gran_y,
-                    b->block_gran, b->sorted_src, b->ctr, b->gcost, b->gchunk, b->plan, b->order, b->heavy, b->gpre, b->gvis, b->gacc, b->box,
+    void *ptrs[] = {b->status, b->digit_total, b->block_cells, b->block_leaves, b->sdep, b->cpos,
+                    b->leaf_first, b->leaf_key, b->leaf_sum, b->tile_range, b->top, b->node4,
+                    b->child, b->nsum, b->gran_first, b->gran_key, b->gran_y, b->block_gran,
+                    b->sorted_src, b->ctr, b->gchunk, b->order, b->gvis, b->gacc, b->box,
                     b->box_part};
     for (void *p : ptrs) (void)hipFree(p);
     *b = BhBuffers{};
@@ -1596,36 +1078,44 @@ hipError_t bh_launch_build(gsim_sim *s, const float2 *pos, const float *mass,
     bh_emit_kernel<<<pb, 256, 0, s->stream>>>(sk, si, pos, mass, vel, perm_in, pos_out, vel_out,
                                               mass_out, perm_out, nk.cells, na, bits,
                                               b.block_cells,
-                                              b.block_leaves, b.sdep, b.cpos, b.prod,
-                                              b.leaf_first, b.leaf_key, b.node4, b.ncount,
-                                              b.sorted_src, b.breaker, b.ctr,
+                                              b.block_leaves, b.sdep, b.cpos,
+                                              b.leaf_first, b.leaf_key, b.node4,
+                                              b.sorted_src, b.ctr,
                                               deep ? b.block_gran : nullptr,
                                               deep ? b.gran_first : nullptr, b.gran_key);
     const uint32_t lb = pb < kLeafBlocks ? pb : kLeafBlocks;
-    bh_leaf_kernel<<<lb, 256, 0, s->stream>>>(b.leaf_first, b.leaf_key, b.prod, sk, na, bits,
-                                              b.cpos, b.breaker, b.ctr, b.leaf_sum, b.tile_range,
-                                              b.sdep, b.node4, b.ncount,
+    bh_leaf_kernel<<<lb, 256, 0, s->stream>>>(b.leaf_first, b.leaf_key, b.cpos, b.ctr, bits,
+                                              b.leaf_sum, b.tile_range, b.node4, b.child,
                                               deep ? b.nsum : nullptr, box, &b.ctr->tiles_busy);
     if (deep) {
         // sparse levels below depth 10, then depth-10 records for the dense path
         for (int d = (int)kDeepBits - 1; d > (int)kTreeDepth; --d)
-            bh_level_kernel<<<pb, 256, 0, s->stream>>>(sk, b.sdep, b.cpos, b.prod, b.ctr, b.node4,
-                                                       b.ncount, b.nsum, d, box);
-        bh_gran_kernel<<<pb, 256, 0, s->stream>>>(sk, b.sdep, b.cpos, b.prod, b.ctr, b.ncount,
+            bh_level_kernel<<<pb, 256, 0, s->stream>>>(sk, b.sdep, b.cpos, b.ctr, b.node4,
+                                                       b.child, b.nsum, d, box);
+        bh_gran_kernel<<<pb, 256, 0, s->stream>>>(sk, b.sdep, b.cpos, b.ctr, b.node4, b.child,
                                                   b.nsum, b.gran_first, b.gran_key, b.leaf_sum,
-                                                  b.gran_y, b.tile_range, &b.ctr->tiles_busy);
+                                                  b.gran_y, b.tile_range, &b.ctr->tiles_busy,
+                                                  box);
         bh_tile_kernel<<<kTiles, 256, 0, s->stream>>>(b.tile_range, b.gran_first, b.gran_key,
                                                       b.leaf_sum, b.sdep, b.cpos, b.node4,
-                                                      b.ncount, b.top, box, b.gran_y, b.ctr);
+                                                      b.child, b.top, box, b.gran_y, b.ctr);
     } else {
         bh_tile_kernel<<<kTiles, 256, 0, s->stream>>>(b.tile_range, b.leaf_first, b.leaf_key,
                                                       b.leaf_sum, b.sdep, b.cpos, b.node4,
-                                                      b.ncount, b.top, box, nullptr, b.ctr);
+                                                      b.child, b.top, box, nullptr, b.ctr);
     }
     return hipGetLastError();
 }
 
-// The static walk's workgroup order (null: index order), re-planned from the
+uint32_t walk_parts(const gsim_sim *s) {
+    const uint32_t groups = (uint32_t)(s->na / s->W), most = s->W / 8;
+    if (groups > kWalkSplitGroups) return 1;
+    uint32_t parts = 2;
+    while (parts < most && 2 * parts * groups <= kWalkFillWaves) parts *= 2;
+    return parts;
+}
+
+// The walk's workgroup order (null: index order), re-planned from the
 // last walk's costs every kOrderReplan steps (costs change slowly) and on
 // every trial step, on the walk's own stream: a plan on the side stream
 // beside the build measured slower (the cross-stream fork and join cost more
@@ -1644,97 +1134,36 @@ hipError_t bh_launch_traverse(gsim_sim *s, const float2 *pos, const float2 *vel,
                               float2 *pos_out, float2 *vel_out, const uint32_t *perm_out) {
     BhBuffers &b = s->bh;
     const uint32_t na = (uint32_t)s->na;
-    const uint32_t grid = (na + 255) / 256;
     const NextKeys nk = next_keys(s, perm_out);
     // the next build reads the cells this walk writes
     b.walk_keys = nk.cells != nullptr;
     if (b.walk_keys) b.kin ^= 1;
     const bool dbg = (s->debug_flags & GSIM_DEBUG_ACCEL) != 0;
     float2 *acc = dbg ? s->accel : nullptr;
+    const uint32_t groups = na / s->W, parts = walk_parts(s);
+    const uint32_t grid = (groups * parts + 3) / 4;
+    const uint32_t *order = parts == 1 ? launch_order(s, groups) : nullptr;
+    const bool wide = b.cap >= kNarrowNodes;
+#define GSIM_WALK(W, R)                                                                        \
+    do {                                                                                       \
+        auto *k = dbg ? (wide ? bh_walk_kernel<W, R, true, true> : bh_walk_kernel<W, R, false, true>) \
+                      : (wide ? bh_walk_kernel<W, R, true, false> : bh_walk_kernel<W, R, false, false>); \
+        k<<<grid, 256, 0, s->stream>>>(b.sorted_src, pos, vel, b.node4, b.child, b.ctr,        \
+                                       pos_out, vel_out, acc, na, (uint32_t)b.cap, s->eps2,    \
+                                       s->theta2, s->kv, s->kp, b.gvis, b.gacc, b.gchunk,      \
+                                       s->xcd_order, nk, order);                               \
+    } while (0)
     if (s->W == 64) {
-        const uint32_t groups = na / 64;
-        if (s->trav_mode & 4u) {
-            bh_cost_scan_kernel<<<1, 1024, 0, s->stream>>>(b.gcost, groups, b.gpre);
-            const uint32_t P = s->trav_segments;
-#define GSIM_BAL(D, S)                                                                          \
-    bh_traverse_bal_kernel<D, S><<<P, 1024, 0, s->stream>>>(                                   \
-        b.sorted_src, pos, vel, b.node4, b.ncount, b.ctr, pos_out, vel_out, acc, na,          \
-        (uint32_t)b.cap, s->eps2, s->theta2, s->kv, s->kp, b.gpre, b.gcost, s->trav_split,   \
-        b.gvis, b.gacc, nk)
-            if (dbg) { if (s->trav_split) GSIM_BAL(true, true); else GSIM_BAL(true, false); }
-            else { if (s->trav_split) GSIM_BAL(false, true); else GSIM_BAL(false, false); }
-#undef GSIM_BAL
-            return hipGetLastError();
-        }
-        const bool persistent = (s->trav_mode & 1u) != 0, staged = (s->trav_mode & 2u) != 0;
-        uint32_t g = grid;
-        // static staged launch with more groups than the GPU holds at once:
-        // last step's heaviest groups go to four-wave workgroups on the side
-        // stream (forked after the plan, joined back below), beside the main
-        // launch, whose later rounds leave them room.  When every group is
-        // resident from the start the side workgroups only find room at the
-        // end and lengthen the launch (two disks at 500k: +5%), so they stay
-        // off there.
-        // The heavy list and the heaviest-first launch order (below) answer
-        // the same tail; with the order active the list only lengthened the
-        // walk (1M, W = 64: two disks 0.91 -> 0.95, galaxy collision 1.21 ->
-        // 1.23 ms per step), so it runs with index order only.
-        const uint8_t *heavy = nullptr;
-        if (!persistent && staged && s->trav_split && s->side && groups > kHeavyMinGroups &&
-            !s->trav_order) {
-            bh_heavy_plan_kernel<<<1, 1024, 0, s->stream>>>(b.gchunk, groups, s->trav_split,
-                                                            kMaxHeavy, b.plan, b.heavy, b.ctr);
-            hipError_t e = hipEventRecord(s->ev_fork, s->stream);
-            if (e == hipSuccess) e = hipStreamWaitEvent(s->side, s->ev_fork, 0);
-            if (e != hipSuccess) return e;
-#define GSIM_HEAVY(D)                                                                        \
-    bh_traverse_heavy_kernel<D><<<kMaxHeavy, 256, 0, s->side>>>(                              \
-        b.plan, b.ctr, b.sorted_src, pos, vel, b.node4, b.ncount, pos_out, vel_out, acc, na, \
-        (uint32_t)b.cap, s->eps2, s->theta2, s->kv, s->kp, b.gvis, b.gacc, b.gchunk, nk)
-            if (dbg) GSIM_HEAVY(true);
-            else GSIM_HEAVY(false);
-#undef GSIM_HEAVY
-            heavy = b.heavy;
-        }
-        const uint32_t *order = persistent ? nullptr : launch_order(s, groups);
-        if (persistent) {
-            // waves_per_simd waves on each of the 1024 SIMDs, at most one per group
-            uint32_t waves = 1024u * s->trav_waves_per_simd;
-            if (waves > groups) waves = groups;
-            g = (waves + 3) / 4;
-        }
-#define GSIM_TRAV(D, S, P)                                                                 \
-    bh_traverse64_kernel<D, S, P><<<g, 256, 0, s->stream>>>(                               \
-        b.sorted_src, pos, vel, b.node4, b.ncount, b.ctr, pos_out, vel_out, acc, na, \
-        (uint32_t)b.cap, s->eps2, s->theta2, s->kv, s->kp, b.gvis, b.gacc, b.gchunk, heavy, \
-        s->xcd_order, nk, order)
-        if (dbg) {
-            if (persistent) { if (staged) GSIM_TRAV(true, true, true); else GSIM_TRAV(true, false, true); }
-            else { if (staged) GSIM_TRAV(true, true, false); else GSIM_TRAV(true, false, false); }
-        } else {
-            if (persistent) { if (staged) GSIM_TRAV(false, true, true); else GSIM_TRAV(false, false, true); }
-            else { if (staged) GSIM_TRAV(false, true, false); else GSIM_TRAV(false, false, false); }
-        }
-#undef GSIM_TRAV
-        if (heavy) {  // the next launch on the stream waits for the heavy list too
-            hipError_t e = hipEventRecord(s->ev_join, s->side);
-            if (e == hipSuccess) e = hipStreamWaitEvent(s->stream, s->ev_join, 0);
-            if (e != hipSuccess) return e;
-        }
+        if (parts == 1) GSIM_WALK(64, 8);
+        else if (parts == 2) GSIM_WALK(64, 4);
+        else if (parts == 4) GSIM_WALK(64, 2);
+        else GSIM_WALK(64, 1);
     } else {
-        const uint32_t g32 = (na / 32 + 3) / 4;  // four 32-particle groups per workgroup
-        const uint32_t *order = launch_order(s, na / 32);
-        if (dbg)
-            bh_traverse32_kernel<true><<<g32, 256, 0, s->stream>>>(
-                b.sorted_src, pos, vel, b.node4, b.ncount, b.ctr, pos_out, vel_out, acc, na,
-                (uint32_t)b.cap, s->eps2, s->theta2, s->kv, s->kp, b.gvis, b.gacc, s->xcd_order,
-                nk, order);
-        else
-            bh_traverse32_kernel<false><<<g32, 256, 0, s->stream>>>(
-                b.sorted_src, pos, vel, b.node4, b.ncount, b.ctr, pos_out, vel_out, acc, na,
-                (uint32_t)b.cap, s->eps2, s->theta2, s->kv, s->kp, b.gvis, b.gacc, s->xcd_order,
-                nk, order);
+        if (parts == 1) GSIM_WALK(32, 4);
+        else if (parts == 2) GSIM_WALK(32, 2);
+        else GSIM_WALK(32, 1);
     }
+#undef GSIM_WALK
     return hipGetLastError();
 }
 

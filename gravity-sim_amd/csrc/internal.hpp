@@ -9,11 +9,9 @@
 //                   partials float2[(sum over groups of B - 16g)*64]
 //   Barnes-Hut      cells uint2[Na] x2 (the sort's input {cell, slot} by particle
 //                   index), keys/idx u32[Na] x2, radix histograms, sdep i8[Na+1],
-//                   cpos u32[Na], prod float4[Na], leaf records,
-//                   tile results,
-//                   breaker u32[cap], node4 float4[cap] {x, y, mass, radius}
-//                   (a particle node's radius word holds minus its run length),
-//                   ncount u32[cap],
+//                   cpos u32[Na], leaf records, tile results,
+//                   node4 float4[cap] {x, y, mass, radius} (a particle's radius
+//                   is 0), child uint4[cap] the cells' children,
 //                   sorted_src u32[Na], device counters
 #pragma once
 
@@ -50,10 +48,8 @@ struct BhCounters {
     uint32_t n_cells;   // cell nodes (cells holding >= 2 particles)
     uint32_t n_nodes;   // n_in + n_cells = counts[0]
     uint32_t n_leaves;  // occupied leaf cells (depth 10, or 15 with 15-bit leaves)
-    uint32_t next_group;         // work counter of the persistent traversal
     uint32_t n_gran;             // 15-bit leaves: occupied depth-10 cells
     uint32_t sort_stall;         // look-back waits that hit their bound (never expected)
-    uint32_t n_heavy;            // static traversal: groups on the heavy list this step
     uint32_t tiles_busy;         // occupied depth-5 tiles
     uint32_t tiles_done;         // occupied tiles reduced (the last one reduces the top)
 };
@@ -73,16 +69,24 @@ constexpr uint32_t kLookGroup = 16;
 // fewer workgroups add into each word; a pass sums the copies.
 constexpr uint32_t kDigitCopies = 8;
 
-// Particle runs a walking wave queues in its LDS before summing them (the
-// staged walk's run stack; the batch may use fewer, BatchTune::run_queue).
+// A walk of at most kWalkSplitGroups groups (two waves a SIMD) takes two waves
+// a group, and more up to kWalkFillWaves waves.  Each wave repeats the group's
+// decisions, so more waves only pay while SIMDs are idle: 60,000 particles at
+// W = 64 (938 groups) took 31 us with 2 waves a group, 36 with 4 and 54 with
+// 8; 20,000 (313 groups) 26 with 4, 29 with 8; 120,000 with a dense core
+// (1,876 groups) 108 with 1, 85 with 2, 96 with 4.
+constexpr uint32_t kWalkSplitGroups = 2048;
+constexpr uint32_t kWalkFillWaves = 2048;
+
+// Node arrays of fewer records than this are addressed by 32-bit byte offsets.
+constexpr size_t kNarrowNodes = (size_t)1 << 28;
+
+// The largest value of BatchTune::run_queue.
 constexpr uint32_t kRunQueue = 64;
 
-// Static traversal: at most this many groups per step go to the heavy list
-// (walked by four waves each beside the main launch).
-constexpr uint32_t kMaxHeavy = 512;
-// ... and only when the launch has more groups than the GPU holds at once
-// (256 CUs x 4 SIMDs x 8 waves of the static traversal).
-constexpr uint32_t kHeavyMinGroups = 8192;
+// child[slot] of a cell node: the subtree sizes of its four quadrants (0:
+// empty, 1: one particle), or for a leaf cell {particles, 0, 0, kLeafMark}.
+constexpr uint32_t kLeafMark = 0xffffffffu;
 
 struct TileCell {  // one cell of the dense tile/top reduction
     uint32_t n, y, f, pad;
@@ -103,19 +107,17 @@ struct BhBuffers {
     uint32_t *status = nullptr;      // [4 * sort_blocks * 256] look-back words per pass
     uint32_t *digit_total = nullptr; // [2][kDigitCopies][4 * 256] per-pass digit totals, two halves
     uint32_t parity = 0;             // the half the next build counts into
-    uint32_t *breaker = nullptr;     // [cap] sorted position where cell node #o starts
     uint32_t *block_cells = nullptr; // [prep_blocks] then scanned
     uint32_t *block_leaves = nullptr;
     int8_t *sdep = nullptr;          // [Na] shared depth with the previous sorted key
     uint32_t *cpos = nullptr;        // [Na] cell nodes starting before sorted position k
-    float4 *prod = nullptr;          // [Na] (m*x, m*y, m, -) in sorted order
     uint32_t *leaf_first = nullptr;  // [Na+1]
     uint32_t *leaf_key = nullptr;    // [Na]
     float4 *leaf_sum = nullptr;      // [Na] (sx, sy, sm, n as bits)
     uint32_t *tile_range = nullptr;  // [2*kTiles] first/end leaf of each depth-5 tile
     TileCell *top = nullptr;         // [kTiles]
     float4 *node4 = nullptr;         // [cap]
-    uint32_t *ncount = nullptr;      // [cap]
+    uint4 *child = nullptr;          // [cap] a cell's children (kLeafMark)
     float4 *nsum = nullptr;          // [cap] 15-bit leaves only: a cell node's
                                      // (sx, sy, sm, particle count as bits)
     // 15-bit leaves only: the occupied depth-10 cells ("granules") that feed
@@ -128,15 +130,9 @@ struct BhBuffers {
     uint32_t *sorted_src = nullptr;  // [Na]
     BhCounters *ctr = nullptr;
     uint32_t sorted_slot = 0;        // which keys/idx buffer holds the sorted result
-    // balanced traversal: each group's walk cost from the previous step and
-    // the exclusive prefix of (cost + 1) that cuts the groups into segments
-    uint32_t *gcost = nullptr;       // [Na/64], zero before the first walk
     uint32_t *gchunk = nullptr;      // [Na/64 + 1] chunks each group summed last step (issue priority)
-    uint32_t *plan = nullptr;        // [kMaxHeavy] the heavy list
-    uint8_t *heavy = nullptr;        // [Na/64 + 1] 1: on the heavy list this step
     uint32_t *order = nullptr;       // [Na/128] static walk's launch order of the workgroups
     bool order_valid = false;        // order holds a plan (a permutation of the units)
-    uint32_t *gpre = nullptr;        // [Na/64 + 1]
     // each group's real-lane node visits and acceptances in the last walk,
     // written by the group's wave and summed on a dump (one same-address
     // atomic per wave cost ~5% of the walk)
@@ -188,20 +184,11 @@ struct gsim_sim {
     gsim_params params{};
     int device = 0;
     hipStream_t stream = nullptr;
-    hipStream_t side = nullptr;        // Barnes-Hut: the heavy list's walks, beside the main one
-    hipEvent_t ev_fork = nullptr, ev_join = nullptr;
     size_t n = 0, na = 0;
     // FP32 constants squared/multiplied on the host as the reference does
     // (DirectSimulation.cpp:179, BarnesHutSimulation.cpp:575-578).
     float eps2 = 0, theta2 = 0, dt = 0, kv = 0, kp = 0;
     uint32_t W = 64;
-    uint32_t trav_waves_per_simd = 8;  // persistent traversal width
-    uint32_t trav_mode = 2;            // bit 0 persistent, bit 1 LDS-staged runs,
-                                       // bit 2 cost-balanced segments (staged);
-                                       // default 2: one wave per group, staged
-    uint32_t trav_segments = 512;      // balanced traversal: workgroups (2 per CU)
-    uint32_t trav_split = 2;           // static: heavy list above this x mean chunk count;
-                                       // balanced: split above this x mean cost (0: never)
     uint32_t bh_box = 0;               // adaptive bounding box instead of the fixed domain
     // Static walk's launch order: order_mode 0 index, 1 heaviest first (by last
     // step's visits), 2 auto: a trial of kOrderTrial steps alternating the
@@ -214,7 +201,7 @@ struct gsim_sim {
     uint32_t order_rec = 0;            // trial steps recorded
     bool order_wait = false;           // the trial's events are outstanding
     uint64_t order_next = 1;           // first step of the next trial
-    uint32_t xcd_order = 1;            // static traversals: each XCD takes runs of this
+    uint32_t xcd_order = 1;            // the walk: each XCD takes runs of this
                                        // many consecutive workgroups (xcd_block; <= 1:
                                        // round-robin)
     uint32_t ds_rcp = 0;               // direct sum: 1/r2 from the transcendental unit
@@ -266,9 +253,12 @@ hipError_t bh_launch_build(gsim_sim *s, const float2 *pos, const float *mass,
 hipError_t bh_launch_traverse(gsim_sim *s, const float2 *pos, const float2 *vel,
                               float2 *pos_out, float2 *vel_out, const uint32_t *perm_out);
 hipError_t bh_launch_morton30(gsim_sim *s, const float2 *pos, uint32_t *out);
-// Whether the handle's walk is a static launch of four-group workgroups,
-// which GSIM_TUNE_BH_ORDER can reorder (W = 32, or W = 64 neither persistent
-// nor balanced).
-inline bool order_launch(const gsim_sim *s) { return s->W == 32 || (s->trav_mode & 5u) == 0; }
+// Waves per vote group of the handle's walk (1, 2, 4 or 8 at W = 64; at most
+// 4 at W = 32), each taking its share of the group's targets: as many as keep
+// the launch within the wave slots of the GPU.
+uint32_t walk_parts(const gsim_sim *s);
+// Whether GSIM_TUNE_BH_ORDER can reorder the walk's workgroups: with one wave
+// per group, four groups each.
+inline bool order_launch(const gsim_sim *s) { return walk_parts(s) == 1; }
 
 }  // namespace gsim

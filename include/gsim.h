@@ -162,28 +162,20 @@ gsim_status gsim_set_ds_shape(gsim_sim *sim, uint32_t targets_per_lane,
 /* Launch tuning that never changes results beyond the documented tolerance
  * (visit/accept counts and trees are unaffected by every knob), and two
  * opt-in options beyond the reference, GSIM_TUNE_BH_ADAPTIVE_BOX and
- * GSIM_TUNE_BH_LEAF_BITS.  The traversal launch knobs (WAVES_PER_SIMD,
- * TRAVERSAL, SEGMENTS, SPLIT) shape the W = 64 launches only: on a Barnes-Hut
- * handle of group width 32 they return GSIM_ERROR_INVALID_ARGUMENT. */
+ * GSIM_TUNE_BH_LEAF_BITS.  WAVES_PER_SIMD, TRAVERSAL, SEGMENTS and SPLIT are
+ * checked and have no further effect: the walk has one launch, shaped by the
+ * number of groups.  On a Barnes-Hut handle of group width 32 they return
+ * GSIM_ERROR_INVALID_ARGUMENT. */
 typedef enum gsim_tuning {
     GSIM_TUNE_DS_RCP = 1,             /* 0/1: 1/r^2 from v_rcp instead of a multiply  */
-    GSIM_TUNE_BH_WAVES_PER_SIMD = 2,  /* 1..8: persistent traversal width             */
-    GSIM_TUNE_BH_TRAVERSAL = 3,       /* bit 0 persistent groups, bit 1 LDS-staged runs
-                                         (2, one wave per group with staged runs, is the
-                                         default); 6 = cost-balanced contiguous
-                                         segments, with dense-core groups split          */
+    GSIM_TUNE_BH_WAVES_PER_SIMD = 2,  /* 1..8; no effect                               */
+    GSIM_TUNE_BH_TRAVERSAL = 3,       /* 0..3 or 6; no effect                          */
     GSIM_TUNE_DS_SYMMETRIC = 4,       /* 0/1: each pair once (Newton's third law); the
                                          default for 16,384 <= Na <= 262,144           */
     GSIM_TUNE_DS_SYM_COLS = 5,        /* symmetric kernel: 1 or 2 column blocks per
                                          wave, 0 = by size                              */
-    GSIM_TUNE_BH_SEGMENTS = 6,        /* balanced traversal: workgroups of 16 waves
-                                         (default 512, two per CU)                      */
-    GSIM_TUNE_BH_SPLIT = 7,           /* groups whose last walk reaches this multiple
-                                         of the mean are walked by 4 waves: in the
-                                         default traversal in index order (chunk
-                                         count, the heaviest 512 at most, beside the
-                                         main launch) and the balanced one (cost);
-                                         0 = never; default 2                          */
+    GSIM_TUNE_BH_SEGMENTS = 6,        /* 1..65536; no effect                           */
+    GSIM_TUNE_BH_SPLIT = 7,           /* 0..1000; no effect                            */
     GSIM_TUNE_BH_ADAPTIVE_BOX = 8,    /* 0/1, beyond the reference and off by default:
                                          each step's tree spans the bounding square of
                                          the particles (centre c, half-size h = extent
@@ -201,23 +193,20 @@ typedef enum gsim_tuning {
                                          the reference's.  Combines with the adaptive
                                          box.  Reallocates the node arrays (synchronous;
                                          they grow by up to 2.5 x Na entries).          */
-    GSIM_TUNE_BH_XCD_ORDER = 10,      /* 0..4096: the static traversals hand each of
-                                         the 8 XCDs (each with its own L2) runs of this
-                                         many consecutive workgroups instead of every
+    GSIM_TUNE_BH_XCD_ORDER = 10,      /* 0..4096: the walk hands each of the 8 XCDs
+                                         (each with its own L2) runs of this many
+                                         consecutive workgroups instead of every
                                          eighth one, so spatially adjacent groups share
                                          an L2 (one contiguous range per XCD once the
                                          runs reach an eighth of the launch); 0 or 1 =
-                                         round-robin, the default: measured at 500k,
-                                         runs of 2-32 change nothing and contiguous
-                                         ranges are 16% slower.  W = 32 and 64.         */
-    GSIM_TUNE_BH_ORDER = 11           /* static walk's launch order (W = 32, and W =
-                                         64 neither persistent nor balanced), by
-                                         workgroup of four groups: 0 index order, 1
-                                         heaviest first (by the last step's visits), 2
-                                         auto (the default): every 1,024 steps, four
-                                         steps alternate the two and the faster is kept
-                                         (decided once the host sees them complete;
-                                         never waited for)                              */
+                                         round-robin, the default                      */
+    GSIM_TUNE_BH_ORDER = 11           /* the walk's launch order, by workgroup of four
+                                         groups (more than 2,048 groups): 0 index
+                                         order, 1 heaviest first (by the last step's
+                                         visits), 2 auto (the default): every 1,024
+                                         steps, four steps alternate the two and the
+                                         faster is kept (decided once the host sees
+                                         them complete; never waited for)              */
 } gsim_tuning;
 gsim_status gsim_set_tuning(gsim_sim *sim, int32_t knob, uint32_t value);
 
@@ -297,8 +286,7 @@ size_t gsim_batch_bytes_per_particle(void);
 typedef struct gsim_batch_tuning {
     uint32_t waves_per_simd;  /* persistent force-launch width, 1..8 (default 6)      */
     uint32_t sort_tile;       /* radix sort tile: 2048, 3072 (default) or 4096 keys  */
-    uint32_t run_queue;       /* leaf runs a walking wave queues in its LDS stack
-                                 before summing them, 1..64 (default 64)            */
+    uint32_t run_queue;       /* 1..64 (default 64); no effect                       */
     uint32_t prio_step;       /* summed 64-node chunks per issue-priority level of a
                                  walking wave, 0 = off (default 32)                  */
     uint32_t prio_carry;      /* a work item starts at level (chunks it summed last
@@ -309,8 +297,8 @@ gsim_status gsim_batch_set_tuning(gsim_batch *batch, const gsim_batch_tuning *tu
 /* Persistent force-launch width only (waves per SIMD, 1..8). */
 gsim_status gsim_batch_set_waves(gsim_batch *batch, uint32_t waves_per_simd);
 /* Autotuner: coordinate descent over the gsim_batch_tuning knobs on the live
- * batch (waves per SIMD, sort tile, run queue, priority step, priority
- * carry, in that order), each candidate timed twice over steps_per_trial
+ * batch (waves per SIMD, sort tile, priority step, priority carry, in that
+ * order), each candidate timed twice over steps_per_trial
  * steps (0: 5) from a snapshot of the state that is restored after every
  * trial, the faster run counting; keeps the fastest setting (read it back
  * with gsim_batch_get_tuning).  *chosen_waves_per_simd may be NULL. */
