@@ -128,9 +128,12 @@ gsim_status ds_reserve_partial(gsim_sim *s, size_t entries) {
     return GSIM_OK;
 }
 
-// Selects the symmetric or the one-sided kernel and sizes its partial sums.
-gsim_status ds_configure(gsim_sim *s, bool sym) {
+// Selects the symmetric or a one-sided form (blocks or slices) and sizes its
+// partial sums.
+gsim_status ds_configure(gsim_sim *s, bool sym, bool block) {
     s->ds_sym = sym ? 1u : 0u;
+    s->ds_block = !sym && block;
+    if (s->ds_block) return GSIM_OK;
     if (sym) {
         s->ds_plan = gsim::ds_sym_plan(s->na, s->ds_sym_cols);
         return ds_reserve_partial(s, s->ds_plan.ipart + s->ds_plan.jpart);
@@ -215,10 +218,15 @@ gsim_status run_steps(gsim_sim *s, uint32_t count) {
             std::swap(s->mass, s->mass_next);
             s->has_tree = true;
         } else {
-            GSIM_HIP(gsim::ds_launch_partial(s, s->pos[in], s->mass));
+            if (s->ds_block)
+                GSIM_HIP(gsim::ds_launch_block(s, s->pos[in], s->vel[in], s->mass, s->pos[out],
+                                               s->vel[out]));
+            else
+                GSIM_HIP(gsim::ds_launch_partial(s, s->pos[in], s->mass));
             if (s->timing) GSIM_HIP(hipEventRecord(ev[1], s->stream));
-            GSIM_HIP(gsim::ds_launch_combine(s, s->pos[in], s->vel[in], s->pos[out],
-                                             s->vel[out]));
+            if (!s->ds_block)
+                GSIM_HIP(gsim::ds_launch_combine(s, s->pos[in], s->vel[in], s->pos[out],
+                                                 s->vel[out]));
         }
         if (s->timing) {
             GSIM_HIP(hipEventRecord(ev[2], s->stream));
@@ -362,7 +370,8 @@ gsim_status gsim_create(const gsim_params *params, const float *pos_xy, const fl
 
     if (params->algorithm == GSIM_DIRECT_SUM) {
         gsim::ds_pick_shape(na, &s->ds_R, &s->ds_S);
-        gsim_status st = ds_configure(s, gsim::ds_sym_default(na));
+        gsim_status st = ds_configure(s, gsim::ds_sym_default(na),
+                                      gsim::ds_block_default(na));
         if (st != GSIM_OK) return bail(st);
     } else {
         e = gsim::bh_alloc(&s->bh, na, gsim::kTreeDepth);
@@ -441,6 +450,8 @@ gsim_status gsim_set_ds_shape(gsim_sim *s, uint32_t R, uint32_t S) {
         return fail(GSIM_ERROR_INVALID_ARGUMENT, "gsim_set_ds_shape: not a direct-sum handle");
     if (R != 1 && R != 2 && R != 4)
         return fail(GSIM_ERROR_INVALID_ARGUMENT, "targets per lane must be 1, 2 or 4");
+    // two targets per lane and slices by size: the default one-sided form
+    const bool block = S == 0 && R == 2 && gsim::ds_block_default(s->na);
     if (S == 0) {
         uint32_t r;
         gsim::ds_pick_shape(s->na, &r, &S);
@@ -451,7 +462,8 @@ gsim_status gsim_set_ds_shape(gsim_sim *s, uint32_t R, uint32_t S) {
     GSIM_HIP(hipStreamSynchronize(s->stream));
     s->ds_R = R;
     s->ds_S = S;
-    return ds_configure(s, false);
+    s->ds_shaped = !block;
+    return ds_configure(s, false, block);
 }
 
 gsim_status gsim_set_tuning(gsim_sim *s, int32_t knob, uint32_t value) {
@@ -534,7 +546,9 @@ gsim_status gsim_set_tuning(gsim_sim *s, int32_t knob, uint32_t value) {
             bool sym = s->ds_sym != 0;
             if (knob == GSIM_TUNE_DS_SYMMETRIC) sym = value != 0;
             else s->ds_sym_cols = value;
-            return ds_configure(s, sym);
+            // a handle given a shape keeps its slices
+            return ds_configure(s, sym, s->ds_shaped ? s->ds_block
+                                                     : gsim::ds_block_default(s->na));
         }
         default:
             return fail(GSIM_ERROR_INVALID_ARGUMENT, "unknown tuning knob %d", knob);

@@ -32,6 +32,15 @@ size_t cell_bound(size_t na) {
     return cells;
 }
 
+// A direct-sum system's share of the batch's admission rule, which allows
+// 4 units a particle of the arena: na for every slice of at least 512 sources.
+size_t ds_share(size_t na) {
+    uint32_t R = 0, S = 0;
+    gsim::ds_pick_shape(na, &R, &S);
+    const size_t jlen = ((na + S - 1) / S + 63) / 64 * 64;
+    return (na + jlen - 1) / jlen * na;
+}
+
 void destroy_graphs(gsim_batch *b) {
     for (auto &g : b->graph) {
         if (g) (void)hipGraphExecDestroy(g);
@@ -44,8 +53,8 @@ void free_batch(gsim_batch *b) {
     if (b->stream) (void)hipStreamSynchronize(b->stream);
     destroy_graphs(b);
     gsim::BatchDevice &d = b->d;
-    void *ptrs[] = {d.pos[0], d.pos[1], d.vel[0], d.vel[1], d.mass, d.partial, d.desc, d.remaining,
-                    d.bh_sys, d.bh_prefix, d.ds_sys, d.ds_prefix, d.items, d.counts, d.stats,
+    void *ptrs[] = {d.pos[0], d.pos[1], d.vel[0], d.vel[1], d.mass, d.desc, d.remaining,
+                    d.bh_sys, d.bh_prefix, d.items, d.counts, d.stats,
                     d.keys[0], d.keys[1], d.idx[0], d.idx[1], d.status, d.digit_total,
                     d.block_cells, d.block_leaves, d.sdep, d.cpos, d.sorted_src,
                     d.leaf_sum, d.leaf_first, d.leaf_key, d.tile_range, d.live_tiles, d.top, d.node4,
@@ -87,10 +96,10 @@ void give_range(gsim_batch *b, uint32_t off, uint32_t len) {
 // Rebuilds and uploads the membership arrays (descriptors, ranks, work items).
 gsim_status upload_membership(gsim_batch *b) {
     std::vector<gsim::SysDesc> desc;
-    std::vector<uint32_t> bh_sys, bh_prefix{0}, ds_sys, ds_prefix{0};
-    std::vector<uint2> items;
+    std::vector<uint32_t> bh_sys, bh_prefix{0};
+    // direct-sum blocks first: the longest items, so that none starts last
+    std::vector<uint2> items, bh_items;
     std::vector<uint32_t> remaining;
-    uint32_t part_off = 0;
     GSIM_HIP(hipStreamSynchronize(b->stream));  // step counts below are exact from here
     for (auto &kv : b->systems) {
         gsim::BatchSystem &s = kv.second;
@@ -124,31 +133,20 @@ gsim_status upload_membership(gsim_batch *b) {
             bh_prefix.push_back(bh_prefix.back() + s.na);
             // one work item per vote group: 64 sorted positions, or 32 at W = 32
             d.w = s.params.group_width;
-            for (uint32_t g = 0; g < s.na / d.w; ++g) items.push_back(make_uint2(di, g));
+            for (uint32_t g = 0; g < s.na / d.w; ++g) bh_items.push_back(make_uint2(di, g));
         } else {
-            uint32_t R = 0, S = 0;
-            gsim::ds_pick_shape(s.na, &R, &S);
-            const uint32_t jlen = (uint32_t)(((s.na + S - 1) / S + 63) / 64 * 64);
-            const uint32_t slices = (s.na + jlen - 1) / jlen;
-            d.ds_jlen = jlen;
-            d.ds_slices = slices;
-            d.ds_part_off = part_off;
-            part_off += slices * s.na;
-            ds_sys.push_back(di);
-            ds_prefix.push_back(ds_prefix.back() + s.na);
-            for (uint32_t tb = 0; tb < (s.na + 127) / 128; ++tb)
-                for (uint32_t sl = 0; sl < slices; ++sl) items.push_back(make_uint2(di, (tb << 16) | sl));
+            for (uint32_t tb = 0; tb < s.na / gsim::kDsBlockTargets; ++tb)
+                items.push_back(make_uint2(di, tb));
         }
         desc.push_back(d);
     }
-    if (items.size() > b->item_capacity || part_off > b->partial_capacity)
+    items.insert(items.end(), bh_items.begin(), bh_items.end());
+    if (items.size() > b->item_capacity)
         return fail(GSIM_ERROR_CAPACITY, "batch work list exceeds its capacity");
     gsim::BatchCounts c{};
     c.n_sys = (uint32_t)desc.size();
     c.n_bh = (uint32_t)bh_sys.size();
     c.n_bh_particles = bh_prefix.back();
-    c.n_ds = (uint32_t)ds_sys.size();
-    c.n_ds_particles = ds_prefix.back();
     c.n_items = (uint32_t)items.size();
     // the acceptance and visit totals carry over
     GSIM_HIP(hipMemcpy(&c.accepts, &b->d.counts->accepts, sizeof(c.accepts), hipMemcpyDeviceToHost));
@@ -159,8 +157,6 @@ gsim_status upload_membership(gsim_batch *b) {
     GSIM_HIP(up(b->d.desc, desc.data(), desc.size() * sizeof(gsim::SysDesc)));
     GSIM_HIP(up(b->d.bh_sys, bh_sys.data(), bh_sys.size() * 4));
     GSIM_HIP(up(b->d.bh_prefix, bh_prefix.data(), bh_prefix.size() * 4));
-    GSIM_HIP(up(b->d.ds_sys, ds_sys.data(), ds_sys.size() * 4));
-    GSIM_HIP(up(b->d.ds_prefix, ds_prefix.data(), ds_prefix.size() * 4));
     GSIM_HIP(up(b->d.items, items.data(), items.size() * sizeof(uint2)));
     // the work items changed: their last-step chunk counts no longer apply
     GSIM_HIP(hipMemsetAsync(b->d.ichunk, 0, sizeof(uint32_t) * b->item_capacity, b->stream));
@@ -246,12 +242,9 @@ gsim_status gsim_batch_create(int32_t device, size_t capacity_particles, uint32_
         GSIM_BALLOC(d.idx[k], cap);
     }
     GSIM_BALLOC(d.mass, cap);
-    GSIM_BALLOC(d.partial, b->partial_capacity);
     GSIM_BALLOC(d.desc, max_systems);
     GSIM_BALLOC(d.bh_sys, max_systems);
     GSIM_BALLOC(d.bh_prefix, max_systems + 1);
-    GSIM_BALLOC(d.ds_sys, max_systems);
-    GSIM_BALLOC(d.ds_prefix, max_systems + 1);
     GSIM_BALLOC(d.items, b->item_capacity);
     GSIM_BALLOC(d.remaining, max_systems);
     GSIM_BALLOC(d.counts, 1);
@@ -315,15 +308,9 @@ gsim_status gsim_batch_add(gsim_batch *b, const gsim_params *p, const float *pos
     const size_t nodes = p->algorithm == GSIM_BARNES_HUT ? na + cell_bound(na) : 0;
     if (b->nodes_reserved + nodes > b->node_capacity)
         return fail(GSIM_ERROR_CAPACITY, "batch node arrays are full");
-    size_t part = 0;
-    if (p->algorithm == GSIM_DIRECT_SUM) {
-        uint32_t R = 0, S = 0;
-        gsim::ds_pick_shape(na, &R, &S);
-        const size_t jlen = ((na + S - 1) / S + 63) / 64 * 64;
-        part = ((na + jlen - 1) / jlen) * na;
-        if (b->partial_used + part > b->partial_capacity)
-            return fail(GSIM_ERROR_CAPACITY, "batch partial-sum space is full");
-    }
+    const size_t part = p->algorithm == GSIM_DIRECT_SUM ? ds_share(na) : 0;
+    if (b->partial_used + part > b->partial_capacity)
+        return fail(GSIM_ERROR_CAPACITY, "batch direct-sum space is full");
     uint32_t off = 0;
     if (!take_range(b, (uint32_t)na, &off))
         return fail(GSIM_ERROR_CAPACITY, "no free arena range of %zu particles", na);
@@ -371,12 +358,7 @@ gsim_status gsim_batch_remove(gsim_batch *b, uint32_t id) {
     const gsim::BatchSystem &s = it->second;
     give_range(b, s.off, s.na);
     b->nodes_reserved -= s.node_reserve;
-    if (s.params.algorithm == GSIM_DIRECT_SUM) {
-        uint32_t R = 0, S = 0;
-        gsim::ds_pick_shape(s.na, &R, &S);
-        const size_t jlen = ((s.na + S - 1) / S + 63) / 64 * 64;
-        b->partial_used -= ((s.na + jlen - 1) / jlen) * s.na;
-    }
+    if (s.params.algorithm == GSIM_DIRECT_SUM) b->partial_used -= ds_share(s.na);
     b->systems.erase(it);
     b->dirty = true;
     return GSIM_OK;
@@ -489,7 +471,7 @@ gsim_status gsim_batch_query(const gsim_batch *b, gsim_batch_info *out) {
 }
 
 size_t gsim_batch_bytes_per_particle(void) {
-    // state 36 B, Barnes-Hut scratch 55 B, 3 node slots x 32 B, partials 32 B
+    // at most: state 36 B, Barnes-Hut scratch 55 B, 3 node slots x 32 B, 32 B
     return 36 + 55 + 3 * 32 + 32;
 }
 

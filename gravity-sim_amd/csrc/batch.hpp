@@ -19,8 +19,6 @@ struct SysDesc {
     float eps2, theta2, kv, kp;      // softening^2, theta^2, velocity and position factors
     float dt, pad0;
     uint32_t bh_rank, sorted_base;   // Barnes-Hut: rank in the global sort, first sorted position
-    uint32_t ds_part_off, ds_jlen;   // direct sum: partial-sum offset (float2) and slice length
-    uint32_t ds_slices;
     uint32_t w;                      // Barnes-Hut vote width: 64 or 32
 };
 
@@ -45,8 +43,6 @@ constexpr uint32_t kForceQueues = 64;
 struct BatchCounts {
     uint32_t n_bh;            // Barnes-Hut systems (ranks)
     uint32_t n_bh_particles;  // sum of their padded counts = sorted positions
-    uint32_t n_ds;            // direct-sum systems
-    uint32_t n_ds_particles;  // sum of their padded counts
     uint32_t n_items;         // work items of the force launch
     uint32_t n_cells;         // cell nodes of all trees (emit)
     uint32_t n_leaves;        // occupied leaves of all trees (emit)
@@ -90,7 +86,7 @@ constexpr uint32_t kBatchRankShift = 21;                   // key = rank << 21 |
 constexpr uint32_t kBatchMaxSystems = 1u << (32 - kBatchRankShift);  // 2048
 constexpr uint32_t kBatchSentinel = 0xffffffffu;
 constexpr uint32_t kMaxForceWaves = 1024u * 8u;  // persistent force launch: 8 waves per SIMD
-// Largest arena: node slots (3 per particle) and partial sums stay within
+// Largest arena: node slots (3 per particle) and offsets stay within
 // 32-bit indices.
 constexpr size_t kBatchMaxParticles = (0x7fffffffull / 8) / 64 * 64;
 
@@ -98,11 +94,9 @@ struct BatchDevice {
     // arena
     float2 *pos[2] = {}, *vel[2] = {};
     float *mass = nullptr;
-    float2 *partial = nullptr;
     // membership
     SysDesc *desc = nullptr;
     uint32_t *bh_sys = nullptr, *bh_prefix = nullptr;  // [max_systems (+1)]
-    uint32_t *ds_sys = nullptr, *ds_prefix = nullptr;
     uint2 *items = nullptr;
     uint32_t *remaining = nullptr;  // steps each system may still take (kUnlimitedSteps = no limit)
     BatchCounts *counts = nullptr;
@@ -145,7 +139,7 @@ struct gsim_batch {
     hipStream_t stream = nullptr;
     size_t capacity = 0;        // particles (padded) in the arena
     size_t node_capacity = 0;   // node slots
-    size_t partial_capacity = 0;
+    size_t partial_capacity = 0;  // direct-sum admission units
     size_t item_capacity = 0;
     uint32_t max_systems = 0;
     size_t tiles_cap = 0, blocks_cap = 0;

@@ -9,11 +9,12 @@
 // by the emit kernel).  The per-system semantics are those of the
 // single-system kernels in bh_kernels.hip (same cells, same canonical order,
 // same reduction association, same vote), so a system's result in a batch is
-// bit-identical to its result alone.  Direct-sum systems use the same slice
-// split as the single-system path for their size, so they match bit for bit
-// as well.
+// bit-identical to its result alone.  Direct-sum systems run the roles of the
+// single-system block kernel (ds_device.hpp), so they match bit for bit as
+// well.
 #include "batch.hpp"
 #include "bh_device.hpp"
+#include "ds_device.hpp"
 #include "radix_device.hpp"
 
 #include <algorithm>
@@ -511,45 +512,72 @@ __device__ void bb_walk_group(uint32_t g, const SysDesc &d, const RankStats &st,
     vel_out[src] = make_float2(nvx, nvy);
 }
 
-// Direct-sum tile: 128 targets (two per lane) x one source slice; the same
-// arithmetic as ds_partial_kernel, so the per-slice partials are identical.
-__device__ void bb_ds_tile(uint32_t sub, const SysDesc &d, const float2 *__restrict__ pos,
-                           const float *__restrict__ mass, float2 *__restrict__ partial) {
-    const uint32_t lane = threadIdx.x & 63;
-    const uint32_t tb = sub >> 16, slice = sub & 0xffffu;
-    const uint32_t t0 = tb * 128 + lane, t1 = t0 + 64;
-    const float2 p0 = t0 < d.na ? pos[d.off + t0] : make_float2(0.0f, 0.0f);
-    const float2 p1 = t1 < d.na ? pos[d.off + t1] : make_float2(0.0f, 0.0f);
-    float ax0 = 0.0f, ay0 = 0.0f, ax1 = 0.0f, ay1 = 0.0f;
-    const uint32_t j0 = d.off + slice * d.ds_jlen;
-    const uint32_t j1 = min(d.off + d.na, j0 + d.ds_jlen);
-    const float eps2 = d.eps2;
-    for (uint32_t j = j0; j < j1; j += 8) {  // slices are whole multiples of 64
-#pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            const float2 s = pos[j + u];
-            const float m = mass[j + u];
-            {
-                const float dx = s.x - p0.x, dy = s.y - p0.y;
-                const float r2 = __builtin_fmaf(dx, dx, __builtin_fmaf(dy, dy, eps2));
-                const float inv = __builtin_amdgcn_rsqf(r2);
-                const float tt = (m * inv) * (inv * inv);
-                ax0 = __builtin_fmaf(dx, tt, ax0);
-                ay0 = __builtin_fmaf(dy, tt, ay0);
-            }
-            {
-                const float dx = s.x - p1.x, dy = s.y - p1.y;
-                const float r2 = __builtin_fmaf(dx, dx, __builtin_fmaf(dy, dy, eps2));
-                const float inv = __builtin_amdgcn_rsqf(r2);
-                const float tt = (m * inv) * (inv * inv);
-                ax1 = __builtin_fmaf(dx, tt, ax1);
-                ay1 = __builtin_fmaf(dy, tt, ay1);
-            }
+// Direct-sum block tb of one system: its 16 targets against every source, role
+// after role, then integrate (ds_block_kernel's additions in its order).
+__device__ void bb_ds_block(uint32_t tb, const SysDesc &d, const float2 *__restrict__ pos_all,
+                            const float2 *__restrict__ vel_all,
+                            const float *__restrict__ mass_all, float2 *__restrict__ pos_out,
+                            float2 *__restrict__ vel_out, bool live) {
+    const uint32_t lane = threadIdx.x & 63, stream = lane & 15u, slot = lane >> 4;
+    const uint32_t mine = 4 * slot + (stream >> 2);  // the target this lane ends with
+    const uint32_t i = d.off + tb * kDsBlockTargets + mine;
+    const bool writes = (lane & 3u) == 0;
+    const float2 p = pos_all[i], v = vel_all[i];
+    if (!live) {  // budget spent: hold the state
+        if (writes) {
+            pos_out[i] = p;
+            vel_out[i] = v;
         }
+        return;
     }
-    float2 *dst = partial + d.ds_part_off + (size_t)slice * d.na;
-    if (t0 < d.na) dst[t0] = make_float2(ax0, ay0);
-    if (t1 < d.na) dst[t1] = make_float2(ax1, ay1);
+    const float2 *const pos = pos_all + d.off;
+    const float *const mass = mass_all + d.off;
+    const uint32_t na = d.na, t0 = tb * kDsBlockTargets;
+    float tx[4], ty[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const float2 q = pos[t0 + 4 * slot + r];
+        tx[r] = q.x;
+        ty[r] = q.y;
+    }
+    float ev = d.eps2;
+    asm volatile("" : "+v"(ev));
+    constexpr uint32_t kStep = 16 * kDsRoles;
+    float bx = 0.0f, by = 0.0f;
+    // the sixteens of role w start at 16 w, 16 w + 256, ...; the next two in
+    // flight, across roles
+    auto next = [&](uint32_t &w, uint32_t &j) {
+        j += kStep;
+        if (j >= na) j = 16 * ++w;
+    };
+    auto load = [&](uint32_t j) { return ds_source(pos, mass, min(j, na - 16) + stream); };
+    uint32_t w = 0, j = 0, w1 = 0, j1 = 0;
+    next(w1, j1);
+    uint32_t w2 = w1, j2 = j1;
+    next(w2, j2);
+    DsSource q0 = load(j), q1 = load(j1);
+    const uint32_t roles = min(kDsRoles, na / 16);  // the others have no source
+    while (w < roles) {
+        float ax[4] = {0.0f, 0.0f, 0.0f, 0.0f}, ay[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+        const uint32_t role = w;
+        while (w == role) {
+            const DsSource c = q0;
+            q0 = q1;
+            q1 = load(j2);
+            ds_add<false>(c, tx, ty, ev, ax, ay);
+            w = w1;
+            j = j1;
+            w1 = w2;
+            j1 = j2;
+            next(w2, j2);
+        }
+        bx = bx + ds_sum_streams(ax, lane);
+        by = by + ds_sum_streams(ay, lane);
+    }
+    if (!writes) return;
+    const float nvx = v.x + bx * d.kv, nvy = v.y + by * d.kv;  // SimShader.comp:68-69
+    pos_out[i] = make_float2(p.x + ((v.x + nvx) * 0.5f) * d.dt, p.y + ((v.y + nvy) * 0.5f) * d.dt);
+    vel_out[i] = make_float2(nvx, nvy);
 }
 
 template <bool kWide>
@@ -560,9 +588,8 @@ __global__ __launch_bounds__(256) void bb_force_kernel(
     const uint32_t *__restrict__ sorted_src, const float2 *__restrict__ pos,
     const float2 *__restrict__ vel, const float *__restrict__ mass,
     const float4 *__restrict__ node4, const uint4 *__restrict__ child,
-    float2 *__restrict__ pos_out, float2 *__restrict__ vel_out, float2 *__restrict__ partial,
-    uint32_t node_cap, unsigned long long *__restrict__ wave_acc, uint32_t *__restrict__ ichunk,
-    BatchTune tune) {
+    float2 *__restrict__ pos_out, float2 *__restrict__ vel_out, uint32_t node_cap,
+    unsigned long long *__restrict__ wave_acc, uint32_t *__restrict__ ichunk, BatchTune tune) {
     __shared__ WalkShared sh[4];
     const uint32_t w = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const uint32_t nitems = counts->n_items;
@@ -596,8 +623,8 @@ __global__ __launch_bounds__(256) void bb_force_kernel(
             else
                 bb_walk_group<64, kWide>(item.y, d, st, sh[w], sorted_src, pos, vel, node4, child,
                                   pos_out, vel_out, node_cap, vis, acc, &ichunk[it], tune);
-        } else if (live) {
-            bb_ds_tile(item.y, d, pos, mass, partial);
+        } else {
+            bb_ds_block(item.y, d, pos, vel, mass, pos_out, vel_out, live);
         }
     }
     if (lane == 0) {
@@ -643,42 +670,10 @@ __global__ __launch_bounds__(256) void bb_finish_kernel(uint32_t *__restrict__ r
     }
 }
 
-// Direct-sum combine + integrate (SimShader.comp:68-69) for every DS particle.
-__global__ __launch_bounds__(256) void bb_ds_combine_kernel(
-    const SysDesc *__restrict__ desc, const uint32_t *__restrict__ remaining,
-    const uint32_t *__restrict__ ds_sys,
-    const uint32_t *__restrict__ ds_prefix, const BatchCounts *__restrict__ counts,
-    const float2 *__restrict__ partial, const float2 *__restrict__ pos,
-    const float2 *__restrict__ vel, float2 *__restrict__ pos_out, float2 *__restrict__ vel_out) {
-    const uint32_t nd = counts->n_ds, n = counts->n_ds_particles;
-    for (uint32_t f = blockIdx.x * 256 + threadIdx.x; f < n; f += gridDim.x * 256) {
-        const uint32_t r = rank_of(ds_prefix, nd, f);
-        const uint32_t di = ds_sys[r];
-        const SysDesc d = desc[di];
-        const uint32_t li = f - ds_prefix[r];
-        if (remaining[di] == 0u) {  // budget spent: hold the state
-            pos_out[d.off + li] = pos[d.off + li];
-            vel_out[d.off + li] = vel[d.off + li];
-            continue;
-        }
-        float ax = 0.0f, ay = 0.0f;
-        for (uint32_t s = 0; s < d.ds_slices; ++s) {
-            const float2 a = partial[d.ds_part_off + (size_t)s * d.na + li];
-            ax = ax + a.x;
-            ay = ay + a.y;
-        }
-        const uint32_t i = d.off + li;
-        const float2 p = pos[i], v = vel[i];
-        const float nvx = v.x + ax * d.kv, nvy = v.y + ay * d.kv;
-        pos_out[i] = make_float2(p.x + ((v.x + nvx) * 0.5f) * d.dt, p.y + ((v.y + nvy) * 0.5f) * d.dt);
-        vel_out[i] = make_float2(nvx, nvy);
-    }
-}
-
 }  // namespace
 
 // One batched step: Barnes-Hut build for all BH systems, one persistent force
-// launch for every system, the direct-sum combine.  Launched onto b->stream
+// launch for every system.  Launched onto b->stream
 // (captured into a graph by the caller).
 hipError_t batch_launch_step(gsim_batch *b, int in, int out) {
     BatchDevice &d = b->d;
@@ -734,12 +729,9 @@ hipError_t batch_launch_step(gsim_batch *b, int in, int out) {
     auto *force = b->node_capacity >= kNarrowNodes ? bb_force_kernel<true> : bb_force_kernel<false>;
     force<<<waves / 4, 256, 0, st>>>(d.items, d.desc, d.remaining, d.stats, d.counts, d.sorted_src,
                                                d.pos[in], d.vel[in], d.mass, d.node4, d.child,
-                                               d.pos[out], d.vel[out], d.partial,
+                                               d.pos[out], d.vel[out],
                                                (uint32_t)b->node_capacity, d.wave_acc, d.ichunk,
                                                tune);
-    bb_ds_combine_kernel<<<g_part, 256, 0, st>>>(d.desc, d.remaining, d.ds_sys, d.ds_prefix,
-                                                 d.counts, d.partial, d.pos[in], d.vel[in],
-                                                 d.pos[out], d.vel[out]);
     bb_finish_kernel<<<8, 256, 0, st>>>(d.remaining, d.counts, d.wave_acc, waves);
     return hipGetLastError();
 }

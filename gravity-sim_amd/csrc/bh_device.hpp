@@ -2,6 +2,7 @@
 #pragma once
 
 #include "internal.hpp"
+#include "lane_ops.hpp"
 
 namespace gsim {
 
@@ -391,13 +392,6 @@ __device__ __forceinline__ uint32_t uniform(uint32_t v) {
 __device__ __forceinline__ uint32_t lane_rank(unsigned long long m) {  // set bits below this lane
     return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
 }
-
-template <int kCtrl>
-__device__ __forceinline__ float dpp(float v) {
-    return __builtin_bit_cast(
-        float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), kCtrl, 0xF, 0xF, true));
-}
-constexpr int kDppXor1 = 0xB1, kDppXor2 = 0x4E, kDppXor7 = 0x141, kDppXor15 = 0x140;
 
 __device__ __forceinline__ float lane_value(float v, uint32_t lane) {
     return __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(v), lane));

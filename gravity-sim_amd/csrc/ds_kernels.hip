@@ -4,7 +4,10 @@
 // a_i = sum_j d * (m_j r^3) with d = p_j - p_i, r = rsqrt(d.d + eps2), then
 // v' = v + a*(dt*G), p' = p + ((v+v')*0.5)*dt.
 //
-// One-sided form -- work split: a target block of 256*R targets (R per lane) times a source
+// Three forms: blocks (below 16,384 particles, one launch a step), symmetric
+// (each pair once, from there on) and one-sided slices.
+//
+// One-sided slices -- work split: a target block of 256*R targets (R per lane) times a source
 // slice of `jlen` particles is one workgroup.  Source particles are read with
 // wave-uniform indices, so they arrive through scalar loads (s_load) and sit
 // in SGPRs: no LDS traffic and no VALU cycles spent on broadcast.  Each slice
@@ -14,6 +17,7 @@
 #include <cstring>
 #include <mutex>
 
+#include "ds_device.hpp"
 #include "internal.hpp"
 
 namespace gsim {
@@ -64,6 +68,71 @@ __global__ __launch_bounds__(kDsThreads) void ds_partial_kernel(
         const uint32_t i = base + r * kDsThreads;
         if (i < na) partial[(size_t)slice * na + i] = make_float2(ax[r], ay[r]);
     }
+}
+
+// Blocks: one workgroup per 16 targets, its 16 waves the roles of ds_device.hpp,
+// so a step is one launch with no partial sums in memory.  What bounds it: the
+// launch and two dependent round trips below ~2,000 particles, the VALU above
+// (4,096 particles: 2.07e12 pairs a second of the 4.6e12 its issue rate allows;
+// 12,288: 3.6e12).
+// Against slices of at least 512 sources (1 to 31 slices) and a combine
+// launch, us a step: 64 particles 7.8 -> 2.8, 1,024 41 -> 4.1, 4,096 51 -> 8.1,
+// 12,288 71 -> 42, 15,040 90 -> 65.
+template <bool kRcp>
+__global__ __launch_bounds__(1024, 8) void ds_block_kernel(
+    const float2 *__restrict__ pos, const float2 *__restrict__ vel,
+    const float *__restrict__ mass, float2 *__restrict__ pos_out, float2 *__restrict__ vel_out,
+    float2 *__restrict__ acc_dbg, uint32_t na, float eps2, float kv, float dt) {
+    __shared__ float2 sum[kDsRoles][kDsBlockTargets];
+    const uint32_t lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const uint32_t stream = lane & 15u, slot = lane >> 4;
+    const uint32_t t0 = blockIdx.x * kDsBlockTargets;  // na is a multiple of 64
+    float tx[4], ty[4], ax[4], ay[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const float2 p = pos[t0 + 4 * slot + r];
+        tx[r] = p.x;
+        ty[r] = p.y;
+        ax[r] = 0.0f;
+        ay[r] = 0.0f;
+    }
+    // the integrated particles, needed at the end
+    const uint32_t i = t0 + (threadIdx.x & (kDsBlockTargets - 1u));
+    const float2 p = pos[i], v = vel[i];
+    float ev = eps2;  // in a vector register: a scalar operand costs the second issue
+    asm volatile("" : "+v"(ev));
+    // sixteen sources at 16 w, 16 w + 256, ..., the next four rounds in flight
+    constexpr uint32_t kAhead = 4, kStep = 16 * kDsRoles;
+    const uint32_t first = 16 * w + stream;
+    DsSource q[kAhead];
+#pragma unroll
+    for (uint32_t u = 0; u < kAhead; ++u)
+        q[u] = ds_source(pos, mass, min(first + u * kStep, na - 16 + stream));
+    for (uint32_t j = 16 * w; j < na; j += kAhead * kStep) {
+#pragma unroll
+        for (uint32_t u = 0; u < kAhead; ++u) {
+            if (j + u * kStep >= na) break;
+            const DsSource c = q[u];
+            q[u] = ds_source(pos, mass, min(j + (u + kAhead) * kStep, na - 16) + stream);
+            ds_add<kRcp>(c, tx, ty, ev, ax, ay);
+        }
+    }
+    const float sx = ds_sum_streams(ax, lane), sy = ds_sum_streams(ay, lane);
+    if ((lane & 3u) == 0) sum[w][4 * slot + (stream >> 2)] = make_float2(sx, sy);
+    __syncthreads();
+    if (threadIdx.x >= kDsBlockTargets) return;
+    float bx = 0.0f, by = 0.0f;
+#pragma unroll
+    for (uint32_t u = 0; u < kDsRoles; ++u) {
+        const float2 a = sum[u][threadIdx.x];
+        bx = bx + a.x;
+        by = by + a.y;
+    }
+    // SimShader.comp:68-69
+    const float nvx = v.x + bx * kv, nvy = v.y + by * kv;
+    pos_out[i] = make_float2(p.x + ((v.x + nvx) * 0.5f) * dt, p.y + ((v.y + nvy) * 0.5f) * dt);
+    vel_out[i] = make_float2(nvx, nvy);
+    if (acc_dbg) acc_dbg[i] = make_float2(bx, by);
 }
 
 __global__ __launch_bounds__(256) void ds_combine_kernel(
@@ -327,6 +396,19 @@ void ds_pick_shape(size_t na, uint32_t *R, uint32_t *S) {
     *S = (uint32_t)s;
 }
 
+bool ds_block_default(size_t na) { return na < kDsSymMinParticles; }
+
+// One launch for the whole step: forces and integration.
+hipError_t ds_launch_block(gsim_sim *s, const float2 *pos, const float2 *vel, const float *mass,
+                           float2 *pos_out, float2 *vel_out) {
+    const uint32_t na = (uint32_t)s->na;
+    float2 *acc = (s->debug_flags & GSIM_DEBUG_ACCEL) ? s->accel : nullptr;
+    auto *k = s->ds_rcp ? ds_block_kernel<true> : ds_block_kernel<false>;
+    k<<<na / kDsBlockTargets, 64 * kDsRoles, 0, s->stream>>>(pos, vel, mass, pos_out, vel_out, acc,
+                                                            na, s->eps2, s->kv, s->dt);
+    return hipGetLastError();
+}
+
 hipError_t ds_launch_partial(gsim_sim *s, const float2 *pos, const float *mass) {
     const uint32_t na = (uint32_t)s->na;
     if (s->ds_sym) {
@@ -376,7 +458,8 @@ hipError_t ds_launch_combine(gsim_sim *s, const float2 *pos, const float2 *vel,
 // ---- allocation-free direct-sum step ---------------------------------------------
 //
 // gsim_ds_step_noalloc runs one one-sided direct-sum step on caller-owned
-// device arrays.  Its only scratch, the per-slice partial accelerations, lives
+// device arrays: in blocks below 16,384 particles, which need no scratch, in
+// slices from there on.  Their only scratch, the per-slice partial accelerations, lives
 // in `scratch`, a file-scope device array that every GPU holds for the life of
 // the process, so the call allocates nothing and can run where hipMalloc
 // cannot (under stream capture, inside a serving loop that forbids it).  In
@@ -428,8 +511,19 @@ gsim_status noalloc_setup(int device, float2 **out) {
 gsim_status noalloc_launch(float2 *part, const gsim_params *p, const float2 *pos,
                            const float2 *vel, const float *mass, float2 *pos_out,
                            float2 *vel_out, uint32_t na, hipStream_t stream) {
+    // the form gsim_step picks for a one-sided handle
+    if (ds_block_default(na)) {
+        const float dt = p->simulation_time;
+        ds_block_kernel<false><<<na / kDsBlockTargets, 64 * kDsRoles, 0, stream>>>(
+            pos, vel, mass, pos_out, vel_out, nullptr, na, p->softening_len * p->softening_len,
+            dt * p->gravitational_const, dt);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess)
+            return fail(GSIM_ERROR_DEVICE, "direct-sum launch failed: %s", hipGetErrorString(e));
+        return GSIM_OK;
+    }
     uint32_t R = 2, S = 1;
-    ds_pick_shape(na, &R, &S);  // the shape gsim_step picks for a one-sided handle
+    ds_pick_shape(na, &R, &S);
     const size_t fit = kNoallocScratchEntries / na;
     if (S > fit) S = (uint32_t)fit;
     const uint32_t jlen = ((na + S - 1) / S + 63) / 64 * 64;

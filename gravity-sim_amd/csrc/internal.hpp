@@ -160,6 +160,9 @@ constexpr size_t kDsSymMinParticles = 16384;   // default range of the symmetric
 constexpr size_t kDsSymMaxParticles = 262144;  // (its partial sums grow as N^2 / 64)
 constexpr size_t kDsSymMinWaves = 32768;       // auto: 2 columns per wave from this many waves
 
+// Targets of one workgroup of the block kernel, and of one batch work item.
+constexpr uint32_t kDsBlockTargets = 16;
+
 struct DsSymPlan {
     uint32_t B = 0, G = 0;      // 64-particle blocks, row groups
     uint32_t cols = 0;          // column blocks per wave (1 or 2)
@@ -218,6 +221,8 @@ struct gsim_sim {
     float2 *partial = nullptr;
     size_t partial_cap = 0;            // float2 entries allocated
     uint32_t ds_R = 1, ds_S = 1, ds_S_used = 1;
+    bool ds_block = false;                 // the block kernel (one launch) instead of slices
+    bool ds_shaped = false;                // gsim_set_ds_shape chose slices
     uint32_t ds_sym = 0, ds_sym_cols = 0;  // symmetric kernel; column blocks per tile (0 auto)
     gsim::DsSymPlan ds_plan{};
     // Barnes-Hut
@@ -238,6 +243,9 @@ namespace gsim {
 // Direct sum (ds_kernels.hip)
 void ds_pick_shape(size_t na, uint32_t *R, uint32_t *S);
 bool ds_sym_default(size_t na);
+bool ds_block_default(size_t na);
+hipError_t ds_launch_block(gsim_sim *s, const float2 *pos, const float2 *vel, const float *mass,
+                           float2 *pos_out, float2 *vel_out);
 DsSymPlan ds_sym_plan(size_t na, uint32_t cols);
 hipError_t ds_launch_partial(gsim_sim *s, const float2 *pos, const float *mass);
 hipError_t ds_launch_combine(gsim_sim *s, const float2 *pos, const float2 *vel,

@@ -153,7 +153,8 @@ gsim_status gsim_set_timing(gsim_sim *sim, int32_t enable);
 gsim_status gsim_get_timing(gsim_sim *sim, gsim_timing *out, int32_t reset);
 
 /* Selects the one-sided direct-sum kernel with this launch shape: targets per
- * lane (1, 2 or 4) and source slices (0 = pick by size).  Results stay within the documented tolerance for every
+ * lane (1, 2 or 4) and source slices (0 = pick by size; with 2 targets per
+ * lane below 16,384 padded particles the block form, one launch a step).  Results stay within the documented tolerance for every
  * shape; the partial sums are combined in slice order, so a shape is
  * deterministic. */
 gsim_status gsim_set_ds_shape(gsim_sim *sim, uint32_t targets_per_lane,

@@ -1,0 +1,49 @@
+"""The direct sum's block form (below 16,384 padded particles) where its split
+changes: fewer sixteens of sources than roles, a ragged last round, one and
+several rounds in flight, the largest size.  Forces within 1e-5 system-relative
+of the FP32 oracle and per particle no further from FP64 than 1.5x the oracle's
+own sums, the integration bit-exact on those forces, and the same bits in a
+batch."""
+import numpy as np
+import pytest
+
+import gsim
+import helpers as H
+import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+EPS2 = H.sq32(0.2)
+
+
+@pytest.mark.parametrize("rcp", [0, 1])
+@pytest.mark.parametrize("n", [1, 64, 250, 256, 300, 1024, 1025, 4160, 16320])
+def test_block_forces_and_batch(n, rcp):
+    print(f"ds block n={n} rcp={rcp}", flush=True)
+    p = gsim.generate("galaxy", n, 50.0, 1.0, 10.0, seed=n)
+    with gsim.Simulation(p, "direct-sum") as s:
+        s.set_debug(gsim.DEBUG_ACCEL)
+        s.set_tuning(gsim.TUNE_DS_RCP, rcp)
+        s.step(1)
+        a = s.dump(gsim.DUMP_ACCEL)[: p.n]
+        g = s.read()
+    pp = p.padded()
+    ref = O.ds_accel_f32(pp.pos, pp.mass, EPS2)[: p.n]
+    ref64 = O.ds_accel_f64(pp.pos, pp.mass, EPS2)[: p.n]
+    if n == 1:
+        assert np.array_equal(a, np.zeros_like(a))
+    else:
+        assert H.system_rel_err(a, ref) <= 1e-5
+        worst = H.per_particle_rel(ref, ref64).max()
+        assert H.per_particle_rel(a, ref64).max() <= max(1.5 * worst, 1e-6)
+    nv = (p.vel + a * np.float32(1e-3)).astype(np.float32)
+    assert np.array_equal(g.vel, nv)
+    assert np.array_equal(g.pos, (p.pos + ((p.vel + nv) * np.float32(0.5)) * np.float32(1e-3))
+                          .astype(np.float32))
+    if rcp:
+        return
+    with gsim.Batch(max(8 * pp.n, 65536), 4) as b:  # its direct-sum admission rule needs 8n
+        k = b.add(p, "direct-sum")
+        b.step(1)
+        q = b.read(k)
+    assert np.array_equal(q.pos, g.pos) and np.array_equal(q.vel, g.vel)
