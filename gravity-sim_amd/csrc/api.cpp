@@ -68,6 +68,7 @@ void free_sim(gsim_sim *s) {
     (void)hipFree(s->partial);
     (void)hipFree(s->accel);
     gsim::bh_free(&s->bh);
+    s->stage.release();
     for (auto &p : s->pending)
         for (hipEvent_t e : p.e) s->event_pool.push_back(e);
     for (hipEvent_t e : s->event_pool) (void)hipEventDestroy(e);
@@ -397,30 +398,36 @@ gsim_status gsim_synchronize(gsim_sim *s) {
     return GSIM_OK;
 }
 
-gsim_status gsim_read(gsim_sim *s, float *pos_xy, float *vel_xy, float *mass) {
+gsim_status gsim_read(gsim_sim *s, float *pos_xy, float *vel_xy, float *mass_out) {
     gsim::clear_error();
     if (!s) return fail(GSIM_ERROR_INVALID_ARGUMENT, "gsim_read: NULL handle");
     GSIM_HIP(hipSetDevice(s->device));
-    GSIM_HIP(hipStreamSynchronize(s->stream));
-    if (!s->perm[0]) {  // direct sum: the caller's order
-        if (pos_xy) GSIM_HIP(hipMemcpy(pos_xy, s->pos[s->cur], sizeof(float2) * s->n, hipMemcpyDeviceToHost));
-        if (vel_xy) GSIM_HIP(hipMemcpy(vel_xy, s->vel[s->cur], sizeof(float2) * s->n, hipMemcpyDeviceToHost));
-        if (mass) GSIM_HIP(hipMemcpy(mass, s->mass, sizeof(float) * s->n, hipMemcpyDeviceToHost));
+    const uint32_t na = (uint32_t)s->na, n = (uint32_t)s->n;
+    const float2 *pos = s->pos[s->cur], *vel = s->vel[s->cur];
+    const float *mass = s->mass;
+    const uint32_t *perm = s->perm[s->cur];  // null for a direct sum
+    if (s->n <= gsim::kReadStageParticles && s->stage.ready()) {
+        const gsim::ReadTarget t = s->stage.target(s->n);
+        GSIM_HIP(gsim::read_launch(pos, vel, mass, perm, na, n, t, nullptr, s->stream));
+        GSIM_HIP(hipStreamSynchronize(s->stream));
+        if (pos_xy) std::memcpy(pos_xy, t.pos, sizeof(float2) * s->n);
+        if (vel_xy) std::memcpy(vel_xy, t.vel, sizeof(float2) * s->n);
+        if (mass_out) std::memcpy(mass_out, t.mass, sizeof(float) * s->n);
         return GSIM_OK;
     }
-    // Barnes-Hut: the state is in the last step's sorted order
-    const size_t na = s->na;
-    std::vector<uint32_t> perm(na);
-    GSIM_HIP(hipMemcpy(perm.data(), s->perm[s->cur], sizeof(uint32_t) * na, hipMemcpyDeviceToHost));
-    std::vector<float> tmp(2 * na);
-    const float *src[3] = {(const float *)s->pos[s->cur], (const float *)s->vel[s->cur], s->mass};
-    float *dst[3] = {pos_xy, vel_xy, mass};
-    for (int a = 0; a < 3; ++a) {
-        if (!dst[a]) continue;
-        const size_t w = a < 2 ? 2 : 1;
-        GSIM_HIP(hipMemcpy(tmp.data(), src[a], sizeof(float) * w * na, hipMemcpyDeviceToHost));
-        unpermute(perm, tmp.data(), dst[a], w, s->n);
+    if (perm) {
+        // Barnes-Hut: the caller's order, in buffers that only a build uses
+        float2 *const stage = (float2 *)s->bh.leaf_sum;
+        const gsim::ReadTarget t{stage, stage + s->na, (float *)s->bh.leaf_key, nullptr};
+        GSIM_HIP(gsim::read_launch(pos, vel, mass, perm, na, n, t, nullptr, s->stream));
+        pos = t.pos;
+        vel = t.vel;
+        mass = t.mass;
     }
+    if (pos_xy) GSIM_HIP(hipMemcpyAsync(pos_xy, pos, sizeof(float2) * s->n, hipMemcpyDeviceToHost, s->stream));
+    if (vel_xy) GSIM_HIP(hipMemcpyAsync(vel_xy, vel, sizeof(float2) * s->n, hipMemcpyDeviceToHost, s->stream));
+    if (mass_out) GSIM_HIP(hipMemcpyAsync(mass_out, mass, sizeof(float) * s->n, hipMemcpyDeviceToHost, s->stream));
+    GSIM_HIP(hipStreamSynchronize(s->stream));
     return GSIM_OK;
 }
 

@@ -60,6 +60,7 @@ void free_batch(gsim_batch *b) {
                     d.leaf_sum, d.leaf_first, d.leaf_key, d.tile_range, d.live_tiles, d.top, d.node4,
                     d.child, d.wave_acc, d.ichunk};
     for (void *p : ptrs) (void)hipFree(p);
+    b->stage.release();
     if (b->stream) (void)hipStreamDestroy(b->stream);
     delete b;
 }
@@ -439,16 +440,33 @@ gsim_status gsim_batch_read(gsim_batch *b, uint32_t id, float *pos_xy, float *ve
     auto it = b->systems.find(id);
     if (it == b->systems.end()) return fail(GSIM_ERROR_INVALID_ARGUMENT, "no system %u in the batch", id);
     GSIM_HIP(hipSetDevice(b->device));
-    GSIM_HIP(hipStreamSynchronize(b->stream));
+    const gsim::BatchSystem &s = it->second;
+    const float2 *pos = b->d.pos[b->cur] + s.off, *vel = b->d.vel[b->cur] + s.off;
+    const float *m = b->d.mass + s.off;
+    const bool staged = s.n <= gsim::kReadStageParticles && b->stage.ready();
+    const gsim::ReadTarget t = staged ? b->stage.target(s.n) : gsim::ReadTarget{};
     uint32_t stall = 0;
-    GSIM_HIP(hipMemcpy(&stall, &b->d.counts->sort_stall, sizeof(stall), hipMemcpyDeviceToHost));
+    if (staged) {
+        GSIM_HIP(gsim::read_launch(pos, vel, m, nullptr, s.na, s.n, t, &b->d.counts->sort_stall,
+                                   b->stream));
+        GSIM_HIP(hipStreamSynchronize(b->stream));
+        stall = *t.stall;
+    } else {
+        GSIM_HIP(hipStreamSynchronize(b->stream));
+        GSIM_HIP(hipMemcpy(&stall, &b->d.counts->sort_stall, sizeof(stall), hipMemcpyDeviceToHost));
+    }
     if (stall)
         return fail(GSIM_ERROR_DEVICE, "radix sort look-back gave up on %u status words: the batch state is invalid",
                     stall);
-    const gsim::BatchSystem &s = it->second;
-    if (pos_xy) GSIM_HIP(hipMemcpy(pos_xy, b->d.pos[b->cur] + s.off, sizeof(float2) * s.n, hipMemcpyDeviceToHost));
-    if (vel_xy) GSIM_HIP(hipMemcpy(vel_xy, b->d.vel[b->cur] + s.off, sizeof(float2) * s.n, hipMemcpyDeviceToHost));
-    if (mass) GSIM_HIP(hipMemcpy(mass, b->d.mass + s.off, sizeof(float) * s.n, hipMemcpyDeviceToHost));
+    if (staged) {
+        if (pos_xy) std::memcpy(pos_xy, t.pos, sizeof(float2) * s.n);
+        if (vel_xy) std::memcpy(vel_xy, t.vel, sizeof(float2) * s.n);
+        if (mass) std::memcpy(mass, t.mass, sizeof(float) * s.n);
+        return GSIM_OK;
+    }
+    if (pos_xy) GSIM_HIP(hipMemcpy(pos_xy, pos, sizeof(float2) * s.n, hipMemcpyDeviceToHost));
+    if (vel_xy) GSIM_HIP(hipMemcpy(vel_xy, vel, sizeof(float2) * s.n, hipMemcpyDeviceToHost));
+    if (mass) GSIM_HIP(hipMemcpy(mass, m, sizeof(float) * s.n, hipMemcpyDeviceToHost));
     return GSIM_OK;
 }
 

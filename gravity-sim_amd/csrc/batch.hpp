@@ -152,6 +152,7 @@ struct gsim_batch {
     int cur = 0;
     hipGraphExec_t graph[2] = {nullptr, nullptr};
     gsim::BatchTune tune;
+    gsim::ReadStage stage;
     uint64_t steps = 0;
     // host mirror of the membership arrays
     std::vector<gsim::SysDesc> h_desc;

@@ -181,6 +181,26 @@ __host__ __device__ inline size_t ds_sym_jbase(uint32_t g, uint32_t B) {
     return (size_t)g * B - (size_t)kDsSymRows * g * (g - (g ? 1u : 0u)) / 2;
 }
 
+// Readback (read_kernels.hip): where the particles go, device memory or pinned
+// host memory, and the pinned block that a handle keeps for small reads (made
+// by the second one, freed with the handle).
+struct ReadTarget {
+    float2 *pos, *vel;
+    float *mass;
+    uint32_t *stall;
+};
+constexpr size_t kReadStageParticles = 16384;
+struct ReadStage {
+    void *block = nullptr;
+    bool read_before = false;
+    bool ready();
+    void release();
+    ReadTarget target(size_t n) const;
+};
+hipError_t read_launch(const float2 *pos, const float2 *vel, const float *mass,
+                       const uint32_t *perm, uint32_t na, uint32_t n, const ReadTarget &out,
+                       const uint32_t *stall, hipStream_t stream);
+
 }  // namespace gsim
 
 struct gsim_sim {
@@ -227,6 +247,7 @@ struct gsim_sim {
     gsim::DsSymPlan ds_plan{};
     // Barnes-Hut
     gsim::BhBuffers bh;
+    gsim::ReadStage stage;
     // debug / timing
     float2 *accel = nullptr;
     uint32_t debug_flags = 0;
