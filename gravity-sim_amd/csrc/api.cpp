@@ -371,8 +371,13 @@ gsim_status gsim_create(const gsim_params *params, const float *pos_xy, const fl
 
     if (params->algorithm == GSIM_DIRECT_SUM) {
         gsim::ds_pick_shape(na, &s->ds_R, &s->ds_S);
-        gsim_status st = ds_configure(s, gsim::ds_sym_default(na),
-                                      gsim::ds_block_default(na));
+        const bool sym = gsim::ds_sym_default(na), block = gsim::ds_block_default(na);
+        gsim_status st = ds_configure(s, sym, block);
+        if (st == GSIM_ERROR_OUT_OF_MEMORY && sym) {  // the slices need far less
+            (void)hipGetLastError();
+            gsim::clear_error();
+            st = ds_configure(s, false, block);
+        }
         if (st != GSIM_OK) return bail(st);
     } else {
         e = gsim::bh_alloc(&s->bh, na, gsim::kTreeDepth);

@@ -13,6 +13,7 @@
 // in SGPRs: no LDS traffic and no VALU cycles spent on broadcast.  Each slice
 // writes a partial acceleration; the combine kernel adds the S partials in
 // slice order (deterministic) and integrates.
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <mutex>
@@ -162,7 +163,7 @@ __global__ __launch_bounds__(256) void ds_combine_kernel(
 // interactions; only its upper triangle is evaluated, each pair (i, j) once,
 // adding  m_j d inv^3  to a_i and  -m_i d inv^3  to a_j (d = p_j - p_i; the
 // pair's r2 and inv are the same numbers from either side).  Row groups of
-// kDsSymRows blocks sit in one wave (each lane holds one particle of every row
+// R blocks sit in one wave (each lane holds one particle of every row
 // block); a workgroup tile is one row group times 4 * `cols` column blocks,
 // `cols` per wave.  For a column
 // block the wave holds one source particle per lane and rotates the sources,
@@ -170,8 +171,8 @@ __global__ __launch_bounds__(256) void ds_combine_kernel(
 // 64 steps every lane has met every source once and each reaction is back in
 // its owner's lane.  Per pair: 12 VALU + 1 v_rsq_f32 for two interactions,
 // against 9 + 1 for one in the one-sided kernel; the 5 rotates per step are
-// shared by the group's 16 rows (16 rows beat 8 by 3-5%: 0.420 against 0.431
-// ms/step at 50k, 1.537 against 1.609 at 100k).
+// shared by the group's rows.  The pairs are kept in the order written: 200,000
+// particles 5,939 -> 5,757 us a step, 45 clocks a pair.
 //
 // Partial sums, both in fixed order: per tile, each row particle's sum over
 // the tile's columns (ipart; the four waves' sums added in wave order through
@@ -192,18 +193,17 @@ __device__ __forceinline__ float ror1(float v) {
 // One column block against the wave's row blocks.  kInGroup: the column lies
 // inside the row group, so rows below it are skipped, the diagonal row is
 // one-sided and only rows above it react.
-template <bool kInGroup>
-__device__ __forceinline__ void ds_sym_column(const float (&ix)[kDsSymRows],
-                                              const float (&iy)[kDsSymRows],
-                                              const float (&im)[kDsSymRows],
-                                              float (&aix)[kDsSymRows], float (&aiy)[kDsSymRows],
-                                              float jx, float jy, float jm, float &ajx_out,
-                                              float &ajy_out, float eps2, uint32_t I0, uint32_t J) {
+template <bool kInGroup, int R>
+__device__ __forceinline__ void ds_sym_column(const float (&ix)[R], const float (&iy)[R],
+                                              const float (&im)[R], float (&aix)[R],
+                                              float (&aiy)[R], float jx, float jy, float jm,
+                                              float &ajx_out, float &ajy_out, float eps2,
+                                              uint32_t I0, uint32_t J) {
     float ajx = 0.0f, ajy = 0.0f;
 #pragma unroll 2
     for (int k = 0; k < 64; ++k) {
 #pragma unroll
-        for (int r = 0; r < kDsSymRows; ++r) {
+        for (int r = 0; r < R; ++r) {
             if (kInGroup && I0 + r > J) continue;
             const float dx = jx - ix[r], dy = jy - iy[r];
             const float r2 = __builtin_fmaf(dx, dx, __builtin_fmaf(dy, dy, eps2));
@@ -217,6 +217,7 @@ __device__ __forceinline__ void ds_sym_column(const float (&ix)[kDsSymRows],
                 ajx = __builtin_fmaf(-dx, tj, ajx);
                 ajy = __builtin_fmaf(-dy, tj, ajy);
             }
+            __builtin_amdgcn_sched_barrier(0);
         }
         jx = ror1(jx);
         jy = ror1(jy);
@@ -240,12 +241,12 @@ __device__ __forceinline__ uint32_t ds_sym_group(uint32_t t, uint32_t G, uint32_
     return lo;
 }
 
+template <int R>
 __global__ __launch_bounds__(256) void ds_sym_kernel(const float2 *__restrict__ pos,
                                                      const float *__restrict__ mass,
                                                      float2 *__restrict__ ipart,
                                                      float2 *__restrict__ jpart, uint32_t B,
                                                      uint32_t G, uint32_t cols, float eps2) {
-    constexpr int R = kDsSymRows;
     __shared__ float2 red[3][R][64];  // row sums of waves 1..3
     const uint32_t lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const uint32_t T = blockIdx.x;  // one tile per workgroup
@@ -268,16 +269,16 @@ __global__ __launch_bounds__(256) void ds_sym_kernel(const float2 *__restrict__ 
         aix[r] = 0.0f;
         aiy[r] = 0.0f;
     }
-    const size_t jrow = ds_sym_jbase(g, B);
+    const size_t jrow = ds_sym_jbase(g, B, R);
     for (uint32_t J = J0; J < J1; ++J) {
         const uint32_t j = J * 64 + lane;
         const float2 q = pos[j];
         const float qm = mass[j];
         float ajx, ajy;
         if (J >= I0 + R)
-            ds_sym_column<false>(ix, iy, im, aix, aiy, q.x, q.y, qm, ajx, ajy, eps2, I0, J);
+            ds_sym_column<false, R>(ix, iy, im, aix, aiy, q.x, q.y, qm, ajx, ajy, eps2, I0, J);
         else
-            ds_sym_column<true>(ix, iy, im, aix, aiy, q.x, q.y, qm, ajx, ajy, eps2, I0, J);
+            ds_sym_column<true, R>(ix, iy, im, aix, aiy, q.x, q.y, qm, ajx, ajy, eps2, I0, J);
         jpart[(jrow + (J - I0)) * 64 + lane] = make_float2(ajx, ajy);
     }
     if (w > 0) {
@@ -303,10 +304,10 @@ __global__ __launch_bounds__(256) void ds_sym_kernel(const float2 *__restrict__ 
 // One workgroup per 64-particle block: its four waves each add a quarter of
 // the block's partial list in order, then the quarters are added in order.
 __global__ __launch_bounds__(256) void ds_sym_combine_kernel(
-    const float2 *__restrict__ ipart, const float2 *__restrict__ jpart, uint32_t B, uint32_t width,
+    const float2 *__restrict__ ipart, const float2 *__restrict__ jpart, uint32_t B, uint32_t R,
+    uint32_t width,
     const float2 *__restrict__ pos, const float2 *__restrict__ vel, float2 *__restrict__ pos_out,
     float2 *__restrict__ vel_out, float2 *__restrict__ acc_dbg, float kv, float dt) {
-    constexpr uint32_t R = kDsSymRows;
     __shared__ float2 q[4][64];
     const uint32_t P = blockIdx.x, lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const uint32_t g = P / R, r = P % R;
@@ -319,7 +320,7 @@ __global__ __launch_bounds__(256) void ds_sym_combine_kernel(
     auto addr = [&](uint32_t e) -> size_t {
         if (e < ni) return ((tb + e) * R + r) * 64 + lane;
         const uint32_t h = e - ni;
-        return (ds_sym_jbase(h, B) + (P - h * R)) * 64 + lane;
+        return (ds_sym_jbase(h, B, R) + (P - h * R)) * 64 + lane;
     };
     float ax = 0.0f, ay = 0.0f;
     uint32_t e = lo;
@@ -361,20 +362,26 @@ __global__ __launch_bounds__(256) void ds_sym_combine_kernel(
 DsSymPlan ds_sym_plan(size_t na, uint32_t cols) {
     DsSymPlan p{};
     p.B = (uint32_t)(na / 64);
-    p.G = (p.B + kDsSymRows - 1) / kDsSymRows;
-    auto tiles = [&](uint32_t width) -> size_t {
-        const uint32_t cb = (p.B + width - 1) / width, step = kDsSymRows / width;
-        return ds_sym_tile_base(p.G, cb, step);
-    };
-    // Two columns per wave once that still gives ~32k waves.  Measured
-    // (ms/step, 1 / 2 columns): 20k 0.101 / 0.118, 50k 0.424 / 0.432, 100k
-    // 1.639 / 1.607.
-    if (cols == 0) cols = tiles(8) * 4 >= kDsSymMinWaves ? 2 : 1;
+    // Few rows make many small tiles, which fill the GPU and end together at
+    // small sizes; many rows share the rotates and shrink the column partials.
+    // Measured (us a step, rows x cols):
+    //             4 x 1   8 x 1  16 x 1  16 x 2  16 x 4
+    //    16,384    61.7    67.2    85.2   112.5
+    //    25,000   117.5   118.5   123.7   157.9
+    //    35,000   210.0   205.1   219.6   231.6
+    //    50,000   414.0   394.2   403.9   421.0   445.5
+    //   100,000  1602    1502    1468    1472    1496
+    //   200,000  6370    5953    5817    5739    5749
+    //   300,001                 13000   12800   12751
+    p.rows = na < 28672 ? 4 : na < 65536 ? 8 : 16;
+    if (cols == 0) cols = na < 131072 ? 1 : na < 262144 ? 2 : 4;
+    cols = std::min(cols, p.rows / 4);  // the width divides the rows
+    p.G = (p.B + p.rows - 1) / p.rows;
     p.cols = cols;
     p.width = 4 * cols;
-    p.ntiles = (uint32_t)tiles(p.width);
-    p.ipart = (size_t)p.ntiles * kDsSymRows * 64;
-    p.jpart = ds_sym_jbase(p.G, p.B) * 64;
+    p.ntiles = (uint32_t)ds_sym_tile_base(p.G, (p.B + p.width - 1) / p.width, p.rows / p.width);
+    p.ipart = (size_t)p.ntiles * p.rows * 64;
+    p.jpart = ds_sym_jbase(p.G, p.B, p.rows) * 64;
     return p;
 }
 
@@ -413,9 +420,9 @@ hipError_t ds_launch_partial(gsim_sim *s, const float2 *pos, const float *mass) 
     const uint32_t na = (uint32_t)s->na;
     if (s->ds_sym) {
         const DsSymPlan &p = s->ds_plan;
-        ds_sym_kernel<<<p.ntiles, 256, 0, s->stream>>>(pos, mass, s->partial,
-                                                       s->partial + p.ipart, p.B, p.G, p.cols,
-                                                       s->eps2);
+        auto *k = p.rows == 4 ? ds_sym_kernel<4> : p.rows == 8 ? ds_sym_kernel<8> : ds_sym_kernel<16>;
+        k<<<p.ntiles, 256, 0, s->stream>>>(pos, mass, s->partial, s->partial + p.ipart, p.B, p.G,
+                                           p.cols, s->eps2);
         return hipGetLastError();
     }
     const uint32_t R = s->ds_R, S = s->ds_S;
@@ -444,7 +451,7 @@ hipError_t ds_launch_combine(gsim_sim *s, const float2 *pos, const float2 *vel,
     if (s->ds_sym) {
         const DsSymPlan &p = s->ds_plan;
         ds_sym_combine_kernel<<<p.B, 256, 0, s->stream>>>(s->partial, s->partial + p.ipart, p.B,
-                                                          p.width, pos, vel, pos_out, vel_out, acc,
+                                                          p.rows, p.width, pos, vel, pos_out, vel_out, acc,
                                                           s->kv, s->dt);
         return hipGetLastError();
     }

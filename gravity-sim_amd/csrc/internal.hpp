@@ -151,34 +151,33 @@ struct PhaseEvents {
     bool bh;
 };
 
-// Symmetric direct sum (ds_kernels.hip): row groups of kDsSymRows 64-particle
+// Symmetric direct sum (ds_kernels.hip): row groups of `rows` 64-particle
 // blocks; a workgroup tile is a row group times `width` = 4 x cols column
-// blocks (width divides kDsSymRows, so the tile count of each group has a
-// closed form).
-constexpr uint32_t kDsSymRows = 16;
-constexpr size_t kDsSymMinParticles = 16384;   // default range of the symmetric kernel
-constexpr size_t kDsSymMaxParticles = 262144;  // (its partial sums grow as N^2 / 64)
-constexpr size_t kDsSymMinWaves = 32768;       // auto: 2 columns per wave from this many waves
+// blocks (width divides rows, so the tile count of each group has a closed
+// form).
+constexpr size_t kDsSymMinParticles = 16384;    // default range of the symmetric kernel
+constexpr size_t kDsSymMaxParticles = 524288;   // (its partial sums grow as N^2: 2.2 GB here)
 
 // Targets of one workgroup of the block kernel, and of one batch work item.
 constexpr uint32_t kDsBlockTargets = 16;
 
 struct DsSymPlan {
     uint32_t B = 0, G = 0;      // 64-particle blocks, row groups
-    uint32_t cols = 0;          // column blocks per wave (1 or 2)
+    uint32_t rows = 0;          // blocks per row group (4, 8 or 16)
+    uint32_t cols = 0;          // column blocks per wave (1, 2 or 4)
     uint32_t width = 0;         // column blocks per workgroup tile (4 x cols)
     uint32_t ntiles = 0;        // workgroups of the force launch
     size_t ipart = 0, jpart = 0;  // float2 entries of the two partial arrays
 };
 
 // First tile of row group g: sum over h < g of ceil((B - R h) / width)
-// = g * cb - step * g (g - 1) / 2 with cb = ceil(B / width), step = R / width.
+// = g * cb - step * g (g - 1) / 2 with cb = ceil(B / width), step = rows / width.
 __host__ __device__ inline size_t ds_sym_tile_base(uint32_t g, uint32_t cb, uint32_t step) {
     return (size_t)g * cb - (size_t)step * g * (g - (g ? 1u : 0u)) / 2;
 }
-// First column-partial row of group g: sum over h < g of (B - R h).
-__host__ __device__ inline size_t ds_sym_jbase(uint32_t g, uint32_t B) {
-    return (size_t)g * B - (size_t)kDsSymRows * g * (g - (g ? 1u : 0u)) / 2;
+// First column-partial row of group g: sum over h < g of (B - rows h).
+__host__ __device__ inline size_t ds_sym_jbase(uint32_t g, uint32_t B, uint32_t rows) {
+    return (size_t)g * B - (size_t)rows * g * (g - (g ? 1u : 0u)) / 2;
 }
 
 // Readback (read_kernels.hip): where the particles go, device memory or pinned

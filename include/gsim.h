@@ -172,9 +172,10 @@ typedef enum gsim_tuning {
     GSIM_TUNE_BH_WAVES_PER_SIMD = 2,  /* 1..8; no effect                               */
     GSIM_TUNE_BH_TRAVERSAL = 3,       /* 0..3 or 6; no effect                          */
     GSIM_TUNE_DS_SYMMETRIC = 4,       /* 0/1: each pair once (Newton's third law); the
-                                         default for 16,384 <= Na <= 262,144           */
+                                         default for 16,384 <= Na <= 524,288 (where its
+                                         partial sums fit in memory)                   */
     GSIM_TUNE_DS_SYM_COLS = 5,        /* symmetric kernel: 1 or 2 column blocks per
-                                         wave, 0 = by size                              */
+                                         wave (at most 1 below 28,672), 0 = by size     */
     GSIM_TUNE_BH_SEGMENTS = 6,        /* 1..65536; no effect                           */
     GSIM_TUNE_BH_SPLIT = 7,           /* 0..1000; no effect                            */
     GSIM_TUNE_BH_ADAPTIVE_BOX = 8,    /* 0/1, beyond the reference and off by default:
