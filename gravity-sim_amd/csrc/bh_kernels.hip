@@ -144,13 +144,11 @@ __global__ __launch_bounds__(kSortThreads) void bh_keys_kernel(
     __shared__ uint32_t h[kPasses][256];
     const uint32_t t = threadIdx.x;
     const uint32_t g = blockIdx.x * kSortThreads + t, stride = gridDim.x * kSortThreads;
-    for (uint32_t j = g; j < 2 * kTiles; j += stride) tile_range[j] = 0;
+    for (uint32_t j = g; j < kTileWords; j += stride) tile_range[j] = 0;
     for (uint32_t j = g; j < kDigitCopies * 1024; j += stride) digit_next[j] = 0;
     for (uint32_t j = g; j < status_words; j += stride) status[j] = 0;
     if (g == 0) {
         ctr->sort_stall = 0;
-        ctr->tiles_busy = 0;
-        ctr->tiles_done = 0;
     }
 #pragma unroll
     for (int p = 0; p < kPasses; ++p) h[p][t] = 0;
@@ -437,7 +435,7 @@ __global__ __launch_bounds__(256) void bh_leaf_kernel(
     const uint32_t *__restrict__ cpos, const BhCounters *__restrict__ ctr, int bits,
     float4 *__restrict__ leaf_sum, uint32_t *__restrict__ tile_range,
     float4 *__restrict__ node4, uint4 *__restrict__ child, float4 *__restrict__ nsum,
-    const float *__restrict__ box, uint32_t *__restrict__ tiles_busy) {
+    const float *__restrict__ box) {
     __shared__ float4 stage[4][64];
     const uint32_t n_in = ctr->n_in, nl = ctr->n_leaves, ncells = ctr->n_cells;
     const bool deep = nsum != nullptr;
@@ -485,7 +483,6 @@ __global__ __launch_bounds__(256) void bh_leaf_kernel(
             const uint32_t T = leaf_key[L] >> 10;
             if (L == 0 || (leaf_key[L - 1] >> 10) != T) {
                 tile_range[2 * T] = L;
-                atomicAdd(tiles_busy, 1u);
             }
             if (L + 1 == nl || (leaf_key[L + 1] >> 10) != T) tile_range[2 * T + 1] = L + 1;
         }
@@ -588,7 +585,7 @@ __global__ __launch_bounds__(256) void bh_gran_kernel(
     const float4 *__restrict__ nsum, const uint32_t *__restrict__ gran_first,
     const uint32_t *__restrict__ gran_key, float4 *__restrict__ gran_sum,
     uint32_t *__restrict__ gran_y, uint32_t *__restrict__ tile_range,
-    uint32_t *__restrict__ tiles_busy, const float *__restrict__ box) {
+    const float *__restrict__ box) {
     const uint32_t n_in = ctr->n_in, n_nodes = ctr->n_nodes, ng = ctr->n_gran;
     const float r0 = box ? box[3] : kFixedR0;
     for (uint32_t L = blockIdx.x * 256 + threadIdx.x; L < ng; L += gridDim.x * 256) {
@@ -610,7 +607,6 @@ __global__ __launch_bounds__(256) void bh_gran_kernel(
         const uint32_t T = gran_key[L] >> 10;
         if (L == 0 || (gran_key[L - 1] >> 10) != T) {
             tile_range[2 * T] = L;
-            atomicAdd(tiles_busy, 1u);
         }
         if (L + 1 == ng || (gran_key[L + 1] >> 10) != T) tile_range[2 * T + 1] = L + 1;
     }
@@ -624,49 +620,111 @@ __device__ __forceinline__ int tile_level_offset(int d) {
     return d == 9 ? 0 : d == 8 ? 256 : d == 7 ? 320 : d == 6 ? 336 : 340;
 }
 
-// The last occupied tile's workgroup to finish (a device-scope counter,
-// zeroed by the keys kernel, against the number of occupied tiles the leaf
-// pass counted) also reduces the 1024 depth-5 cells to the root and writes
-// depths 4..0, so the top needs no launch of its own.  Only occupied tiles
-// write their record to `top` (fenced before they count); empty tiles return
-// at once, and the last workgroup takes their empty record from tile_range.
+// A tile's record for the workgroup that reduces the top, on any XCD: each
+// word is stored at the scope of the device and has arrived before the call
+// returns, and is loaded at that scope, past the XCD's own L2.  A fence would
+// write that whole L2 back, once a tile.
+__device__ __forceinline__ void publish_top(TileCell *to, const TileCell &c) {
+    uint32_t *w = reinterpret_cast<uint32_t *>(to);
+    status_store(w + 0, c.n);
+    status_store(w + 1, c.y);
+    status_store(w + 2, c.f);
+    status_store(w + 4, __float_as_uint(c.sx));
+    status_store(w + 5, __float_as_uint(c.sy));
+    status_store(w + 6, __float_as_uint(c.sm));
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+}
+
+__device__ __forceinline__ TileCell published_top(const TileCell *from) {
+    const uint32_t *w = reinterpret_cast<const uint32_t *>(from);
+    TileCell c;
+    c.n = status_load(w + 0);
+    c.y = status_load(w + 1);
+    c.f = status_load(w + 2);
+    c.pad = 0u;
+    c.sx = __uint_as_float(status_load(w + 4));
+    c.sy = __uint_as_float(status_load(w + 5));
+    c.sm = __uint_as_float(status_load(w + 6));
+    c.pad2 = 0.0f;
+    return c;
+}
+
+// The last occupied tile's workgroup to finish also reduces the 1024 depth-5
+// cells to the root and writes depths 4..0, so the top needs no launch of its
+// own.  Occupied tiles publish their record, then count themselves done in
+// their group of 32 tiles; the last of a group counts the group done, and the
+// last group's workgroup goes on.  How many to expect is read from tile_range.
+// One counter for all tiles is a chain of 1024 same-address atomics across the
+// XCDs, and the fence it needs writes an L2 back for each.  Empty tiles return
+// at once; their empty record comes from tile_range.
+// Bound by latency: its chain of loads, six levels and two counts.  53.3 ->
+// 14.5 us with every tile occupied (200,000 particles, adaptive box), 12.7 ->
+// 8.1 us at 500,000 in the fixed domain, 16.3 -> 8.2 us at 5,000: the counters
+// a cache line apart 57 -> 22, the smaller LDS image and the loads ahead of it
+// the rest.
 __global__ __launch_bounds__(256) void bh_tile_kernel(
-    const uint32_t *__restrict__ tile_range, const uint32_t *__restrict__ leaf_first,
+    uint32_t *__restrict__ tile_range, const uint32_t *__restrict__ leaf_first,
     const uint32_t *__restrict__ leaf_key, const float4 *__restrict__ leaf_sum,
     const int8_t *__restrict__ sdep, const uint32_t *__restrict__ cpos,
     float4 *__restrict__ node4, uint4 *__restrict__ child, TileCell *__restrict__ top,
-    const float *__restrict__ box, const uint32_t *__restrict__ leaf_y,
-    BhCounters *__restrict__ ctr) {
+    const float *__restrict__ box, const uint32_t *__restrict__ leaf_y) {
     // leaf_y (15-bit leaves): the depth-10 records are granules whose subtree
     // size is given; otherwise leaves of n particles, y = n + [n >= 2].  The
     // depth-10 nodes themselves are already written.
-    __shared__ TileCell l10[1024];
+    // the depth-10 cells {sums, particles} and {subtree size, first particle}:
+    // 35 KB with `up`, so all 1024 workgroups are resident (four a CU)
+    __shared__ float4 sum10[1024];
+    __shared__ uint2 yf10[1024];
     __shared__ TileCell up[341];
-    __shared__ uint32_t last;
+    __shared__ uint32_t last, wave_groups[4];
     const uint32_t T = blockIdx.x, t = threadIdx.x;
     const uint32_t lb = tile_range[2 * T], le = tile_range[2 * T + 1];
     if (lb == le) return;  // the whole workgroup: an empty tile
+    uint32_t *const done = tile_range + 2 * kTiles;  // 32 words apart; the groups' last
+    const uint2 *const range = reinterpret_cast<const uint2 *>(tile_range);
+    uint32_t expect = 0;  // occupied tiles of this tile's group
+    if (t >= 192) {  // the wave that publishes: it emits fewest cells
+        const uint2 r = range[(T & ~31u) + (t & 31u)];
+        expect = (uint32_t)__popcll(__ballot(t < 224 && r.x != r.y));
+    }
     const float r0 = box ? box[3] : kFixedR0;
-    for (uint32_t c = t; c < 1024; c += 256)
-        l10[c] = TileCell{0u, 0u, 0xffffffffu, 0u, 0.0f, 0.0f, 0.0f, 0.0f};
-    lds_barrier();
     // a tile holds at most 1024 leaves (granules): four per thread, loaded
     // together
+    struct Leaf {
+        float4 s;
+        uint32_t k, f, y;
+    };
+    auto leaf = [&](uint32_t u) {
+        const uint32_t L = min(lb + t + 256 * u, le - 1);
+        return Leaf{leaf_sum[L], leaf_key[L], leaf_first[L], leaf_y ? leaf_y[L] : 0u};
+    };
+    const Leaf a0 = leaf(0), a1 = leaf(1), a2 = leaf(2), a3 = leaf(3);
 #pragma unroll
     for (uint32_t u = 0; u < 4; ++u) {
-        const uint32_t L = lb + t + 256 * u;
-        if (L >= le) break;
-        const uint32_t c = leaf_key[L] & 1023u;
-        const float4 s = leaf_sum[L];
-        const uint32_t n = __float_as_uint(s.w);
-        const uint32_t y = leaf_y ? leaf_y[L] : n + (n >= 2u ? 1u : 0u);
-        l10[c] = TileCell{n, y, leaf_first[L], 0u, s.x, s.y, s.z, 0.0f};
+        sum10[t + 256 * u] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        yf10[t + 256 * u] = make_uint2(0u, 0xffffffffu);
     }
     lds_barrier();
-    {
-        const uint32_t c = t;  // 256 depth-9 cells
-        up[c] = reduce4(l10[4 * c], l10[4 * c + 1], l10[4 * c + 2], l10[4 * c + 3]);
-    }
+    auto place = [&](uint32_t u, const Leaf &a) {
+        if (lb + t + 256 * u >= le) return;
+        const uint32_t c = a.k & 1023u, n = __float_as_uint(a.s.w);
+        sum10[c] = a.s;
+        yf10[c] = make_uint2(leaf_y ? a.y : n + (n >= 2u ? 1u : 0u), a.f);
+    };
+    place(0, a0);
+    place(1, a1);
+    place(2, a2);
+    place(3, a3);
+    lds_barrier();
+    auto kid = [&](uint32_t u) {  // of depth-9 cell t
+        const float4 s = sum10[4 * t + u];
+        const uint2 q = yf10[4 * t + u];
+        return TileCell{__float_as_uint(s.w), q.x, q.y, 0u, s.x, s.y, s.z, 0.0f};
+    };
+    const TileCell k0 = kid(0), k1 = kid(1), k2 = kid(2), k3 = kid(3);
+    const uint4 sizes9 = make_uint4(k0.y, k1.y, k2.y, k3.y);
+    const TileCell c9 = reduce4(k0, k1, k2, k3);
+    up[t] = c9;
     lds_barrier();
     for (int d = 8; d >= 5; --d) {
         const uint32_t cnt = 1u << (2 * (d - 5));
@@ -676,33 +734,47 @@ __global__ __launch_bounds__(256) void bh_tile_kernel(
                                 up[oc + 4 * t + 3]);
         lds_barrier();
     }
-    for (uint32_t c = t; c < 341; c += 256) {
-        const int d = c < 256 ? 9 : c < 320 ? 8 : c < 336 ? 7 : c < 340 ? 6 : 5;
-        const TileCell *kids =
-            d == 9 ? l10 + 4 * c : up + tile_level_offset(d + 1) + 4 * (c - tile_level_offset(d));
+    if (t == 192) {
+        publish_top(top + T, up[340]);
+        last = atomicAdd(done + T / 32 * 32, 1u) + 1u == expect ? 1u : 0u;
+    }
+    if (t < 85) {  // depths 8..5
+        const uint32_t c = 256 + t;
+        const int d = c < 320 ? 8 : c < 336 ? 7 : c < 340 ? 6 : 5;
+        const TileCell *kids = up + tile_level_offset(d + 1) + 4 * (c - tile_level_offset(d));
         emit_cell(up[c], d, sizes4(kids), sdep, cpos, node4, child, r0);
     }
-    if (t == 0) {
-        top[T] = up[340];
-        __threadfence();  // top[T] before the count (release)
-        last = atomicAdd(&ctr->tiles_done, 1u) + 1u == ctr->tiles_busy ? 1u : 0u;
-    }
-    // a full barrier: thread 0's acquire of the other tiles' top[] is handed
-    // on to the whole workgroup
-    __syncthreads();
+    emit_cell(c9, 9, sizes9, sdep, cpos, node4, child, r0);
+    lds_barrier();
     if (!last) return;
-    __threadfence();  // every tile's top[] after the count (acquire)
+    const uint4 ra = reinterpret_cast<const uint4 *>(tile_range)[2 * t];
+    const uint4 rb = reinterpret_cast<const uint4 *>(tile_range)[2 * t + 1];
+    const bool in0 = ra.x != ra.y, in1 = ra.z != ra.w, in2 = rb.x != rb.y, in3 = rb.z != rb.w;
+    // groups with an occupied tile: eight threads a group, eight groups a wave
+    unsigned long long m = __ballot(in0 || in1 || in2 || in3);
+    m |= m >> 4;
+    m |= m >> 2;
+    m |= m >> 1;
+    if ((t & 63) == 0)
+        wave_groups[t >> 6] = (uint32_t)__popcll(m & 0x0101010101010101ull);
+    lds_barrier();
+    if (t == 0)
+        last = atomicAdd(done + 32 * 32, 1u) + 1u ==
+                       wave_groups[0] + wave_groups[1] + wave_groups[2] + wave_groups[3]
+                   ? 1u
+                   : 0u;
+    lds_barrier();
+    if (!last) return;
+    asm volatile("" ::: "memory");  // no record is read before the counts
     // depths 4..0 in `up` at the offsets of depths 9..5
-    TileCell c4[4];
-#pragma unroll
-    for (uint32_t u = 0; u < 4; ++u) {
-        const uint32_t q = 4 * t + u;
-        c4[u] = tile_range[2 * q] != tile_range[2 * q + 1]
-                    ? top[q]
-                    : TileCell{0u, 0u, 0xffffffffu, 0u, 0.0f, 0.0f, 0.0f, 0.0f};
-    }
-    up[t] = reduce4(c4[0], c4[1], c4[2], c4[3]);
-    emit_cell(up[t], 4, sizes4(c4), sdep, cpos, node4, child, r0);
+    const TileCell empty{0u, 0u, 0xffffffffu, 0u, 0.0f, 0.0f, 0.0f, 0.0f};
+    const TileCell t0 = in0 ? published_top(top + 4 * t) : empty;
+    const TileCell t1 = in1 ? published_top(top + 4 * t + 1) : empty;
+    const TileCell t2 = in2 ? published_top(top + 4 * t + 2) : empty;
+    const TileCell t3 = in3 ? published_top(top + 4 * t + 3) : empty;
+    const TileCell c4 = reduce4(t0, t1, t2, t3);
+    up[t] = c4;
+    emit_cell(c4, 4, make_uint4(t0.y, t1.y, t2.y, t3.y), sdep, cpos, node4, child, r0);
     lds_barrier();
     for (int d = 3; d >= 0; --d) {
         const uint32_t cnt = 1u << (2 * d);
@@ -967,7 +1039,7 @@ hipError_t bh_alloc(BhBuffers *b, size_t na, uint32_t bits) {
     GSIM_ALLOC(b->leaf_first, na + 1);
     GSIM_ALLOC(b->leaf_key, na);
     GSIM_ALLOC(b->leaf_sum, na);
-    GSIM_ALLOC(b->tile_range, 2 * kTiles);
+    GSIM_ALLOC(b->tile_range, kTileWords);
     GSIM_ALLOC(b->top, kTiles);
     GSIM_ALLOC(b->node4, b->cap);
     GSIM_ALLOC(b->child, b->cap);
@@ -1086,7 +1158,7 @@ hipError_t bh_launch_build(gsim_sim *s, const float2 *pos, const float *mass,
     const uint32_t lb = pb < kLeafBlocks ? pb : kLeafBlocks;
     bh_leaf_kernel<<<lb, 256, 0, s->stream>>>(b.leaf_first, b.leaf_key, b.cpos, b.ctr, bits,
                                               b.leaf_sum, b.tile_range, b.node4, b.child,
-                                              deep ? b.nsum : nullptr, box, &b.ctr->tiles_busy);
+                                              deep ? b.nsum : nullptr, box);
     if (deep) {
         // sparse levels below depth 10, then depth-10 records for the dense path
         for (int d = (int)kDeepBits - 1; d > (int)kTreeDepth; --d)
@@ -1094,15 +1166,14 @@ hipError_t bh_launch_build(gsim_sim *s, const float2 *pos, const float *mass,
                                                        b.child, b.nsum, d, box);
         bh_gran_kernel<<<pb, 256, 0, s->stream>>>(sk, b.sdep, b.cpos, b.ctr, b.node4, b.child,
                                                   b.nsum, b.gran_first, b.gran_key, b.leaf_sum,
-                                                  b.gran_y, b.tile_range, &b.ctr->tiles_busy,
-                                                  box);
+                                                  b.gran_y, b.tile_range, box);
         bh_tile_kernel<<<kTiles, 256, 0, s->stream>>>(b.tile_range, b.gran_first, b.gran_key,
                                                       b.leaf_sum, b.sdep, b.cpos, b.node4,
-                                                      b.child, b.top, box, b.gran_y, b.ctr);
+                                                      b.child, b.top, box, b.gran_y);
     } else {
         bh_tile_kernel<<<kTiles, 256, 0, s->stream>>>(b.tile_range, b.leaf_first, b.leaf_key,
                                                       b.leaf_sum, b.sdep, b.cpos, b.node4,
-                                                      b.child, b.top, box, nullptr, b.ctr);
+                                                      b.child, b.top, box, nullptr);
     }
     return hipGetLastError();
 }

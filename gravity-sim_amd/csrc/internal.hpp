@@ -42,6 +42,7 @@ constexpr uint32_t kDeepBits = 15;
 constexpr uint32_t kKilledKeyDeep = 1u << 30;  // sorts after every 30-bit cell
 constexpr uint32_t kTileDepth = 5;          // tile kernel: one depth-5 cell per workgroup
 constexpr uint32_t kTiles = 1u << (2 * kTileDepth);
+constexpr uint32_t kTileWords = 2 * kTiles + 33 * 32;  // BhBuffers::tile_range
 
 struct BhCounters {
     uint32_t n_in;      // particles inside the domain (padding included)
@@ -50,8 +51,6 @@ struct BhCounters {
     uint32_t n_leaves;  // occupied leaf cells (depth 10, or 15 with 15-bit leaves)
     uint32_t n_gran;             // 15-bit leaves: occupied depth-10 cells
     uint32_t sort_stall;         // look-back waits that hit their bound (never expected)
-    uint32_t tiles_busy;         // occupied depth-5 tiles
-    uint32_t tiles_done;         // occupied tiles reduced (the last one reduces the top)
 };
 
 // Radix sort passes (single and batched builds): tiles of kSortTile keys,
@@ -114,7 +113,9 @@ struct BhBuffers {
     uint32_t *leaf_first = nullptr;  // [Na+1]
     uint32_t *leaf_key = nullptr;    // [Na]
     float4 *leaf_sum = nullptr;      // [Na] (sx, sy, sm, n as bits)
-    uint32_t *tile_range = nullptr;  // [2*kTiles] first/end leaf of each depth-5 tile
+    // [kTileWords] first/end leaf of each depth-5 tile, then the counts of the
+    // tiles reduced, of each group of 32 tiles and of the groups, 32 words apart
+    uint32_t *tile_range = nullptr;
     TileCell *top = nullptr;         // [kTiles]
     float4 *node4 = nullptr;         // [cap]
     uint4 *child = nullptr;          // [cap] a cell's children (kLeafMark)

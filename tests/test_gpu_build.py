@@ -1,0 +1,55 @@
+"""The Barnes-Hut build where its kernels change shape: every node array equals
+the oracle's, bit for bit, on the first step and on a third one (whose counters
+and look-back words the steps before it have used)."""
+import numpy as np
+import pytest
+
+import gsim
+import helpers as H
+import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+TILE = 1000.0 / 32  # edge of a depth-5 cell of the fixed domain
+
+
+def _same_tree(pos, mass, bits=10, steps=3):
+    # padded here: the padding moves with the others, and is read back
+    p = gsim.Particles(pos, np.zeros_like(pos), mass).padded()
+    with gsim.Simulation(p, "barnes-hut") as s:
+        if bits != 10:
+            s.set_tuning(gsim.TUNE_BH_LEAF_BITS, bits)
+        for k in range(steps):
+            pp = s.read() if k else p
+            s.step(1)
+            if k in (0, steps - 1):
+                t = s.tree()
+                ot, nn, _, _, _ = O.bh_build(pp.pos, pp.mass, bits=bits)
+                assert t["total"] == nn, k
+                for key in ("sorted_src", "counts", "radii", "node_mass", "node_pos"):
+                    assert np.array_equal(t[key], ot[key]), (k, key)
+
+
+def _tiles(which, per, seed):
+    """`per` particles in each depth-5 cell (by its Morton index) of `which`."""
+    rng = np.random.default_rng(seed)
+    x = np.zeros(len(which), np.int64)
+    y = np.zeros(len(which), np.int64)
+    for b in range(5):
+        x |= ((which >> (2 * b)) & 1) << b
+        y |= ((which >> (2 * b + 1)) & 1) << b
+    corner = np.stack([x, y], 1) * TILE - 500.0
+    pos = np.repeat(corner, per, 0) + rng.uniform(0.05, 0.95, (len(which) * per, 2)) * TILE
+    return pos.astype(np.float32), rng.uniform(1, 10, len(pos)).astype(np.float32)
+
+
+@pytest.mark.parametrize("bits", [10, 15])
+@pytest.mark.parametrize("name,which,per", [
+    ("one", np.array([1023]), 1), ("one-full", np.array([37]), 1500),
+    ("first-of-each-32", np.arange(0, 1024, 32), 3), ("one-32", np.arange(64, 96), 2),
+    ("two-of-33", np.array([0, 32]), 5), ("every", np.arange(1024), 1),
+    ("every-9", np.arange(1024), 9)])
+def test_tree_for_every_pattern_of_occupied_tiles(name, which, per, bits):
+    print(f"tiles {name} bits={bits}", flush=True)
+    pos, mass = _tiles(which, per, len(which) + per)
+    _same_tree(pos, mass, bits)
