@@ -277,30 +277,95 @@ __global__ __launch_bounds__(256) void bh_prep_kernel(const uint32_t *__restrict
     }
 }
 
+// What the emission of a sorted position reads and writes.
+struct EmitArgs {
+    const float2 *pos, *vel;  // last step's order
+    const float *mass;
+    const uint32_t *perm_in;
+    float2 *pos_out, *vel_out;
+    float *mass_out;
+    uint32_t *perm_out;
+    uint2 *ncells;  // the next build's cells (nullptr: not kept)
+    uint32_t na;
+    int bits;
+    int8_t *sdep;
+    uint32_t *cpos, *leaf_first, *leaf_key;
+    float4 *node4;
+    uint32_t *sorted_src;
+    BhCounters *ctr;
+    uint32_t *gran_first, *gran_key;  // 15-bit leaves only, else nullptr
+};
+
+// Sorted position k: the particle of slot i in last step's order (p, m, the
+// caller's index orig), with C cells, L leaves and G occupied depth-10 cells
+// before it; k is its slot in the next order.
+__device__ __forceinline__ void emit_position(const EmitArgs &e, const PosInfo &q, uint32_t k,
+                                              uint32_t i, float2 p, float m, uint32_t orig,
+                                              uint32_t C, uint32_t L, uint32_t G) {
+    e.perm_out[k] = orig;
+    if (!q.inside) {
+        // killed (InitShader.comp:110-117): not walked; the reference leaves
+        // vel_out stale, here it keeps the input velocity
+        const float kk = -kSimSize * 2.0f;
+        e.pos_out[k] = make_float2(kk, kk);
+        e.vel_out[k] = e.vel[i];
+        e.mass_out[k] = 0.0f;
+        if (e.ncells)  // the next build's cell, where the walk writes the others
+            e.ncells[orig] = make_uint2(e.bits == (int)kDeepBits ? kKilledKeyDeep : kKilledKey, k);
+        e.sorted_src[k] = e.na;  // ClearShader.comp:81-82 sentinel
+        if (k == 0) {            // nothing inside the domain
+            e.ctr->n_in = 0;
+            e.ctr->n_cells = 0;
+            e.ctr->n_nodes = 0;
+            e.ctr->n_leaves = 0;
+            e.ctr->n_gran = 0;
+            e.leaf_first[0] = 0;
+            if (e.gran_first) e.gran_first[0] = 0;
+        }
+        return;
+    }
+    e.mass_out[k] = m;
+    const uint32_t slot = k + C + q.ns;
+    // ParticleSortShader.comp:99-107 (canonical order)
+    e.node4[slot] = make_float4(p.x, p.y, m, 0.0f);
+    e.sorted_src[k] = i;
+    e.sdep[k] = (int8_t)q.sk;
+    e.cpos[k] = C;
+    if (q.lf) {
+        e.leaf_first[L] = k;
+        e.leaf_key[L] = q.key;
+    }
+    if (e.gran_first && q.g10) {
+        e.gran_first[G] = k;
+        e.gran_key[G] = q.key >> 10;  // the 20-bit cell
+    }
+    if (q.sk1 < 0) {  // last in-domain position
+        e.ctr->n_in = k + 1;
+        e.ctr->n_cells = C + q.ns;
+        e.ctr->n_nodes = k + 1 + C + q.ns;
+        e.ctr->n_leaves = L + q.lf;
+        e.leaf_first[L + q.lf] = k + 1;
+        e.ctr->n_gran = G + (q.g10 ? 1u : 0u);
+        if (e.gran_first) e.gran_first[G + (q.g10 ? 1u : 0u)] = k + 1;
+    }
+}
+
 // block_cells, block_leaves (and block_gran): bh_prep_kernel's per-block
 // counts; each block adds up those of the blocks before it (integer sums, a
 // few loads per thread) instead of a separate scan launch.
 __global__ __launch_bounds__(256) void bh_emit_kernel(
-    const uint32_t *__restrict__ keys, const uint32_t *__restrict__ sidx,
-    const float2 *__restrict__ pos, const float *__restrict__ mass,
-    const float2 *__restrict__ vel, const uint32_t *__restrict__ perm_in,
-    float2 *__restrict__ pos_out, float2 *__restrict__ vel_out, float *__restrict__ mass_out,
-    uint32_t *__restrict__ perm_out, uint2 *__restrict__ ncells, uint32_t na, int bits,
+    const uint32_t *__restrict__ keys, const uint32_t *__restrict__ sidx, EmitArgs e,
     const uint32_t *__restrict__ block_cells, const uint32_t *__restrict__ block_leaves,
-    int8_t *__restrict__ sdep, uint32_t *__restrict__ cpos,
-    uint32_t *__restrict__ leaf_first, uint32_t *__restrict__ leaf_key,
-    float4 *__restrict__ node4, uint32_t *__restrict__ sorted_src,
-    BhCounters *__restrict__ ctr, const uint32_t *__restrict__ block_gran,
-    uint32_t *__restrict__ gran_first, uint32_t *__restrict__ gran_key) {
+    const uint32_t *__restrict__ block_gran) {
+    const uint32_t na = e.na;
     __shared__ uint32_t wa[4], wb[4], wc[4], pa[4], pb[4], pc[4];
     const uint32_t k = blockIdx.x * 256 + threadIdx.x;
     // the particle now at sorted position k, from its slot i of the last
-    // step's order (nearly the same order, so nearly sequential reads); k is
-    // its slot in the next order
+    // step's order (nearly the same order, so nearly sequential reads)
     const uint32_t i = k < na ? sidx[k] : 0u;
-    const float2 p = k < na ? pos[i] : make_float2(0.0f, 0.0f);
-    const float m = k < na ? mass[i] : 0.0f;
-    const uint32_t orig = k < na ? perm_in[i] : 0u;
+    const float2 p = k < na ? e.pos[i] : make_float2(0.0f, 0.0f);
+    const float m = k < na ? e.mass[i] : 0.0f;
+    const uint32_t orig = k < na ? e.perm_in[i] : 0u;
     // the counts of the blocks before this one, eight loads per thread at once
     uint32_t xa = 0, xb = 0, xc = 0;
     for (uint32_t j0 = threadIdx.x; j0 < blockIdx.x; j0 += 8 * 256) {
@@ -320,7 +385,7 @@ __global__ __launch_bounds__(256) void bh_emit_kernel(
             xc += vc[u];
         }
     }
-    const PosInfo q = pos_info(keys, na, k, bits);
+    const PosInfo q = pos_info(keys, na, k, e.bits);
     uint32_t a = q.ns, b = q.lf;
     wave_scan2(a, b);
     const unsigned long long gb = __ballot(q.g10);
@@ -349,53 +414,194 @@ __global__ __launch_bounds__(256) void bh_emit_kernel(
         eb += wb[w];
         ec += wc[w];
     }
-    if (k >= na) return;
-    perm_out[k] = orig;
-    if (!q.inside) {
-        // killed (InitShader.comp:110-117): not walked; the reference leaves
-        // vel_out stale, here it keeps the input velocity
-        const float kk = -kSimSize * 2.0f;
-        pos_out[k] = make_float2(kk, kk);
-        vel_out[k] = vel[i];
-        mass_out[k] = 0.0f;
-        if (ncells)  // the next build's cell, where the walk writes the others
-            ncells[orig] = make_uint2(bits == (int)kDeepBits ? kKilledKeyDeep : kKilledKey, k);
-        sorted_src[k] = na;  // ClearShader.comp:81-82 sentinel
-        if (k == 0) {        // nothing inside the domain
-            ctr->n_in = 0;
-            ctr->n_cells = 0;
-            ctr->n_nodes = 0;
-            ctr->n_leaves = 0;
-            ctr->n_gran = 0;
-            leaf_first[0] = 0;
-            if (gran_first) gran_first[0] = 0;
+    if (k < na) emit_position(e, q, k, i, p, m, orig, ea, eb, ec);
+}
+
+// ---- 1.-4. in one workgroup: small builds ---------------------------------------
+
+// Keys, sort, slot scan and emission of up to kSmallBuild particles by one
+// workgroup of 16 waves.  Below that size each of the six launches it stands
+// in for (keys, three sort passes, prep, emit) is bound by its own launch and
+// its chain of loads; here the keys stay in LDS between the passes (digits of
+// 7 bits, three passes; 15-bit leaves: 8 bits, four).  The limit is the LDS
+// (64 KB of keys, indices and digit counts at 8,192 particles).
+// It is bound by the vector units of its one CU (a ranking of 64 keys is 28
+// operations) and, for the rest, by latency.  The whole build in us, six
+// launches against this one: 64 particles 43 -> 20, 1,000 46 -> 24, 4,096
+// 51 -> 33, 8,192 52 -> 45; 15-bit leaves and adaptive box 59 -> 37, 74 -> 50,
+// 89 -> 65, 92 -> 85.
+constexpr uint32_t kSmallBuild = 8192;
+constexpr uint32_t kSmallWaves = 16;
+constexpr uint32_t kSmallRows = kSmallBuild / (64 * kSmallWaves);  // keys per lane, at most
+
+// A wave holds `rows` consecutive rows of 64 positions; cells and kWalk as in
+// bh_keys_kernel, keys_out: the sorted keys.
+template <bool kBox, bool kDeep, bool kWalk>
+__global__ __launch_bounds__(64 * kSmallWaves) void bh_small_kernel(
+    EmitArgs e, uint2 *__restrict__ cells, uint32_t *__restrict__ keys_out,
+    uint32_t *__restrict__ tile_range, const float *__restrict__ box) {
+    constexpr uint32_t kBits = kDeep ? 8 : 7, kPasses = kDeep ? 4 : 3, kDigits = 1u << kBits;
+    constexpr uint32_t kNone = 0xffffffffu;
+    __shared__ uint32_t skey[kSmallBuild];
+    __shared__ uint16_t sval[kSmallBuild];
+    __shared__ uint32_t count[kSmallWaves * kDigits];
+    __shared__ uint32_t wsum[kSmallWaves], wgran[kSmallWaves];
+    const uint32_t na = e.na, t = threadIdx.x, lane = t & 63;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const uint32_t rows = (na + 64 * kSmallWaves - 1) / (64 * kSmallWaves);
+    const uint32_t first = wave * rows * 64 + lane;  // row r: position first + 64 r
+    for (uint32_t j = t; j < kTileWords; j += 64 * kSmallWaves) tile_range[j] = 0;
+    if (t == 0) e.ctr->sort_stall = 0;
+    uint32_t key[kSmallRows], val[kSmallRows], rank[kSmallRows];
+    if constexpr (!kWalk) {
+        float2 p[kSmallRows];
+        uint32_t o[kSmallRows];
+#pragma unroll
+        for (uint32_t r = 0; r < kSmallRows; ++r) {
+            const uint32_t k = first + 64 * r;
+            if (r >= rows || k >= na) continue;
+            p[r] = e.pos[k];
+            o[r] = e.perm_in[k];
         }
-        return;
+#pragma unroll
+        for (uint32_t r = 0; r < kSmallRows; ++r) {
+            const uint32_t k = first + 64 * r;
+            if (r >= rows || k >= na) continue;
+            const float x = p[r].x, y = p[r].y;
+            uint32_t c;
+            if (kDeep) c = kBox ? cell30_box(x, y, box[0], box[1], box[2]) : cell30(x, y);
+            else c = kBox ? cell20_box(x, y, box[0], box[1], box[2]) : cell20(x, y);
+            if (c == kNone) c = kDeep ? kKilledKeyDeep : kKilledKey;
+            cells[o[r]] = make_uint2(c, k);
+            skey[o[r]] = c;
+            sval[o[r]] = (uint16_t)k;
+        }
+        lds_barrier();
     }
-    mass_out[k] = m;
-    const uint32_t C = ea, L = eb;
-    const uint32_t slot = k + C + q.ns;
-    // ParticleSortShader.comp:99-107 (canonical order)
-    node4[slot] = make_float4(p.x, p.y, m, 0.0f);
-    sorted_src[k] = i;
-    sdep[k] = (int8_t)q.sk;
-    cpos[k] = C;
-    if (q.lf) {
-        leaf_first[L] = k;
-        leaf_key[L] = q.key;
+#pragma unroll
+    for (uint32_t r = 0; r < kSmallRows; ++r) {
+        const uint32_t k = first + 64 * r;
+        key[r] = kNone;
+        val[r] = 0;
+        if (r < rows && k < na) {
+            if (kWalk) {
+                const uint2 kv = cells[k];
+                key[r] = kv.x;
+                val[r] = kv.y;
+            } else {
+                key[r] = skey[k];
+                val[r] = sval[k];
+            }
+        }
     }
-    if (gran_first && q.g10) {
-        gran_first[ec] = k;
-        gran_key[ec] = q.key >> 10;  // the 20-bit cell
+    uint32_t *const mine = count + wave * kDigits;
+#pragma unroll 1
+    for (uint32_t pass = 0; pass < kPasses; ++pass) {
+        const uint32_t shift = pass * kBits;
+#pragma unroll
+        for (uint32_t d = 0; d < kDigits; d += 64) mine[d + lane] = 0;
+        wave_lds_order();
+        // ranks within the wave, a row after the other
+#pragma unroll
+        for (uint32_t r = 0; r < kSmallRows; ++r) {
+            if (r >= rows) break;
+            const bool valid = key[r] != kNone;
+            const uint32_t d = (key[r] >> shift) & (kDigits - 1);
+            const uint64_t m = digit_peers<(int)kBits>(d, valid);
+            const uint32_t before = (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
+            const uint32_t n = mine[d];
+            rank[r] = n + before;
+            wave_lds_order();
+            if (valid && before == 0) mine[d] = n + (uint32_t)__popcll(m);
+            wave_lds_order();
+        }
+        lds_barrier();
+        // digit t: where each wave's keys of it go
+        uint32_t n[kSmallWaves], sum = 0, unused = 0;
+        if (t < kDigits) {
+#pragma unroll
+            for (uint32_t w = 0; w < kSmallWaves; ++w) n[w] = count[w * kDigits + t];
+#pragma unroll
+            for (uint32_t w = 0; w < kSmallWaves; ++w) sum += n[w];
+        }
+        uint32_t at = sum;
+        if (t < kDigits) {
+            wave_scan2(at, unused);
+            if (lane == 63) wsum[wave] = at;
+        }
+        lds_barrier();
+        if (t < kDigits) {
+            at -= sum;
+            for (uint32_t w = 0; w < wave; ++w) at += wsum[w];
+#pragma unroll
+            for (uint32_t w = 0; w < kSmallWaves; ++w) {
+                count[w * kDigits + t] = at;
+                at += n[w];
+            }
+        }
+        lds_barrier();
+#pragma unroll
+        for (uint32_t r = 0; r < kSmallRows; ++r) {
+            if (r >= rows || key[r] == kNone) continue;
+            const uint32_t to = mine[(key[r] >> shift) & (kDigits - 1)] + rank[r];
+            skey[to] = key[r];
+            sval[to] = (uint16_t)val[r];
+        }
+        lds_barrier();
+#pragma unroll
+        for (uint32_t r = 0; r < kSmallRows; ++r) {
+            const uint32_t k = first + 64 * r;
+            if (r >= rows || k >= na) continue;
+            key[r] = skey[k];
+            val[r] = sval[k];
+        }
     }
-    if (q.sk1 < 0) {  // last in-domain position
-        ctr->n_in = k + 1;
-        ctr->n_cells = C + q.ns;
-        ctr->n_nodes = k + 1 + C + q.ns;
-        ctr->n_leaves = L + q.lf;
-        leaf_first[L + q.lf] = k + 1;
-        ctr->n_gran = ec + (q.g10 ? 1u : 0u);
-        if (gran_first) gran_first[ec + (q.g10 ? 1u : 0u)] = k + 1;
+    // the particles of the sorted positions, all loads ahead of the scan
+    float2 p[kSmallRows];
+    float m[kSmallRows];
+    uint32_t orig[kSmallRows];
+#pragma unroll
+    for (uint32_t r = 0; r < kSmallRows; ++r) {
+        if (r >= rows || key[r] == kNone) continue;
+        p[r] = e.pos[val[r]];
+        m[r] = e.mass[val[r]];
+        orig[r] = e.perm_in[val[r]];
+    }
+    // cells and leaves before each position: cells in the low 18 bits (at most
+    // 16 a particle), leaves above (at most one)
+    uint32_t ahead[kSmallRows], gahead[kSmallRows], run = 0, grun = 0;
+#pragma unroll
+    for (uint32_t r = 0; r < kSmallRows; ++r) {
+        if (r >= rows) break;
+        const PosInfo q = pos_info(skey, na, first + 64 * r, e.bits);
+        const uint32_t own = q.ns | q.lf << 18;
+        uint32_t incl = own, unused = 0;
+        wave_scan2(incl, unused);
+        ahead[r] = run + incl - own;
+        run += __builtin_amdgcn_readlane(incl, 63);
+        const unsigned long long g = __ballot(q.g10);
+        gahead[r] = grun + (uint32_t)__popcll(g & ((1ull << lane) - 1ull));
+        grun += (uint32_t)__popcll(g);
+    }
+    if (lane == 0) {
+        wsum[wave] = run;
+        wgran[wave] = grun;
+    }
+    lds_barrier();
+    uint32_t base = 0, gbase = 0;
+    for (uint32_t w = 0; w < wave; ++w) {
+        base += wsum[w];
+        gbase += wgran[w];
+    }
+#pragma unroll
+    for (uint32_t r = 0; r < kSmallRows; ++r) {
+        const uint32_t k = first + 64 * r;
+        if (r >= rows || k >= na) continue;
+        const uint32_t a = base + ahead[r];
+        const PosInfo q = pos_info(skey, na, k, e.bits);
+        keys_out[k] = key[r];
+        emit_position(e, q, k, val[r], p[r], m[r], orig[r], a & 0x3ffffu, a >> 18,
+                      gbase + gahead[r]);
     }
 }
 
@@ -1107,54 +1313,63 @@ hipError_t bh_launch_build(gsim_sim *s, const float2 *pos, const float *mass,
         bh_box_final_kernel<<<1, 256, 0, s->stream>>>(b.box_part, nparts, b.box);
         box = b.box;
     }
-    // one tile of kSortTile keys per workgroup, in the keys kernel and in
-    // every pass; each pass's status holds its tile words, then its group words
-    const uint32_t nblk = (na + kSortTile - 1) / kSortTile;
-    const uint32_t kblk = nblk;
-    const uint32_t pass_words = (nblk + (nblk + kLookGroup - 1) / kLookGroup) * 256u;
-    const int passes = deep ? 4 : 3;
-    const uint32_t status_words = (uint32_t)passes * pass_words;
-    // digit totals alternate between two halves by build parity
-    uint32_t *const totals = b.digit_total + kDigitCopies * 1024 * b.parity;
-    uint32_t *const totals_next = b.digit_total + kDigitCopies * 1024 * (b.parity ^ 1u);
-    b.parity ^= 1u;
     // the sort's input: written by the last walk (fixed domain), else here
     const int kin = b.kin;
     const bool walk = b.walk_keys && !box;
     b.kcells = kin;
-#define GSIM_KEYS(B, D, W)                                                                    \
-    bh_keys_kernel<B, D, kSortRounds, W><<<kblk, kSortThreads, 0, s->stream>>>(                \
-        pos, perm_in, na, b.cells[kin], b.tile_range, totals, totals_next, b.status,          \
-        status_words, b.ctr, box)
-    if (box) { if (deep) GSIM_KEYS(true, true, false); else GSIM_KEYS(true, false, false); }
-    else if (walk) { if (deep) GSIM_KEYS(false, true, true); else GSIM_KEYS(false, false, true); }
-    else { if (deep) GSIM_KEYS(false, true, false); else GSIM_KEYS(false, false, false); }
-#undef GSIM_KEYS
-    // 20-bit keys: cells[kin] -> keys[0] -> keys[1] -> keys[0]; 30-bit keys take
-    // a fourth pass -> keys[1].  cells[kin] keeps the per-particle cells.
-    const int in_of[4] = {-1, 0, 1, 0}, out_of[4] = {0, 1, 0, 1};
-    for (int pass = 0; pass < passes; ++pass) {
-        const int i = in_of[pass], o = out_of[pass];
-        uint32_t *const st = b.status + (size_t)pass * pass_words;
-        radix_onesweep_kernel<kSortRounds><<<nblk, kSortThreads, 0, s->stream>>>(
-            i < 0 ? nullptr : b.keys[i], i < 0 ? nullptr : b.idx[i], i < 0 ? b.cells[kin] : nullptr,
-            b.keys[o], b.idx[o], na, 8u * pass, totals + 256 * pass, st,
-            &b.ctr->sort_stall);
-    }
     b.sorted_slot = deep ? 1 : 0;
     const uint32_t *sk = b.keys[b.sorted_slot], *si = b.idx[b.sorted_slot];
     const uint32_t pb = (uint32_t)b.prep_blocks;
-    bh_prep_kernel<<<pb, 256, 0, s->stream>>>(sk, na, bits, b.block_cells, b.block_leaves,
-                                              deep ? b.block_gran : nullptr);
     const NextKeys nk = next_keys(s, perm_out);
-    bh_emit_kernel<<<pb, 256, 0, s->stream>>>(sk, si, pos, mass, vel, perm_in, pos_out, vel_out,
-                                              mass_out, perm_out, nk.cells, na, bits,
-                                              b.block_cells,
-                                              b.block_leaves, b.sdep, b.cpos,
-                                              b.leaf_first, b.leaf_key, b.node4,
-                                              b.sorted_src, b.ctr,
-                                              deep ? b.block_gran : nullptr,
-                                              deep ? b.gran_first : nullptr, b.gran_key);
+    const EmitArgs emit{pos,       vel,     mass,           perm_in,      pos_out,   vel_out,
+                        mass_out,  perm_out, nk.cells,      na,           bits,      b.sdep,
+                        b.cpos,    b.leaf_first, b.leaf_key, b.node4,     b.sorted_src, b.ctr,
+                        deep ? b.gran_first : nullptr, b.gran_key};
+    if (na <= kSmallBuild) {
+        uint32_t *const ko = b.keys[b.sorted_slot];
+#define GSIM_SMALL(B, D, W)                                                                   \
+    bh_small_kernel<B, D, W><<<1, 64 * kSmallWaves, 0, s->stream>>>(emit, b.cells[kin], ko,    \
+                                                                    b.tile_range, box)
+        if (box) { if (deep) GSIM_SMALL(true, true, false); else GSIM_SMALL(true, false, false); }
+        else if (walk) { if (deep) GSIM_SMALL(false, true, true); else GSIM_SMALL(false, false, true); }
+        else { if (deep) GSIM_SMALL(false, true, false); else GSIM_SMALL(false, false, false); }
+#undef GSIM_SMALL
+    } else {
+        // one tile of kSortTile keys per workgroup, in the keys kernel and in
+        // every pass; each pass's status holds its tile words, then its group words
+        const uint32_t nblk = (na + kSortTile - 1) / kSortTile;
+        const uint32_t kblk = nblk;
+        const uint32_t pass_words = (nblk + (nblk + kLookGroup - 1) / kLookGroup) * 256u;
+        const int passes = deep ? 4 : 3;
+        const uint32_t status_words = (uint32_t)passes * pass_words;
+        // digit totals alternate between two halves by build parity
+        uint32_t *const totals = b.digit_total + kDigitCopies * 1024 * b.parity;
+        uint32_t *const totals_next = b.digit_total + kDigitCopies * 1024 * (b.parity ^ 1u);
+        b.parity ^= 1u;
+#define GSIM_KEYS(B, D, W)                                                                    \
+        bh_keys_kernel<B, D, kSortRounds, W><<<kblk, kSortThreads, 0, s->stream>>>(                \
+            pos, perm_in, na, b.cells[kin], b.tile_range, totals, totals_next, b.status,          \
+            status_words, b.ctr, box)
+        if (box) { if (deep) GSIM_KEYS(true, true, false); else GSIM_KEYS(true, false, false); }
+        else if (walk) { if (deep) GSIM_KEYS(false, true, true); else GSIM_KEYS(false, false, true); }
+        else { if (deep) GSIM_KEYS(false, true, false); else GSIM_KEYS(false, false, false); }
+#undef GSIM_KEYS
+        // 20-bit keys: cells[kin] -> keys[0] -> keys[1] -> keys[0]; 30-bit keys take
+        // a fourth pass -> keys[1].  cells[kin] keeps the per-particle cells.
+        const int in_of[4] = {-1, 0, 1, 0}, out_of[4] = {0, 1, 0, 1};
+        for (int pass = 0; pass < passes; ++pass) {
+            const int i = in_of[pass], o = out_of[pass];
+            uint32_t *const st = b.status + (size_t)pass * pass_words;
+            radix_onesweep_kernel<kSortRounds><<<nblk, kSortThreads, 0, s->stream>>>(
+                i < 0 ? nullptr : b.keys[i], i < 0 ? nullptr : b.idx[i], i < 0 ? b.cells[kin] : nullptr,
+                b.keys[o], b.idx[o], na, 8u * pass, totals + 256 * pass, st,
+                &b.ctr->sort_stall);
+        }
+        bh_prep_kernel<<<pb, 256, 0, s->stream>>>(sk, na, bits, b.block_cells, b.block_leaves,
+                                                  deep ? b.block_gran : nullptr);
+        bh_emit_kernel<<<pb, 256, 0, s->stream>>>(sk, si, emit, b.block_cells, b.block_leaves,
+                                                  deep ? b.block_gran : nullptr);
+    }
     const uint32_t lb = pb < kLeafBlocks ? pb : kLeafBlocks;
     bh_leaf_kernel<<<lb, 256, 0, s->stream>>>(b.leaf_first, b.leaf_key, b.cpos, b.ctr, bits,
                                               b.leaf_sum, b.tile_range, b.node4, b.child,

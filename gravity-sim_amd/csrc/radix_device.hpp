@@ -50,15 +50,21 @@ __device__ __forceinline__ void status_store(uint32_t *p, uint32_t v) {
     __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Lanes of this wave whose digit equals this lane's (valid lanes only).
+// Lanes of this wave whose kBits-bit digit equals this lane's (valid lanes only).
+template <int kBits = 8>
 __device__ __forceinline__ uint64_t digit_peers(uint32_t d, bool valid) {
-    uint64_t m = __ballot(valid);
+    // per bit: the lanes that have it (a scalar mask), against this lane's bit
+    // spread over a word; each half of the mask is one three-input operation
+    const uint64_t v = __ballot(valid);
+    uint32_t lo = (uint32_t)v, hi = (uint32_t)(v >> 32);
 #pragma unroll
-    for (int bit = 0; bit < 8; ++bit) {
-        const bool set = (d >> bit) & 1u;
-        const uint64_t bb = __ballot(set);
-        m &= set ? bb : ~bb;
+    for (int bit = 0; bit < kBits; ++bit) {
+        const uint32_t own = (uint32_t)((int)(d << (31 - bit)) >> 31);
+        const uint64_t bb = __ballot((int)own < 0);
+        lo &= ~((uint32_t)bb ^ own);
+        hi &= ~((uint32_t)(bb >> 32) ^ own);
     }
+    const uint64_t m = (uint64_t)hi << 32 | lo;
     return m;
 }
 

@@ -13,18 +13,21 @@ pytestmark = pytest.mark.gpu
 TILE = 1000.0 / 32  # edge of a depth-5 cell of the fixed domain
 
 
-def _same_tree(pos, mass, bits=10, steps=3):
+def _same_tree(pos, mass, bits=10, steps=3, boxed=False):
     # padded here: the padding moves with the others, and is read back
     p = gsim.Particles(pos, np.zeros_like(pos), mass).padded()
     with gsim.Simulation(p, "barnes-hut") as s:
         if bits != 10:
             s.set_tuning(gsim.TUNE_BH_LEAF_BITS, bits)
+        if boxed:
+            s.set_tuning(gsim.TUNE_BH_ADAPTIVE_BOX, 1)
         for k in range(steps):
             pp = s.read() if k else p
             s.step(1)
             if k in (0, steps - 1):
                 t = s.tree()
-                ot, nn, _, _, _ = O.bh_build(pp.pos, pp.mass, bits=bits)
+                ot, nn, _, _, _ = O.bh_build(pp.pos, pp.mass, bits=bits,
+                                           box=O.bh_box(pp.pos) if boxed else None)
                 assert t["total"] == nn, k
                 for key in ("sorted_src", "counts", "radii", "node_mass", "node_pos"):
                     assert np.array_equal(t[key], ot[key]), (k, key)
@@ -53,3 +56,17 @@ def test_tree_for_every_pattern_of_occupied_tiles(name, which, per, bits):
     print(f"tiles {name} bits={bits}", flush=True)
     pos, mass = _tiles(which, per, len(which) + per)
     _same_tree(pos, mass, bits)
+
+
+@pytest.mark.parametrize("bits,boxed", [(10, False), (15, False), (10, True), (15, True)])
+@pytest.mark.parametrize("n", [1, 65, 1024, 1025, 5000, 8127, 8192, 8193])
+def test_tree_on_both_sides_of_the_one_workgroup_build(n, bits, boxed):
+    """Up to 8,192 particles one workgroup sorts and emits them: rows of 64 that
+    end anywhere, equal keys, particles outside the domain, and one size more."""
+    print(f"small build n={n} bits={bits} boxed={boxed}", flush=True)
+    rng = np.random.default_rng(n)
+    pos = rng.normal(0, 150, (n, 2)).astype(np.float32)
+    pos[: n // 3] = rng.normal(31.2, 0.2, (n // 3, 2))
+    pos[n // 3: n // 3 + n // 50] = 7.5
+    pos[n // 2: n // 2 + n // 40] = [600, 0]
+    _same_tree(pos, rng.uniform(1, 10, n).astype(np.float32), bits, 4, boxed)
