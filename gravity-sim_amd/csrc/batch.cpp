@@ -163,6 +163,11 @@ gsim_status upload_membership(gsim_batch *b) {
     GSIM_HIP(hipMemsetAsync(b->d.ichunk, 0, sizeof(uint32_t) * b->item_capacity, b->stream));
     GSIM_HIP(up(b->d.remaining, remaining.data(), remaining.size() * 4));
     GSIM_HIP(up(b->d.counts, &c, sizeof(c)));
+    const uint32_t slots = c.n_bh_particles / gsim::kBatchSortTileMin + c.n_bh;  // any tile size
+    if (slots > b->sort_slots) {
+        destroy_graphs(b);
+        b->sort_slots = 2 * slots;
+    }
     b->h_desc = desc;
     b->h_counts = c;
     b->dirty = false;
@@ -227,7 +232,7 @@ gsim_status gsim_batch_create(int32_t device, size_t capacity_particles, uint32_
     b->node_capacity = 3 * cap + 64;
     b->partial_capacity = 4 * cap;
     b->item_capacity = cap / 8 + cap / 64 + 16 * (size_t)max_systems + 64;
-    b->tiles_cap = (cap + gsim::kBatchSortTileMin - 1) / gsim::kBatchSortTileMin;
+    b->tiles_cap = cap / gsim::kBatchSortTileMin + max_systems;  // slots: one more a system
     b->blocks_cap = (cap + 255) / 256;
     b->free_ranges[0] = (uint32_t)cap;
     hipError_t e = hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking);
@@ -250,8 +255,8 @@ gsim_status gsim_batch_create(int32_t device, size_t capacity_particles, uint32_
     GSIM_BALLOC(d.remaining, max_systems);
     GSIM_BALLOC(d.counts, 1);
     GSIM_BALLOC(d.stats, max_systems);
-    GSIM_BALLOC(d.status, 2 * 256 * b->tiles_cap);
-    GSIM_BALLOC(d.digit_total, 4 * 256);
+    GSIM_BALLOC(d.status, 2 * 2 * 256 * b->tiles_cap);
+    GSIM_BALLOC(d.digit_total, (size_t)max_systems * gsim::kBatchPasses * 256);
     GSIM_BALLOC(d.block_cells, b->blocks_cap);
     GSIM_BALLOC(d.block_leaves, b->blocks_cap);
     GSIM_BALLOC(d.sdep, cap);
@@ -269,6 +274,8 @@ gsim_status gsim_batch_create(int32_t device, size_t capacity_particles, uint32_
     GSIM_BALLOC(d.ichunk, b->item_capacity);
 #undef GSIM_BALLOC
     if (e == hipSuccess) e = hipMemset(d.counts, 0, sizeof(gsim::BatchCounts));
+    if (e == hipSuccess)
+        e = hipMemset(d.digit_total, 0, sizeof(uint32_t) * max_systems * gsim::kBatchPasses * 256);
     if (e == hipSuccess) e = hipMemset(d.wave_acc, 0, sizeof(unsigned long long) * 2 * gsim::kMaxForceWaves);
     if (e == hipSuccess) e = hipMemset(d.ichunk, 0, sizeof(uint32_t) * b->item_capacity);
     if (e == hipSuccess) e = hipMemset(d.child, 0, sizeof(uint4) * b->node_capacity);

@@ -49,7 +49,6 @@ struct BatchCounts {
     uint32_t n_sys;           // all systems (direct sum and Barnes-Hut)
     uint32_t pad;
     uint32_t sort_stall;      // radix look-back waits that hit their bound (never expected)
-    uint32_t sort_tile[4];    // tile counter of each radix pass
     uint32_t n_live[kLiveLists];  // (system, depth-5 tile) pairs holding leaves, per list
     uint32_t qnext[kForceQueues];  // force launch: items taken from each queue (zeroed each step)
     unsigned long long accepts;  // Barnes-Hut real-lane acceptances, all steps
@@ -63,9 +62,11 @@ constexpr uint32_t kUnlimitedSteps = 0xffffffffu;
 
 // Radix tiles of the batched sort: sort_rounds keys per thread (8, 12 or 16:
 // tiles of 2,048, 3,072 or 4,096 keys; 12 by default, the autotuner picks).
-// The look-back status words are sized for the smallest tile.
+// The look-back status words are sized for the smallest tile.  Each system is
+// sorted by itself on its 21 bits of cell and killed bit, in three passes.
 constexpr int kBatchSortRoundsDefault = 12;
 constexpr int kBatchSortTileMin = 8 * kSortThreads;
+constexpr uint32_t kBatchPasses = 3;
 
 // Launch parameters of a batched step that never change results (the
 // autotuner's knobs): persistent force-launch width, radix tile size, leaf
@@ -103,8 +104,8 @@ struct BatchDevice {
     RankStats *stats = nullptr;
     // Barnes-Hut scratch over all sorted positions
     uint32_t *keys[2] = {}, *idx[2] = {};
-    uint32_t *status = nullptr;       // [2][tiles_cap * 256] radix look-back words, by pass parity
-    uint32_t *digit_total = nullptr;  // [4 * 256] per-pass digit totals
+    uint32_t *status = nullptr;       // [2][tile, group][tiles_cap * 256] radix look-back words, by pass parity
+    uint32_t *digit_total = nullptr;  // [max_systems][kBatchPasses * 256] digit totals, zero between steps
     uint32_t *ichunk = nullptr;       // [item_capacity] chunks each work item summed last step (issue priority)
     uint32_t *block_cells = nullptr, *block_leaves = nullptr;
     int8_t *sdep = nullptr;
@@ -143,6 +144,10 @@ struct gsim_batch {
     size_t item_capacity = 0;
     uint32_t max_systems = 0;
     size_t tiles_cap = 0, blocks_cap = 0;
+    // sort slots the graphs launch: what the members need, with room to grow
+    // (not what the arena could hold: an idle slot is a workgroup that starts
+    // and ends, three times a step); more drops the graphs
+    uint32_t sort_slots = 256;
     gsim::BatchDevice d;
     std::map<uint32_t, gsim::BatchSystem> systems;  // id -> system
     std::map<uint32_t, uint32_t> free_ranges;       // arena offset -> length (units of particles)

@@ -25,21 +25,46 @@ namespace {
 constexpr uint32_t kCellMask = (1u << 20) - 1u;
 constexpr uint32_t kKilledBit = 1u << 20;
 
-// Largest r in [0, n) with prefix[r] <= f (prefix ascending, prefix[0] = 0).
-__device__ __forceinline__ uint32_t rank_of(const uint32_t *__restrict__ prefix, uint32_t n,
-                                            uint32_t f) {
-    uint32_t lo = 0, hi = n;  // answer in [lo, hi)
-    while (hi - lo > 1) {
-        const uint32_t mid = (lo + hi) >> 1;
-        if (prefix[mid] <= f) lo = mid;
-        else hi = mid;
+// ---- keys and sort -----------------------------------------------------------
+// The particles come grouped by system (rank), so each system is sorted by
+// itself, on the 21 bits of cell and killed bit alone: three passes instead of
+// the four that keys with the rank in them take, digit totals per system, and
+// look-back chains no longer than a system.  The radix tiles never cross a
+// system: rank r's are the sort slots from bh_prefix[r] / tile keys + r on (at
+// least as many as it needs), one workgroup a slot in launch order: the counter
+// that dealt the tiles before was a chain of same-address atomics.
+// Bound by latency.  48 systems of 1,000 to 64,000 particles: keys and sort
+// 95 -> 45 us a step (a pass 19.4 -> 12.2), 12 systems up to 200,000: 101 -> 40
+// (22.2 -> 10.9).
+
+// The tile of a sort slot.
+struct SortSeg {
+    uint32_t r;              // rank
+    uint32_t first, n;       // the system's sorted positions
+    uint32_t slot0;          // its first slot
+    uint32_t tile, tiles;    // this slot's tile of the system's tiles (tile >= tiles: none)
+};
+
+// Found by the whole workgroup (synchronises it): rank r's thread sees that
+// the slot is r's.
+__device__ __forceinline__ SortSeg sort_seg(const uint32_t *__restrict__ prefix, uint32_t nb,
+                                            uint32_t slot, uint32_t tile_keys, SortSeg &sh) {
+    if (threadIdx.x == 0) sh = SortSeg{0u, 0u, 0u, 0u, 0u, 0u};
+    lds_barrier();
+    for (uint32_t r = threadIdx.x; r < nb; r += kSortThreads) {
+        const uint32_t f = prefix[r], e = prefix[r + 1];
+        const uint32_t s0 = f / tile_keys + r, s1 = e / tile_keys + r + 1;
+        if (slot >= s0 && (slot < s1 || r + 1 == nb))
+            sh = SortSeg{r, f, e - f, s0, slot - s0, (e - f + tile_keys - 1) / tile_keys};
     }
-    return lo;
+    lds_barrier();
+    return sh;
 }
 
-// ---- keys ------------------------------------------------------------------
-
-__global__ __launch_bounds__(256) void bb_keys_kernel(
+// Every particle's key (rank << 21 | cell; input of pass 0), the digit totals
+// of its system's passes, and the step's clears.
+template <int kR>
+__global__ __launch_bounds__(kSortThreads) void bb_keys_kernel(
     const SysDesc *__restrict__ desc, const uint32_t *__restrict__ bh_sys,
     const uint32_t *__restrict__ bh_prefix, const uint32_t *__restrict__ remaining,
     BatchCounts *__restrict__ counts,
@@ -47,115 +72,94 @@ __global__ __launch_bounds__(256) void bb_keys_kernel(
     const float2 *__restrict__ vel, float2 *__restrict__ vel_out, uint32_t *__restrict__ keys,
     uint32_t *__restrict__ idx, uint32_t *__restrict__ tile_range,
     RankStats *__restrict__ stats, uint32_t *__restrict__ digit_total,
-    uint32_t *__restrict__ status, uint32_t tile_keys) {
-    const uint32_t nb = counts->n_bh, n = counts->n_bh_particles;
-    const uint32_t tid = blockIdx.x * 256 + threadIdx.x, stride = gridDim.x * 256;
+    uint32_t *__restrict__ status, size_t group_words) {
+    __shared__ uint32_t h[kBatchPasses][256];
+    __shared__ SortSeg seg_sh;
+    constexpr uint32_t kTile = kR * kSortThreads;
+    const uint32_t nb = counts->n_bh, th = threadIdx.x;
+    const uint32_t tid = blockIdx.x * kSortThreads + th, stride = gridDim.x * kSortThreads;
     for (uint32_t t = tid; t < nb * 2 * kTiles; t += stride) tile_range[t] = 0;
     for (uint32_t t = tid; t < nb; t += stride) stats[t] = RankStats{0u, 0u, 0u, 0u};
-    for (uint32_t t = tid; t < 4 * 256; t += stride) digit_total[t] = 0;
     for (uint32_t t = tid; t < kLiveLists; t += stride) counts->n_live[t] = 0;
-    // the first radix pass's look-back words (each pass clears the next one's)
-    const uint32_t status_words = (n + tile_keys - 1) / tile_keys * 256;
-    for (uint32_t t = tid; t < status_words; t += stride) status[t] = 0;
     if (tid == 0) {
         counts->n_cells = 0;
         counts->n_leaves = 0;
         counts->sort_stall = 0;
     }
-    if (tid < 4) counts->sort_tile[tid] = 0;
-    for (uint32_t f = tid; f < n; f += stride) {
-        const uint32_t r = rank_of(bh_prefix, nb, f);
-        const uint32_t di = bh_sys[r];
-        const SysDesc &d = desc[di];
-        const uint32_t i = d.off + (f - bh_prefix[r]);
-        const float2 p = pos[i];
-        if (remaining[di] == 0u) {
+#pragma unroll
+    for (uint32_t p = 0; p < kBatchPasses; ++p) h[p][th] = 0;
+    const SortSeg seg = sort_seg(bh_prefix, nb, blockIdx.x, kTile, seg_sh);  // synchronises
+    if (seg.tile >= seg.tiles) return;
+    // the first radix pass's look-back words (each pass clears the next one's)
+    status[(size_t)blockIdx.x * 256 + th] = 0;
+    status[group_words + (size_t)blockIdx.x * 256 + th] = 0;
+    const uint32_t di = bh_sys[seg.r], off = desc[di].off;
+    const bool spent = remaining[di] == 0u;
+    const uint32_t base = seg.tile * kTile + th, rank_bits = seg.r << kBatchRankShift;
+    float2 p[kR];
+#pragma unroll
+    for (int r = 0; r < kR; ++r) {
+        const uint32_t f = base + r * kSortThreads;
+        p[r] = f < seg.n ? pos[off + f] : make_float2(0.0f, 0.0f);
+    }
+#pragma unroll
+    for (int r = 0; r < kR; ++r) {
+        const uint32_t f = base + r * kSortThreads;
+        if (f >= seg.n) break;
+        const uint32_t i = off + f;
+        uint32_t c = kKilledBit;
+        if (spent) {
             // Budget spent: the system keeps its state exactly (no kill of
             // particles that left the domain on its last step) and builds an
             // empty tree, so the force launch skips it.
-            pos_out[i] = p;
+            pos_out[i] = p[r];
             vel_out[i] = vel[i];
-            keys[f] = (r << kBatchRankShift) | kKilledBit;
-            idx[f] = i;
-            continue;
+        } else {
+            c = cell20(p[r].x, p[r].y);
+            if (c == 0xffffffffu) {  // InitShader.comp:110-117
+                const float k = -kSimSize * 2.0f;
+                pos[i] = make_float2(k, k);
+                pos_out[i] = make_float2(k, k);
+                mass[i] = 0.0f;
+                vel_out[i] = vel[i];
+                c = kKilledBit;
+            }
         }
-        uint32_t c = cell20(p.x, p.y);
-        if (c == 0xffffffffu) {  // InitShader.comp:110-117
-            const float k = -kSimSize * 2.0f;
-            pos[i] = make_float2(k, k);
-            pos_out[i] = make_float2(k, k);
-            mass[i] = 0.0f;
-            vel_out[i] = vel[i];
-            c = kKilledBit;
-        }
-        keys[f] = (r << kBatchRankShift) | c;
-        idx[f] = i;
+        keys[seg.first + f] = rank_bits | c;
+        idx[seg.first + f] = i;
+        hist_add<kBatchPasses>(h, rank_bits | c);
+    }
+    lds_barrier();
+    uint32_t *const total = digit_total + (size_t)seg.r * kBatchPasses * 256;
+#pragma unroll
+    for (uint32_t q = 0; q < kBatchPasses; ++q) {
+        const uint32_t c = h[q][th];
+        if (c) atomicAdd(&total[q * 256 + th], c);
     }
 }
 
-// ---- stable LSD radix sort over all sorted positions (4 x 8 bits) -----------
-// One-sweep passes (radix_device.hpp) with persistent workgroups: the live
-// tile count comes from device memory.
-
-// digit_total[pass * 256 + d] += keys of digit d in pass `pass`; the per-wave
-// aggregation matters here: a wave's keys usually share one system, so the
-// upper digits repeat across the wave.
-template <int kR>
-__global__ __launch_bounds__(kSortThreads) void bb_hist_kernel(
-    const uint32_t *__restrict__ keys, const BatchCounts *__restrict__ counts,
-    uint32_t *__restrict__ digit_total) {
-    constexpr uint32_t kTile = kR * kSortThreads;
-    __shared__ uint32_t h[4][256];
-    const uint32_t t = threadIdx.x;
-#pragma unroll
-    for (int p = 0; p < 4; ++p) h[p][t] = 0;
-    __syncthreads();
-    const uint32_t n = counts->n_bh_particles;
-    for (uint32_t base = blockIdx.x * kTile; base < n; base += gridDim.x * kTile) {
-        uint32_t k[kR];
-#pragma unroll
-        for (int r = 0; r < kR; ++r) {
-            const uint32_t i = base + r * kSortThreads + t;
-            k[r] = i < n ? keys[i] : 0u;
-        }
-#pragma unroll
-        for (int r = 0; r < kR; ++r)
-            hist_add<4, true>(h, k[r], base + r * kSortThreads + t < n);
-    }
-    __syncthreads();
-#pragma unroll
-    for (int p = 0; p < 4; ++p) {
-        const uint32_t c = h[p][t];
-        if (c) atomicAdd(&digit_total[p * 256 + t], c);
-    }
-}
-
-// Pass `pass` (digit (key >> 8 pass) & 255): workgroups take tiles from
-// counts->sort_tile[pass] until the live tiles run out.  status: this pass's
-// [tiles][256] look-back words, zeroed; status_next: the next pass's, zeroed
-// here tile by tile.
+// Pass `pass` (digit (key >> 8 pass) & 255).  status: this pass's look-back
+// words by slot, zeroed, the groups' group_words after the tiles' (a system's
+// groups from its first slot on); status_next: the next pass's, zeroed here.
 template <int kR>
 __global__ __launch_bounds__(kSortThreads) void bb_onesweep_kernel(
     const uint32_t *__restrict__ keys_in, const uint32_t *__restrict__ idx_in,
     uint32_t *__restrict__ keys_out, uint32_t *__restrict__ idx_out,
-    BatchCounts *__restrict__ counts, uint32_t pass, const uint32_t *__restrict__ digit_total,
-    uint32_t *__restrict__ status, uint32_t *__restrict__ status_next) {
+    const uint32_t *__restrict__ bh_prefix, BatchCounts *__restrict__ counts, uint32_t pass,
+    const uint32_t *__restrict__ digit_total, uint32_t *__restrict__ status,
+    uint32_t *__restrict__ status_next, size_t group_words) {
     __shared__ SortShared<true, kR> sh;
-    constexpr uint32_t kTile = kR * kSortThreads;
-    const uint32_t n = counts->n_bh_particles;
-    const uint32_t ntiles = (n + kTile - 1) / kTile;
-    const uint32_t gbase = digit_base(digit_total + 256 * pass, sh);  // synchronises
-    for (;;) {
-        if (threadIdx.x == 0) sh.tile = atomicAdd(&counts->sort_tile[pass], 1u);
-        sort_tile_clear(sh);
-        __syncthreads();
-        const uint32_t tile = sh.tile;
-        if (tile >= ntiles) break;
-        status_next[(size_t)tile * 256 + threadIdx.x] = 0;
-        sort_tile<true>(keys_in, idx_in, keys_out, idx_out, n, 8u * pass, tile, gbase, status,
-                  &counts->sort_stall, sh);
-        __syncthreads();
-    }
+    __shared__ SortSeg seg_sh;
+    sort_tile_clear(sh);
+    const SortSeg g = sort_seg(bh_prefix, counts->n_bh, blockIdx.x, kR * kSortThreads, seg_sh);
+    if (g.tile >= g.tiles) return;
+    status_next[(size_t)blockIdx.x * 256 + threadIdx.x] = 0;
+    status_next[group_words + (size_t)blockIdx.x * 256 + threadIdx.x] = 0;
+    uint32_t *const st = status + (size_t)g.slot0 * 256;
+    sort_tile<true, kR>(keys_in + g.first, idx_in + g.first, keys_out + g.first, idx_out + g.first,
+                        g.n, 8u * pass, g.tile, g.tiles, st, st + group_words,
+                        digit_total + ((size_t)g.r * kBatchPasses + pass) * 256, 1u, 0u,
+                        &counts->sort_stall, sh);
 }
 
 // ---- slot scan and emission ----------------------------------------------------
@@ -194,9 +198,14 @@ __device__ __forceinline__ BPos bpos_info(const uint32_t *__restrict__ keys, uin
 __global__ __launch_bounds__(256) void bb_prep_kernel(const uint32_t *__restrict__ keys,
                                                       const BatchCounts *__restrict__ counts,
                                                       uint32_t *__restrict__ block_cells,
-                                                      uint32_t *__restrict__ block_leaves) {
+                                                      uint32_t *__restrict__ block_leaves,
+                                                      uint32_t *__restrict__ digit_total) {
     __shared__ uint32_t wa[4], wb[4];
     const uint32_t n = counts->n_bh_particles;
+    // the sort is done: its digit totals are cleared for the next step's
+    const uint32_t words = counts->n_bh * kBatchPasses * 256;
+    for (uint32_t t = blockIdx.x * 256 + threadIdx.x; t < words; t += gridDim.x * 256)
+        digit_total[t] = 0;
     const uint32_t nblocks = (n + 255) / 256;
     const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     for (uint32_t blk = blockIdx.x; blk < nblocks; blk += gridDim.x) {
@@ -678,39 +687,34 @@ __global__ __launch_bounds__(256) void bb_finish_kernel(uint32_t *__restrict__ r
 hipError_t batch_launch_step(gsim_batch *b, int in, int out) {
     BatchDevice &d = b->d;
     hipStream_t st = b->stream;
-    const uint32_t g_part = (uint32_t)std::min<size_t>((b->capacity + 255) / 256, 4096);
     const uint32_t live_per_list = (uint32_t)(((size_t)b->max_systems * kTiles + kLiveLists - 1) / kLiveLists);
     const BatchTune &tune = b->tune;
     const uint32_t rounds = tune.sort_rounds;
     if (rounds != 8 && rounds != 12 && rounds != 16) return hipErrorInvalidValue;
-    const uint32_t tile_keys = rounds * kSortThreads;
-    const size_t tiles = (b->capacity + tile_keys - 1) / tile_keys;  // <= tiles_cap
-    const uint32_t g_tiles = (uint32_t)std::min<size_t>(tiles, 2048);
-    const uint32_t g_hist = (uint32_t)std::min<size_t>(tiles, 1024);
-    bb_keys_kernel<<<g_part, 256, 0, st>>>(d.desc, d.bh_sys, d.bh_prefix, d.remaining, d.counts, d.pos[in],
-                                           d.mass, d.pos[out], d.vel[in], d.vel[out], d.keys[0],
-                                           d.idx[0], d.tile_range, d.stats, d.digit_total,
-                                           d.status, tile_keys);
+    // passes: keys[0] -> keys[1] -> keys[0] -> keys[1]; look-back words
+    // alternate between the two status halves (tile words, group words)
+    const size_t group_words = 256 * b->tiles_cap, half = 2 * group_words;
 #define GSIM_BB_SORT(R)                                                                          \
     do {                                                                                         \
-        bb_hist_kernel<R><<<g_hist, kSortThreads, 0, st>>>(d.keys[0], d.counts, d.digit_total); \
-        for (int pass = 0; pass < 4; ++pass) {                                                   \
+        bb_keys_kernel<R><<<b->sort_slots, kSortThreads, 0, st>>>(                               \
+            d.desc, d.bh_sys, d.bh_prefix, d.remaining, d.counts, d.pos[in], d.mass, d.pos[out], \
+            d.vel[in], d.vel[out], d.keys[0], d.idx[0], d.tile_range, d.stats, d.digit_total,    \
+            d.status, group_words);                                                              \
+        for (uint32_t pass = 0; pass < kBatchPasses; ++pass) {                                   \
             const int i = pass & 1, o = i ^ 1;                                                   \
-            bb_onesweep_kernel<R><<<g_tiles, kSortThreads, 0, st>>>(                              \
-                d.keys[i], d.idx[i], d.keys[o], d.idx[o], d.counts, (uint32_t)pass,              \
-                d.digit_total, d.status + half * (pass & 1), d.status + half * ((pass + 1) & 1)); \
+            bb_onesweep_kernel<R><<<b->sort_slots, kSortThreads, 0, st>>>(                       \
+                d.keys[i], d.idx[i], d.keys[o], d.idx[o], d.bh_prefix, d.counts, pass,           \
+                d.digit_total, d.status + half * i, d.status + half * o, group_words);           \
         }                                                                                        \
     } while (0)
-    // 4 passes: keys[0] -> keys[1] -> keys[0] -> keys[1] -> keys[0]; look-back
-    // words alternate between the two status halves
-    const size_t half = 256 * b->tiles_cap;
     if (rounds == 8) GSIM_BB_SORT(8);
     else if (rounds == 12) GSIM_BB_SORT(12);
     else GSIM_BB_SORT(16);
 #undef GSIM_BB_SORT
-    const uint32_t *sk = d.keys[0], *si = d.idx[0];
+    const uint32_t *sk = d.keys[kBatchPasses & 1], *si = d.idx[kBatchPasses & 1];
     const uint32_t g_blk = (uint32_t)std::min<size_t>(b->blocks_cap, 4096);
-    bb_prep_kernel<<<g_blk, 256, 0, st>>>(sk, d.counts, d.block_cells, d.block_leaves);
+    bb_prep_kernel<<<g_blk, 256, 0, st>>>(sk, d.counts, d.block_cells, d.block_leaves,
+                                          d.digit_total);
     bb_block_scan_kernel<<<2, 1024, 0, st>>>(d.block_cells, d.block_leaves, d.counts);
     bb_emit_kernel<<<g_blk, 256, 0, st>>>(sk, si, d.pos[in], d.mass, d.counts, d.bh_prefix,
                                           d.block_cells, d.block_leaves, d.sdep, d.cpos,

@@ -163,7 +163,7 @@ __global__ __launch_bounds__(kSortThreads) void bh_keys_kernel(
         }
 #pragma unroll
         for (int r = 0; r < kR; ++r)
-            if (base + r * kSortThreads + t < na) hist_add<kPasses, false>(h, c[r], true);
+            if (base + r * kSortThreads + t < na) hist_add<kPasses>(h, c[r]);
     } else {
     float2 pr[kR];
     uint32_t orig[kR];
@@ -183,7 +183,7 @@ __global__ __launch_bounds__(kSortThreads) void bh_keys_kernel(
         else c = kBox ? cell20_box(p.x, p.y, box[0], box[1], box[2]) : cell20(p.x, p.y);
         if (c == 0xffffffffu) c = kDeep ? kKilledKeyDeep : kKilledKey;
         cells[orig[r]] = make_uint2(c, i);
-        hist_add<kPasses, false>(h, c, true);
+        hist_add<kPasses>(h, c);
     }
     }
     lds_barrier();
@@ -214,9 +214,9 @@ __global__ __launch_bounds__(kSortThreads) void radix_onesweep_kernel(
     // Tile = workgroup index.  A tile only waits for lower tiles, which the
     // dispatcher starts first, and a pass's workgroups all fit on the GPU at
     // once, so every wait ends (and each is bounded besides).
-    sort_tile<false, kR, true>(keys_in, idx_in, keys_out, idx_out, n, shift, blockIdx.x, 0u,
-                               status, stall, sh, gridDim.x, status + (size_t)gridDim.x * 256,
-                               digit_total, kDigitCopies, 1024u, cells_in);
+    sort_tile<false, kR>(keys_in, idx_in, keys_out, idx_out, n, shift, blockIdx.x, gridDim.x,
+                         status, status + (size_t)gridDim.x * 256, digit_total, kDigitCopies,
+                         1024u, stall, sh, cells_in);
 }
 
 // ---- 3./4. slot scan and emission --------------------------------------------

@@ -1,9 +1,9 @@
 // One-sweep stable LSD radix sort pieces shared by the single-system build
 // (bh_kernels.hip) and the batched build (batch_kernels.hip).
 //
-// A pass sorts tiles of kSortTile (key, value) pairs on one 8-bit digit.  A
-// workgroup takes the next tile from a counter, so every lower tile belongs to
-// a workgroup that is already running.  Within the tile, key r * 256 + t
+// A pass sorts tiles of kSortTile (key, value) pairs on one 8-bit digit, one
+// tile per workgroup in launch order, so every lower tile belongs to a
+// workgroup that has started before.  Within the tile, key r * 256 + t
 // (round r, thread t) is ranked among the equal digits of its wave by
 // ballots; the per-(round, wave, digit) counts go to LDS and thread d scans
 // digit d's counts in (round, wave) order, which is input order, so the sort
@@ -11,12 +11,10 @@
 // kStage the tile is staged in LDS in digit order and written out from there,
 // so consecutive lanes store consecutive positions of a digit's run (pays for
 // many tiles of spatially clustered keys; without it each key is stored
-// straight to its position).  The tile publishes its counts in one status word per (tile, digit) -- 0 (not
-// yet counted), kStA | the tile's count, kStP | the inclusive prefix over
-// tiles 0..tile -- and sums its predecessors' words back to the first kStP
-// (decoupled look-back).  A tile publishes kStA before it reads any
-// predecessor, so every wait ends; waits are bounded all the same
-// (kSpinLimit re-reads, counted in *stall).
+// straight to its position).  The tile's words (0: not yet counted, kStA | a
+// count, kStP | an inclusive prefix) are summed by grouped_prefix.  A tile
+// publishes its count before it reads any predecessor, so every wait ends;
+// waits are bounded all the same (kSpinLimit re-reads, counted in *stall).
 #pragma once
 #include "bh_device.hpp"
 #include "internal.hpp"
@@ -24,7 +22,6 @@
 namespace gsim {
 
 constexpr uint32_t kStA = 1u << 30, kStP = 2u << 30, kStVal = kStA - 1u;
-constexpr int kLookWindow = 4;             // predecessors read at once per digit
 constexpr uint32_t kSpinLimit = 1u << 20;  // bound on re-reads of one status word
 
 // kR: rounds of kSortThreads keys per tile (kSortRounds unless the launch
@@ -39,7 +36,6 @@ struct SortShared {
     uint32_t first[256];             // tile position of the first key of each digit
     uint32_t adj[256];               // output position - tile position, per digit
     uint32_t wsum[4];
-    uint32_t tile;
 };
 
 __device__ __forceinline__ uint32_t status_load(const uint32_t *p) {
@@ -68,31 +64,11 @@ __device__ __forceinline__ uint64_t digit_peers(uint32_t d, bool valid) {
     return m;
 }
 
-// Adds the digits of kPasses passes of `key` to the LDS histograms h, one
-// atomic per lane; with kUniform, one atomic for a digit that every valid
-// lane of the wave shares (the upper digits of keys grouped by system).
-template <int kPasses, bool kUniform>
-__device__ __forceinline__ void hist_add(uint32_t (*h)[256], uint32_t key, bool valid) {
-    if (!kUniform) {
+// Adds the digits of kPasses passes of `key` to the LDS histograms h.
+template <int kPasses>
+__device__ __forceinline__ void hist_add(uint32_t (*h)[256], uint32_t key) {
 #pragma unroll
-        for (int p = 0; p < kPasses; ++p)
-            if (valid) atomicAdd(&h[p][(key >> (8 * p)) & 255u], 1u);
-        return;
-    }
-    const uint64_t live = __ballot(valid);
-    if (!live) return;
-    const int first = __builtin_ctzll(live);
-    const uint32_t lane = threadIdx.x & 63;
-#pragma unroll
-    for (int p = 0; p < kPasses; ++p) {
-        const uint32_t d = (key >> (8 * p)) & 255u;
-        const uint32_t d0 = __shfl(d, first, 64);
-        if (__ballot(valid && d != d0) == 0) {
-            if (lane == (uint32_t)first) atomicAdd(&h[p][d], (uint32_t)__popcll(live));
-        } else if (valid) {
-            atomicAdd(&h[p][d], 1u);
-        }
-    }
+    for (int p = 0; p < kPasses; ++p) atomicAdd(&h[p][(key >> (8 * p)) & 255u], 1u);
 }
 
 // Adds predecessors j, j-1, ..., j-kW+1 of this digit's chain to *excl until
@@ -137,16 +113,6 @@ __device__ __forceinline__ void look_back(const uint32_t *st, int j, uint32_t *e
         }
         __builtin_amdgcn_s_sleep(1);
     }
-}
-
-// Exclusive prefix of this pass's digit totals for digit threadIdx.x
-// (synchronises the workgroup).
-template <bool kStage, int kR>
-__device__ __forceinline__ uint32_t digit_base(const uint32_t *__restrict__ digit_total,
-                                               SortShared<kStage, kR> &sh) {
-    const uint32_t total = digit_total[threadIdx.x];
-    uint32_t all = 0;
-    return block_scan256(total, &all, sh.wsum) - total;
 }
 
 // Clears this thread's column of sh.slot (sort_tile's precondition, ordered
@@ -212,35 +178,30 @@ __device__ __forceinline__ uint32_t grouped_prefix(uint32_t *st, uint32_t *gst, 
     return gex + inner;
 }
 
-// Sorts tile `tile` of keys_in/idx_in on digit (key >> shift) & 255 into
-// keys_out/idx_out.  gbase: digit_base() of this thread's digit; status: this
-// pass's [tiles][256] words; sh.slot cleared by sort_tile_clear() before a
-// barrier.  Ends with sh in use: a barrier must precede its next use.
-// kGrouped: grouped_prefix instead of the tile-by-tile look-back (tiles: the
-// pass's tile count; gstatus: its [groups][256] words, zeroed); with totals
-// (this pass's digit totals, split over `copies` copies `copy_stride` words
-// apart) gbase is not given but computed here, the totals loaded ahead of the
-// keys and scanned once the tile is ranked.  packed_in: the input as {key,
+// Sorts tile `tile` of `tiles` of keys_in/idx_in on digit (key >> shift) & 255
+// into keys_out/idx_out.  status, gstatus: the pass's [tiles][256] and
+// [groups][256] words, zeroed; totals: the pass's digit totals, split over
+// `copies` copies `copy_stride` words apart, loaded ahead of the keys and
+// scanned once the tile is ranked; sh.slot cleared by sort_tile_clear() (the
+// tile's first barrier follows its ranking).  packed_in: the input as {key,
 // index} pairs instead of keys_in/idx_in.
-template <bool kStage, int kR, bool kGrouped = false>
+template <bool kStage, int kR>
 __device__ __forceinline__ void sort_tile(const uint32_t *__restrict__ keys_in,
                                           const uint32_t *__restrict__ idx_in,
                                           uint32_t *__restrict__ keys_out,
                                           uint32_t *__restrict__ idx_out, uint32_t n,
-                                          uint32_t shift, uint32_t tile, uint32_t gbase,
+                                          uint32_t shift, uint32_t tile, uint32_t tiles,
                                           uint32_t *__restrict__ status,
-                                          uint32_t *__restrict__ stall,
-                                          SortShared<kStage, kR> &sh, uint32_t tiles = 0,
-                                          uint32_t *__restrict__ gstatus = nullptr,
-                                          const uint32_t *__restrict__ totals = nullptr,
-                                          uint32_t copies = 0, uint32_t copy_stride = 0,
+                                          uint32_t *__restrict__ gstatus,
+                                          const uint32_t *__restrict__ totals, uint32_t copies,
+                                          uint32_t copy_stride, uint32_t *__restrict__ stall,
+                                          SortShared<kStage, kR> &sh,
                                           const uint2 *__restrict__ packed_in = nullptr) {
     constexpr int kRows = SortShared<kStage, kR>::kRows;
     const uint32_t t = threadIdx.x, wave = t >> 6, lane = t & 63;
     const uint32_t base = tile * SortShared<kStage, kR>::kTile;
     uint32_t total = 0;
-    if (kGrouped && totals)
-        for (uint32_t c = 0; c < copies; ++c) total += totals[c * copy_stride + t];
+    for (uint32_t c = 0; c < copies; ++c) total += totals[c * copy_stride + t];
     uint32_t key[kR], val[kR], rank[kR];
 #pragma unroll
     for (int r = 0; r < kR; ++r) {
@@ -271,31 +232,14 @@ __device__ __forceinline__ void sort_tile(const uint32_t *__restrict__ keys_in,
         sh.slot[k * 256 + t] = c;
         c += x;
     }
-    if (kGrouped && totals) {
-        uint32_t all = 0;
-        gbase = block_scan256(total, &all, sh.wsum) - total;  // synchronises
-    }
+    uint32_t all = 0;
+    const uint32_t gbase = block_scan256(total, &all, sh.wsum) - total;  // synchronises
     uint32_t tile_n = 0, first = 0;
     if (kStage) {
         first = block_scan256(c, &tile_n, sh.wsum) - c;  // synchronises
         sh.first[t] = first;
     }
-    uint32_t *const st = status + t;  // this digit's word of tile j: st[j * 256]
-    uint32_t excl = 0;
-    if (kGrouped) {
-        excl = grouped_prefix(st, gstatus + t, tile, tiles, c, stall);
-    } else {
-        status_store(st + (size_t)tile * 256, (tile ? kStA : kStP) | c);
-        if (tile) {
-            int j = (int)tile - 1;
-            bool done = false;
-            while (!done) {
-                look_back<kLookWindow>(st, j, &excl, &done, stall);
-                j -= kLookWindow;
-            }
-            status_store(st + (size_t)tile * 256, kStP | (excl + c));
-        }
-    }
+    const uint32_t excl = grouped_prefix(status + t, gstatus + t, tile, tiles, c, stall);
     sh.adj[t] = gbase + excl - first;
     lds_barrier();
     if (!kStage) {

@@ -70,3 +70,36 @@ def test_tree_on_both_sides_of_the_one_workgroup_build(n, bits, boxed):
     pos[n // 3: n // 3 + n // 50] = 7.5
     pos[n // 2: n // 2 + n // 40] = [600, 0]
     _same_tree(pos, rng.uniform(1, 10, n).astype(np.float32), bits, 4, boxed)
+
+
+@pytest.mark.parametrize("tile", [2048, 3072, 4096])
+def test_batch_sorted_by_system_equals_each_system_alone(tile):
+    """Systems that end one below, at and one above a radix tile, a group of 16
+    tiles, two groups, with particles outside the domain; then members that need
+    more sort slots than the first steps' launches had.  Same bits as alone."""
+    sizes = [64, tile - 64, tile, tile + 64, 5 * 64, 16 * tile, 16 * tile + 64, 33 * tile, 1]
+    batch = gsim.Batch(1400000, 32)
+    batch.set_tuning(sort_tile=tile)
+    alone, ids = [], []
+
+    def add(n, seed, preset="exponential-disk"):
+        p = gsim.generate(preset, n, 120.0, 1.0, 10.0, seed=seed)
+        p.pos[: n // 50] = [700, 0]
+        alone.append(gsim.Simulation(p, "barnes-hut", accuracy_parameter=1.0))
+        ids.append(batch.add(p, "barnes-hut", accuracy_parameter=1.0))
+
+    for k, n in enumerate(sizes):
+        print(f"batch tile={tile} n={n}", flush=True)
+        add(n, k)
+    for extra in ([], [300000, 300000, 200000]):
+        for k, n in enumerate(extra):
+            add(n, 100 + k, "galaxy")
+        batch.step(3)
+        for a, k in zip(alone, ids):
+            a.step(3)
+            x, y = a.read(), batch.read(k)
+            assert np.array_equal(x.pos, y.pos) and np.array_equal(x.vel, y.vel)
+            assert np.array_equal(x.mass, y.mass)
+    for a in alone:
+        a.close()
+    batch.close()
