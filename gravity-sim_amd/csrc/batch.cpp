@@ -61,6 +61,9 @@ void free_batch(gsim_batch *b) {
                     d.child, d.wave_acc, d.ichunk};
     for (void *p : ptrs) (void)hipFree(p);
     b->stage.release();
+    if (b->fork) (void)hipEventDestroy(b->fork);
+    if (b->join) (void)hipEventDestroy(b->join);
+    if (b->side) (void)hipStreamDestroy(b->side);
     if (b->stream) (void)hipStreamDestroy(b->stream);
     delete b;
 }
@@ -98,7 +101,6 @@ void give_range(gsim_batch *b, uint32_t off, uint32_t len) {
 gsim_status upload_membership(gsim_batch *b) {
     std::vector<gsim::SysDesc> desc;
     std::vector<uint32_t> bh_sys, bh_prefix{0};
-    // direct-sum blocks first: the longest items, so that none starts last
     std::vector<uint2> items, bh_items;
     std::vector<uint32_t> remaining;
     GSIM_HIP(hipStreamSynchronize(b->stream));  // step counts below are exact from here
@@ -149,6 +151,7 @@ gsim_status upload_membership(gsim_batch *b) {
     c.n_bh = (uint32_t)bh_sys.size();
     c.n_bh_particles = bh_prefix.back();
     c.n_items = (uint32_t)items.size();
+    c.n_ds = c.n_items - (uint32_t)bh_items.size();
     // the acceptance and visit totals carry over
     GSIM_HIP(hipMemcpy(&c.accepts, &b->d.counts->accepts, sizeof(c.accepts), hipMemcpyDeviceToHost));
     GSIM_HIP(hipMemcpy(&c.visits, &b->d.counts->visits, sizeof(c.visits), hipMemcpyDeviceToHost));
@@ -167,6 +170,10 @@ gsim_status upload_membership(gsim_batch *b) {
     if (slots > b->sort_slots) {
         destroy_graphs(b);
         b->sort_slots = 2 * slots;
+    }
+    if (c.n_ds && !b->has_ds) {
+        destroy_graphs(b);
+        b->has_ds = true;
     }
     b->h_desc = desc;
     b->h_counts = c;
@@ -236,6 +243,9 @@ gsim_status gsim_batch_create(int32_t device, size_t capacity_particles, uint32_
     b->blocks_cap = (cap + 255) / 256;
     b->free_ranges[0] = (uint32_t)cap;
     hipError_t e = hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking);
+    if (e == hipSuccess) e = hipStreamCreateWithFlags(&b->side, hipStreamNonBlocking);
+    if (e == hipSuccess) e = hipEventCreateWithFlags(&b->fork, hipEventDisableTiming);
+    if (e == hipSuccess) e = hipEventCreateWithFlags(&b->join, hipEventDisableTiming);
     gsim::BatchDevice &d = b->d;
 #define GSIM_BALLOC(ptr, count)                                                          \
     do {                                                                                 \

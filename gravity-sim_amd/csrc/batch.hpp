@@ -35,7 +35,12 @@ struct RankStats {
 // one counter for all of them serialises thousands of same-address atomics.
 constexpr uint32_t kLiveLists = 64;
 
-// The force launch's work list is dealt to kForceQueues interleaved queues
+// Workgroups of the direct-sum launch: one to a CU, so that the build beside it
+// finds room (128: 328 us a step of the mix above bb_ds_kernel, 192: 314, 256:
+// 311, 512: 330, 2,048: 318; on the build's own stream, 512: 337).
+constexpr uint32_t kBatchDsBlocks = 256;
+
+// The walk launch's work list is dealt to kForceQueues interleaved queues
 // (item i to queue i mod kForceQueues); the waves of queue q take its items
 // one at a time from a counter, so a wave that drew light items takes more.
 constexpr uint32_t kForceQueues = 64;
@@ -43,11 +48,11 @@ constexpr uint32_t kForceQueues = 64;
 struct BatchCounts {
     uint32_t n_bh;            // Barnes-Hut systems (ranks)
     uint32_t n_bh_particles;  // sum of their padded counts = sorted positions
-    uint32_t n_items;         // work items of the force launch
+    uint32_t n_items;         // work items, direct-sum blocks first
+    uint32_t n_ds;            // direct-sum blocks
     uint32_t n_cells;         // cell nodes of all trees (emit)
     uint32_t n_leaves;        // occupied leaves of all trees (emit)
     uint32_t n_sys;           // all systems (direct sum and Barnes-Hut)
-    uint32_t pad;
     uint32_t sort_stall;      // radix look-back waits that hit their bound (never expected)
     uint32_t n_live[kLiveLists];  // (system, depth-5 tile) pairs holding leaves, per list
     uint32_t qnext[kForceQueues];  // force launch: items taken from each queue (zeroed each step)
@@ -138,6 +143,9 @@ struct BatchSystem {
 struct gsim_batch {
     int device = 0;
     hipStream_t stream = nullptr;
+    hipStream_t side = nullptr;  // the direct sums, beside the build (captured with it)
+    hipEvent_t fork = nullptr, join = nullptr;
+    bool has_ds = false;         // the graphs hold the direct-sum launch
     size_t capacity = 0;        // particles (padded) in the arena
     size_t node_capacity = 0;   // node slots
     size_t partial_capacity = 0;  // direct-sum admission units

@@ -480,7 +480,7 @@ __global__ __launch_bounds__(1024) void bb_top_kernel(const TileCell *__restrict
     }
 }
 
-// ---- one persistent force launch for every system ------------------------------
+// ---- force: a launch for the direct sums, a persistent one for the walks --------
 
 // Barnes-Hut group g of one system: the walk of bh_kernels.hip over the
 // system's node range with its own constants, one wave per group.
@@ -521,72 +521,43 @@ __device__ void bb_walk_group(uint32_t g, const SysDesc &d, const RankStats &st,
     vel_out[src] = make_float2(nvx, nvy);
 }
 
-// Direct-sum block tb of one system: its 16 targets against every source, role
-// after role, then integrate (ds_block_kernel's additions in its order).
-__device__ void bb_ds_block(uint32_t tb, const SysDesc &d, const float2 *__restrict__ pos_all,
-                            const float2 *__restrict__ vel_all,
-                            const float *__restrict__ mass_all, float2 *__restrict__ pos_out,
-                            float2 *__restrict__ vel_out, bool live) {
-    const uint32_t lane = threadIdx.x & 63, stream = lane & 15u, slot = lane >> 4;
-    const uint32_t mine = 4 * slot + (stream >> 2);  // the target this lane ends with
-    const uint32_t i = d.off + tb * kDsBlockTargets + mine;
-    const bool writes = (lane & 3u) == 0;
-    const float2 p = pos_all[i], v = vel_all[i];
-    if (!live) {  // budget spent: hold the state
-        if (writes) {
-            pos_out[i] = p;
-            vel_out[i] = v;
+// The direct-sum systems' blocks of 16 targets (items [0, n_ds)), a workgroup a
+// block: ds_block_kernel's additions in its order.  The blocks of one system
+// follow each other, so that stepping by the grid spreads each system over all
+// workgroups.  Bound by the VALU (2.7e12 pairs a second).  One wave a block,
+// role after role, inside the walks' launch took the time of the largest
+// system's blocks: 25 systems of 1,030 to 6,128 particles alone 203 -> 136 us a
+// step (the empty build's launches are 50 of each); with 23 Barnes-Hut systems
+// 345 -> 311.
+__global__ __launch_bounds__(64 * kDsRoles, 8) void bb_ds_kernel(
+    const uint2 *__restrict__ items, const SysDesc *__restrict__ desc,
+    const uint32_t *__restrict__ remaining, const BatchCounts *__restrict__ counts,
+    const float2 *__restrict__ pos, const float2 *__restrict__ vel,
+    const float *__restrict__ mass, float2 *__restrict__ pos_out, float2 *__restrict__ vel_out) {
+    __shared__ float2 sum[kDsRoles][kDsBlockTargets];
+    const uint32_t n = counts->n_ds;
+    for (uint32_t it = blockIdx.x; it < n; it += gridDim.x) {
+        const uint2 item = items[it];
+        const SysDesc d = desc[item.x];
+        const bool live = remaining[item.x] != 0u;
+        const uint32_t t0 = item.y * kDsBlockTargets;
+        const uint32_t i = d.off + t0 + (threadIdx.x & (kDsBlockTargets - 1u));
+        const float2 p = pos[i], v = vel[i];
+        if (live) ds_block_role<false>(pos + d.off, mass + d.off, d.na, t0, d.eps2, sum);
+        lds_barrier();
+        if (threadIdx.x < kDsBlockTargets) {
+            float2 po = p, vo = v;  // budget spent: hold the state
+            if (live) {
+                const float2 b = ds_block_sum(sum, threadIdx.x);
+                vo = make_float2(v.x + b.x * d.kv, v.y + b.y * d.kv);  // SimShader.comp:68-69
+                po = make_float2(p.x + ((v.x + vo.x) * 0.5f) * d.dt,
+                                 p.y + ((v.y + vo.y) * 0.5f) * d.dt);
+            }
+            pos_out[i] = po;
+            vel_out[i] = vo;
         }
-        return;
+        lds_barrier();
     }
-    const float2 *const pos = pos_all + d.off;
-    const float *const mass = mass_all + d.off;
-    const uint32_t na = d.na, t0 = tb * kDsBlockTargets;
-    float tx[4], ty[4];
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        const float2 q = pos[t0 + 4 * slot + r];
-        tx[r] = q.x;
-        ty[r] = q.y;
-    }
-    float ev = d.eps2;
-    asm volatile("" : "+v"(ev));
-    constexpr uint32_t kStep = 16 * kDsRoles;
-    float bx = 0.0f, by = 0.0f;
-    // the sixteens of role w start at 16 w, 16 w + 256, ...; the next two in
-    // flight, across roles
-    auto next = [&](uint32_t &w, uint32_t &j) {
-        j += kStep;
-        if (j >= na) j = 16 * ++w;
-    };
-    auto load = [&](uint32_t j) { return ds_source(pos, mass, min(j, na - 16) + stream); };
-    uint32_t w = 0, j = 0, w1 = 0, j1 = 0;
-    next(w1, j1);
-    uint32_t w2 = w1, j2 = j1;
-    next(w2, j2);
-    DsSource q0 = load(j), q1 = load(j1);
-    const uint32_t roles = min(kDsRoles, na / 16);  // the others have no source
-    while (w < roles) {
-        float ax[4] = {0.0f, 0.0f, 0.0f, 0.0f}, ay[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-        const uint32_t role = w;
-        while (w == role) {
-            const DsSource c = q0;
-            q0 = q1;
-            q1 = load(j2);
-            ds_add<false>(c, tx, ty, ev, ax, ay);
-            w = w1;
-            j = j1;
-            w1 = w2;
-            j1 = j2;
-            next(w2, j2);
-        }
-        bx = bx + ds_sum_streams(ax, lane);
-        by = by + ds_sum_streams(ay, lane);
-    }
-    if (!writes) return;
-    const float nvx = v.x + bx * d.kv, nvy = v.y + by * d.kv;  // SimShader.comp:68-69
-    pos_out[i] = make_float2(p.x + ((v.x + nvx) * 0.5f) * d.dt, p.y + ((v.y + nvy) * 0.5f) * d.dt);
-    vel_out[i] = make_float2(nvx, nvy);
 }
 
 template <bool kWide>
@@ -595,13 +566,13 @@ __global__ __launch_bounds__(256) void bb_force_kernel(
     const uint32_t *__restrict__ remaining, const RankStats *__restrict__ stats,
     BatchCounts *__restrict__ counts,
     const uint32_t *__restrict__ sorted_src, const float2 *__restrict__ pos,
-    const float2 *__restrict__ vel, const float *__restrict__ mass,
+    const float2 *__restrict__ vel,
     const float4 *__restrict__ node4, const uint4 *__restrict__ child,
     float2 *__restrict__ pos_out, float2 *__restrict__ vel_out, uint32_t node_cap,
     unsigned long long *__restrict__ wave_acc, uint32_t *__restrict__ ichunk, BatchTune tune) {
     __shared__ WalkShared sh[4];
     const uint32_t w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const uint32_t nitems = counts->n_items;
+    const uint32_t nitems = counts->n_items, n_ds = counts->n_ds;
     // this wave's queue (kForceQueues queues, each shared by the waves of
     // one residue): items are taken one at a time, the next one's ticket
     // drawn before the current item is walked
@@ -615,26 +586,22 @@ __global__ __launch_bounds__(256) void bb_force_kernel(
     unsigned long long acc = 0, vis = 0;
     uint32_t next = draw();
     while (true) {
-        const uint32_t it = q + kForceQueues * next;
+        const uint32_t it = n_ds + q + kForceQueues * next;
         if (it >= nitems) break;  // the queue is drained (every later ticket is beyond too)
         next = draw();
         const uint2 item = items[it];
         const SysDesc d = desc[item.x];
         const bool live = remaining[item.x] != 0u;
-        if (d.algo == GSIM_BARNES_HUT) {
-            const RankStats st = stats[d.bh_rank];
-            // no particle inside the domain, or a spent budget (the keys
-            // kernel has already written the system's output)
-            if (!live || st.n_in == 0) continue;
-            if (d.w == 32)
-                bb_walk_group<32, kWide>(item.y, d, st, sh[w], sorted_src, pos, vel, node4, child,
-                                  pos_out, vel_out, node_cap, vis, acc, &ichunk[it], tune);
-            else
-                bb_walk_group<64, kWide>(item.y, d, st, sh[w], sorted_src, pos, vel, node4, child,
-                                  pos_out, vel_out, node_cap, vis, acc, &ichunk[it], tune);
-        } else {
-            bb_ds_block(item.y, d, pos, vel, mass, pos_out, vel_out, live);
-        }
+        const RankStats st = stats[d.bh_rank];
+        // no particle inside the domain, or a spent budget (the keys
+        // kernel has already written the system's output)
+        if (!live || st.n_in == 0) continue;
+        if (d.w == 32)
+            bb_walk_group<32, kWide>(item.y, d, st, sh[w], sorted_src, pos, vel, node4, child,
+                                     pos_out, vel_out, node_cap, vis, acc, &ichunk[it], tune);
+        else
+            bb_walk_group<64, kWide>(item.y, d, st, sh[w], sorted_src, pos, vel, node4, child,
+                                     pos_out, vel_out, node_cap, vis, acc, &ichunk[it], tune);
     }
     if (lane == 0) {
         wave_acc[blockIdx.x * 4 + w] = acc;
@@ -681,13 +648,23 @@ __global__ __launch_bounds__(256) void bb_finish_kernel(uint32_t *__restrict__ r
 
 }  // namespace
 
-// One batched step: Barnes-Hut build for all BH systems, one persistent force
-// launch for every system.  Launched onto b->stream
+// One batched step: the direct sums on a stream beside the Barnes-Hut build of
+// all BH systems, whose launches leave most of the GPU idle; then the walks.  Launched onto b->stream
 // (captured into a graph by the caller).
 hipError_t batch_launch_step(gsim_batch *b, int in, int out) {
     BatchDevice &d = b->d;
     hipStream_t st = b->stream;
     const uint32_t live_per_list = (uint32_t)(((size_t)b->max_systems * kTiles + kLiveLists - 1) / kLiveLists);
+    if (b->has_ds) {
+        hipError_t e = hipEventRecord(b->fork, st);
+        if (e == hipSuccess) e = hipStreamWaitEvent(b->side, b->fork, 0);
+        if (e != hipSuccess) return e;
+        bb_ds_kernel<<<kBatchDsBlocks, 64 * kDsRoles, 0, b->side>>>(
+            d.items, d.desc, d.remaining, d.counts, d.pos[in], d.vel[in], d.mass, d.pos[out],
+            d.vel[out]);
+        e = hipEventRecord(b->join, b->side);
+        if (e != hipSuccess) return e;
+    }
     const BatchTune &tune = b->tune;
     const uint32_t rounds = tune.sort_rounds;
     if (rounds != 8 && rounds != 12 && rounds != 16) return hipErrorInvalidValue;
@@ -732,10 +709,14 @@ hipError_t batch_launch_step(gsim_batch *b, int in, int out) {
     const uint32_t waves = 1024u * b->tune.waves_per_simd;
     auto *force = b->node_capacity >= kNarrowNodes ? bb_force_kernel<true> : bb_force_kernel<false>;
     force<<<waves / 4, 256, 0, st>>>(d.items, d.desc, d.remaining, d.stats, d.counts, d.sorted_src,
-                                               d.pos[in], d.vel[in], d.mass, d.node4, d.child,
+                                               d.pos[in], d.vel[in], d.node4, d.child,
                                                d.pos[out], d.vel[out],
                                                (uint32_t)b->node_capacity, d.wave_acc, d.ichunk,
                                                tune);
+    if (b->has_ds) {  // the finish counts the step as taken
+        hipError_t e = hipStreamWaitEvent(st, b->join, 0);
+        if (e != hipSuccess) return e;
+    }
     bb_finish_kernel<<<8, 256, 0, st>>>(d.remaining, d.counts, d.wave_acc, waves);
     return hipGetLastError();
 }

@@ -85,55 +85,19 @@ __global__ __launch_bounds__(1024, 8) void ds_block_kernel(
     const float *__restrict__ mass, float2 *__restrict__ pos_out, float2 *__restrict__ vel_out,
     float2 *__restrict__ acc_dbg, uint32_t na, float eps2, float kv, float dt) {
     __shared__ float2 sum[kDsRoles][kDsBlockTargets];
-    const uint32_t lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const uint32_t stream = lane & 15u, slot = lane >> 4;
     const uint32_t t0 = blockIdx.x * kDsBlockTargets;  // na is a multiple of 64
-    float tx[4], ty[4], ax[4], ay[4];
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        const float2 p = pos[t0 + 4 * slot + r];
-        tx[r] = p.x;
-        ty[r] = p.y;
-        ax[r] = 0.0f;
-        ay[r] = 0.0f;
-    }
     // the integrated particles, needed at the end
     const uint32_t i = t0 + (threadIdx.x & (kDsBlockTargets - 1u));
     const float2 p = pos[i], v = vel[i];
-    float ev = eps2;  // in a vector register: a scalar operand costs the second issue
-    asm volatile("" : "+v"(ev));
-    // sixteen sources at 16 w, 16 w + 256, ..., the next four rounds in flight
-    constexpr uint32_t kAhead = 4, kStep = 16 * kDsRoles;
-    const uint32_t first = 16 * w + stream;
-    DsSource q[kAhead];
-#pragma unroll
-    for (uint32_t u = 0; u < kAhead; ++u)
-        q[u] = ds_source(pos, mass, min(first + u * kStep, na - 16 + stream));
-    for (uint32_t j = 16 * w; j < na; j += kAhead * kStep) {
-#pragma unroll
-        for (uint32_t u = 0; u < kAhead; ++u) {
-            if (j + u * kStep >= na) break;
-            const DsSource c = q[u];
-            q[u] = ds_source(pos, mass, min(j + (u + kAhead) * kStep, na - 16) + stream);
-            ds_add<kRcp>(c, tx, ty, ev, ax, ay);
-        }
-    }
-    const float sx = ds_sum_streams(ax, lane), sy = ds_sum_streams(ay, lane);
-    if ((lane & 3u) == 0) sum[w][4 * slot + (stream >> 2)] = make_float2(sx, sy);
+    ds_block_role<kRcp>(pos, mass, na, t0, eps2, sum);
     __syncthreads();
     if (threadIdx.x >= kDsBlockTargets) return;
-    float bx = 0.0f, by = 0.0f;
-#pragma unroll
-    for (uint32_t u = 0; u < kDsRoles; ++u) {
-        const float2 a = sum[u][threadIdx.x];
-        bx = bx + a.x;
-        by = by + a.y;
-    }
+    const float2 b = ds_block_sum(sum, threadIdx.x);
     // SimShader.comp:68-69
-    const float nvx = v.x + bx * kv, nvy = v.y + by * kv;
+    const float nvx = v.x + b.x * kv, nvy = v.y + b.y * kv;
     pos_out[i] = make_float2(p.x + ((v.x + nvx) * 0.5f) * dt, p.y + ((v.y + nvy) * 0.5f) * dt);
     vel_out[i] = make_float2(nvx, nvy);
-    if (acc_dbg) acc_dbg[i] = make_float2(bx, by);
+    if (acc_dbg) acc_dbg[i] = b;
 }
 
 __global__ __launch_bounds__(256) void ds_combine_kernel(
