@@ -212,7 +212,14 @@ gsim_status run_steps(gsim_sim *s, uint32_t count) {
                                               s->vel[out], s->perm[out]));
             if (trial) {
                 GSIM_HIP(hipEventRecord(s->order_ev[2 * s->order_rec + 1], s->stream));
-                if (++s->order_rec == gsim::kOrderTrial) s->order_wait = true;
+                if (++s->order_rec == gsim::kOrderTrial) {
+                    s->order_wait = true;
+                    // until the outcome is read: a caller that queues many
+                    // steps gets no poll in between.  20 steps of 1,000,000
+                    // particles (galaxy) 1,023 us each against 1,560 in index
+                    // order; where index order is the faster it is by 1%.
+                    s->trav_order = 1;
+                }
             } else {
                 order_poll(s);
             }

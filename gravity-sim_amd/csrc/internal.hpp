@@ -31,7 +31,7 @@ constexpr float kSimSize = 500.0f;
 constexpr uint32_t kTreeSize = 1024;
 constexpr uint32_t kTreeDepth = 10;
 // GSIM_TUNE_BH_ORDER = 2 (auto): every kOrderPeriod steps, kOrderTrial
-// consecutive W = 32 steps alternate heaviest-first and index order
+// consecutive steps alternate heaviest-first and index order
 constexpr uint32_t kOrderTrial = 4;
 constexpr uint64_t kOrderPeriod = 1024;
 constexpr uint64_t kOrderReplan = 8;  // steps between plans of the order
@@ -216,7 +216,8 @@ struct gsim_sim {
     // Static walk's launch order: order_mode 0 index, 1 heaviest first (by last
     // step's visits), 2 auto: a trial of kOrderTrial steps alternating the
     // two, timed by events, keeps the faster once the host sees the trial's
-    // last event complete (polled at each later step; never waited for)
+    // last event complete (polled at each later step; never waited for),
+    // heaviest first until then
     uint32_t order_mode = 2;
     uint32_t trav_order = 0;           // the order the next walk uses (0/1)
     bool order_fresh = false;          // this step is a trial step: plan afresh
