@@ -1223,7 +1223,7 @@ hipError_t bh_alloc(BhBuffers *b, size_t na, uint32_t bits) {
     b->na = na;
     b->bits = bits;
     b->cap = bh_capacity(na, bits);
-    b->sort_blocks = (na + kSortTile - 1) / kSortTile;
+    b->sort_blocks = sort_tiles(na);
     b->prep_blocks = (na + 255) / 256;
     hipError_t e = hipSuccess;
 #define GSIM_ALLOC(ptr, count)                                                  \
@@ -1335,10 +1335,9 @@ hipError_t bh_launch_build(gsim_sim *s, const float2 *pos, const float *mass,
         else { if (deep) GSIM_SMALL(false, true, false); else GSIM_SMALL(false, false, false); }
 #undef GSIM_SMALL
     } else {
-        // one tile of kSortTile keys per workgroup, in the keys kernel and in
-        // every pass; each pass's status holds its tile words, then its group words
-        const uint32_t nblk = (na + kSortTile - 1) / kSortTile;
-        const uint32_t kblk = nblk;
+        // one tile per workgroup, in the keys kernel and in every pass; each
+        // pass's status holds its tile words, then its group words
+        const uint32_t nblk = (uint32_t)sort_tiles(na);
         const uint32_t pass_words = (nblk + (nblk + kLookGroup - 1) / kLookGroup) * 256u;
         const int passes = deep ? 4 : 3;
         const uint32_t status_words = (uint32_t)passes * pass_words;
@@ -1346,25 +1345,32 @@ hipError_t bh_launch_build(gsim_sim *s, const float2 *pos, const float *mass,
         uint32_t *const totals = b.digit_total + kDigitCopies * 1024 * b.parity;
         uint32_t *const totals_next = b.digit_total + kDigitCopies * 1024 * (b.parity ^ 1u);
         b.parity ^= 1u;
-#define GSIM_KEYS(B, D, W)                                                                    \
-        bh_keys_kernel<B, D, kSortRounds, W><<<kblk, kSortThreads, 0, s->stream>>>(                \
-            pos, perm_in, na, b.cells[kin], b.tile_range, totals, totals_next, b.status,          \
-            status_words, b.ctr, box)
-        if (box) { if (deep) GSIM_KEYS(true, true, false); else GSIM_KEYS(true, false, false); }
-        else if (walk) { if (deep) GSIM_KEYS(false, true, true); else GSIM_KEYS(false, false, true); }
-        else { if (deep) GSIM_KEYS(false, true, false); else GSIM_KEYS(false, false, false); }
-#undef GSIM_KEYS
         // 20-bit keys: cells[kin] -> keys[0] -> keys[1] -> keys[0]; 30-bit keys take
         // a fourth pass -> keys[1].  cells[kin] keeps the per-particle cells.
         const int in_of[4] = {-1, 0, 1, 0}, out_of[4] = {0, 1, 0, 1};
-        for (int pass = 0; pass < passes; ++pass) {
-            const int i = in_of[pass], o = out_of[pass];
-            uint32_t *const st = b.status + (size_t)pass * pass_words;
-            radix_onesweep_kernel<kSortRounds><<<nblk, kSortThreads, 0, s->stream>>>(
-                i < 0 ? nullptr : b.keys[i], i < 0 ? nullptr : b.idx[i], i < 0 ? b.cells[kin] : nullptr,
-                b.keys[o], b.idx[o], na, 8u * pass, totals + 256 * pass, st,
-                &b.ctr->sort_stall);
-        }
+#define GSIM_KEYS(R, B, D, W)                                                                  \
+    bh_keys_kernel<B, D, R, W><<<nblk, kSortThreads, 0, s->stream>>>(                           \
+        pos, perm_in, na, b.cells[kin], b.tile_range, totals, totals_next, b.status,           \
+        status_words, b.ctr, box)
+#define GSIM_SORT(R)                                                                           \
+    do {                                                                                       \
+        if (box) { if (deep) GSIM_KEYS(R, true, true, false); else GSIM_KEYS(R, true, false, false); } \
+        else if (walk) { if (deep) GSIM_KEYS(R, false, true, true); else GSIM_KEYS(R, false, false, true); } \
+        else { if (deep) GSIM_KEYS(R, false, true, false); else GSIM_KEYS(R, false, false, false); } \
+        for (int pass = 0; pass < passes; ++pass) {                                            \
+            const int i = in_of[pass], o = out_of[pass];                                       \
+            radix_onesweep_kernel<R><<<nblk, kSortThreads, 0, s->stream>>>(                    \
+                i < 0 ? nullptr : b.keys[i], i < 0 ? nullptr : b.idx[i],                       \
+                i < 0 ? b.cells[kin] : nullptr, b.keys[o], b.idx[o], na, 8u * pass,            \
+                totals + 256 * pass, b.status + (size_t)pass * pass_words, &b.ctr->sort_stall); \
+        }                                                                                      \
+    } while (0)
+        const uint32_t rounds = sort_rounds(na);
+        if (rounds == 2) GSIM_SORT(2);
+        else if (rounds == 4) GSIM_SORT(4);
+        else GSIM_SORT(8);
+#undef GSIM_SORT
+#undef GSIM_KEYS
         bh_prep_kernel<<<pb, 256, 0, s->stream>>>(sk, na, bits, b.block_cells, b.block_leaves,
                                                   deep ? b.block_gran : nullptr);
         bh_emit_kernel<<<pb, 256, 0, s->stream>>>(sk, si, emit, b.block_cells, b.block_leaves,

@@ -53,12 +53,22 @@ struct BhCounters {
     uint32_t sort_stall;         // look-back waits that hit their bound (never expected)
 };
 
-// Radix sort passes (single and batched builds): tiles of kSortTile keys,
-// kSortRounds per thread of a kSortThreads workgroup.  Look-back status
-// buffers hold 256 words per tile.
+// Radix sort passes (single and batched builds): tiles of kSortThreads keys a
+// round.  Look-back status buffers hold 256 words per tile.
 constexpr int kSortThreads = 256;
-constexpr int kSortRounds = 8;
-constexpr int kSortTile = kSortThreads * kSortRounds;
+// Rounds of the single build: as few as leave a tile a CU, two at least, and
+// eight where the tiles outnumber the CUs, so that the chain of look-backs
+// stays short.  Build in us at 2 / 4 / 8 rounds: 20,000 particles 46.7 / 48.5 /
+// 50.6, 100,000 53.6 / 55.5 / 59.7, 200,000 65.4 / 62.1 / 66.2, 300,000 71.7 /
+// 69.3 / 69.1, 500,000 94 / 80.8 / 77.8, 1,000,000 147 / 119 / 108 (12 rounds
+// 116).
+constexpr uint32_t sort_rounds(size_t na) {
+    return na <= 256 * 2 * kSortThreads ? 2 : na <= 256 * 4 * kSortThreads ? 4 : 8;
+}
+constexpr size_t sort_tiles(size_t na) {
+    const size_t tile = sort_rounds(na) * kSortThreads;
+    return (na + tile - 1) / tile;
+}
 // Tiles per group of the radix passes' two-level look-back; each pass's
 // status words hold its tile words, then one group word set per kLookGroup
 // tiles.

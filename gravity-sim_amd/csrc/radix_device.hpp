@@ -1,7 +1,7 @@
 // One-sweep stable LSD radix sort pieces shared by the single-system build
 // (bh_kernels.hip) and the batched build (batch_kernels.hip).
 //
-// A pass sorts tiles of kSortTile (key, value) pairs on one 8-bit digit, one
+// A pass sorts tiles of kR * kSortThreads (key, value) pairs on one 8-bit digit, one
 // tile per workgroup in launch order, so every lower tile belongs to a
 // workgroup that has started before.  Within the tile, key r * 256 + t
 // (round r, thread t) is ranked among the equal digits of its wave by
@@ -24,9 +24,8 @@ namespace gsim {
 constexpr uint32_t kStA = 1u << 30, kStP = 2u << 30, kStVal = kStA - 1u;
 constexpr uint32_t kSpinLimit = 1u << 20;  // bound on re-reads of one status word
 
-// kR: rounds of kSortThreads keys per tile (kSortRounds unless the launch
-// picks another tile size).
-template <bool kStage, int kR = kSortRounds>
+// kR: rounds of kSortThreads keys per tile.
+template <bool kStage, int kR>
 struct SortShared {
     static constexpr int kRows = kR * (kSortThreads / 64);
     static constexpr int kTile = kR * kSortThreads;

@@ -103,3 +103,11 @@ def test_batch_sorted_by_system_equals_each_system_alone(tile):
     for a in alone:
         a.close()
     batch.close()
+
+
+@pytest.mark.parametrize("bits,boxed", [(10, False), (15, True)])
+@pytest.mark.parametrize("n", [131072, 131073, 262144, 262145])
+def test_tree_on_both_sides_of_a_change_of_radix_tile(n, bits, boxed):
+    print(f"radix tile n={n} bits={bits}", flush=True)
+    p = gsim.generate("galaxy-collision", n, 130.0, 1.0, 10.0, seed=n)
+    _same_tree(p.pos, p.mass, bits, 2, boxed)
