@@ -41,8 +41,11 @@ namespace {
 // ---- 1. keys ----------------------------------------------------------------
 
 // ---- 0. adaptive bounding box (opt-in; beyond the reference) -------------------
-// Extremes of the finite positions: per-block partials, then one block that
-// also applies the box formula {cx, cy, h, r0} (order-independent, so exact).
+// Extremes of the finite positions: per-block partials, reduced by every
+// workgroup of the keys kernel, which applies the box formula {cx, cy, h, r0}
+// (order-independent, so exact).  One block's launch for it took 4.6 us (build
+// with the box, 100,000 particles: 60.7 -> 59.1); up to kSmallBuild particles
+// the one workgroup takes the extremes itself (1,000: 31.6 -> 27.2).
 
 __device__ __forceinline__ void minmax4_wave(float &a, float &b, float &c, float &d) {
 #pragma unroll
@@ -83,39 +86,31 @@ __global__ __launch_bounds__(256) void bh_box_partial_kernel(const float2 *__res
     }
 }
 
-__global__ __launch_bounds__(256) void bh_box_final_kernel(const float4 *__restrict__ part,
-                                                           uint32_t nparts,
-                                                           float *__restrict__ box) {
-    __shared__ float4 wv[4];
-    float x0 = __builtin_inff(), x1 = -__builtin_inff(), y0 = __builtin_inff(),
-          y1 = -__builtin_inff();
-    for (uint32_t i = threadIdx.x; i < nparts; i += 256) {
-        const float4 r = part[i];
-        x0 = fminf(x0, r.x);
-        x1 = fmaxf(x1, r.y);
-        y0 = fminf(y0, r.z);
-        y1 = fmaxf(y1, r.w);
-    }
-    minmax4_wave(x0, x1, y0, y1);
-    if ((threadIdx.x & 63) == 0) wv[threadIdx.x >> 6] = make_float4(x0, x1, y0, y1);
-    lds_barrier();
-    if (threadIdx.x != 0) return;
-    for (int w = 1; w < 4; ++w) {
-        wv[0].x = fminf(wv[0].x, wv[w].x);
-        wv[0].y = fmaxf(wv[0].y, wv[w].y);
-        wv[0].z = fminf(wv[0].z, wv[w].z);
-        wv[0].w = fmaxf(wv[0].w, wv[w].w);
-    }
-    float xmin = wv[0].x, xmax = wv[0].y, ymin = wv[0].z, ymax = wv[0].w;
+// Centre, half edge and r0 of the box around extremes x0 <= x1, y0 <= y1.
+__device__ __forceinline__ float4 box_of(float xmin, float xmax, float ymin, float ymax) {
     if (!(xmin <= xmax)) xmin = xmax = ymin = ymax = 0.0f;  // no finite particle
     const float cx = (xmin + xmax) * 0.5f, cy = (ymin + ymax) * 0.5f;
     const float w = fmaxf(xmax - xmin, ymax - ymin);
     float h = w * 0.501953125f;  // half the extent plus 2^-9: the farthest maps below 1024
     if (!(h >= 1e-3f)) h = 1e-3f;
-    box[0] = cx;
-    box[1] = cy;
-    box[2] = h;
-    box[3] = (h * h) * 2.0f;
+    return make_float4(cx, cy, h, (h * h) * 2.0f);
+}
+
+// The box around every wave's extremes, in every thread of a workgroup of
+// kWaves waves (synchronises it).
+template <uint32_t kWaves>
+__device__ __forceinline__ float4 box_of_group(float x0, float x1, float y0, float y1,
+                                               float4 (&wv)[kWaves]) {
+    minmax4_wave(x0, x1, y0, y1);
+    if ((threadIdx.x & 63) == 0) wv[threadIdx.x >> 6] = make_float4(x0, x1, y0, y1);
+    lds_barrier();
+    float4 r = wv[0];
+#pragma unroll
+    for (uint32_t w = 1; w < kWaves; ++w) {
+        const float4 o = wv[w];
+        r = make_float4(fminf(r.x, o.x), fmaxf(r.y, o.y), fminf(r.z, o.z), fmaxf(r.w, o.w));
+    }
+    return box_of(r.x, r.y, r.z, r.w);
 }
 
 // kDeep: 30-bit keys of the 32768^2 grid (15-bit leaves) instead of 20-bit cells.
@@ -139,7 +134,7 @@ __global__ __launch_bounds__(kSortThreads) void bh_keys_kernel(
     uint2 *__restrict__ cells, uint32_t *__restrict__ tile_range,
     uint32_t *__restrict__ digit_total, uint32_t *__restrict__ digit_next,
     uint32_t *__restrict__ status, uint32_t status_words, BhCounters *__restrict__ ctr,
-    const float *__restrict__ box) {
+    const float4 *__restrict__ box_part, uint32_t box_parts, float4 *__restrict__ box) {
     constexpr int kPasses = kDeep ? 4 : 3;
     __shared__ uint32_t h[kPasses][256];
     const uint32_t t = threadIdx.x;
@@ -152,7 +147,16 @@ __global__ __launch_bounds__(kSortThreads) void bh_keys_kernel(
     }
 #pragma unroll
     for (int p = 0; p < kPasses; ++p) h[p][t] = 0;
-    lds_barrier();
+    float4 bx = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    if constexpr (kBox) {
+        __shared__ float4 wv[kSortThreads / 64];
+        const float inf = __builtin_inff();
+        const float4 q = t < box_parts ? box_part[t] : make_float4(inf, -inf, inf, -inf);
+        bx = box_of_group(q.x, q.y, q.z, q.w, wv);  // synchronises
+        if (g == 0) *box = bx;
+    } else {
+        lds_barrier();
+    }
     const uint32_t base = blockIdx.x * (kR * kSortThreads);
     if constexpr (kWalk) {
         uint32_t c[kR];
@@ -179,8 +183,8 @@ __global__ __launch_bounds__(kSortThreads) void bh_keys_kernel(
         if (i >= na) continue;
         const float2 p = pr[r];
         uint32_t c;
-        if (kDeep) c = kBox ? cell30_box(p.x, p.y, box[0], box[1], box[2]) : cell30(p.x, p.y);
-        else c = kBox ? cell20_box(p.x, p.y, box[0], box[1], box[2]) : cell20(p.x, p.y);
+        if (kDeep) c = kBox ? cell30_box(p.x, p.y, bx.x, bx.y, bx.z) : cell30(p.x, p.y);
+        else c = kBox ? cell20_box(p.x, p.y, bx.x, bx.y, bx.z) : cell20(p.x, p.y);
         if (c == 0xffffffffu) c = kDeep ? kKilledKeyDeep : kKilledKey;
         cells[orig[r]] = make_uint2(c, i);
         hist_add<kPasses>(h, c);
@@ -439,7 +443,7 @@ constexpr uint32_t kSmallRows = kSmallBuild / (64 * kSmallWaves);  // keys per l
 template <bool kBox, bool kDeep, bool kWalk>
 __global__ __launch_bounds__(64 * kSmallWaves) void bh_small_kernel(
     EmitArgs e, uint2 *__restrict__ cells, uint32_t *__restrict__ keys_out,
-    uint32_t *__restrict__ tile_range, const float *__restrict__ box) {
+    uint32_t *__restrict__ tile_range, float4 *__restrict__ box) {
     constexpr uint32_t kBits = kDeep ? 8 : 7, kPasses = kDeep ? 4 : 3, kDigits = 1u << kBits;
     constexpr uint32_t kNone = 0xffffffffu;
     __shared__ uint32_t skey[kSmallBuild];
@@ -463,14 +467,30 @@ __global__ __launch_bounds__(64 * kSmallWaves) void bh_small_kernel(
             p[r] = e.pos[k];
             o[r] = e.perm_in[k];
         }
+        float4 bx = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        if constexpr (kBox) {  // as bh_box_partial_kernel
+            __shared__ float4 wv[kSmallWaves];
+            float x0 = __builtin_inff(), x1 = -x0, y0 = x0, y1 = -x0;
+#pragma unroll
+            for (uint32_t r = 0; r < kSmallRows; ++r) {
+                if (r >= rows || first + 64 * r >= na) continue;
+                if (!__builtin_isfinite(p[r].x) || !__builtin_isfinite(p[r].y)) continue;
+                x0 = fminf(x0, p[r].x);
+                x1 = fmaxf(x1, p[r].x);
+                y0 = fminf(y0, p[r].y);
+                y1 = fmaxf(y1, p[r].y);
+            }
+            bx = box_of_group(x0, x1, y0, y1, wv);
+            if (t == 0) *box = bx;
+        }
 #pragma unroll
         for (uint32_t r = 0; r < kSmallRows; ++r) {
             const uint32_t k = first + 64 * r;
             if (r >= rows || k >= na) continue;
             const float x = p[r].x, y = p[r].y;
             uint32_t c;
-            if (kDeep) c = kBox ? cell30_box(x, y, box[0], box[1], box[2]) : cell30(x, y);
-            else c = kBox ? cell20_box(x, y, box[0], box[1], box[2]) : cell20(x, y);
+            if (kDeep) c = kBox ? cell30_box(x, y, bx.x, bx.y, bx.z) : cell30(x, y);
+            else c = kBox ? cell20_box(x, y, bx.x, bx.y, bx.z) : cell20(x, y);
             if (c == kNone) c = kDeep ? kKilledKeyDeep : kKilledKey;
             cells[o[r]] = make_uint2(c, k);
             skey[o[r]] = c;
@@ -1303,16 +1323,11 @@ hipError_t bh_launch_build(gsim_sim *s, const float2 *pos, const float *mass,
                            float2 *vel_out, float *mass_out, uint32_t *perm_out) {
     BhBuffers &b = s->bh;
     const uint32_t na = (uint32_t)s->na;
-    const uint32_t g256 = (na + 255) / 256;
     const bool deep = b.bits == kDeepBits;
     const int bits = (int)b.bits;
-    const float *box = nullptr;
-    if (s->bh_box) {
-        const uint32_t nparts = std::min<uint32_t>(g256, kBoxParts);
-        bh_box_partial_kernel<<<nparts, 256, 0, s->stream>>>(pos, na, b.box_part);
-        bh_box_final_kernel<<<1, 256, 0, s->stream>>>(b.box_part, nparts, b.box);
-        box = b.box;
-    }
+    // adaptive box: written by the kernel that makes the keys
+    const float *box = s->bh_box ? b.box : nullptr;
+    float4 *const box4 = reinterpret_cast<float4 *>(b.box);
     // the sort's input: written by the last walk (fixed domain), else here
     const int kin = b.kin;
     const bool walk = b.walk_keys && !box;
@@ -1329,7 +1344,7 @@ hipError_t bh_launch_build(gsim_sim *s, const float2 *pos, const float *mass,
         uint32_t *const ko = b.keys[b.sorted_slot];
 #define GSIM_SMALL(B, D, W)                                                                   \
     bh_small_kernel<B, D, W><<<1, 64 * kSmallWaves, 0, s->stream>>>(emit, b.cells[kin], ko,    \
-                                                                    b.tile_range, box)
+                                                                    b.tile_range, box4)
         if (box) { if (deep) GSIM_SMALL(true, true, false); else GSIM_SMALL(true, false, false); }
         else if (walk) { if (deep) GSIM_SMALL(false, true, true); else GSIM_SMALL(false, false, true); }
         else { if (deep) GSIM_SMALL(false, true, false); else GSIM_SMALL(false, false, false); }
@@ -1338,6 +1353,8 @@ hipError_t bh_launch_build(gsim_sim *s, const float2 *pos, const float *mass,
         // one tile per workgroup, in the keys kernel and in every pass; each
         // pass's status holds its tile words, then its group words
         const uint32_t nblk = (uint32_t)sort_tiles(na);
+        const uint32_t nparts = std::min<uint32_t>((na + 255) / 256, kBoxParts);
+        if (box) bh_box_partial_kernel<<<nparts, 256, 0, s->stream>>>(pos, na, b.box_part);
         const uint32_t pass_words = (nblk + (nblk + kLookGroup - 1) / kLookGroup) * 256u;
         const int passes = deep ? 4 : 3;
         const uint32_t status_words = (uint32_t)passes * pass_words;
@@ -1351,7 +1368,7 @@ hipError_t bh_launch_build(gsim_sim *s, const float2 *pos, const float *mass,
 #define GSIM_KEYS(R, B, D, W)                                                                  \
     bh_keys_kernel<B, D, R, W><<<nblk, kSortThreads, 0, s->stream>>>(                           \
         pos, perm_in, na, b.cells[kin], b.tile_range, totals, totals_next, b.status,           \
-        status_words, b.ctr, box)
+        status_words, b.ctr, b.box_part, nparts, box4)
 #define GSIM_SORT(R)                                                                           \
     do {                                                                                       \
         if (box) { if (deep) GSIM_KEYS(R, true, true, false); else GSIM_KEYS(R, true, false, false); } \
