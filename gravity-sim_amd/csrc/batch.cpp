@@ -275,7 +275,7 @@ gsim_status gsim_batch_create(int32_t device, size_t capacity_particles, uint32_
     GSIM_BALLOC(d.leaf_sum, cap);
     GSIM_BALLOC(d.leaf_first, cap + 1);
     GSIM_BALLOC(d.leaf_key, cap);
-    GSIM_BALLOC(d.tile_range, 2 * (size_t)gsim::kTiles * max_systems);
+    GSIM_BALLOC(d.tile_range, (size_t)gsim::kTileWords * max_systems);
     GSIM_BALLOC(d.live_tiles, (size_t)gsim::kTiles * max_systems);
     GSIM_BALLOC(d.top, (size_t)gsim::kTiles * max_systems);
     GSIM_BALLOC(d.node4, b->node_capacity);

@@ -840,183 +840,17 @@ __global__ __launch_bounds__(256) void bh_gran_kernel(
 
 // ---- 6./7. dense reduction per tile, then the top ------------------------------
 
-// Level offsets inside `up`: depth 9 at 0 (256 cells), 8 at 256 (64),
-// 7 at 320 (16), 6 at 336 (4), 5 at 340 (1).
-__device__ __forceinline__ int tile_level_offset(int d) {
-    return d == 9 ? 0 : d == 8 ? 256 : d == 7 ? 320 : d == 6 ? 336 : 340;
-}
-
-// A tile's record for the workgroup that reduces the top, on any XCD: each
-// word is stored at the scope of the device and has arrived before the call
-// returns, and is loaded at that scope, past the XCD's own L2.  A fence would
-// write that whole L2 back, once a tile.
-__device__ __forceinline__ void publish_top(TileCell *to, const TileCell &c) {
-    uint32_t *w = reinterpret_cast<uint32_t *>(to);
-    status_store(w + 0, c.n);
-    status_store(w + 1, c.y);
-    status_store(w + 2, c.f);
-    status_store(w + 4, __float_as_uint(c.sx));
-    status_store(w + 5, __float_as_uint(c.sy));
-    status_store(w + 6, __float_as_uint(c.sm));
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-}
-
-__device__ __forceinline__ TileCell published_top(const TileCell *from) {
-    const uint32_t *w = reinterpret_cast<const uint32_t *>(from);
-    TileCell c;
-    c.n = status_load(w + 0);
-    c.y = status_load(w + 1);
-    c.f = status_load(w + 2);
-    c.pad = 0u;
-    c.sx = __uint_as_float(status_load(w + 4));
-    c.sy = __uint_as_float(status_load(w + 5));
-    c.sm = __uint_as_float(status_load(w + 6));
-    c.pad2 = 0.0f;
-    return c;
-}
-
-// The last occupied tile's workgroup to finish also reduces the 1024 depth-5
-// cells to the root and writes depths 4..0, so the top needs no launch of its
-// own.  Occupied tiles publish their record, then count themselves done in
-// their group of 32 tiles; the last of a group counts the group done, and the
-// last group's workgroup goes on.  How many to expect is read from tile_range.
-// One counter for all tiles is a chain of 1024 same-address atomics across the
-// XCDs, and the fence it needs writes an L2 back for each.  Empty tiles return
-// at once; their empty record comes from tile_range.
-// Bound by latency: its chain of loads, six levels and two counts.  53.3 ->
-// 14.5 us with every tile occupied (200,000 particles, adaptive box), 12.7 ->
-// 8.1 us at 500,000 in the fixed domain, 16.3 -> 8.2 us at 5,000: the counters
-// a cache line apart 57 -> 22, the smaller LDS image and the loads ahead of it
-// the rest.
 __global__ __launch_bounds__(256) void bh_tile_kernel(
     uint32_t *__restrict__ tile_range, const uint32_t *__restrict__ leaf_first,
     const uint32_t *__restrict__ leaf_key, const float4 *__restrict__ leaf_sum,
     const int8_t *__restrict__ sdep, const uint32_t *__restrict__ cpos,
     float4 *__restrict__ node4, uint4 *__restrict__ child, TileCell *__restrict__ top,
     const float *__restrict__ box, const uint32_t *__restrict__ leaf_y) {
-    // leaf_y (15-bit leaves): the depth-10 records are granules whose subtree
-    // size is given; otherwise leaves of n particles, y = n + [n >= 2].  The
-    // depth-10 nodes themselves are already written.
-    // the depth-10 cells {sums, particles} and {subtree size, first particle}:
-    // 35 KB with `up`, so all 1024 workgroups are resident (four a CU)
-    __shared__ float4 sum10[1024];
-    __shared__ uint2 yf10[1024];
-    __shared__ TileCell up[341];
-    __shared__ uint32_t last, wave_groups[4];
-    const uint32_t T = blockIdx.x, t = threadIdx.x;
-    const uint32_t lb = tile_range[2 * T], le = tile_range[2 * T + 1];
-    if (lb == le) return;  // the whole workgroup: an empty tile
-    uint32_t *const done = tile_range + 2 * kTiles;  // 32 words apart; the groups' last
-    const uint2 *const range = reinterpret_cast<const uint2 *>(tile_range);
-    uint32_t expect = 0;  // occupied tiles of this tile's group
-    if (t >= 192) {  // the wave that publishes: it emits fewest cells
-        const uint2 r = range[(T & ~31u) + (t & 31u)];
-        expect = (uint32_t)__popcll(__ballot(t < 224 && r.x != r.y));
-    }
-    const float r0 = box ? box[3] : kFixedR0;
-    // a tile holds at most 1024 leaves (granules): four per thread, loaded
-    // together
-    struct Leaf {
-        float4 s;
-        uint32_t k, f, y;
-    };
-    auto leaf = [&](uint32_t u) {
-        const uint32_t L = min(lb + t + 256 * u, le - 1);
-        return Leaf{leaf_sum[L], leaf_key[L], leaf_first[L], leaf_y ? leaf_y[L] : 0u};
-    };
-    const Leaf a0 = leaf(0), a1 = leaf(1), a2 = leaf(2), a3 = leaf(3);
-#pragma unroll
-    for (uint32_t u = 0; u < 4; ++u) {
-        sum10[t + 256 * u] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        yf10[t + 256 * u] = make_uint2(0u, 0xffffffffu);
-    }
-    lds_barrier();
-    auto place = [&](uint32_t u, const Leaf &a) {
-        if (lb + t + 256 * u >= le) return;
-        const uint32_t c = a.k & 1023u, n = __float_as_uint(a.s.w);
-        sum10[c] = a.s;
-        yf10[c] = make_uint2(leaf_y ? a.y : n + (n >= 2u ? 1u : 0u), a.f);
-    };
-    place(0, a0);
-    place(1, a1);
-    place(2, a2);
-    place(3, a3);
-    lds_barrier();
-    auto kid = [&](uint32_t u) {  // of depth-9 cell t
-        const float4 s = sum10[4 * t + u];
-        const uint2 q = yf10[4 * t + u];
-        return TileCell{__float_as_uint(s.w), q.x, q.y, 0u, s.x, s.y, s.z, 0.0f};
-    };
-    const TileCell k0 = kid(0), k1 = kid(1), k2 = kid(2), k3 = kid(3);
-    const uint4 sizes9 = make_uint4(k0.y, k1.y, k2.y, k3.y);
-    const TileCell c9 = reduce4(k0, k1, k2, k3);
-    up[t] = c9;
-    lds_barrier();
-    for (int d = 8; d >= 5; --d) {
-        const uint32_t cnt = 1u << (2 * (d - 5));
-        const int o = tile_level_offset(d), oc = tile_level_offset(d + 1);
-        if (t < cnt)
-            up[o + t] = reduce4(up[oc + 4 * t], up[oc + 4 * t + 1], up[oc + 4 * t + 2],
-                                up[oc + 4 * t + 3]);
-        lds_barrier();
-    }
-    if (t == 192) {
-        publish_top(top + T, up[340]);
-        last = atomicAdd(done + T / 32 * 32, 1u) + 1u == expect ? 1u : 0u;
-    }
-    if (t < 85) {  // depths 8..5
-        const uint32_t c = 256 + t;
-        const int d = c < 320 ? 8 : c < 336 ? 7 : c < 340 ? 6 : 5;
-        const TileCell *kids = up + tile_level_offset(d + 1) + 4 * (c - tile_level_offset(d));
-        emit_cell(up[c], d, sizes4(kids), sdep, cpos, node4, child, r0);
-    }
-    emit_cell(c9, 9, sizes9, sdep, cpos, node4, child, r0);
-    lds_barrier();
-    if (!last) return;
-    const uint4 ra = reinterpret_cast<const uint4 *>(tile_range)[2 * t];
-    const uint4 rb = reinterpret_cast<const uint4 *>(tile_range)[2 * t + 1];
-    const bool in0 = ra.x != ra.y, in1 = ra.z != ra.w, in2 = rb.x != rb.y, in3 = rb.z != rb.w;
-    // groups with an occupied tile: eight threads a group, eight groups a wave
-    unsigned long long m = __ballot(in0 || in1 || in2 || in3);
-    m |= m >> 4;
-    m |= m >> 2;
-    m |= m >> 1;
-    if ((t & 63) == 0)
-        wave_groups[t >> 6] = (uint32_t)__popcll(m & 0x0101010101010101ull);
-    lds_barrier();
-    if (t == 0)
-        last = atomicAdd(done + 32 * 32, 1u) + 1u ==
-                       wave_groups[0] + wave_groups[1] + wave_groups[2] + wave_groups[3]
-                   ? 1u
-                   : 0u;
-    lds_barrier();
-    if (!last) return;
-    asm volatile("" ::: "memory");  // no record is read before the counts
-    // depths 4..0 in `up` at the offsets of depths 9..5
-    const TileCell empty{0u, 0u, 0xffffffffu, 0u, 0.0f, 0.0f, 0.0f, 0.0f};
-    const TileCell t0 = in0 ? published_top(top + 4 * t) : empty;
-    const TileCell t1 = in1 ? published_top(top + 4 * t + 1) : empty;
-    const TileCell t2 = in2 ? published_top(top + 4 * t + 2) : empty;
-    const TileCell t3 = in3 ? published_top(top + 4 * t + 3) : empty;
-    const TileCell c4 = reduce4(t0, t1, t2, t3);
-    up[t] = c4;
-    emit_cell(c4, 4, make_uint4(t0.y, t1.y, t2.y, t3.y), sdep, cpos, node4, child, r0);
-    lds_barrier();
-    for (int d = 3; d >= 0; --d) {
-        const uint32_t cnt = 1u << (2 * d);
-        const int o = tile_level_offset(d + 5), oc = tile_level_offset(d + 6);
-        if (t < cnt)
-            up[o + t] = reduce4(up[oc + 4 * t], up[oc + 4 * t + 1], up[oc + 4 * t + 2],
-                                up[oc + 4 * t + 3]);
-        lds_barrier();
-    }
-    if (t < 85) {  // depths 3..0
-        const uint32_t c = 256 + t;
-        const int d = c < 320 ? 3 : c < 336 ? 2 : c < 340 ? 1 : 0;
-        const TileCell *kids =
-            up + tile_level_offset(d + 6) + 4 * (c - tile_level_offset(d + 5));
-        emit_cell(up[c], d, sizes4(kids), sdep, cpos, node4, child, r0);
-    }
+    __shared__ TileShared sh;
+    const uint32_t T = blockIdx.x;
+    if (tile_range[2 * T] == tile_range[2 * T + 1]) return;  // the whole workgroup: empty
+    reduce_tile(T, tile_range, leaf_first, leaf_key, leaf_sum, leaf_y, sdep, cpos, node4, child,
+                top, box ? box[3] : kFixedR0, sh);
 }
 
 // ---- 8. traversal + integrate ----------------------------------------------------

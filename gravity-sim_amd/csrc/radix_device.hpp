@@ -37,14 +37,6 @@ struct SortShared {
     uint32_t wsum[4];
 };
 
-__device__ __forceinline__ uint32_t status_load(const uint32_t *p) {
-    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-__device__ __forceinline__ void status_store(uint32_t *p, uint32_t v) {
-    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
 // Lanes of this wave whose kBits-bit digit equals this lane's (valid lanes only).
 template <int kBits = 8>
 __device__ __forceinline__ uint64_t digit_peers(uint32_t d, bool valid) {
