@@ -58,7 +58,7 @@ void free_batch(gsim_batch *b) {
                     d.keys[0], d.keys[1], d.idx[0], d.idx[1], d.status, d.digit_total,
                     d.block_cells, d.block_leaves, d.sdep, d.cpos, d.sorted_src,
                     d.leaf_sum, d.leaf_first, d.leaf_key, d.tile_range, d.live_tiles, d.top, d.node4,
-                    d.child, d.wave_acc, d.ichunk};
+                    d.child, d.wave_acc, d.ichunk, d.qnext};
     for (void *p : ptrs) (void)hipFree(p);
     b->stage.release();
     if (b->fork) (void)hipEventDestroy(b->fork);
@@ -264,6 +264,7 @@ gsim_status gsim_batch_create(int32_t device, size_t capacity_particles, uint32_
     GSIM_BALLOC(d.items, b->item_capacity);
     GSIM_BALLOC(d.remaining, max_systems);
     GSIM_BALLOC(d.counts, 1);
+    GSIM_BALLOC(d.qnext, gsim::kForceQueues * gsim::kQueueStride);
     GSIM_BALLOC(d.stats, max_systems);
     GSIM_BALLOC(d.status, 2 * 2 * 256 * b->tiles_cap);
     GSIM_BALLOC(d.digit_total, (size_t)max_systems * gsim::kBatchPasses * 256);
@@ -284,6 +285,8 @@ gsim_status gsim_batch_create(int32_t device, size_t capacity_particles, uint32_
     GSIM_BALLOC(d.ichunk, b->item_capacity);
 #undef GSIM_BALLOC
     if (e == hipSuccess) e = hipMemset(d.counts, 0, sizeof(gsim::BatchCounts));
+    if (e == hipSuccess)
+        e = hipMemset(d.qnext, 0, sizeof(uint32_t) * gsim::kForceQueues * gsim::kQueueStride);
     if (e == hipSuccess)
         e = hipMemset(d.digit_total, 0, sizeof(uint32_t) * max_systems * gsim::kBatchPasses * 256);
     if (e == hipSuccess) e = hipMemset(d.wave_acc, 0, sizeof(unsigned long long) * 2 * gsim::kMaxForceWaves);

@@ -44,6 +44,7 @@ constexpr uint32_t kBatchDsBlocks = 256;
 // (item i to queue i mod kForceQueues); the waves of queue q take its items
 // one at a time from a counter, so a wave that drew light items takes more.
 constexpr uint32_t kForceQueues = 64;
+constexpr uint32_t kQueueStride = 32;  // words between their counters: a cache line each
 
 struct BatchCounts {
     uint32_t n_bh;            // Barnes-Hut systems (ranks)
@@ -55,7 +56,6 @@ struct BatchCounts {
     uint32_t n_sys;           // all systems (direct sum and Barnes-Hut)
     uint32_t sort_stall;      // radix look-back waits that hit their bound (never expected)
     uint32_t n_live[kLiveLists];  // (system, depth-5 tile) pairs holding leaves, per list
-    uint32_t qnext[kForceQueues];  // force launch: items taken from each queue (zeroed each step)
     unsigned long long accepts;  // Barnes-Hut real-lane acceptances, all steps
     unsigned long long visits;   // Barnes-Hut real-lane node visits, all steps
 };
@@ -106,6 +106,7 @@ struct BatchDevice {
     uint2 *items = nullptr;
     uint32_t *remaining = nullptr;  // steps each system may still take (kUnlimitedSteps = no limit)
     BatchCounts *counts = nullptr;
+    uint32_t *qnext = nullptr;  // [kForceQueues * kQueueStride] items drawn from each queue (zeroed each step)
     RankStats *stats = nullptr;
     // Barnes-Hut scratch over all sorted positions
     uint32_t *keys[2] = {}, *idx[2] = {};
