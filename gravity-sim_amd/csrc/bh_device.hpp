@@ -647,48 +647,29 @@ __device__ __forceinline__ T tree_record(const T *__restrict__ base, uint32_t sl
                  : *reinterpret_cast<const T *>(reinterpret_cast<const char *>(base) + slot * 16u);
 }
 
-// Four sources for each stream from a block of 32 list entries: stream s
-// takes entries 4s .. 4s + 3.
-struct SourceBlock {
-    f3v q[4];
-};
-
-template <bool kWide>
-__device__ __forceinline__ SourceBlock load_block(const WalkShared &sh, uint32_t block,
-                                                  uint32_t stream,
-                                                  const float4 *__restrict__ node4) {
-    const uint4 i = sh.list4[block * 8 + stream];
-    SourceBlock b;
-    b.q[0] = load_source<kWide>(node4, i.x);
-    b.q[1] = load_source<kWide>(node4, i.y);
-    b.q[2] = load_source<kWide>(node4, i.z);
-    b.q[3] = load_source<kWide>(node4, i.w);
-    return b;
-}
-
-template <int R>
-__device__ __forceinline__ void add_block(const SourceBlock &b, const float (&tx)[R],
-                                          const float (&ty)[R], float eps2, float (&ax)[R],
-                                          float (&ay)[R]) {
-#pragma unroll
-    for (int j = 0; j < 4; ++j) add_source<R>(b.q[j], tx, ty, eps2, ax, ay);
-}
-
-// The whole blocks of 32 of the first `count` list entries, each block's
-// loads in flight while the block before is summed.
+// The whole blocks of 32 of the first list entries: stream s takes entries
+// 4s .. 4s + 3 of each.  Two sources a stream are loaded while the two before
+// are summed; four at a time held 24 registers instead of 12 and made 500,000
+// particles (galaxy, W = 64) 245 us a walk, not 236.
 template <int R, bool kWide>
 __device__ __forceinline__ void sum_blocks(const WalkShared &sh, uint32_t blocks, uint32_t stream,
                                            const float4 *__restrict__ node4, const float (&tx)[R],
                                            const float (&ty)[R], float eps2, float (&ax)[R],
                                            float (&ay)[R]) {
     if (!blocks) return;
-    SourceBlock a = load_block<kWide>(sh, 0, stream, node4);
-    for (uint32_t b = 0; b < blocks; b += 2) {
-        const SourceBlock c = load_block<kWide>(sh, min(b + 1, blocks - 1), stream, node4);
-        add_block<R>(a, tx, ty, eps2, ax, ay);
-        if (b + 1 == blocks) break;
-        a = load_block<kWide>(sh, min(b + 2, blocks - 1), stream, node4);
-        add_block<R>(c, tx, ty, eps2, ax, ay);
+    const uint2 *const pairs = reinterpret_cast<const uint2 *>(sh.list4) + 2 * stream;
+    uint2 k = pairs[0];
+    f3v a0 = load_source<kWide>(node4, k.x), a1 = load_source<kWide>(node4, k.y);
+    for (uint32_t b = 0; b < blocks; ++b) {
+        k = pairs[16 * b + 1];
+        const f3v c0 = load_source<kWide>(node4, k.x), c1 = load_source<kWide>(node4, k.y);
+        add_source<R>(a0, tx, ty, eps2, ax, ay);
+        add_source<R>(a1, tx, ty, eps2, ax, ay);
+        k = pairs[16 * min(b + 1, blocks - 1)];
+        a0 = load_source<kWide>(node4, k.x);
+        a1 = load_source<kWide>(node4, k.y);
+        add_source<R>(c0, tx, ty, eps2, ax, ay);
+        add_source<R>(c1, tx, ty, eps2, ax, ay);
     }
 }
 
