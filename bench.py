@@ -41,9 +41,9 @@ VALU_LANE_OPS = 256 * 64 * 2.4e9  # one FP32 op per lane per clock, lane-ops/s
 DS_FLOP_PER_PAIR = 14             # 2 sub, 2 FMA, rsqrt, 3 mul, 2 FMA (one-sided interaction)
 DS_LANEOPS_PER_PAIR = 10
 # symmetric kernel: per unordered pair 12 VALU + 1 rsq, plus 5 DPP rotates per
-# 16 pairs (counted in its ISA); B(B+1)/2 block pairs of 64 x 64 (diagonal
-# blocks one-sided)
-DS_SYM_ISSUED_PER_PAIR = 13.3125
+# 8 pairs (8 row blocks a wave at this size); B(B+1)/2 block pairs of 64 x 64
+# (diagonal blocks one-sided)
+DS_SYM_ISSUED_PER_PAIR = 13.625
 # HBM bytes per ds_sym_kernel launch at 50,048 particles: rocprofv3 FETCH_SIZE
 # x 2 + WRITE_SIZE x 1 (factors from a 256 MiB copy), 2 x 2,417 + 48,950 KiB;
 # profiles/ds50k_bh500k_counters.md
@@ -202,7 +202,7 @@ def bench_barnes_hut(steps: int, warmup: int, leaf_bits: int = 10, box: bool = F
                    "adaptive_box": box},
         "roofline": {
             "bound": "valu",
-            "kernel": f"bh_traverse{width}_kernel",
+            "kernel": "bh_walk_kernel",
             "achieved": achieved,
             "peak": PEAK_FP32_TFLOPS,
             "unit": "TFLOP/s",
@@ -285,7 +285,7 @@ def bench_batched(steps: int, serial_steps: int = 20) -> dict:
                    "one_by_one_steps": serial_steps,
                    "autotuned": dict(picks, seconds=tune_s,
                                      method="coordinate descent over waves per SIMD, sort "
-                                            "tile, run queue, priority step and carry; each "
+                                            "tile, priority step and carry; each "
                                             "candidate 2 x 5 steps from a restored snapshot")},
     }
 
