@@ -103,6 +103,7 @@ gsim_status upload_membership(gsim_batch *b) {
     std::vector<uint32_t> bh_sys, bh_prefix{0};
     std::vector<uint2> items, bh_items;
     std::vector<uint32_t> remaining;
+    uint64_t ds_pairs = 0;
     GSIM_HIP(hipStreamSynchronize(b->stream));  // step counts below are exact from here
     for (auto &kv : b->systems) {
         gsim::BatchSystem &s = kv.second;
@@ -138,6 +139,7 @@ gsim_status upload_membership(gsim_batch *b) {
             d.w = s.params.group_width;
             for (uint32_t g = 0; g < s.na / d.w; ++g) bh_items.push_back(make_uint2(di, g));
         } else {
+            ds_pairs += (uint64_t)s.na * s.na;
             for (uint32_t tb = 0; tb < s.na / gsim::kDsBlockTargets; ++tb)
                 items.push_back(make_uint2(di, tb));
         }
@@ -152,6 +154,8 @@ gsim_status upload_membership(gsim_batch *b) {
     c.n_bh_particles = bh_prefix.back();
     c.n_items = (uint32_t)items.size();
     c.n_ds = c.n_items - (uint32_t)bh_items.size();
+    c.ds_groups = ds_pairs > gsim::kBatchDsPairs * c.n_bh_particles ? gsim::kBatchDsBlocks
+                                                                   : gsim::kBatchDsBeside;
     // the acceptance and visit totals carry over
     GSIM_HIP(hipMemcpy(&c.accepts, &b->d.counts->accepts, sizeof(c.accepts), hipMemcpyDeviceToHost));
     GSIM_HIP(hipMemcpy(&c.visits, &b->d.counts->visits, sizeof(c.visits), hipMemcpyDeviceToHost));

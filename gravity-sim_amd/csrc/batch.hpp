@@ -35,10 +35,16 @@ struct RankStats {
 // one counter for all of them serialises thousands of same-address atomics.
 constexpr uint32_t kLiveLists = 64;
 
-// Workgroups of the direct-sum launch: one to a CU, so that the build beside it
-// finds room (128: 328 us a step of the mix above bb_ds_kernel, 192: 314, 256:
-// 311, 512: 330, 2,048: 318; on the build's own stream, 512: 337).
-constexpr uint32_t kBatchDsBlocks = 256;
+// Workgroups of the direct-sum launch, and how many of them take blocks: one to
+// a CU, so that the build beside it finds room, where the direct sums are a
+// small part of the step; all, several to a CU, where they outlast the build.
+// Us a step beside / all, by direct-sum pairs per Barnes-Hut particle: 417 392 /
+// 427, 450 236 / 255, 1,875 168 / 182, 2,000 447 / 439, 5,400 492 / 434, 27,000
+// 472 / 406, no Barnes-Hut system 832 / 697.  256 beside: 128 +5%, 192 +1%, 512
+// +6% at the mix above bb_ds_kernel.
+constexpr uint32_t kBatchDsBlocks = 1024;
+constexpr uint32_t kBatchDsBeside = 256;
+constexpr uint64_t kBatchDsPairs = 1900;
 
 // The walk launch's work list is dealt to kForceQueues interleaved queues
 // (item i to queue i mod kForceQueues); the waves of queue q take its items
@@ -51,6 +57,8 @@ struct BatchCounts {
     uint32_t n_bh_particles;  // sum of their padded counts = sorted positions
     uint32_t n_items;         // work items, direct-sum blocks first
     uint32_t n_ds;            // direct-sum blocks
+    uint32_t ds_groups;       // workgroups that take them (<= kBatchDsBlocks)
+    uint32_t pad;
     uint32_t n_cells;         // cell nodes of all trees (emit)
     uint32_t n_leaves;        // occupied leaves of all trees (emit)
     uint32_t n_sys;           // all systems (direct sum and Barnes-Hut)

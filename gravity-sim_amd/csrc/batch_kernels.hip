@@ -462,10 +462,10 @@ __device__ void bb_walk_group(uint32_t g, const SysDesc &d, const RankStats &st,
 // The direct-sum systems' blocks of 16 targets (items [0, n_ds)), a workgroup a
 // block: ds_block_kernel's additions in its order.  The blocks of one system
 // follow each other, so that stepping by the grid spreads each system over all
-// workgroups.  Bound by the VALU (2.7e12 pairs a second).  One wave a block,
-// role after role, inside the walks' launch took the time of the largest
-// system's blocks: 25 systems of 1,030 to 6,128 particles alone 203 -> 136 us a
-// step (the empty build's launches are 50 of each); with 23 Barnes-Hut systems
+// workgroups.  Bound by the VALU (alone 3.3e12 pairs a second).  One wave a
+// block, role after role, inside the walks' launch took the time of the largest
+// system's blocks: 25 systems of 1,030 to 6,128 particles alone 203 -> 123 us a
+// step (the empty build's launches are 50 of each), with 23 Barnes-Hut systems
 // 345 -> 311.
 __global__ __launch_bounds__(64 * kDsRoles, 8) void bb_ds_kernel(
     const uint2 *__restrict__ items, const SysDesc *__restrict__ desc,
@@ -473,8 +473,9 @@ __global__ __launch_bounds__(64 * kDsRoles, 8) void bb_ds_kernel(
     const float2 *__restrict__ pos, const float2 *__restrict__ vel,
     const float *__restrict__ mass, float2 *__restrict__ pos_out, float2 *__restrict__ vel_out) {
     __shared__ float2 sum[kDsRoles][kDsBlockTargets];
-    const uint32_t n = counts->n_ds;
-    for (uint32_t it = blockIdx.x; it < n; it += gridDim.x) {
+    const uint32_t n = counts->n_ds, stride = counts->ds_groups;
+    if (blockIdx.x >= stride) return;
+    for (uint32_t it = blockIdx.x; it < n; it += stride) {
         const uint2 item = items[it];
         const SysDesc d = desc[item.x];
         const bool live = remaining[item.x] != 0u;

@@ -111,3 +111,26 @@ def test_tree_on_both_sides_of_a_change_of_radix_tile(n, bits, boxed):
     print(f"radix tile n={n} bits={bits}", flush=True)
     p = gsim.generate("galaxy-collision", n, 130.0, 1.0, 10.0, seed=n)
     _same_tree(p.pos, p.mass, bits, 2, boxed)
+
+
+@pytest.mark.parametrize("bh", [0, 64, 16000])
+def test_batch_direct_sums_beside_and_without_a_build(bh):
+    """The direct-sum launch with all its workgroups taking blocks (no or few
+    Barnes-Hut particles) and with one a CU; a system whose budget is spent
+    holds its state.  Same bits as alone."""
+    print(f"batch direct sums bh={bh}", flush=True)
+    batch = gsim.Batch(400000, 32)
+    alone, ids = [], []
+    for k, n in enumerate([64, 1000, 16 * 257, 6128] + ([bh] if bh else [])):
+        p = gsim.generate("random", n, 60.0, 1.0, 10.0, seed=k)
+        algo = "barnes-hut" if bh and k == 4 else "direct-sum"
+        alone.append(gsim.Simulation(p, algo))
+        ids.append(batch.add(p, algo))
+    batch.set_steps(ids[0], 2)
+    batch.step(3)
+    for k, (a, i) in enumerate(zip(alone, ids)):
+        a.step(2 if k == 0 else 3)
+        x, y = a.read(), batch.read(i)
+        assert np.array_equal(x.pos, y.pos) and np.array_equal(x.vel, y.vel)
+        a.close()
+    batch.close()
