@@ -45,15 +45,14 @@ DS_LANEOPS_PER_PAIR = 10
 # (diagonal blocks one-sided)
 DS_SYM_ISSUED_PER_PAIR = 13.625
 # HBM bytes per ds_sym_kernel launch at 50,048 particles: rocprofv3 FETCH_SIZE
-# x 2 + WRITE_SIZE x 1 (factors from a 256 MiB copy), 2 x 2,417 + 48,950 KiB;
+# x 2 + WRITE_SIZE x 1 (factors from a 256 MiB copy), 2 x 2,384 + 58,110 KiB;
 # profiles/ds50k_bh500k_counters.md
-DS_TRAFFIC_BYTES = (2 * 2417 + 48950) * 1024
-# HBM bytes per traversal launch at 500,032 particles (same counters, median
-# over the steady steps, state in sorted order), by group width:
-# bh_traverse64_kernel (one wave per group, staged runs) 2 x 44,890 + 25,530
-# KiB; bh_traverse32_kernel (one 32-particle group per wave) 2 x 44,310 +
-# 25,060 KiB
-BH_TRAFFIC_BYTES = {64: (2 * 44890 + 25530) * 1024, 32: (2 * 44310 + 25060) * 1024}
+DS_TRAFFIC_BYTES = (2 * 2384 + 58110) * 1024
+# HBM bytes per walk launch at 500,032 particles (same counters, median over
+# the steady steps, state in sorted order), by group width: bh_walk_kernel with
+# one wave per group, 2 x 45,590 + 25,260 KiB at W = 64, 2 x 48,760 + 25,180 at
+# W = 32
+BH_TRAFFIC_BYTES = {64: (2 * 45590 + 25260) * 1024, 32: (2 * 48760 + 25180) * 1024}
 BH_FLOP_VISIT, BH_FLOP_ACCEPT = 7, 8     # 2 sub + 2 FMA + theta-mul; rsqrt + 3 mul + 2 FMA
 BH_LANEOPS_VISIT, BH_LANEOPS_ACCEPT = 6, 6
 REF_DS_MS_50K = 3.602             # reference README.md:18 (RTX 3070), ms/step at 50,000
