@@ -208,7 +208,8 @@ typedef enum gsim_tuning {
                                          visits), 2 auto (the default): every 1,024
                                          steps, four steps alternate the two and the
                                          faster is kept (decided once the host sees
-                                         them complete; never waited for)              */
+                                         them complete; never waited for; heaviest
+                                         first until then)                             */
 } gsim_tuning;
 gsim_status gsim_set_tuning(gsim_sim *sim, int32_t knob, uint32_t value);
 
@@ -238,10 +239,11 @@ gsim_status gsim_ds_step_noalloc(const gsim_params *params, const float *pos_xy,
 /* ---- batched form: many independent systems stepped together ---------------
  * A batch is one device arena holding many systems of uneven size (direct sum
  * or Barnes-Hut, each with its own parameters).  Every stage of a step runs
- * as one launch over all systems (Barnes-Hut systems share one radix sort and
- * one node array; one persistent launch computes every system's forces), and
- * the whole step is replayed from a captured hipGraph.  Membership can change
- * between steps without re-capturing.  A system's results are bit-identical
+ * as one launch over all systems (Barnes-Hut systems share one node array; the
+ * direct sums run beside their build), and the whole step is replayed from a
+ * captured hipGraph.  Membership can change between steps; the graph is
+ * captured again only when the members outgrow twice what they were, or the
+ * first direct-sum system joins.  A system's results are bit-identical
  * to stepping it alone with gsim_step (the same group width, 32 or 64, and
  * the default launch shape).
  * Direct-sum systems of 16,384 or more padded particles are refused: they
