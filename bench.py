@@ -61,7 +61,7 @@ REF_BH_MS_500K = 2.853            # reference README.md:19, ms/step at 500,000
 DS_N = WL.DS_N
 BH_N = WL.BH_N
 ERR_SAMPLE = 2048                 # targets of the FP64 error sample
-CPU_THREADS_MAX = 16              # the GPU box's host share for one GPU
+CPU_THREADS_MAX = 16              # the host threads that go with one GPU
 
 
 def log(msg: str) -> None:
@@ -551,8 +551,8 @@ def main() -> int:
         copy_calibration()
         return 0
     if args.gpus != 1 or int(os.environ.get("WORLD_SIZE", "1")) != 1:
-        print("bench.py measures one GPU only: every GPU box of this build has one GPU and "
-              "the simulation step has no multi-GPU path; run with --gpus 1.", file=sys.stderr)
+        print("bench.py measures one GPU only: the simulation step has no multi-GPU path; "
+              "run with --gpus 1.", file=sys.stderr)
         return 2
     log(f"direct-sum 50k: warmup {args.warmup}, steps {args.steps}")
     ds = bench_direct_sum(args.steps, args.warmup)
