@@ -82,13 +82,11 @@ constexpr int kBatchSortTileMin = 8 * kSortThreads;
 constexpr uint32_t kBatchPasses = 3;
 
 // Launch parameters of a batched step that never change results (the
-// autotuner's knobs): persistent force-launch width, radix tile size, leaf
-// runs a wave queues before summing them (its LDS run stack), and the walk's
-// issue-priority step and carry divisor (0: off).
+// autotuner's knobs): persistent walk-launch width, radix tile size and the
+// walk's issue-priority step and carry divisor (0: off).
 struct BatchTune {
-    // 6 of the force kernel's 7 resident waves per SIMD: on the 256-system
-    // mix 2.36 ms per step against 2.91 with 7 and 2.78 with 8 (a second
-    // round of waves)
+    // waves of the walk launch (four a SIMD are resident at once): 48 systems
+    // of 1,030 to 63,279 particles 360 us a step with 4, 344 with 6, 346 with 8
     uint32_t waves_per_simd = 6;
     uint32_t sort_rounds = kBatchSortRoundsDefault;
     uint32_t run_queue = 64;   // <= kRunQueue (kept for the interface: the walk has no run queue)

@@ -2,9 +2,9 @@
 // reads its sizes from device memory (BatchCounts), so a step captured once
 // in a hipGraph serves any membership that fits the arena.
 //
-// Barnes-Hut systems share one stable radix sort on (rank << 21 | cell):
-// sorted positions group by system, and because node slots are
-// position + scanned cell-node count, each system's pre-order tree lands
+// Barnes-Hut systems are sorted each by itself, by cell, at consecutive sorted
+// positions (keys rank << 21 | cell), and because node slots are position +
+// scanned cell-node count, each system's pre-order tree lands
 // contiguously in one global node array ([root, end_slot) per rank, recorded
 // by the emit kernel).  The per-system semantics are those of the
 // single-system kernels in bh_kernels.hip (same cells, same canonical order,

@@ -9,8 +9,10 @@
 //   1. keys      20-bit Morton cell per particle (InitShader.comp:80-98); the
 //                out-of-domain kill of InitShader.comp:110-117.
 //   2. sort      stable LSD radix sort of (cell, index), 3 passes of 8 bits,
-//                so a leaf's particles are in ascending index order: one
-//                histogram launch, then one launch per pass (look-back).
+//                so a leaf's particles are in ascending index order: the
+//                keys kernel counts the digits, then one launch per pass
+//                (look-back).  Up to kSmallBuild particles steps 1 to 4 are
+//                one launch of one workgroup.
 //   3. prep      s(k) = depth shared by sorted keys k-1 and k; the cell nodes
 //                that start at k are the depths in (s(k), s(k+1)], so an
 //                exclusive scan C(k) of their number gives every pre-order
@@ -36,9 +38,6 @@
 
 namespace gsim {
 namespace {
-
-
-// ---- 1. keys ----------------------------------------------------------------
 
 // ---- 0. adaptive bounding box (opt-in; beyond the reference) -------------------
 // Extremes of the finite positions: per-block partials, reduced by every
@@ -112,6 +111,8 @@ __device__ __forceinline__ float4 box_of_group(float x0, float x1, float y0, flo
     }
     return box_of(r.x, r.y, r.z, r.w);
 }
+
+// ---- 1. keys ----------------------------------------------------------------
 
 // kDeep: 30-bit keys of the 32768^2 grid (15-bit leaves) instead of 20-bit cells.
 // One block of kR x kSortThreads particles (kR per thread) per workgroup.
