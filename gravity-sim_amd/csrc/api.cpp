@@ -115,31 +115,48 @@ gsim_status drain_timing(gsim_sim *s) {
 }
 
 // Grows the partial-sum buffer to hold `entries` float2 (the caller has
-// synchronised the stream).
+// synchronised the stream).  On failure the handle keeps a buffer of the size
+// it had, unless not even that can be had again once it was given up.
 gsim_status ds_reserve_partial(gsim_sim *s, size_t entries) {
     if (entries <= s->partial_cap) return GSIM_OK;
-    (void)hipFree(s->partial);
-    s->partial = nullptr;
-    s->partial_cap = 0;
-    hipError_t e = hipMalloc((void **)&s->partial, sizeof(float2) * entries);
+    float2 *fresh = nullptr;
+    hipError_t e = hipMalloc((void **)&fresh, sizeof(float2) * entries);
+    if (e != hipSuccess && s->partial) {  // both at once may be too much
+        (void)hipGetLastError();
+        (void)hipFree(s->partial);
+        s->partial = nullptr;
+        e = hipMalloc((void **)&fresh, sizeof(float2) * entries);
+        if (e != hipSuccess) {
+            (void)hipGetLastError();
+            if (hipMalloc((void **)&s->partial, sizeof(float2) * s->partial_cap) != hipSuccess) {
+                (void)hipGetLastError();
+                s->partial = nullptr;
+                s->partial_cap = 0;
+            }
+        }
+    }
     if (e != hipSuccess)
         return fail(GSIM_ERROR_OUT_OF_MEMORY, "direct-sum partial sums (%zu bytes): %s",
                     sizeof(float2) * entries, hipGetErrorString(e));
+    (void)hipFree(s->partial);
+    s->partial = fresh;
     s->partial_cap = entries;
     return GSIM_OK;
 }
 
-// Selects the symmetric or a one-sided form (blocks or slices) and sizes its
-// partial sums.
-gsim_status ds_configure(gsim_sim *s, bool sym, bool block) {
-    s->ds_sym = sym ? 1u : 0u;
-    s->ds_block = !sym && block;
-    if (s->ds_block) return GSIM_OK;
-    if (sym) {
-        s->ds_plan = gsim::ds_sym_plan(s->na, s->ds_sym_cols);
-        return ds_reserve_partial(s, s->ds_plan.ipart + s->ds_plan.jpart);
-    }
-    return ds_reserve_partial(s, s->na * s->ds_S);
+// Partial sums that a direct-sum form writes in one step.
+size_t ds_entries(const gsim_sim *s, const gsim::DsForm &f) {
+    if (f.sym) return f.plan.ipart + f.plan.jpart;
+    return f.block ? 0 : s->na * f.S;
+}
+
+// Gives the handle a direct-sum form (symmetric, blocks or slices) and sizes
+// its partial sums; a form whose sums cannot be had leaves the last one.
+gsim_status ds_configure(gsim_sim *s, gsim::DsForm f) {
+    if (f.sym) f.plan = gsim::ds_sym_plan(s->na, f.sym_cols);
+    const gsim_status st = ds_reserve_partial(s, ds_entries(s, f));
+    if (st == GSIM_OK) s->ds = f;
+    return st;
 }
 
 // GSIM_TUNE_BH_ORDER = 2: whether this step's walk is a trial walk (and with
@@ -226,13 +243,15 @@ gsim_status run_steps(gsim_sim *s, uint32_t count) {
             std::swap(s->mass, s->mass_next);
             s->has_tree = true;
         } else {
-            if (s->ds_block)
+            if (ds_entries(s, s->ds) > s->partial_cap)  // lost to a form that did not fit
+                return fail(GSIM_ERROR_OUT_OF_MEMORY, "the handle has no direct-sum partial sums");
+            if (s->ds.one_launch())
                 GSIM_HIP(gsim::ds_launch_block(s, s->pos[in], s->vel[in], s->mass, s->pos[out],
                                                s->vel[out]));
             else
                 GSIM_HIP(gsim::ds_launch_partial(s, s->pos[in], s->mass));
             if (s->timing) GSIM_HIP(hipEventRecord(ev[1], s->stream));
-            if (!s->ds_block)
+            if (!s->ds.one_launch())
                 GSIM_HIP(gsim::ds_launch_combine(s, s->pos[in], s->vel[in], s->pos[out],
                                                  s->vel[out]));
         }
@@ -377,13 +396,16 @@ gsim_status gsim_create(const gsim_params *params, const float *pos_xy, const fl
     if (e != hipSuccess) return bail(hip_fail(e, "upload"));
 
     if (params->algorithm == GSIM_DIRECT_SUM) {
-        gsim::ds_pick_shape(na, &s->ds_R, &s->ds_S);
-        const bool sym = gsim::ds_sym_default(na), block = gsim::ds_block_default(na);
-        gsim_status st = ds_configure(s, sym, block);
-        if (st == GSIM_ERROR_OUT_OF_MEMORY && sym) {  // the slices need far less
+        gsim::DsForm f;
+        gsim::ds_pick_shape(na, &f.R, &f.S);
+        f.sym = gsim::ds_sym_default(na);
+        f.block = gsim::ds_block_default(na);
+        gsim_status st = ds_configure(s, f);
+        if (st == GSIM_ERROR_OUT_OF_MEMORY && f.sym) {  // the slices need far less
             (void)hipGetLastError();
             gsim::clear_error();
-            st = ds_configure(s, false, block);
+            f.sym = false;
+            st = ds_configure(s, f);
         }
         if (st != GSIM_OK) return bail(st);
     } else {
@@ -479,10 +501,12 @@ gsim_status gsim_set_ds_shape(gsim_sim *s, uint32_t R, uint32_t S) {
         return fail(GSIM_ERROR_INVALID_ARGUMENT, "slices must be <= 256 and <= Na/64");
     GSIM_HIP(hipSetDevice(s->device));
     GSIM_HIP(hipStreamSynchronize(s->stream));
-    s->ds_R = R;
-    s->ds_S = S;
-    s->ds_shaped = !block;
-    return ds_configure(s, false, block);
+    gsim::DsForm f = s->ds;
+    f.R = R;
+    f.S = S;
+    f.sym = false;
+    f.block = block;
+    return ds_configure(s, f);
 }
 
 gsim_status gsim_set_tuning(gsim_sim *s, int32_t knob, uint32_t value) {
@@ -562,12 +586,10 @@ gsim_status gsim_set_tuning(gsim_sim *s, int32_t knob, uint32_t value) {
                 return fail(GSIM_ERROR_INVALID_ARGUMENT, "column blocks per wave must be 0, 1 or 2");
             GSIM_HIP(hipSetDevice(s->device));
             GSIM_HIP(hipStreamSynchronize(s->stream));
-            bool sym = s->ds_sym != 0;
-            if (knob == GSIM_TUNE_DS_SYMMETRIC) sym = value != 0;
-            else s->ds_sym_cols = value;
-            // a handle given a shape keeps its slices
-            return ds_configure(s, sym, s->ds_shaped ? s->ds_block
-                                                     : gsim::ds_block_default(s->na));
+            gsim::DsForm f = s->ds;  // one-sided, it is what it was
+            if (knob == GSIM_TUNE_DS_SYMMETRIC) f.sym = value != 0;
+            else f.sym_cols = value;
+            return ds_configure(s, f);
         }
         default:
             return fail(GSIM_ERROR_INVALID_ARGUMENT, "unknown tuning knob %d", knob);

@@ -382,14 +382,14 @@ hipError_t ds_launch_block(gsim_sim *s, const float2 *pos, const float2 *vel, co
 
 hipError_t ds_launch_partial(gsim_sim *s, const float2 *pos, const float *mass) {
     const uint32_t na = (uint32_t)s->na;
-    if (s->ds_sym) {
-        const DsSymPlan &p = s->ds_plan;
+    if (s->ds.sym) {
+        const DsSymPlan &p = s->ds.plan;
         auto *k = p.rows == 4 ? ds_sym_kernel<4> : p.rows == 8 ? ds_sym_kernel<8> : ds_sym_kernel<16>;
         k<<<p.ntiles, 256, 0, s->stream>>>(pos, mass, s->partial, s->partial + p.ipart, p.B, p.G,
                                            p.cols, s->eps2);
         return hipGetLastError();
     }
-    const uint32_t R = s->ds_R, S = s->ds_S;
+    const uint32_t R = s->ds.R, S = s->ds.S;
     // slice length: multiple of 64 covering na in S pieces
     uint32_t jlen = (uint32_t)(((na + S - 1) / S + 63) / 64 * 64);
     const uint32_t slices = (na + jlen - 1) / jlen;
@@ -412,8 +412,8 @@ hipError_t ds_launch_combine(gsim_sim *s, const float2 *pos, const float2 *vel,
                              float2 *pos_out, float2 *vel_out) {
     const uint32_t na = (uint32_t)s->na;
     float2 *acc = (s->debug_flags & GSIM_DEBUG_ACCEL) ? s->accel : nullptr;
-    if (s->ds_sym) {
-        const DsSymPlan &p = s->ds_plan;
+    if (s->ds.sym) {
+        const DsSymPlan &p = s->ds.plan;
         ds_sym_combine_kernel<<<p.B, 256, 0, s->stream>>>(s->partial, s->partial + p.ipart, p.B,
                                                           p.rows, p.width, pos, vel, pos_out, vel_out, acc,
                                                           s->kv, s->dt);

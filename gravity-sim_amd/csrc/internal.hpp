@@ -181,6 +181,16 @@ struct DsSymPlan {
     size_t ipart = 0, jpart = 0;  // float2 entries of the two partial arrays
 };
 
+// A handle's direct-sum form.
+struct DsForm {
+    bool sym = false;       // the symmetric kernel, else one-sided:
+    bool block = false;     // the block kernel (one launch a step) or slices
+    uint32_t R = 1, S = 1;  // slices: targets per lane, slices
+    uint32_t sym_cols = 0;  // symmetric: column blocks per wave (0: by size)
+    DsSymPlan plan{};
+    bool one_launch() const { return !sym && block; }
+};
+
 // First tile of row group g: sum over h < g of ceil((B - R h) / width)
 // = g * cb - step * g (g - 1) / 2 with cb = ceil(B / width), step = rows / width.
 __host__ __device__ inline size_t ds_sym_tile_base(uint32_t g, uint32_t cb, uint32_t step) {
@@ -251,11 +261,8 @@ struct gsim_sim {
     // direct sum
     float2 *partial = nullptr;
     size_t partial_cap = 0;            // float2 entries allocated
-    uint32_t ds_R = 1, ds_S = 1, ds_S_used = 1;
-    bool ds_block = false;                 // the block kernel (one launch) instead of slices
-    bool ds_shaped = false;                // gsim_set_ds_shape chose slices
-    uint32_t ds_sym = 0, ds_sym_cols = 0;  // symmetric kernel; column blocks per tile (0 auto)
-    gsim::DsSymPlan ds_plan{};
+    gsim::DsForm ds;
+    uint32_t ds_S_used = 1;
     // Barnes-Hut
     gsim::BhBuffers bh;
     gsim::ReadStage stage;

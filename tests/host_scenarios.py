@@ -1,0 +1,87 @@
+"""What libgsim's host code does when something fails: each scenario runs in a
+process of its own against the HIP runtime of native/fake_hip.cpp, where device
+memory is host memory and kernels only leave their names.
+
+    python host_scenarios.py <fake_hip.so> <scenario>
+"""
+import ctypes as C
+import os
+import sys
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+sys.path.insert(0, os.path.join(ROOT, "gravity-sim_amd", "python"))
+
+fake = None  # the runtime
+gsim = None
+
+OUT_OF_MEMORY = 2
+
+
+def _load(path):
+    global fake, gsim
+    fake = C.CDLL(path, mode=C.RTLD_GLOBAL)  # ahead of libgsim.so
+    fake.fake_limit.argtypes = [C.c_size_t]
+    fake.fake_live.restype = C.c_size_t
+    fake.fake_launches.restype = fake.fake_faults.restype = C.c_char_p
+    import gsim as module
+    gsim = module
+
+
+def _launched(call):
+    """The kernels that `call` launches."""
+    fake.fake_forget()
+    call()
+    return fake.fake_launches().decode()
+
+
+def _refused(status, call):
+    try:
+        call()
+    except gsim.GsimError as e:
+        assert e.status == status, e
+        return
+    raise AssertionError("not refused")
+
+
+def failed_form_keeps_the_last():
+    """A direct-sum form whose partial sums do not fit is refused, and the
+    handle goes on in the form it had."""
+    for n, kernel, asks in (
+            # slices, too large for the default symmetric form
+            (600_000, "ds_partial_kernel", lambda s: s.set_tuning(gsim.TUNE_DS_SYMMETRIC, 1)),
+            # symmetric; many slices need more
+            (20_000, "ds_sym_kernel", lambda s: s.set_ds_shape(4, 256)),
+            # blocks, which have no partial sums at all
+            (10_000, "ds_block_kernel", lambda s: s.set_ds_shape(1, 100)),
+            (10_000, "ds_block_kernel", lambda s: s.set_tuning(gsim.TUNE_DS_SYMMETRIC, 1))):
+        with gsim.Simulation(gsim.generate("random", n, 100.0, 1.0, 10.0), "direct-sum") as s:
+            before = _launched(lambda: s.step(1))
+            assert kernel in before, (n, before)
+            fake.fake_limit(fake.fake_live())
+            _refused(OUT_OF_MEMORY, lambda: asks(s))
+            assert _launched(lambda: s.step(1)) == before
+            fake.fake_limit(2 ** 64 - 1)
+            assert _launched(lambda: s.step(1)) == before
+            asks(s)  # and with memory it is granted
+            assert _launched(lambda: s.step(1)) != before
+    with gsim.Simulation(gsim.generate("random", 20_000, 100.0, 1.0, 10.0), "direct-sum") as s:
+        s.set_ds_shape(4, 200)  # 32 MB of partial sums
+        fake.fake_limit(fake.fake_live() + (20 << 20))  # 41 fit, but not beside the 32
+        s.set_ds_shape(4, 256)
+        fake.fake_limit(2 ** 64 - 1)
+        assert "ds_partial_kernel" in _launched(lambda: s.step(1))
+    with gsim.Simulation(gsim.generate("random", 20_000, 100.0, 1.0, 10.0), "direct-sum") as s:
+        s.set_ds_shape(4, 100)
+        fake.fake_limit(0)  # neither the new sums nor the old ones again
+        _refused(OUT_OF_MEMORY, lambda: s.set_ds_shape(4, 256))
+        _refused(OUT_OF_MEMORY, lambda: s.step(1))
+        fake.fake_limit(2 ** 64 - 1)
+        s.set_ds_shape(4, 100)
+        s.step(1)
+
+
+if __name__ == "__main__":
+    _load(sys.argv[1])
+    globals()[sys.argv[2]]()
+    assert not fake.fake_faults(), fake.fake_faults().decode()
+    print("ok")
