@@ -215,6 +215,8 @@ gsim_status run_steps(gsim_sim *s, uint32_t count) {
             GSIM_HIP(hipEventRecord(ev[0], s->stream));
         }
         if (bh) {
+            if (!s->bh.ctr)  // lost to a leaf depth that did not fit
+                return fail(GSIM_ERROR_OUT_OF_MEMORY, "the handle has no Barnes-Hut buffers");
             // the walk's workgroup order is fixed for the whole step; a trial
             // step is timed whole
             const bool trial = order_trial_step(s);
@@ -449,6 +451,21 @@ gsim_status gsim_read(gsim_sim *s, float *pos_xy, float *vel_xy, float *mass_out
         if (mass_out) std::memcpy(mass_out, t.mass, sizeof(float) * s->n);
         return GSIM_OK;
     }
+    if (perm && !s->bh.leaf_sum) {  // no buffers (GSIM_TUNE_BH_LEAF_BITS): order on the host
+        std::vector<uint32_t> order(na);
+        std::vector<float> tmp(2 * (size_t)na);
+        GSIM_HIP(hipStreamSynchronize(s->stream));
+        GSIM_HIP(hipMemcpy(order.data(), perm, sizeof(uint32_t) * na, hipMemcpyDeviceToHost));
+        const float *src[3] = {(const float *)pos, (const float *)vel, mass};
+        float *dst[3] = {pos_xy, vel_xy, mass_out};
+        for (int a = 0; a < 3; ++a) {
+            if (!dst[a]) continue;
+            const size_t w = a < 2 ? 2 : 1;
+            GSIM_HIP(hipMemcpy(tmp.data(), src[a], sizeof(float) * w * na, hipMemcpyDeviceToHost));
+            unpermute(order, tmp.data(), dst[a], w, n);
+        }
+        return GSIM_OK;
+    }
     if (perm) {
         // Barnes-Hut: the caller's order, in buffers that only a build uses
         float2 *const stage = (float2 *)s->bh.leaf_sum;
@@ -547,12 +564,18 @@ gsim_status gsim_set_tuning(gsim_sim *s, int32_t knob, uint32_t value) {
             GSIM_HIP(hipSetDevice(s->device));
             GSIM_HIP(hipStreamSynchronize(s->stream));
             // the node arrays are sized for the depth: reallocate them
+            const uint32_t last = s->bh.bits;
             gsim::bh_free(&s->bh);
             s->has_tree = false;
             const hipError_t e = gsim::bh_alloc(&s->bh, s->na, value);
             if (e != hipSuccess) {
+                (void)hipGetLastError();
                 gsim::bh_free(&s->bh);
-                (void)gsim::bh_alloc(&s->bh, s->na, gsim::kTreeDepth);
+                // without even the last depth's, the state can be read and no step taken
+                if (last && gsim::bh_alloc(&s->bh, s->na, last) != hipSuccess) {
+                    (void)hipGetLastError();
+                    gsim::bh_free(&s->bh);
+                }
                 return fail(GSIM_ERROR_OUT_OF_MEMORY, "Barnes-Hut buffers for %u-bit leaves: %s",
                             value, hipGetErrorString(e));
             }
@@ -635,6 +658,8 @@ gsim_status gsim_debug_dump(gsim_sim *s, int32_t what, void *buf, size_t bytes, 
     }
     if (s->params.algorithm != GSIM_BARNES_HUT)
         return fail(GSIM_ERROR_INVALID_ARGUMENT, "dump %d needs a Barnes-Hut handle", what);
+    if (!s->bh.ctr)
+        return fail(GSIM_ERROR_OUT_OF_MEMORY, "the handle has no Barnes-Hut buffers");
     gsim::BhCounters ctr{};
     GSIM_HIP(hipMemcpy(&ctr, s->bh.ctr, sizeof(ctr), hipMemcpyDeviceToHost));
     if (ctr.sort_stall)

@@ -80,6 +80,27 @@ def failed_form_keeps_the_last():
         s.step(1)
 
 
+def lost_tree_buffers():
+    """A leaf depth that does not fit leaves the last one; without memory for
+    either the state can still be read, and no step is taken."""
+    p = gsim.generate("galaxy", 20_000, 100.0, 1.0, 10.0)  # more than a read stages
+    with gsim.Simulation(p, "barnes-hut") as s:
+        fake.fake_limit(fake.fake_live())
+        _refused(OUT_OF_MEMORY, lambda: s.set_tuning(gsim.TUNE_BH_LEAF_BITS, 15))
+        fake.fake_limit(2 ** 64 - 1)
+        assert "bh_leaf_kernel" in _launched(lambda: s.step(1))
+    with gsim.Simulation(p, "barnes-hut") as s:
+        fake.fake_limit(0)
+        _refused(OUT_OF_MEMORY, lambda: s.set_tuning(gsim.TUNE_BH_LEAF_BITS, 15))
+        q = s.read()
+        assert (q.pos == p.pos).all() and (q.vel == p.vel).all() and (q.mass == p.mass).all()
+        _refused(OUT_OF_MEMORY, lambda: s.step(1))
+        _refused(OUT_OF_MEMORY, lambda: s.dump(gsim.DUMP_CELLS))
+        fake.fake_limit(2 ** 64 - 1)
+        s.set_tuning(gsim.TUNE_BH_LEAF_BITS, 10)
+        assert "bh_walk_kernel" in _launched(lambda: s.step(1))
+
+
 if __name__ == "__main__":
     _load(sys.argv[1])
     globals()[sys.argv[2]]()

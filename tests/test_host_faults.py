@@ -11,7 +11,7 @@ import gsim
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 
-SCENARIOS = ["failed_form_keeps_the_last"]
+SCENARIOS = ["failed_form_keeps_the_last", "lost_tree_buffers"]
 
 
 @pytest.fixture(scope="module")
