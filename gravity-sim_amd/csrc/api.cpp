@@ -560,7 +560,7 @@ gsim_status gsim_set_tuning(gsim_sim *s, int32_t knob, uint32_t value) {
                 return fail(GSIM_ERROR_INVALID_ARGUMENT, "not a Barnes-Hut handle");
             if (value != gsim::kTreeDepth && value != gsim::kDeepBits)
                 return fail(GSIM_ERROR_INVALID_ARGUMENT, "leaf bits must be 10 or 15");
-            if (value == s->bh.bits) return GSIM_OK;
+            if (s->bh.ctr && value == s->bh.bits) return GSIM_OK;
             GSIM_HIP(hipSetDevice(s->device));
             GSIM_HIP(hipStreamSynchronize(s->stream));
             // the node arrays are sized for the depth: reallocate them
@@ -572,7 +572,7 @@ gsim_status gsim_set_tuning(gsim_sim *s, int32_t knob, uint32_t value) {
                 (void)hipGetLastError();
                 gsim::bh_free(&s->bh);
                 // without even the last depth's, the state can be read and no step taken
-                if (last && gsim::bh_alloc(&s->bh, s->na, last) != hipSuccess) {
+                if (gsim::bh_alloc(&s->bh, s->na, last) != hipSuccess) {
                     (void)hipGetLastError();
                     gsim::bh_free(&s->bh);
                 }
