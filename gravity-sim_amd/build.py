@@ -1,6 +1,6 @@
-"""Builds libgsim.so (HIP kernels for gfx950 + the C-ABI host runtime) and the
-gravity-sim command-line tool, in-tree under gravity-sim_amd/lib and
-gravity-sim_amd/bin.
+"""Builds libgsim.so (HIP kernels for gfx950 + the C-ABI host runtime), the
+gravity-sim command-line tool and the tests' access to a handle, in-tree under
+gravity-sim_amd/lib and gravity-sim_amd/bin.
 
 Usage: python gravity-sim_amd/build.py [--jobs N]
 """
@@ -23,6 +23,9 @@ LIBDIR = os.path.join(PKG, "lib")
 BINDIR = os.path.join(PKG, "bin")
 LIBGSIM = os.path.join(LIBDIR, "libgsim.so")
 CLI = os.path.join(BINDIR, "gravity-sim")
+# what the tests reach into a handle with (tests/native/handle_access.cpp)
+ACCESS_SRC = os.path.join(ROOT, "tests", "native", "handle_access.cpp")
+ACCESS = os.path.join(LIBDIR, "libgsim_access.so")
 
 HIPCC = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
 ARCH = "gfx950"
@@ -87,14 +90,22 @@ def build_cli() -> str:
     return CLI
 
 
+def build_access() -> str:
+    if not os.path.exists(ACCESS_SRC):
+        return ""
+    _run([HIPCC, f"--offload-arch={ARCH}", "--cuda-host-only", *COMMON, "-shared", ACCESS_SRC,
+          "-o", ACCESS])
+    return ACCESS
+
+
 def main(argv: list[str] | None = None) -> int:
     ap = argparse.ArgumentParser()
     ap.add_argument("--jobs", type=int, default=4)
     args = ap.parse_args(argv)
     print(build_lib(args.jobs))
-    cli = build_cli()
-    if cli:
-        print(cli)
+    for built in (build_cli(), build_access()):
+        if built:
+            print(built)
     return 0
 
 

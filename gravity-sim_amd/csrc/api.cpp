@@ -159,6 +159,15 @@ gsim_status ds_configure(gsim_sim *s, gsim::DsForm f) {
     return st;
 }
 
+// A sort that gave up has spoilt the state for good.
+gsim_status check_sort(gsim_sim *s, uint32_t stall) {
+    if (stall) s->sort_stall = stall;
+    if (!s->sort_stall) return GSIM_OK;
+    return fail(GSIM_ERROR_DEVICE,
+                "radix sort look-back gave up on %u status words: the state is invalid",
+                s->sort_stall);
+}
+
 // GSIM_TUNE_BH_ORDER = 2: whether this step's walk is a trial walk (and with
 // which order); otherwise the walk keeps the order picked last.
 bool order_trial_step(gsim_sim *s) {
@@ -442,10 +451,14 @@ gsim_status gsim_read(gsim_sim *s, float *pos_xy, float *vel_xy, float *mass_out
     const float2 *pos = s->pos[s->cur], *vel = s->vel[s->cur];
     const float *mass = s->mass;
     const uint32_t *perm = s->perm[s->cur];  // null for a direct sum
+    const uint32_t *sorted = s->bh.ctr ? &s->bh.ctr->sort_stall : nullptr;
+    uint32_t stall = 0;
     if (s->n <= gsim::kReadStageParticles && s->stage.ready()) {
         const gsim::ReadTarget t = s->stage.target(s->n);
-        GSIM_HIP(gsim::read_launch(pos, vel, mass, perm, na, n, t, nullptr, s->stream));
+        GSIM_HIP(gsim::read_launch(pos, vel, mass, perm, na, n, t, sorted, s->stream));
         GSIM_HIP(hipStreamSynchronize(s->stream));
+        const gsim_status st = check_sort(s, sorted ? *t.stall : 0);
+        if (st != GSIM_OK) return st;
         if (pos_xy) std::memcpy(pos_xy, t.pos, sizeof(float2) * s->n);
         if (vel_xy) std::memcpy(vel_xy, t.vel, sizeof(float2) * s->n);
         if (mass_out) std::memcpy(mass_out, t.mass, sizeof(float) * s->n);
@@ -454,6 +467,8 @@ gsim_status gsim_read(gsim_sim *s, float *pos_xy, float *vel_xy, float *mass_out
     if (perm && !s->bh.leaf_sum) {  // no buffers (GSIM_TUNE_BH_LEAF_BITS): order on the host
         std::vector<uint32_t> order(na);
         std::vector<float> tmp(2 * (size_t)na);
+        const gsim_status st = check_sort(s, 0);
+        if (st != GSIM_OK) return st;
         GSIM_HIP(hipStreamSynchronize(s->stream));
         GSIM_HIP(hipMemcpy(order.data(), perm, sizeof(uint32_t) * na, hipMemcpyDeviceToHost));
         const float *src[3] = {(const float *)pos, (const float *)vel, mass};
@@ -475,11 +490,13 @@ gsim_status gsim_read(gsim_sim *s, float *pos_xy, float *vel_xy, float *mass_out
         vel = t.vel;
         mass = t.mass;
     }
+    if (sorted)
+        GSIM_HIP(hipMemcpyAsync(&stall, sorted, sizeof(stall), hipMemcpyDeviceToHost, s->stream));
     if (pos_xy) GSIM_HIP(hipMemcpyAsync(pos_xy, pos, sizeof(float2) * s->n, hipMemcpyDeviceToHost, s->stream));
     if (vel_xy) GSIM_HIP(hipMemcpyAsync(vel_xy, vel, sizeof(float2) * s->n, hipMemcpyDeviceToHost, s->stream));
     if (mass_out) GSIM_HIP(hipMemcpyAsync(mass_out, mass, sizeof(float) * s->n, hipMemcpyDeviceToHost, s->stream));
     GSIM_HIP(hipStreamSynchronize(s->stream));
-    return GSIM_OK;
+    return check_sort(s, stall);
 }
 
 gsim_status gsim_destroy(gsim_sim *s) {
@@ -565,6 +582,12 @@ gsim_status gsim_set_tuning(gsim_sim *s, int32_t knob, uint32_t value) {
             GSIM_HIP(hipStreamSynchronize(s->stream));
             // the node arrays are sized for the depth: reallocate them
             const uint32_t last = s->bh.bits;
+            if (s->bh.ctr) {  // the count goes with the buffers
+                uint32_t stall = 0;
+                GSIM_HIP(hipMemcpy(&stall, &s->bh.ctr->sort_stall, sizeof(stall), hipMemcpyDeviceToHost));
+                (void)check_sort(s, stall);
+                gsim::clear_error();
+            }
             gsim::bh_free(&s->bh);
             s->has_tree = false;
             const hipError_t e = gsim::bh_alloc(&s->bh, s->na, value);
@@ -662,9 +685,8 @@ gsim_status gsim_debug_dump(gsim_sim *s, int32_t what, void *buf, size_t bytes, 
         return fail(GSIM_ERROR_OUT_OF_MEMORY, "the handle has no Barnes-Hut buffers");
     gsim::BhCounters ctr{};
     GSIM_HIP(hipMemcpy(&ctr, s->bh.ctr, sizeof(ctr), hipMemcpyDeviceToHost));
-    if (ctr.sort_stall)
-        return fail(GSIM_ERROR_DEVICE, "radix sort look-back gave up on %u status words: the tree is invalid",
-                    ctr.sort_stall);
+    const gsim_status sorted = check_sort(s, ctr.sort_stall);
+    if (sorted != GSIM_OK) return sorted;
     const size_t nodes = s->has_tree ? ctr.n_nodes : 0;
     switch (what) {
         case GSIM_DUMP_CELLS: {

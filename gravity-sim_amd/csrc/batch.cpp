@@ -97,6 +97,20 @@ void give_range(gsim_batch *b, uint32_t off, uint32_t len) {
     }
 }
 
+// Steps that system s has taken.
+uint64_t steps_taken(const gsim_batch *b, const gsim::BatchSystem &s) {
+    const uint64_t taken = b->steps - s.added_at;
+    return s.target == ~0ull ? taken : std::min<uint64_t>(taken, s.target);
+}
+
+// The sort gave up since the last upload: every system that stepped is spoilt
+// for good (`stall` is forgotten with the upload, which lets new ones in).
+void note_stall(gsim_batch *b, uint32_t stall) {
+    if (!stall) return;
+    for (auto &kv : b->systems)
+        if (steps_taken(b, kv.second) > 0) kv.second.spoilt = true;
+}
+
 // Rebuilds and uploads the membership arrays (descriptors, ranks, work items).
 gsim_status upload_membership(gsim_batch *b) {
     std::vector<gsim::SysDesc> desc;
@@ -105,10 +119,12 @@ gsim_status upload_membership(gsim_batch *b) {
     std::vector<uint32_t> remaining;
     uint64_t ds_pairs = 0;
     GSIM_HIP(hipStreamSynchronize(b->stream));  // step counts below are exact from here
+    gsim::BatchCounts last{};
+    GSIM_HIP(hipMemcpy(&last, b->d.counts, sizeof(last), hipMemcpyDeviceToHost));
+    note_stall(b, last.sort_stall);
     for (auto &kv : b->systems) {
         gsim::BatchSystem &s = kv.second;
-        const uint64_t taken = b->steps - s.added_at;
-        s.steps = s.target == ~0ull ? taken : std::min<uint64_t>(taken, s.target);
+        s.steps = steps_taken(b, s);
         remaining.push_back(s.target == ~0ull ? gsim::kUnlimitedSteps
                                               : (uint32_t)std::min<uint64_t>(s.target - s.steps,
                                                                              gsim::kUnlimitedSteps - 1));
@@ -156,9 +172,8 @@ gsim_status upload_membership(gsim_batch *b) {
     c.n_ds = c.n_items - (uint32_t)bh_items.size();
     c.ds_groups = ds_pairs > gsim::kBatchDsPairs * c.n_bh_particles ? gsim::kBatchDsBlocks
                                                                    : gsim::kBatchDsBeside;
-    // the acceptance and visit totals carry over
-    GSIM_HIP(hipMemcpy(&c.accepts, &b->d.counts->accepts, sizeof(c.accepts), hipMemcpyDeviceToHost));
-    GSIM_HIP(hipMemcpy(&c.visits, &b->d.counts->visits, sizeof(c.visits), hipMemcpyDeviceToHost));
+    c.accepts = last.accepts;
+    c.visits = last.visits;
     auto up = [&](void *dst, const void *src, size_t bytes) -> hipError_t {
         return bytes ? hipMemcpy(dst, src, bytes, hipMemcpyHostToDevice) : hipSuccess;
     };
@@ -409,8 +424,7 @@ gsim_status gsim_batch_set_steps(gsim_batch *b, uint32_t id, uint64_t more_steps
     GSIM_HIP(hipSetDevice(b->device));
     GSIM_HIP(hipStreamSynchronize(b->stream));
     gsim::BatchSystem &s = it->second;
-    const uint64_t taken = b->steps - s.added_at;
-    const uint64_t done = s.target == ~0ull ? taken : std::min<uint64_t>(taken, s.target);
+    const uint64_t done = steps_taken(b, s);
     // re-anchor so that `done` steps stay counted and `more_steps` remain
     s.added_at = b->steps - done;
     s.target = more_steps == ~0ull ? ~0ull : done + more_steps;
@@ -423,9 +437,7 @@ gsim_status gsim_batch_steps_done(gsim_batch *b, uint32_t id, uint64_t *steps) {
     if (!b || !steps) return fail(GSIM_ERROR_INVALID_ARGUMENT, "gsim_batch_steps_done: NULL argument");
     auto it = b->systems.find(id);
     if (it == b->systems.end()) return fail(GSIM_ERROR_INVALID_ARGUMENT, "no system %u in the batch", id);
-    const gsim::BatchSystem &s = it->second;
-    const uint64_t taken = b->steps - s.added_at;
-    *steps = s.target == ~0ull ? taken : std::min<uint64_t>(taken, s.target);
+    *steps = steps_taken(b, it->second);
     return GSIM_OK;
 }
 
@@ -479,9 +491,9 @@ gsim_status gsim_batch_read(gsim_batch *b, uint32_t id, float *pos_xy, float *ve
         GSIM_HIP(hipStreamSynchronize(b->stream));
         GSIM_HIP(hipMemcpy(&stall, &b->d.counts->sort_stall, sizeof(stall), hipMemcpyDeviceToHost));
     }
-    if (stall)
-        return fail(GSIM_ERROR_DEVICE, "radix sort look-back gave up on %u status words: the batch state is invalid",
-                    stall);
+    note_stall(b, stall);
+    if (s.spoilt)
+        return fail(GSIM_ERROR_DEVICE, "a radix sort look-back gave up: the system's state is invalid");
     if (staged) {
         if (pos_xy) std::memcpy(pos_xy, t.pos, sizeof(float2) * s.n);
         if (vel_xy) std::memcpy(vel_xy, t.vel, sizeof(float2) * s.n);
@@ -591,6 +603,8 @@ gsim_status gsim_batch_autotune(gsim_batch *b, uint32_t steps_per_trial, uint32_
     // ... and add to the acceptance and visit totals: restore those too
     unsigned long long work0[2] = {0, 0};
     GSIM_HIP(hipMemcpy(work0, &b->d.counts->accepts, sizeof(work0), hipMemcpyDeviceToHost));
+    uint32_t stall0 = 0;
+    GSIM_HIP(hipMemcpy(&stall0, &b->d.counts->sort_stall, sizeof(stall0), hipMemcpyDeviceToHost));
     auto restore = [&]() -> hipError_t {
         hipError_t r = hipStreamSynchronize(b->stream);
         if (r == hipSuccess) r = hipMemcpy(b->d.pos[cur0], snap_pos, sizeof(float2) * cap, hipMemcpyDeviceToDevice);
@@ -600,6 +614,8 @@ gsim_status gsim_batch_autotune(gsim_batch *b, uint32_t steps_per_trial, uint32_
             r = hipMemcpy(b->d.remaining, rem_snapshot.data(), 4 * rem_snapshot.size(), hipMemcpyHostToDevice);
         if (r == hipSuccess)
             r = hipMemcpy(&b->d.counts->accepts, work0, sizeof(work0), hipMemcpyHostToDevice);
+        if (r == hipSuccess)
+            r = hipMemcpy(&b->d.counts->sort_stall, &stall0, sizeof(stall0), hipMemcpyHostToDevice);
         b->cur = cur0;
         b->steps = steps0;
         return r;

@@ -62,7 +62,8 @@ struct BatchCounts {
     uint32_t n_cells;         // cell nodes of all trees (emit)
     uint32_t n_leaves;        // occupied leaves of all trees (emit)
     uint32_t n_sys;           // all systems (direct sum and Barnes-Hut)
-    uint32_t sort_stall;      // radix look-back waits that hit their bound (never expected)
+    uint32_t sort_stall;      // radix look-back waits that hit their bound since the
+                              // membership was uploaded (never expected)
     uint32_t n_live[kLiveLists];  // (system, depth-5 tile) pairs holding leaves, per list
     unsigned long long accepts;  // Barnes-Hut real-lane acceptances, all steps
     unsigned long long visits;   // Barnes-Hut real-lane node visits, all steps
@@ -143,6 +144,7 @@ struct BatchSystem {
     uint64_t steps = 0;          // steps taken (exact after a synchronisation)
     uint64_t added_at = 0;       // batch step count when the system joined
     uint64_t target = ~0ull;     // total steps to take (~0 = unlimited)
+    bool spoilt = false;         // it stepped while the sort gave up: its state is invalid
 };
 
 }  // namespace gsim

@@ -84,7 +84,6 @@ __global__ __launch_bounds__(kSortThreads) void bb_keys_kernel(
     if (tid == 0) {
         counts->n_cells = 0;
         counts->n_leaves = 0;
-        counts->sort_stall = 0;
     }
 #pragma unroll
     for (uint32_t p = 0; p < kBatchPasses; ++p) h[p][th] = 0;
@@ -233,6 +232,8 @@ __global__ __launch_bounds__(1024) void bb_block_scan_kernel(uint32_t *__restric
     scan_inplace_1024(blockIdx.x == 0 ? a : b, (counts->n_bh_particles + 255) / 256, wsum);
 }
 
+// Where a look-back of the sort gave up, its output is no permutation: every
+// particle is taken as outside (no tree, no walk; bh_emit_kernel).
 __global__ __launch_bounds__(256) void bb_emit_kernel(
     const uint32_t *__restrict__ keys, const uint32_t *__restrict__ sidx,
     const float2 *__restrict__ pos, const float *__restrict__ mass,
@@ -246,13 +247,15 @@ __global__ __launch_bounds__(256) void bb_emit_kernel(
     const uint32_t n = counts->n_bh_particles;
     const uint32_t nblocks = (n + 255) / 256;
     const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const bool stalled = counts->sort_stall != 0u;
     for (uint32_t blk = blockIdx.x; blk < nblocks; blk += gridDim.x) {
         const uint32_t k = blk * 256 + threadIdx.x;
         // the particle's gather does not depend on the scan below: start it first
-        const uint32_t i = k < n ? sidx[k] : 0u;
+        const uint32_t i = k < n && !stalled ? sidx[k] : 0u;
         const float2 p = k < n ? pos[i] : make_float2(0.0f, 0.0f);
         const float m = k < n ? mass[i] : 0.0f;
-        const BPos q = bpos_info(keys, n, k);
+        BPos q = bpos_info(keys, n, k);
+        if (stalled) q.inside = false;
         uint32_t a = q.ns, b = q.lf;
         wave_scan2(a, b);
         if (lane == 63) {
@@ -268,7 +271,7 @@ __global__ __launch_bounds__(256) void bb_emit_kernel(
         }
         __syncthreads();
         if (k >= n) continue;
-        if (k + 1 == n) {  // totals over all systems, and the end of the last leaf
+        if (k + 1 == n && !stalled) {  // totals over all systems, and the end of the last leaf
             counts->n_cells = C + q.ns;
             counts->n_leaves = L + q.lf;
             leaf_first[L + q.lf] = q.inside ? k + 1 : n;

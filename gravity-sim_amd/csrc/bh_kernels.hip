@@ -134,8 +134,8 @@ __global__ __launch_bounds__(kSortThreads) void bh_keys_kernel(
     const float2 *__restrict__ pos, const uint32_t *__restrict__ perm, uint32_t na,
     uint2 *__restrict__ cells, uint32_t *__restrict__ tile_range,
     uint32_t *__restrict__ digit_total, uint32_t *__restrict__ digit_next,
-    uint32_t *__restrict__ status, uint32_t status_words, BhCounters *__restrict__ ctr,
-    const float4 *__restrict__ box_part, uint32_t box_parts, float4 *__restrict__ box) {
+    uint32_t *__restrict__ status, uint32_t status_words, const float4 *__restrict__ box_part,
+    uint32_t box_parts, float4 *__restrict__ box) {
     constexpr int kPasses = kDeep ? 4 : 3;
     __shared__ uint32_t h[kPasses][256];
     const uint32_t t = threadIdx.x;
@@ -143,9 +143,6 @@ __global__ __launch_bounds__(kSortThreads) void bh_keys_kernel(
     for (uint32_t j = g; j < kTileWords; j += stride) tile_range[j] = 0;
     for (uint32_t j = g; j < kDigitCopies * 1024; j += stride) digit_next[j] = 0;
     for (uint32_t j = g; j < status_words; j += stride) status[j] = 0;
-    if (g == 0) {
-        ctr->sort_stall = 0;
-    }
 #pragma unroll
     for (int p = 0; p < kPasses; ++p) h[p][t] = 0;
     float4 bx = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
@@ -216,9 +213,9 @@ __global__ __launch_bounds__(kSortThreads) void radix_onesweep_kernel(
     uint32_t *__restrict__ stall) {
     __shared__ SortShared<false, kR> sh;
     sort_tile_clear(sh);  // the tile's first barrier follows its ranking
-    // Tile = workgroup index.  A tile only waits for lower tiles, which the
-    // dispatcher starts first, and a pass's workgroups all fit on the GPU at
-    // once, so every wait ends (and each is bounded besides).
+    // Tile = workgroup index: a tile only waits for lower ones, and every wait
+    // ends (radix_device.hpp), also where a pass has more workgroups than fit
+    // on the GPU at once (four a CU, from about 2,000,000 particles on).
     sort_tile<false, kR>(keys_in, idx_in, keys_out, idx_out, n, shift, blockIdx.x, gridDim.x,
                          status, status + (size_t)gridDim.x * 256, digit_total, kDigitCopies,
                          1024u, stall, sh, cells_in);
@@ -357,7 +354,10 @@ __device__ __forceinline__ void emit_position(const EmitArgs &e, const PosInfo &
 
 // block_cells, block_leaves (and block_gran): bh_prep_kernel's per-block
 // counts; each block adds up those of the blocks before it (integer sums, a
-// few loads per thread) instead of a separate scan launch.
+// few loads per thread) instead of a separate scan launch.  Where a look-back
+// of the sort ever gave up (sort_stall), its output names slots that do not
+// exist and has no order: every particle is taken as killed in place, so that
+// nothing after this is out of bounds, and the handle's reads fail from then on.
 __global__ __launch_bounds__(256) void bh_emit_kernel(
     const uint32_t *__restrict__ keys, const uint32_t *__restrict__ sidx, EmitArgs e,
     const uint32_t *__restrict__ block_cells, const uint32_t *__restrict__ block_leaves,
@@ -367,7 +367,8 @@ __global__ __launch_bounds__(256) void bh_emit_kernel(
     const uint32_t k = blockIdx.x * 256 + threadIdx.x;
     // the particle now at sorted position k, from its slot i of the last
     // step's order (nearly the same order, so nearly sequential reads)
-    const uint32_t i = k < na ? sidx[k] : 0u;
+    const bool stalled = e.ctr->sort_stall != 0u;
+    const uint32_t i = k >= na ? 0u : stalled ? k : sidx[k];
     const float2 p = k < na ? e.pos[i] : make_float2(0.0f, 0.0f);
     const float m = k < na ? e.mass[i] : 0.0f;
     const uint32_t orig = k < na ? e.perm_in[i] : 0u;
@@ -390,7 +391,8 @@ __global__ __launch_bounds__(256) void bh_emit_kernel(
             xc += vc[u];
         }
     }
-    const PosInfo q = pos_info(keys, na, k, e.bits);
+    PosInfo q = pos_info(keys, na, k, e.bits);
+    if (stalled) q.inside = false;
     uint32_t a = q.ns, b = q.lf;
     wave_scan2(a, b);
     const unsigned long long gb = __ballot(q.g10);
@@ -456,7 +458,6 @@ __global__ __launch_bounds__(64 * kSmallWaves) void bh_small_kernel(
     const uint32_t rows = (na + 64 * kSmallWaves - 1) / (64 * kSmallWaves);
     const uint32_t first = wave * rows * 64 + lane;  // row r: position first + 64 r
     for (uint32_t j = t; j < kTileWords; j += 64 * kSmallWaves) tile_range[j] = 0;
-    if (t == 0) e.ctr->sort_stall = 0;
     uint32_t key[kSmallRows], val[kSmallRows], rank[kSmallRows];
     if constexpr (!kWalk) {
         float2 p[kSmallRows];
@@ -1203,7 +1204,7 @@ hipError_t bh_launch_build(gsim_sim *s, const float2 *pos, const float *mass,
 #define GSIM_KEYS(R, B, D, W)                                                                  \
     bh_keys_kernel<B, D, R, W><<<nblk, kSortThreads, 0, s->stream>>>(                           \
         pos, perm_in, na, b.cells[kin], b.tile_range, totals, totals_next, b.status,           \
-        status_words, b.ctr, b.box_part, nparts, box4)
+        status_words, b.box_part, nparts, box4)
 #define GSIM_SORT(R)                                                                           \
     do {                                                                                       \
         if (box) { if (deep) GSIM_KEYS(R, true, true, false); else GSIM_KEYS(R, true, false, false); } \

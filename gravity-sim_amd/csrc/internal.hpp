@@ -50,7 +50,8 @@ struct BhCounters {
     uint32_t n_nodes;   // n_in + n_cells = counts[0]
     uint32_t n_leaves;  // occupied leaf cells (depth 10, or 15 with 15-bit leaves)
     uint32_t n_gran;             // 15-bit leaves: occupied depth-10 cells
-    uint32_t sort_stall;         // look-back waits that hit their bound (never expected)
+    uint32_t sort_stall;         // look-back waits that hit their bound since the buffers
+                                 // were made (never expected)
 };
 
 // Radix sort passes (single and batched builds): tiles of kSortThreads keys a
@@ -265,6 +266,7 @@ struct gsim_sim {
     uint32_t ds_S_used = 1;
     // Barnes-Hut
     gsim::BhBuffers bh;
+    uint32_t sort_stall = 0;           // of bh and the buffers before it, as last read
     gsim::ReadStage stage;
     // debug / timing
     float2 *accel = nullptr;

@@ -2,8 +2,10 @@
 // (bh_kernels.hip) and the batched build (batch_kernels.hip).
 //
 // A pass sorts tiles of kR * kSortThreads (key, value) pairs on one 8-bit digit, one
-// tile per workgroup in launch order, so every lower tile belongs to a
-// workgroup that has started before.  Within the tile, key r * 256 + t
+// tile per workgroup in launch order.  Each XCD starts its workgroups in that
+// order, so of the tiles not yet done the lowest runs or is the next that its
+// XCD starts, whatever else runs beside the sort, and it waits for no other:
+// the tiles finish one after another at worst.  Within the tile, key r * 256 + t
 // (round r, thread t) is ranked among the equal digits of its wave by
 // ballots; the per-(round, wave, digit) counts go to LDS and thread d scans
 // digit d's counts in (round, wave) order, which is input order, so the sort
@@ -14,7 +16,8 @@
 // straight to its position).  The tile's words (0: not yet counted, kStA | a
 // count, kStP | an inclusive prefix) are summed by grouped_prefix.  A tile
 // publishes its count before it reads any predecessor, so every wait ends;
-// waits are bounded all the same (kSpinLimit re-reads, counted in *stall).
+// waits are bounded all the same (kSpinLimit re-reads, counted in *stall, which
+// the emission and the reads look at).
 #pragma once
 #include "bh_device.hpp"
 #include "internal.hpp"

@@ -2,6 +2,9 @@
 checks, and seeded inputs."""
 from __future__ import annotations
 
+import ctypes as C
+import os
+
 import numpy as np
 
 SIM_SIZE = np.float32(500.0)
@@ -252,3 +255,26 @@ def dyadic_particles(n: int, seed: int, spread: int = 40):
     mass = rng.integers(1, 8, size=n).astype(np.float32)
     vel = np.zeros((n, 2), np.float32)
     return pos, vel, mass
+
+
+# ---- inside a handle (native/handle_access.cpp) ------------------------------
+
+_access = None
+
+
+def handle_access():
+    global _access
+    if _access is None:
+        import gsim
+        gsim.load_library()
+        _access = C.CDLL(os.path.join(os.path.dirname(gsim.LIB_PATH), "libgsim_access.so"))
+    return _access
+
+
+def put_sort_stall(handle, count: int) -> None:
+    """As if `count` look-backs of the handle's radix sort had given up."""
+    import gsim
+    handle.synchronize()
+    f = (handle_access().access_batch_sort_stall if isinstance(handle, gsim.Batch)
+         else handle_access().access_sort_stall)
+    assert f(handle._h, C.c_uint32(count)) == 0

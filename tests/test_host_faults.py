@@ -11,7 +11,8 @@ import gsim
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 
-SCENARIOS = ["failed_form_keeps_the_last", "lost_tree_buffers"]
+SCENARIOS = ["failed_form_keeps_the_last", "lost_tree_buffers",
+             "given_up_sort_is_never_read"]
 
 
 @pytest.fixture(scope="module")
