@@ -396,7 +396,7 @@ gsim_status gsim_create(const gsim_params *params, const float *pos_xy, const fl
             e = hipMemcpy(s->vel[k], hv.data(), sizeof(float) * 2 * na, hipMemcpyHostToDevice);
     }
     if (e == hipSuccess) e = hipMemcpy(s->mass, hm.data(), sizeof(float) * na, hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = hipMemset(s->accel, 0, sizeof(float2) * na);
+    if (e == hipSuccess) e = hipMemsetAsync(s->accel, 0, sizeof(float2) * na, s->stream);
     if (e == hipSuccess && s->perm[0]) {
         // the caller's order to start with
         std::vector<uint32_t> id(na);
@@ -420,7 +420,7 @@ gsim_status gsim_create(const gsim_params *params, const float *pos_xy, const fl
         }
         if (st != GSIM_OK) return bail(st);
     } else {
-        e = gsim::bh_alloc(&s->bh, na, gsim::kTreeDepth);
+        e = gsim::bh_alloc(&s->bh, na, gsim::kTreeDepth, s->stream);
         if (e != hipSuccess)
             return bail(fail(GSIM_ERROR_OUT_OF_MEMORY, "Barnes-Hut buffers: %s", hipGetErrorString(e)));
     }
@@ -590,12 +590,12 @@ gsim_status gsim_set_tuning(gsim_sim *s, int32_t knob, uint32_t value) {
             }
             gsim::bh_free(&s->bh);
             s->has_tree = false;
-            const hipError_t e = gsim::bh_alloc(&s->bh, s->na, value);
+            const hipError_t e = gsim::bh_alloc(&s->bh, s->na, value, s->stream);
             if (e != hipSuccess) {
                 (void)hipGetLastError();
                 gsim::bh_free(&s->bh);
                 // without even the last depth's, the state can be read and no step taken
-                if (gsim::bh_alloc(&s->bh, s->na, last) != hipSuccess) {
+                if (gsim::bh_alloc(&s->bh, s->na, last, s->stream) != hipSuccess) {
                     (void)hipGetLastError();
                     gsim::bh_free(&s->bh);
                 }

@@ -303,15 +303,17 @@ gsim_status gsim_batch_create(int32_t device, size_t capacity_particles, uint32_
     GSIM_BALLOC(d.wave_acc, 2 * gsim::kMaxForceWaves);
     GSIM_BALLOC(d.ichunk, b->item_capacity);
 #undef GSIM_BALLOC
-    if (e == hipSuccess) e = hipMemset(d.counts, 0, sizeof(gsim::BatchCounts));
-    if (e == hipSuccess)
-        e = hipMemset(d.qnext, 0, sizeof(uint32_t) * gsim::kForceQueues * gsim::kQueueStride);
-    if (e == hipSuccess)
-        e = hipMemset(d.digit_total, 0, sizeof(uint32_t) * max_systems * gsim::kBatchPasses * 256);
-    if (e == hipSuccess) e = hipMemset(d.wave_acc, 0, sizeof(unsigned long long) * 2 * gsim::kMaxForceWaves);
-    if (e == hipSuccess) e = hipMemset(d.ichunk, 0, sizeof(uint32_t) * b->item_capacity);
-    if (e == hipSuccess) e = hipMemset(d.child, 0, sizeof(uint4) * b->node_capacity);
-    if (e == hipSuccess) e = hipMemset(d.node4, 0, sizeof(float4) * b->node_capacity);
+    // on the batch's stream, which does not wait for the null stream
+    auto clear = [&](void *p, size_t bytes) {
+        if (e == hipSuccess) e = hipMemsetAsync(p, 0, bytes, b->stream);
+    };
+    clear(d.counts, sizeof(gsim::BatchCounts));
+    clear(d.qnext, sizeof(uint32_t) * gsim::kForceQueues * gsim::kQueueStride);
+    clear(d.digit_total, sizeof(uint32_t) * max_systems * gsim::kBatchPasses * 256);
+    clear(d.wave_acc, sizeof(unsigned long long) * 2 * gsim::kMaxForceWaves);
+    clear(d.ichunk, sizeof(uint32_t) * b->item_capacity);
+    clear(d.child, sizeof(uint4) * b->node_capacity);
+    clear(d.node4, sizeof(float4) * b->node_capacity);
     if (e != hipSuccess) {
         gsim_status st = fail(GSIM_ERROR_OUT_OF_MEMORY, "batch allocation failed: %s", hipGetErrorString(e));
         free_batch(b);
@@ -616,6 +618,7 @@ gsim_status gsim_batch_autotune(gsim_batch *b, uint32_t steps_per_trial, uint32_
             r = hipMemcpy(&b->d.counts->accepts, work0, sizeof(work0), hipMemcpyHostToDevice);
         if (r == hipSuccess)
             r = hipMemcpy(&b->d.counts->sort_stall, &stall0, sizeof(stall0), hipMemcpyHostToDevice);
+        if (r == hipSuccess) r = hipStreamSynchronize(nullptr);
         b->cur = cur0;
         b->steps = steps0;
         return r;
@@ -623,6 +626,8 @@ gsim_status gsim_batch_autotune(gsim_batch *b, uint32_t steps_per_trial, uint32_
     if (e == hipSuccess) e = hipMemcpy(snap_pos, b->d.pos[cur0], sizeof(float2) * cap, hipMemcpyDeviceToDevice);
     if (e == hipSuccess) e = hipMemcpy(snap_vel, b->d.vel[cur0], sizeof(float2) * cap, hipMemcpyDeviceToDevice);
     if (e == hipSuccess) e = hipMemcpy(snap_mass, b->d.mass, sizeof(float) * cap, hipMemcpyDeviceToDevice);
+    // copies on the device return before they are done
+    if (e == hipSuccess) e = hipStreamSynchronize(nullptr);
     gsim_status st = GSIM_OK;
     // One trial: the candidate's graphs are captured and warmed by one step,
     // then `steps_per_trial` steps are timed, twice, each from the snapshot;

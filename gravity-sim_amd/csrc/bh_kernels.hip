@@ -1075,7 +1075,7 @@ size_t bh_capacity(size_t na, uint32_t bits) {
     return na + cells + 64;
 }
 
-hipError_t bh_alloc(BhBuffers *b, size_t na, uint32_t bits) {
+hipError_t bh_alloc(BhBuffers *b, size_t na, uint32_t bits, hipStream_t stream) {
     b->na = na;
     b->bits = bits;
     b->cap = bh_capacity(na, bits);
@@ -1121,13 +1121,14 @@ hipError_t bh_alloc(BhBuffers *b, size_t na, uint32_t bits) {
     GSIM_ALLOC(b->gvis, na / 32 + 1);  // one slot per group of W = 32 or 64
     GSIM_ALLOC(b->gacc, na / 32 + 1);
 #undef GSIM_ALLOC
-    if (e == hipSuccess) e = hipMemset(b->ctr, 0, sizeof(BhCounters));
-    if (e == hipSuccess) e = hipMemset(b->digit_total, 0, sizeof(uint32_t) * 2 * kDigitCopies * 1024);
-    if (e == hipSuccess) e = hipMemset(b->gchunk, 0, sizeof(uint32_t) * (na / 64 + 1));
-    if (e == hipSuccess) e = hipMemset(b->gvis, 0, sizeof(unsigned long long) * (na / 32 + 1));
-    if (e == hipSuccess) e = hipMemset(b->gacc, 0, sizeof(unsigned long long) * (na / 32 + 1));
-    if (e == hipSuccess) e = hipMemset(b->child, 0, sizeof(uint4) * b->cap);
-    if (e == hipSuccess) e = hipMemset(b->node4, 0, sizeof(float4) * b->cap);
+    if (e == hipSuccess) e = hipMemsetAsync(b->ctr, 0, sizeof(BhCounters), stream);
+    if (e == hipSuccess)
+        e = hipMemsetAsync(b->digit_total, 0, sizeof(uint32_t) * 2 * kDigitCopies * 1024, stream);
+    if (e == hipSuccess) e = hipMemsetAsync(b->gchunk, 0, sizeof(uint32_t) * (na / 64 + 1), stream);
+    if (e == hipSuccess) e = hipMemsetAsync(b->gvis, 0, sizeof(unsigned long long) * (na / 32 + 1), stream);
+    if (e == hipSuccess) e = hipMemsetAsync(b->gacc, 0, sizeof(unsigned long long) * (na / 32 + 1), stream);
+    if (e == hipSuccess) e = hipMemsetAsync(b->child, 0, sizeof(uint4) * b->cap, stream);
+    if (e == hipSuccess) e = hipMemsetAsync(b->node4, 0, sizeof(float4) * b->cap, stream);
     return e;
 }
 

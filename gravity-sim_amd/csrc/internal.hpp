@@ -294,7 +294,9 @@ hipError_t ds_launch_combine(gsim_sim *s, const float2 *pos, const float2 *vel,
 
 // Barnes-Hut (bh_kernels.hip)
 size_t bh_capacity(size_t na, uint32_t bits);
-hipError_t bh_alloc(BhBuffers *b, size_t na, uint32_t bits);
+// Clears its buffers on `stream`, without waiting: a memset of the null stream
+// returns before it is done, and the handle's stream does not wait for that one.
+hipError_t bh_alloc(BhBuffers *b, size_t na, uint32_t bits, hipStream_t stream);
 void bh_free(BhBuffers *b);
 hipError_t bh_launch_build(gsim_sim *s, const float2 *pos, const float *mass,
                            const uint32_t *perm_in, float2 *pos_out, const float2 *vel,

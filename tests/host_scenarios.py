@@ -136,6 +136,24 @@ def given_up_sort_is_never_read():
         b.read(new)
 
 
+def new_buffers_are_cleared_before_use():
+    """No step starts beside the clearing of the buffers it uses, or beside a
+    copy that keeps the state."""
+    p = gsim.generate("galaxy", 9_000, 100.0, 1.0, 10.0)
+    for algorithm in ("direct-sum", "barnes-hut"):
+        with gsim.Simulation(p, algorithm) as s:
+            s.step(1)
+            if algorithm == "barnes-hut":
+                s.set_tuning(gsim.TUNE_BH_LEAF_BITS, 15)
+                s.step(1)
+    with gsim.Batch(100_000, 8) as b:
+        for algorithm in ("direct-sum", "barnes-hut"):
+            b.add(p, algorithm)
+        b.step(1)
+        b.autotune(1)
+        b.step(1)
+
+
 if __name__ == "__main__":
     _load(sys.argv[1])
     globals()[sys.argv[2]]()

@@ -23,6 +23,9 @@ size_t live = 0, limit = ~(size_t)0;
 std::string launches, faults;
 std::set<void *> capturing, spoiled;  // streams in capture; captures made invalid
 unsigned capture_delay_us = 0, instantiated = 0;
+// Memsets and copies on the device return before they are done; the library's
+// streams do not wait for the null stream.
+bool null_busy = false;
 char token;  // every stream, event and graph but the null stream is some address
 
 void fault(const std::string &what) { faults += what + "\n"; }
@@ -92,6 +95,10 @@ hipError_t copy(void *d, const void *s, size_t n) {
 
 extern "C" {
 
+static void starts_on(hipStream_t st) {
+    if (st && null_busy) fault("work starts beside an unfinished one of the null stream");
+}
+
 // ---- what a test asks for and looks at ---------------------------------------
 void fake_limit(size_t bytes) { limit = bytes; }  // of device memory held at once
 size_t fake_live() { return live; }
@@ -135,6 +142,7 @@ hipError_t hipLaunchKernel(const void *f, dim3, dim3, void **args, size_t, hipSt
         std::lock_guard<std::recursive_mutex> lk(mu);
         const std::string &name = kernels[f];
         launches += name + "\n";
+        if (!capturing.count(st)) starts_on(st);
         auto is = [&](const char *k) { return name.find(k) != std::string::npos; };
         if (is("read_kernel")) read_particles(args);
         if ((is("ds_partial_kernel") || is("ds_sym_kernel")) && !arg<void *>(args, 2))
@@ -156,16 +164,22 @@ hipError_t hipHostFree(void *p) {
     std::free(p);
     return hipSuccess;
 }
-hipError_t hipMemcpy(void *d, const void *s, size_t n, hipMemcpyKind) { return copy(d, s, n); }
-hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind, hipStream_t) {
+hipError_t hipMemcpy(void *d, const void *s, size_t n, hipMemcpyKind kind) {
+    null_busy = kind == hipMemcpyDeviceToDevice;  // the others wait for all before
     return copy(d, s, n);
 }
-hipError_t hipMemset(void *d, int v, size_t n) {
+hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind, hipStream_t st) {
+    starts_on(st);
+    return copy(d, s, n);
+}
+hipError_t hipMemsetAsync(void *d, int v, size_t n, hipStream_t st) {
     if (n && !d) return hipErrorInvalidValue;
+    starts_on(st);
+    if (!st) null_busy = true;
     if (n) std::memset(d, v, n);
     return hipSuccess;
 }
-hipError_t hipMemsetAsync(void *d, int v, size_t n, hipStream_t) { return hipMemset(d, v, n); }
+hipError_t hipMemset(void *d, int v, size_t n) { return hipMemsetAsync(d, v, n, nullptr); }
 
 hipError_t hipGetDevice(int *d) {
     *d = 0;
@@ -198,6 +212,7 @@ hipError_t hipStreamDestroy(hipStream_t s) {
 }
 hipError_t hipStreamSynchronize(hipStream_t s) {
     std::lock_guard<std::recursive_mutex> lk(mu);
+    if (!s) null_busy = false;
     if (!capturing.count(s)) return hipSuccess;
     spoiled.insert(s);
     fault("a stream under capture is waited for");
@@ -223,7 +238,10 @@ hipError_t hipGraphInstantiate(hipGraphExec_t *e, hipGraph_t, hipGraphNode_t *, 
     *e = (hipGraphExec_t)fresh();
     return hipSuccess;
 }
-hipError_t hipGraphLaunch(hipGraphExec_t, hipStream_t) { return hipSuccess; }
+hipError_t hipGraphLaunch(hipGraphExec_t, hipStream_t st) {
+    starts_on(st);
+    return hipSuccess;
+}
 hipError_t hipGraphDestroy(hipGraph_t g) {
     std::free(g);
     return hipSuccess;
