@@ -63,6 +63,12 @@ struct gsim_server {
     std::map<uint64_t, Request *> running;  // (arena << 32 | batch id) -> request
     std::vector<double> latencies_ms;
     uint64_t completed = 0, failed = 0, batch_steps = 0, ds_interactions = 0;
+    // Barnes-Hut acceptances and visits of all arenas, as last read.  Only the
+    // worker touches an arena that it steps (its stream may be under capture):
+    // a query asks it and waits for the next reading, at most a chunk of steps.
+    uint64_t accepts = 0, visits = 0, totals_read = 0;
+    uint32_t totals_wanted = 0;
+    std::condition_variable cv_totals;
     Clock::time_point first_submit, last_done;
     bool any_submit = false;
     char worker_error[256] = {0};
@@ -74,6 +80,20 @@ namespace {
 constexpr uint64_t kChunkSteps = 8;
 
 size_t padded(size_t n) { return (n + 63) / 64 * 64; }
+
+// Reads the arenas' totals (under the lock, no arena being stepped); a failure
+// leaves the last ones.
+void read_totals(gsim_server *s) {
+    uint64_t accepts = 0, visits = 0;
+    for (gsim_batch *b : s->arenas) {
+        uint64_t a = 0, v = 0;
+        if (gsim_batch_accepts(b, &a) != GSIM_OK || gsim_batch_visits(b, &v) != GSIM_OK) return;
+        accepts += a;
+        visits += v;
+    }
+    s->accepts = accepts;
+    s->visits = visits;
+}
 
 void worker_loop(gsim_server *s) {
     std::unique_lock<std::mutex> lk(s->mu);
@@ -134,8 +154,14 @@ void worker_loop(gsim_server *s) {
         for (size_t a = 0; a < s->arenas.size() && st == GSIM_OK; ++a)
             if (busy[a]) st = gsim_batch_synchronize(s->arenas[a]);
         lk.lock();
-        if (st != GSIM_OK) {
+        if (st != GSIM_OK)
             std::snprintf(s->worker_error, sizeof(s->worker_error), "%s", gsim_last_error());
+        if (s->totals_wanted) {
+            read_totals(s);
+            ++s->totals_read;
+            s->cv_totals.notify_all();
+        }
+        if (st != GSIM_OK) {
             for (auto &kv : s->running) {
                 kv.second->state = 3;
                 kv.second->done = Clock::now();
@@ -347,9 +373,19 @@ gsim_status gsim_server_drain(gsim_server *s, double timeout_s, int32_t *idle) {
 gsim_status gsim_server_query(gsim_server *s, gsim_server_info *out) {
     gsim::clear_error();
     if (!s || !out) return fail(GSIM_ERROR_INVALID_ARGUMENT, "gsim_server_query: NULL argument");
-    uint64_t accepts = 0;
     {
-        std::lock_guard<std::mutex> lk(s->mu);
+        std::unique_lock<std::mutex> lk(s->mu);
+        if (s->running.empty()) {  // the worker steps nothing without the lock
+            read_totals(s);
+            gsim::clear_error();
+        } else {
+            const uint64_t seen = s->totals_read;
+            ++s->totals_wanted;
+            s->cv_totals.wait(lk, [&] { return s->totals_read != seen || s->stop; });
+            --s->totals_wanted;
+        }
+        out->bh_interactions = s->accepts;
+        out->bh_visits = s->visits;
         out->completed = s->completed;
         out->failed = s->failed;
         out->queued = s->queue.size();
@@ -364,16 +400,6 @@ gsim_status gsim_server_query(gsim_server *s, gsim_server_info *out) {
         out->ds_interactions = s->ds_interactions;
         out->capacity_particles = s->capacity;
     }
-    uint64_t visits = 0;
-    for (gsim_batch *b : s->arenas) {
-        uint64_t a = 0, v = 0;
-        gsim_batch_accepts(b, &a);
-        gsim_batch_visits(b, &v);
-        accepts += a;
-        visits += v;
-    }
-    out->bh_interactions = accepts;
-    out->bh_visits = visits;
     out->arenas = (uint32_t)s->arenas.size();
     return GSIM_OK;
 }
@@ -386,6 +412,7 @@ gsim_status gsim_server_destroy(gsim_server *s) {
         s->stop = true;
     }
     s->cv_work.notify_all();
+    s->cv_totals.notify_all();
     if (s->worker.joinable()) s->worker.join();
     for (gsim_batch *b : s->arenas) gsim_batch_destroy(b);
     delete s;

@@ -7,6 +7,7 @@ memory is host memory and kernels only leave their names.
 import ctypes as C
 import os
 import sys
+import time
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 for sub in ("gravity-sim_amd/python", "tests", "oracle"):
@@ -152,6 +153,26 @@ def new_buffers_are_cleared_before_use():
         b.step(1)
         b.autotune(1)
         b.step(1)
+
+
+def query_beside_a_capture():
+    """A query from a client's thread leaves the worker's capture alone, and
+    returns what had been counted."""
+    fake.fake_capture_delay(2_000)  # microseconds a captured launch: 30 ms a graph
+    budget = 200_000 * gsim.Batch.bytes_per_particle()
+    ps = [gsim.generate("galaxy", n, 100.0, 1.0, 10.0) for n in (9_000, 700, 12_000, 300)]
+    with gsim.Server(budget, max_systems=64) as srv:
+        rids = []
+        for p, algorithm in zip(ps, ("barnes-hut", "direct-sum", "barnes-hut", "direct-sum")):
+            rids.append(srv.submit(p, 20, algorithm))
+            until = time.monotonic() + 0.2
+            while time.monotonic() < until:
+                srv.stats()
+        assert srv.drain(60.0)
+        stats = srv.stats()
+        assert (stats["completed"], stats["failed"]) == (4, 0), stats
+        for r in rids:
+            assert srv.wait(r, 1.0)
 
 
 if __name__ == "__main__":

@@ -12,7 +12,8 @@ import gsim
 HERE = os.path.dirname(os.path.abspath(__file__))
 
 SCENARIOS = ["failed_form_keeps_the_last", "lost_tree_buffers",
-             "given_up_sort_is_never_read", "new_buffers_are_cleared_before_use"]
+             "given_up_sort_is_never_read", "new_buffers_are_cleared_before_use",
+             "query_beside_a_capture"]
 
 
 @pytest.fixture(scope="module")
