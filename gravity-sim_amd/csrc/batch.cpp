@@ -190,6 +190,11 @@ gsim_status upload_membership(gsim_batch *b) {
         destroy_graphs(b);
         b->sort_slots = 2 * slots;
     }
+    const bool wide = b->nodes_reserved >= b->narrow_nodes;
+    if (wide != b->wide) {
+        destroy_graphs(b);
+        b->wide = wide;
+    }
     if (c.n_ds && !b->has_ds) {
         destroy_graphs(b);
         b->has_ds = true;

@@ -155,6 +155,8 @@ struct gsim_batch {
     hipStream_t side = nullptr;  // the direct sums, beside the build (captured with it)
     hipEvent_t fork = nullptr, join = nullptr;
     bool has_ds = false;         // the graphs hold the direct-sum launch
+    bool wide = false;           // the graphs' walk addresses nodes by slot
+    size_t narrow_nodes = gsim::kNarrowNodes;  // (tests lower it)
     size_t capacity = 0;        // particles (padded) in the arena
     size_t node_capacity = 0;   // node slots
     size_t partial_capacity = 0;  // direct-sum admission units

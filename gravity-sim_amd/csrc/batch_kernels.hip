@@ -653,7 +653,7 @@ hipError_t batch_launch_step(gsim_batch *b, int in, int out) {
                                            d.sdep, d.cpos, d.counts, d.live_tiles, live_per_list,
                                            d.node4, d.child, d.top);
     const uint32_t waves = 1024u * b->tune.waves_per_simd;
-    auto *force = b->node_capacity >= kNarrowNodes ? bb_force_kernel<true> : bb_force_kernel<false>;
+    auto *force = b->wide ? bb_force_kernel<true> : bb_force_kernel<false>;
     force<<<waves / 4, 256, 0, st>>>(d.items, d.desc, d.remaining, d.stats, d.counts, d.sorted_src,
                                                d.pos[in], d.vel[in], d.node4, d.child,
                                                d.pos[out], d.vel[out],

@@ -620,8 +620,8 @@ __device__ __forceinline__ void add_source(f3v q, const float (&tx)[R], const fl
     }
 }
 
-// A list entry: the byte offset of the node's record, or with kWide (node
-// arrays of 4 GiB and more) its slot.
+// A list entry: the byte offset of the node's record, or with kWide (trees
+// that reach beyond 4 GiB of records, kNarrowNodes) its slot.
 template <bool kWide>
 __device__ __forceinline__ uint32_t source_key(uint32_t slot) {
     return kWide ? slot : slot * 16u;

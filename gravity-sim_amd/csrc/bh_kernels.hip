@@ -1289,7 +1289,7 @@ hipError_t bh_launch_traverse(gsim_sim *s, const float2 *pos, const float2 *vel,
     const uint32_t groups = na / s->W, parts = walk_parts(s);
     const uint32_t grid = (groups * parts + 3) / 4;
     const uint32_t *order = parts == 1 ? launch_order(s, groups) : nullptr;
-    const bool wide = b.cap >= kNarrowNodes;
+    const bool wide = b.cap >= s->narrow_nodes;
 #define GSIM_WALK(W, R)                                                                        \
     do {                                                                                       \
         auto *k = dbg ? (wide ? bh_walk_kernel<W, R, true, true> : bh_walk_kernel<W, R, false, true>) \

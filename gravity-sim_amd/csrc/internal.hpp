@@ -88,7 +88,9 @@ constexpr uint32_t kDigitCopies = 8;
 constexpr uint32_t kWalkSplitGroups = 2048;
 constexpr uint32_t kWalkFillWaves = 2048;
 
-// Node arrays of fewer records than this are addressed by 32-bit byte offsets.
+// Walks over fewer node slots than this address them by 32-bit byte offsets
+// (16 bytes a record), others by slot.  Counted are the slots that the handle's
+// tree, or the batch's members, can use.
 constexpr size_t kNarrowNodes = (size_t)1 << 28;
 
 // The largest value of BatchTune::run_queue.
@@ -266,6 +268,7 @@ struct gsim_sim {
     uint32_t ds_S_used = 1;
     // Barnes-Hut
     gsim::BhBuffers bh;
+    size_t narrow_nodes = gsim::kNarrowNodes;  // (tests lower it)
     uint32_t sort_stall = 0;           // of bh and the buffers before it, as last read
     gsim::ReadStage stage;
     // debug / timing

@@ -242,8 +242,9 @@ gsim_status gsim_ds_step_noalloc(const gsim_params *params, const float *pos_xy,
  * as one launch over all systems (Barnes-Hut systems share one node array; the
  * direct sums run beside their build), and the whole step is replayed from a
  * captured hipGraph.  Membership can change between steps; the graph is
- * captured again only when the members outgrow twice what they were, or the
- * first direct-sum system joins.  A system's results are bit-identical
+ * captured again only when the members outgrow twice what they were, the
+ * first direct-sum system joins, or the members' trees come to need, or no
+ * longer need, more than 4 GiB of node records.  A system's results are bit-identical
  * to stepping it alone with gsim_step (the same group width, 32 or 64, and
  * the default launch shape).
  * Direct-sum systems of 16,384 or more padded particles are refused: they

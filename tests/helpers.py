@@ -278,3 +278,12 @@ def put_sort_stall(handle, count: int) -> None:
     f = (handle_access().access_batch_sort_stall if isinstance(handle, gsim.Batch)
          else handle_access().access_sort_stall)
     assert f(handle._h, C.c_uint32(count)) == 0
+
+
+def put_narrow_nodes(handle, nodes: int) -> None:
+    """Node slots from which on the handle's walk takes the wide form."""
+    import gsim
+    f = (handle_access().access_batch_narrow_nodes if isinstance(handle, gsim.Batch)
+         else handle_access().access_narrow_nodes)
+    f.argtypes, f.restype = [C.c_void_p, C.c_size_t], None
+    f(handle._h, nodes)

@@ -175,6 +175,21 @@ def query_beside_a_capture():
             assert srv.wait(r, 1.0)
 
 
+def walk_form_by_the_members():
+    """The batch's walk takes the wide form by what its members can use, not by
+    the size of the arena."""
+    narrow, wide = "bb_force_kernelILb0E", "bb_force_kernelILb1E"
+    with gsim.Batch(100_000_000, 8) as b:  # 300,000,064 node slots
+        b.add(gsim.generate("galaxy", 9_000, 100.0, 1.0, 10.0), "barnes-hut")
+        names = _launched(lambda: b.step(2))
+        assert narrow in names and wide not in names, names
+        helpers.put_narrow_nodes(b, b.info()["nodes_reserved"])
+        names = _launched(lambda: b.step(2))
+        assert wide in names and narrow not in names, names
+        helpers.put_narrow_nodes(b, b.info()["nodes_reserved"] + 1)
+        assert narrow in _launched(lambda: b.step(1))
+
+
 if __name__ == "__main__":
     _load(sys.argv[1])
     globals()[sys.argv[2]]()

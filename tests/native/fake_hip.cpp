@@ -4,6 +4,7 @@
 // libgsim.so, it answers that library's HIP calls.  Failures are asked for by
 // the fake_* functions.
 #include <hip/hip_runtime_api.h>
+#include <sys/mman.h>
 
 #include <chrono>
 #include <cstdlib>
@@ -176,7 +177,14 @@ hipError_t hipMemsetAsync(void *d, int v, size_t n, hipStream_t st) {
     if (n && !d) return hipErrorInvalidValue;
     starts_on(st);
     if (!st) null_busy = true;
-    if (n) std::memset(d, v, n);
+    if (!v && n > ((size_t)64 << 20)) {  // give the pages back instead of touching them
+        const uintptr_t p = (uintptr_t)d, a = (p + 4095) / 4096 * 4096, b = (p + n) / 4096 * 4096;
+        std::memset(d, 0, a - p);
+        madvise((void *)a, b - a, MADV_DONTNEED);
+        std::memset((void *)b, 0, p + n - b);
+    } else if (n) {
+        std::memset(d, v, n);
+    }
     return hipSuccess;
 }
 hipError_t hipMemset(void *d, int v, size_t n) { return hipMemsetAsync(d, v, n, nullptr); }

@@ -19,4 +19,11 @@ int access_batch_sort_stall(gsim_batch *b, uint32_t v) {
     return put(&b->d.counts->sort_stall, &v, 4);
 }
 
+// Walks address nodes by slot from this many on.
+void access_narrow_nodes(gsim_sim *s, size_t n) { s->narrow_nodes = n; }
+void access_batch_narrow_nodes(gsim_batch *b, size_t n) {
+    b->narrow_nodes = n;
+    b->dirty = true;
+}
+
 }  // extern "C"
