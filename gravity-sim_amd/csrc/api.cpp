@@ -114,11 +114,23 @@ gsim_status drain_timing(gsim_sim *s) {
     return GSIM_OK;
 }
 
-// Grows the partial-sum buffer to hold `entries` float2 (the caller has
-// synchronised the stream).  On failure the handle keeps a buffer of the size
-// it had, unless not even that can be had again once it was given up.
+// Gives the partial-sum buffer room for `entries` float2, and memory back where
+// it has more than twice that (the caller has synchronised the stream).  On
+// failure the handle keeps a buffer of the size it had, unless not even that
+// can be had again once it was given up.
 gsim_status ds_reserve_partial(gsim_sim *s, size_t entries) {
-    if (entries <= s->partial_cap) return GSIM_OK;
+    if (entries <= s->partial_cap) {
+        if (2 * entries >= s->partial_cap) return GSIM_OK;
+        float2 *less = nullptr;
+        if (entries && hipMalloc((void **)&less, sizeof(float2) * entries) != hipSuccess) {
+            (void)hipGetLastError();
+            return GSIM_OK;  // what is there is enough
+        }
+        (void)hipFree(s->partial);
+        s->partial = less;
+        s->partial_cap = entries;
+        return GSIM_OK;
+    }
     float2 *fresh = nullptr;
     hipError_t e = hipMalloc((void **)&fresh, sizeof(float2) * entries);
     if (e != hipSuccess && s->partial) {  // both at once may be too much

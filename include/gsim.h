@@ -172,8 +172,12 @@ typedef enum gsim_tuning {
     GSIM_TUNE_BH_WAVES_PER_SIMD = 2,  /* 1..8; no effect                               */
     GSIM_TUNE_BH_TRAVERSAL = 3,       /* 0..3 or 6; no effect                          */
     GSIM_TUNE_DS_SYMMETRIC = 4,       /* 0/1: each pair once (Newton's third law); the
-                                         default for 16,384 <= Na <= 524,288 (where its
-                                         partial sums fit in memory)                   */
+                                         default for 16,384 <= Na <= 524,288.  Its
+                                         partial sums take 9 MB at 16,384 particles,
+                                         60 MB at 50,000, 0.20 GB at 100,000, 0.54 at
+                                         262,144, 0.71 at 300,000 and 2.2 at 524,288;
+                                         where gsim_create cannot have them the handle
+                                         is one-sided, and 0 gives them back           */
     GSIM_TUNE_DS_SYM_COLS = 5,        /* symmetric kernel: 1 or 2 column blocks per
                                          wave (at most 1 below 28,672), 0 = by size     */
     GSIM_TUNE_BH_SEGMENTS = 6,        /* 1..65536; no effect                           */

@@ -190,6 +190,27 @@ def walk_form_by_the_members():
         assert narrow in _launched(lambda: b.step(1))
 
 
+def partial_sums_without_room_and_given_back():
+    """A large direct sum is one-sided where the symmetric form's partial sums
+    do not fit, and gives them back when it is made one-sided."""
+    p = gsim.generate("random", 400_000, 100.0, 1.0, 10.0)
+    at = fake.fake_live()
+    with gsim.Simulation(p, "direct-sum") as s:
+        assert "ds_sym_kernel" in _launched(lambda: s.step(1))
+        with_sums = fake.fake_live() - at
+        s.set_tuning(gsim.TUNE_DS_SYMMETRIC, 0)
+        without = fake.fake_live() - at
+        assert without < with_sums / 10, (with_sums, without)
+        s.step(1)
+    assert fake.fake_live() == at
+    fake.fake_limit(at + with_sums // 2)
+    with gsim.Simulation(p, "direct-sum") as s:
+        names = _launched(lambda: s.step(1))
+        assert "ds_partial_kernel" in names and "ds_sym_kernel" not in names
+        _refused(OUT_OF_MEMORY, lambda: s.set_tuning(gsim.TUNE_DS_SYMMETRIC, 1))
+        assert _launched(lambda: s.step(1)) == names
+
+
 if __name__ == "__main__":
     _load(sys.argv[1])
     globals()[sys.argv[2]]()
