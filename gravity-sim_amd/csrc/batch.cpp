@@ -573,7 +573,10 @@ gsim_status gsim_batch_set_tuning(gsim_batch *b, const gsim_batch_tuning *t) {
     n.run_queue = t->run_queue;
     n.prio_step = t->prio_step;
     n.prio_carry = t->prio_carry;
+    const uint32_t last_queue = b->tune.run_queue;
+    b->tune.run_queue = n.run_queue;  // shapes no launch
     if (std::memcmp(&n, &b->tune, sizeof(n)) != 0) {
+        b->tune.run_queue = last_queue;
         GSIM_HIP(hipSetDevice(b->device));
         GSIM_HIP(hipStreamSynchronize(b->stream));
         destroy_graphs(b);  // the launch parameters are baked into the graphs

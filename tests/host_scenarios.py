@@ -211,6 +211,20 @@ def partial_sums_without_room_and_given_back():
         assert _launched(lambda: s.step(1)) == names
 
 
+def knob_without_effect_keeps_the_graphs():
+    """run_queue shapes no launch any more: setting it captures nothing again."""
+    with gsim.Batch(20_000, 8) as b:
+        b.add(gsim.generate("galaxy", 9_000, 100.0, 1.0, 10.0), "barnes-hut")
+        b.step(2)
+        graphs = fake.fake_instantiated()
+        b.set_tuning(run_queue=16)
+        b.step(2)
+        assert b.tuning()["run_queue"] == 16 and fake.fake_instantiated() == graphs
+        b.set_tuning(run_queue=32, waves_per_simd=4)
+        b.step(2)
+        assert b.tuning()["run_queue"] == 32 and fake.fake_instantiated() == graphs + 2
+
+
 if __name__ == "__main__":
     _load(sys.argv[1])
     globals()[sys.argv[2]]()
