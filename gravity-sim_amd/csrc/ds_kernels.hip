@@ -338,8 +338,9 @@ DsSymPlan ds_sym_plan(size_t na, uint32_t cols) {
     //   200,000  6370    5953    5817    5739    5749
     //   300,001                 13000   12800   12751
     p.rows = na < 28672 ? 4 : na < 65536 ? 8 : 16;
-    if (cols == 0) cols = na < 131072 ? 1 : na < 262144 ? 2 : 4;
-    cols = std::min(cols, p.rows / 4);  // the width divides the rows
+    // the width divides the rows: columns asked for have rows enough
+    if (cols == 0) cols = std::min(p.rows / 4, na < 131072 ? 1u : na < 262144 ? 2u : 4u);
+    else p.rows = std::max(p.rows, 4 * cols);
     p.G = (p.B + p.rows - 1) / p.rows;
     p.cols = cols;
     p.width = 4 * cols;

@@ -179,7 +179,7 @@ typedef enum gsim_tuning {
                                          where gsim_create cannot have them the handle
                                          is one-sided, and 0 gives them back           */
     GSIM_TUNE_DS_SYM_COLS = 5,        /* symmetric kernel: 1 or 2 column blocks per
-                                         wave (at most 1 below 28,672), 0 = by size     */
+                                         wave, 0 = by size                              */
     GSIM_TUNE_BH_SEGMENTS = 6,        /* 1..65536; no effect                           */
     GSIM_TUNE_BH_SPLIT = 7,           /* 0..1000; no effect                            */
     GSIM_TUNE_BH_ADAPTIVE_BOX = 8,    /* 0/1, beyond the reference and off by default:

@@ -225,6 +225,16 @@ def knob_without_effect_keeps_the_graphs():
         assert b.tuning()["run_queue"] == 32 and fake.fake_instantiated() == graphs + 2
 
 
+def columns_asked_for_are_taken():
+    """Two column blocks a wave need eight row blocks, also where the size alone
+    would take four."""
+    for n, rows in ((20_000, (4, 4, 8)), (40_000, (8, 8, 8)), (70_000, (16, 16, 16))):
+        with gsim.Simulation(gsim.generate("random", n, 100.0, 1.0, 10.0), "direct-sum") as s:
+            for cols, r in zip((0, 1, 2), rows):
+                s.set_tuning(gsim.TUNE_DS_SYM_COLS, cols)
+                assert f"ds_sym_kernelILi{r}E" in _launched(lambda: s.step(1)), (n, cols)
+
+
 if __name__ == "__main__":
     _load(sys.argv[1])
     globals()[sys.argv[2]]()

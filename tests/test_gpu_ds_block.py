@@ -69,3 +69,19 @@ def test_symmetric_forces_at_every_tile_shape(n):
     # momentum: every pair gave equal and opposite pulls
     f = (a.astype(np.float64) * p.mass[:, None])
     assert np.linalg.norm(f.sum(0)) <= 1e-5 * np.linalg.norm(f, axis=1).sum()
+
+
+@pytest.mark.parametrize("cols", [1, 2])
+@pytest.mark.parametrize("n", [16384, 20000, 28607, 40000])
+def test_symmetric_forces_with_the_columns_asked_for(n, cols):
+    """As by size, with each number of column blocks a wave."""
+    print(f"ds symmetric n={n} cols={cols}", flush=True)
+    p = gsim.generate("exponential-disk", n, 100.0, 1.0, 10.0, seed=n)
+    with gsim.Simulation(p, "direct-sum") as s:
+        s.set_debug(gsim.DEBUG_ACCEL)
+        s.set_tuning(gsim.TUNE_DS_SYM_COLS, cols)
+        s.step(1)
+        a = s.dump(gsim.DUMP_ACCEL)[: p.n]
+    pp = p.padded()
+    t = np.linspace(0, n - 1, 512).astype(np.uint32)
+    assert H.system_rel_err(a[t], O.ds_accel_f64_at(pp.pos, pp.mass, EPS2, t)) <= 1e-5
