@@ -287,3 +287,19 @@ def put_narrow_nodes(handle, nodes: int) -> None:
          else handle_access().access_narrow_nodes)
     f.argtypes, f.restype = [C.c_void_p, C.c_size_t], None
     f(handle._h, nodes)
+
+
+def launch_order(sim, units: int):
+    """The workgroup order the walk was last launched in, or None without a plan."""
+    sim.synchronize()
+    out = np.empty(units, np.uint32)
+    r = handle_access().access_order(sim._h, out.ctypes.data_as(C.c_void_p), C.c_size_t(units))
+    assert r in (0, 1)
+    return out if r == 0 else None
+
+
+def direct_sum_launch(batch):
+    """(workgroups that take direct-sum blocks, the blocks) of the last membership."""
+    g, n = C.c_uint32(), C.c_uint32()
+    handle_access().access_batch_direct_sums(batch._h, C.byref(g), C.byref(n))
+    return g.value, n.value

@@ -26,4 +26,18 @@ void access_batch_narrow_nodes(gsim_batch *b, size_t n) {
     b->dirty = true;
 }
 
+// The walk's launch order (`units` workgroups); 0 if there is a plan.
+int access_order(gsim_sim *s, uint32_t *out, size_t units) {
+    if (!s->bh.order_valid) return 1;
+    return hipMemcpy(out, s->bh.order, sizeof(uint32_t) * units, hipMemcpyDeviceToHost) == hipSuccess
+               ? 0
+               : 2;
+}
+
+// Workgroups that take direct-sum blocks, and the blocks.
+void access_batch_direct_sums(const gsim_batch *b, uint32_t *groups, uint32_t *blocks) {
+    *groups = b->h_counts.ds_groups;
+    *blocks = b->h_counts.n_ds;
+}
+
 }  // extern "C"
