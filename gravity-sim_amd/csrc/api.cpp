@@ -678,6 +678,12 @@ gsim_status gsim_debug_dump(gsim_sim *s, int32_t what, void *buf, size_t bytes, 
     GSIM_HIP(hipSetDevice(s->device));
     GSIM_HIP(hipStreamSynchronize(s->stream));
     const size_t na = s->na;
+    gsim::BhCounters ctr{};
+    if (s->bh.ctr) {
+        GSIM_HIP(hipMemcpy(&ctr, s->bh.ctr, sizeof(ctr), hipMemcpyDeviceToHost));
+        const gsim_status sorted = check_sort(s, ctr.sort_stall);
+        if (sorted != GSIM_OK) return sorted;
+    }
     if (what == GSIM_DUMP_ACCEL) {
         *written = sizeof(float2) * na;
         if (!buf || bytes < *written) return fail(GSIM_ERROR_CAPACITY, "buffer too small");
@@ -695,10 +701,6 @@ gsim_status gsim_debug_dump(gsim_sim *s, int32_t what, void *buf, size_t bytes, 
         return fail(GSIM_ERROR_INVALID_ARGUMENT, "dump %d needs a Barnes-Hut handle", what);
     if (!s->bh.ctr)
         return fail(GSIM_ERROR_OUT_OF_MEMORY, "the handle has no Barnes-Hut buffers");
-    gsim::BhCounters ctr{};
-    GSIM_HIP(hipMemcpy(&ctr, s->bh.ctr, sizeof(ctr), hipMemcpyDeviceToHost));
-    const gsim_status sorted = check_sort(s, ctr.sort_stall);
-    if (sorted != GSIM_OK) return sorted;
     const size_t nodes = s->has_tree ? ctr.n_nodes : 0;
     switch (what) {
         case GSIM_DUMP_CELLS: {

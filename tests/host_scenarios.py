@@ -118,6 +118,7 @@ def given_up_sort_is_never_read():
             for _ in range(3):
                 _refused(DEVICE, s.read)
             _refused(DEVICE, lambda: s.dump(gsim.DUMP_CELLS))
+            _refused(DEVICE, lambda: s.dump(gsim.DUMP_ACCEL))
             s.set_tuning(gsim.TUNE_BH_LEAF_BITS, 15)
             _refused(DEVICE, s.read)
     with gsim.Batch(100_000, 8) as b:
