@@ -38,7 +38,9 @@ constexpr uint32_t kLiveLists = 64;
 // Workgroups of the direct-sum launch, and how many of them take blocks: one to
 // a CU, so that the build beside it finds room, where the direct sums are a
 // small part of the step; all, several to a CU, where they outlast the build.
-// Us a step beside / all, by direct-sum pairs per Barnes-Hut particle: 417 392 /
+// The line lies between seven mixes whose builds and walks differ in more than
+// this ratio, so it is a fit, no model of which side takes longer: a mix near it
+// may be on the slower side by some per cent.  Us a step beside / all, by direct-sum pairs per Barnes-Hut particle: 417 392 /
 // 427, 450 236 / 255, 1,875 168 / 182, 2,000 447 / 439, 5,400 492 / 434, 27,000
 // 472 / 406, no Barnes-Hut system 832 / 697.  256 beside: 128 +5%, 192 +1%, 512
 // +6% at the mix above bb_ds_kernel.

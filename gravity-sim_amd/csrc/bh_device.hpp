@@ -191,6 +191,14 @@ __device__ __forceinline__ int tile_level_offset(int d) {
 // word is stored at the scope of the device and has arrived before the call
 // returns, and is loaded at that scope, past the XCD's own L2.  A fence would
 // write that whole L2 back, once a tile.
+// The order comes from the machine, not from the language, whose relaxed
+// accesses promise it for one word only.  It rests on the memory model of
+// gfx940 to gfx950 (LLVM's AMDGPU guide): a store with sc1, which a store at
+// device scope is, writes through the L2, and vmcnt counts it off once it is
+// visible to the device, so s_waitcnt vmcnt(0) before the counter's atomic
+// orders the two, as a release at that scope does for its own write-back; the
+// reader's loads with sc1 are issued after the counter's value has returned
+// (it decides the branch that leads to them) and take no line of their L2.
 __device__ __forceinline__ void publish_top(TileCell *to, const TileCell &c) {
     uint32_t *w = reinterpret_cast<uint32_t *>(to);
     status_store(w + 0, c.n);
@@ -335,7 +343,7 @@ __device__ __forceinline__ void reduce_tile(
                    : 0u;
     lds_barrier();
     if (!sh.last) return;
-    asm volatile("" ::: "memory");  // no record is read before the counts
+    asm volatile("" ::: "memory");  // holds the compiler to it: counts, then records
     // depths 4..0 in `up` at the offsets of depths 9..5
     const TileCell empty{0u, 0u, 0xffffffffu, 0u, 0.0f, 0.0f, 0.0f, 0.0f};
     const TileCell t0 = in0 ? published_top(top + 4 * t) : empty;

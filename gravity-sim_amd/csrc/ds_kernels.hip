@@ -74,8 +74,8 @@ __global__ __launch_bounds__(kDsThreads) void ds_partial_kernel(
 // Blocks: one workgroup per 16 targets, its 16 waves the roles of ds_device.hpp,
 // so a step is one launch with no partial sums in memory.  What bounds it: the
 // launch and two dependent round trips below ~2,000 particles, the VALU above
-// (4,096 particles: 2.07e12 pairs a second of the 4.6e12 its issue rate allows;
-// 12,288: 3.6e12).
+// (4,096 particles: 2.07e12 pairs a second of the 4.6e12 that 34 clocks a pair
+// allow at 2.4 GHz; 12,288: 3.6e12).
 // Against slices of at least 512 sources (1 to 31 slices) and a combine
 // launch, us a step: 64 particles 7.8 -> 2.8, 1,024 41 -> 4.1, 4,096 51 -> 8.1,
 // 12,288 71 -> 42, 15,040 90 -> 65.
@@ -136,7 +136,7 @@ __global__ __launch_bounds__(256) void ds_combine_kernel(
 // its owner's lane.  Per pair: 12 VALU + 1 v_rsq_f32 for two interactions,
 // against 9 + 1 for one in the one-sided kernel; the 5 rotates per step are
 // shared by the group's rows.  The pairs are kept in the order written: 200,000
-// particles 5,939 -> 5,757 us a step, 45 clocks a pair.
+// particles 5,939 -> 5,757 us a step, 45 clocks of 2.4 GHz a pair.
 //
 // Partial sums, both in fixed order: per tile, each row particle's sum over
 // the tile's columns (ipart; the four waves' sums added in wave order through

@@ -104,9 +104,12 @@ typedef enum gsim_dump {
 
 /* Timing phases returned by gsim_get_timing (milliseconds, summed). */
 typedef struct gsim_timing {
-    double force_ms;      /* direct-sum force kernel / Barnes-Hut traversal   */
+    double force_ms;      /* direct-sum force kernel / Barnes-Hut traversal, which
+                           * integrates too, as does the direct sum in its block
+                           * form (below 16,384 padded particles)              */
     double build_ms;      /* Barnes-Hut: keys, sort and tree build            */
-    double integrate_ms;  /* direct-sum partial-sum combine and integrate     */
+    double integrate_ms;  /* direct-sum partial-sum combine and integrate; about
+                           * 0 in the block form                               */
     double step_ms;       /* whole steps                                       */
     uint64_t steps;       /* steps covered                                     */
     uint64_t force_launches;
@@ -220,9 +223,9 @@ gsim_status gsim_set_tuning(gsim_sim *sim, int32_t knob, uint32_t value);
 /* ---- allocation-free direct-sum step ---------------------------------------
  * No counterpart in the reference.  For callers that cannot allocate device
  * memory (code under HIP stream capture, serving loops that forbid hipMalloc):
- * one direct-sum step, the one-sided kernels of gsim_step with the slice count
- * gsim_set_ds_shape(sim, 2, 0) picks (capped so slices x n fits the scratch),
- * on caller-owned DEVICE arrays of n particles (n a nonzero multiple of 64;
+ * one direct-sum step in the form that gsim_set_ds_shape(sim, 2, 0) picks:
+ * blocks below 16,384 particles, else slices (capped so slices x n fits the
+ * scratch), on caller-owned DEVICE arrays of n particles (n a nonzero multiple of 64;
  * pad with {0,0,0,0,0} particles as gsim_create does).  Inputs are read and
  * the outputs written on `stream` (a hipStream_t; NULL = the null stream) of
  * params->device, asynchronously; outputs must not alias inputs.  G,
@@ -232,8 +235,9 @@ gsim_status gsim_set_tuning(gsim_sim *sim, int32_t knob, uint32_t value);
  * GSIM_NOALLOC_SCRATCH_BYTES that each GPU the call runs on holds until the
  * process ends, so n is at most GSIM_NOALLOC_SCRATCH_BYTES / 8 (4,194,304);
  * larger n returns GSIM_ERROR_CAPACITY.  The call allocates nothing.  Every
- * call on one GPU shares that GPU's array: calls that overlap on one GPU (two
- * streams, two threads) race and must be serialised by the caller. */
+ * call of 16,384 particles or more on one GPU shares that GPU's array: such
+ * calls that overlap on one GPU (two streams, two threads) race and must be
+ * serialised by the caller. */
 #define GSIM_NOALLOC_SCRATCH_BYTES (32u << 20)
 gsim_status gsim_ds_step_noalloc(const gsim_params *params, const float *pos_xy,
                                  const float *vel_xy, const float *mass,
