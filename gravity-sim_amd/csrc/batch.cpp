@@ -217,10 +217,13 @@ gsim_status launch_steps(gsim_batch *b, uint32_t count) {
                 if (g) (void)hipGraphDestroy(g);
                 return hip_fail(e, "batched step launch");
             }
-            GSIM_HIP(e2);
+            if (e2 != hipSuccess) return hip_fail(e2, "hipStreamEndCapture");
             e = hipGraphInstantiate(&b->graph[in], g, nullptr, nullptr, 0);
             (void)hipGraphDestroy(g);
-            GSIM_HIP(e);
+            if (e != hipSuccess) {
+                b->graph[in] = nullptr;
+                return hip_fail(e, "hipGraphInstantiate");
+            }
         }
         GSIM_HIP(hipGraphLaunch(b->graph[in], b->stream));
         b->cur ^= 1;

@@ -163,8 +163,10 @@ void worker_loop(gsim_server *s) {
         }
         if (st != GSIM_OK) {
             for (auto &kv : s->running) {
-                kv.second->state = 3;
-                kv.second->done = Clock::now();
+                Request *r = kv.second;
+                (void)gsim_batch_remove(s->arenas[r->arena], r->batch_id);  // its space
+                r->state = 3;
+                r->done = Clock::now();
                 ++s->failed;
             }
             s->running.clear();
@@ -186,6 +188,8 @@ void worker_loop(gsim_server *s) {
             gsim_batch *b = s->arenas[r->arena];
             const gsim_status rs = gsim_batch_read(b, r->batch_id, r->pos.data(), r->vel.data(),
                                                    r->mass.data());
+            if (rs != GSIM_OK)
+                std::snprintf(s->worker_error, sizeof(s->worker_error), "%s", gsim_last_error());
             gsim_batch_remove(b, r->batch_id);
             s->running.erase((uint64_t)r->arena << 32 | r->batch_id);
             s->active_particles -= padded(r->n);

@@ -236,6 +236,25 @@ def columns_asked_for_are_taken():
                 assert f"ds_sym_kernelILi{r}E" in _launched(lambda: s.step(1)), (n, cols)
 
 
+def failed_requests_leave_their_space():
+    """Requests that fail with a step, or with the read of their result, say why
+    and make room for the next ones."""
+    p = gsim.generate("galaxy", 15_000, 100.0, 1.0, 10.0)
+    with gsim.Server(20_000 * gsim.Batch.bytes_per_particle(), max_systems=4) as srv:
+        fake.fake_refuse_graphs(1)
+        for _ in range(2):
+            rid = srv.submit(p, 3, "barnes-hut")
+            try:
+                assert srv.wait(rid, 20.0)
+                state = "done"
+            except gsim.GsimError as e:
+                assert "hipGraphInstantiate" in str(e), e
+                state = "failed"
+        assert state == "done"
+        stats = srv.stats()
+        assert (stats["completed"], stats["failed"]) == (1, 1), stats
+
+
 if __name__ == "__main__":
     _load(sys.argv[1])
     globals()[sys.argv[2]]()

@@ -23,7 +23,7 @@ std::map<void *, size_t> blocks;              // live device allocations
 size_t live = 0, limit = ~(size_t)0;
 std::string launches, faults;
 std::set<void *> capturing, spoiled;  // streams in capture; captures made invalid
-unsigned capture_delay_us = 0, instantiated = 0;
+unsigned capture_delay_us = 0, instantiated = 0, refused_graphs = 0;
 // Memsets and copies on the device return before they are done; the library's
 // streams do not wait for the null stream.
 bool null_busy = false;
@@ -104,6 +104,7 @@ static void starts_on(hipStream_t st) {
 void fake_limit(size_t bytes) { limit = bytes; }  // of device memory held at once
 size_t fake_live() { return live; }
 void fake_capture_delay(unsigned us) { capture_delay_us = us; }  // a launch under capture
+void fake_refuse_graphs(unsigned n) { refused_graphs = n; }  // the next n instantiations
 void fake_forget() { launches.clear(); }
 const char *fake_launches() { return launches.c_str(); }  // names, a line each
 const char *fake_faults() { return faults.c_str(); }
@@ -242,6 +243,10 @@ hipError_t hipStreamEndCapture(hipStream_t s, hipGraph_t *g) {
 }
 hipError_t hipGraphInstantiate(hipGraphExec_t *e, hipGraph_t, hipGraphNode_t *, char *, size_t) {
     std::lock_guard<std::recursive_mutex> lk(mu);
+    if (refused_graphs) {
+        --refused_graphs;
+        return hipErrorUnknown;
+    }
     ++instantiated;
     *e = (hipGraphExec_t)fresh();
     return hipSuccess;

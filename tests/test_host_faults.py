@@ -15,7 +15,8 @@ SCENARIOS = ["failed_form_keeps_the_last", "lost_tree_buffers",
              "given_up_sort_is_never_read", "new_buffers_are_cleared_before_use",
              "query_beside_a_capture", "walk_form_by_the_members",
              "partial_sums_without_room_and_given_back",
-             "knob_without_effect_keeps_the_graphs", "columns_asked_for_are_taken"]
+             "knob_without_effect_keeps_the_graphs", "columns_asked_for_are_taken",
+             "failed_requests_leave_their_space"]
 
 
 @pytest.fixture(scope="module")
